@@ -22,11 +22,11 @@ struct KernelSpec {
 // Entries with requires_def come before the plain entry of the same name.
 static const KernelSpec kKernelTable[] = {
     // ---- ops (Q2_AQ / Q2_SC / Q2_AB: the two-pass mode's residual offsets, the reference's -D names; 0 = one pass)
-    {"ops", "quant_rows", nullptr, "piiiipppi", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
+    {"ops", "quant_rows", nullptr, "piiiipppii", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
     {"ops", "rmsnorm_quant", nullptr, "pipiiifppppii", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
     {"ops", "swiglu_quant", nullptr, "piiipppiii", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
-    {"ops", "rmsnorm_quant_r16", nullptr, "pipiiifppppii", {nullptr}, {{nullptr, 0, false}}, 256},
-    {"ops", "swiglu_quant_r16", nullptr, "piiipppiii", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"ops", "swiglu_quant_tile", nullptr, "piiipppiiii", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
+    {"ops", "rmsnorm_quant_wave", nullptr, "pipiiifppppii", {nullptr}, {{nullptr, 0, false}}, 256},
     {"ops", "add_norm_quant", nullptr, "pppiffpiipppii", {nullptr}, {{"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"Q2_AB", 0, false}, {nullptr, 0, false}}, 256},
     {"ops", "act_usum", nullptr, "ppip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"ops", "q4k_wscales", nullptr, "pziip", {nullptr}, {{nullptr, 0, false}}, 256},

@@ -12,56 +12,43 @@
 // layouts q2_aq bytes / q2_sc floats / q2_ab shorts further on in the three buffers, for a second matmul pass that
 // accumulates into the first one's output.
 //
-// Mapping: a work-group of 256 threads takes one superblock (256 values) of 64 token rows.  Thread t holds 16
+// Mapping: a work-group of 256 threads takes one superblock (256 values) of 16 or 64 token rows.  Thread t holds 16
 // consecutive values of one row (16 threads = one row's superblock, read as one contiguous KiB); the two threads of a
 // 32-block exchange their maxima with one cross-lane move.  Scales and sums go through LDS so that they leave as
-// runs of 64 consecutive tokens (the token-minor layout the matmuls read).
+// runs of 16 or 64 consecutive tokens (the token-minor layout the matmuls read).
 #include "quant.h"
 
-// Shared tail of the row kernels: stores one tile's scales and sums token-minor.
+// Shared tail of the tile kernels: stores one tile's scales and sums token-minor (rows: 16 or 64).
 struct QuantTile {
   float asc[8][64];
   short sum[16][64];
 };
 
-__device__ inline void store_tile_scales(const QuantTile& lds, int s, int m0, int M, int act32, float* asc,
+__device__ inline void store_tile_scales(const QuantTile& lds, int s, int m0, int rows, int M, int act32, float* asc,
                                          short* absum) {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, lr = rows == 64 ? 6 : 4, r = t & (rows - 1);
+  if (m0 + r >= M) return;
   if (act32) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = t + 256 * i, b = idx >> 6, r = idx & 63;
-      if (m0 + r < M) asc[((size_t)s * 8 + b) * M + m0 + r] = lds.asc[b][r];
-    }
-  } else if (t < 64) {
-    if (m0 + t < M) asc[(size_t)s * M + m0 + t] = lds.asc[0][t];
+    for (int b = t >> lr; b < 8; b += 256 >> lr) asc[((size_t)s * 8 + b) * M + m0 + r] = lds.asc[b][r];
+  } else if (t < rows) {
+    asc[(size_t)s * M + m0 + r] = lds.asc[0][r];
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = t + 256 * i, h = idx >> 6, r = idx & 63;
-    if (m0 + r < M) absum[((size_t)s * 16 + h) * M + m0 + r] = lds.sum[h][r];
-  }
+  for (int h = t >> lr; h < 16; h += 256 >> lr) absum[((size_t)s * 16 + h) * M + m0 + r] = lds.sum[h][r];
 }
 
-// quant_rows: x [T][ldx] f32 -> aq / asc / absum for M rows (rows >= T zero).  grid (K/256, ceil(M/64)), local 256.
-extern "C" __global__ __launch_bounds__(256) void quant_rows(const float* __restrict__ x, int ldx, int K, int M, int T,
-                                                             signed char* __restrict__ aq, float* __restrict__ asc,
-                                                             short* __restrict__ absum, int act32, int q2_aq, int q2_sc,
-                                                             int q2_ab) {
+// One tile: superblock s of rows m0 .. m0 + rows - 1; load(v, m) gives a thread's 16 values of row m < T.
+template <typename Load>
+__device__ inline void quant_tile(Load load, int s, int m0, int rows, int K, int M, int T, signed char* __restrict__ aq,
+                                  float* __restrict__ asc, short* __restrict__ absum, int act32, int q2_aq, int q2_sc,
+                                  int q2_ab) {
   __shared__ QuantTile lds, lds2;
-  const int s = blockIdx.x, m0 = blockIdx.y * 64;
   const int lane16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
 #pragma unroll 1
-  for (int p = 0; p < 4; ++p) {
-    const int r = p * 16 + rg, m = m0 + r;
+  for (int p = 0; p < rows; p += 16) {
+    const int r = p + rg, m = m0 + r;
     float v[16];
     if (m < T) {
-      const float4* src = (const float4*)(x + (size_t)m * ldx + s * 256 + 16 * lane16);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 f = src[i];
-        v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
-      }
+      load(v, m);
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i) v[i] = 0.0f;
@@ -91,8 +78,26 @@ extern "C" __global__ __launch_bounds__(256) void quant_rows(const float* __rest
     }
   }
   __syncthreads();
-  store_tile_scales(lds, s, m0, M, act32, asc, absum);
-  if (q2_aq) store_tile_scales(lds2, s, m0, M, act32, asc + q2_sc, absum + q2_ab);
+  store_tile_scales(lds, s, m0, rows, M, act32, asc, absum);
+  if (q2_aq) store_tile_scales(lds2, s, m0, rows, M, act32, asc + q2_sc, absum + q2_ab);
+}
+
+// quant_rows: x [T][ldx] f32 -> aq / asc / absum for M rows (rows >= T zero).  grid (K/256, ceil(M / rows)), local 256;
+// rows, 16 or 64, is the launcher's choice.
+extern "C" __global__ __launch_bounds__(256) void quant_rows(const float* __restrict__ x, int ldx, int K, int M, int T,
+                                                             signed char* __restrict__ aq, float* __restrict__ asc,
+                                                             short* __restrict__ absum, int act32, int rows, int q2_aq,
+                                                             int q2_sc, int q2_ab) {
+  const int s = blockIdx.x;
+  auto load = [&](float (&v)[16], int m) {
+    const float4* src = (const float4*)(x + (size_t)m * ldx + s * 256 + 16 * (threadIdx.x & 15));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 f = src[i];
+      v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+    }
+  };
+  quant_tile(load, s, blockIdx.y * rows, rows, K, M, T, aq, asc, absum, act32, q2_aq, q2_sc, q2_ab);
 }
 
 // ---- the two fused producers.  A work-group of 256 threads per row (or several along x, each taking a share of the
@@ -459,164 +464,127 @@ extern "C" __global__ __launch_bounds__(256) void q4k_wscales_int(const uint8_t*
   }
 }
 
-// ---- the fused producers over chunks of many rows: a work-group takes 16 consecutive rows one after the other and
-// keeps their scales and sums in LDS, [block][16 rows], so that the token-minor arrays are written in pieces of 16
-// rows (64 and 32 bytes) instead of one element per block and row from a work-group per row, whose 480 scattered
-// stores a row were most of that form's memory transactions.  One-pass engines, M a multiple of 16, rows of up to
-// R16_KMAX (R16_KMAX_NORM) values.
-#define R16_KMAX 20480      // swiglu_quant_r16 (80 KiB of LDS: two work-groups a compute unit)
-#define R16_KMAX_NORM 16384 // rmsnorm_quant_r16 (64 KiB, and the row sum's four floats)
-template <int KMAX> struct R16Stage {
-  float sc[KMAX / 32 * 16];
-  short sum[KMAX / 16 * 16];
-};
-// a thread's 16 values of superblock s of row r of the 16: quantized, the int8 values stored, scale and sum staged
-template <int KMAX>
-__device__ inline void r16_quant(R16Stage<KMAX>& st, const float* v, int s, int lane16, int r, int m, int K, int act32,
-                                 signed char* __restrict__ aq) {
-  const float amax = block_amax(v, act32);
-  uint4 pk;
-  int sum;
-  quant16(v, amax, pk, sum, nullptr);
-  *(uint4*)(aq + (size_t)m * K + s * 256 + 16 * lane16) = pk;
-  st.sum[(s * 16 + lane16) * 16 + r] = (short)sum;
-  if (act32) {
-    if ((lane16 & 1) == 0) st.sc[(s * 8 + (lane16 >> 1)) * 16 + r] = amax / 127.0f;
-  } else if (lane16 == 0) {
-    st.sc[s * 16 + r] = amax / 127.0f;
-  }
-}
-// the staged scales and sums of rows m0 .. m0 + 15 out to asc [blocks][M] and absum [K / 16][M]
-template <int KMAX>
-__device__ inline void r16_flush(const R16Stage<KMAX>& st, int m0, int M, int K, int act32, float* __restrict__ asc,
-                                 short* __restrict__ absum) {
-  __syncthreads();
-  const int nb = act32 ? K >> 5 : K >> 8;
-  for (int i = threadIdx.x; i < nb * 16; i += 256) asc[(size_t)(i >> 4) * M + m0 + (i & 15)] = st.sc[i];
-  for (int i = threadIdx.x; i < (K >> 4) * 8; i += 256)
-    *(uint32_t*)(absum + (size_t)(i >> 3) * M + m0 + 2 * (i & 7)) = *(const uint32_t*)(st.sum + (i >> 3) * 16 + 2 * (i & 7));
-}
-
-// rmsnorm_quant over 16 rows a work-group: grid (256, M / 16).  A row stays in registers between its sum of squares
-// and its quantization, and the next row's loads are in flight meanwhile.
-extern "C" __global__ __launch_bounds__(256, 2) void rmsnorm_quant_r16(const float* __restrict__ x, int row_off,
-                                                                       const float* __restrict__ w, int K, int M,
-                                                                       int M_valid, float eps, signed char* __restrict__ aq,
-                                                                       float* __restrict__ asc, short* __restrict__ absum,
-                                                                       float* __restrict__ hout, int write_h, int act32) {
-  __shared__ float red[4];
-  __shared__ R16Stage<R16_KMAX_NORM> st;
-  const int m0 = blockIdx.y * 16;
-  const int lane16 = threadIdx.x & 15, sub = threadIdx.x >> 4, nsb = K >> 8;
-  constexpr int MAXU = R16_KMAX_NORM / 4096;  // superblocks a thread holds
-  auto load = [&](float4 (&xv)[MAXU][4], int m) {
-    const bool valid = m < M_valid;
-    const float* xr = x + (size_t)((valid ? m : 0) + row_off) * K;
+// swiglu_quant over a chunk: no value depends on another superblock of its row, so the tiles of quant_rows do (rows, 16
+// or 64, the launcher's choice), and every size fills the chip; 16 whole rows a work-group, the form before, took 123 us
+// at 384 x 17408, now 13.2 (1024: 125 -> 28, 4096 x 5120: 43.5 -> 33, 8192 x 5120: 91.4 -> 90.9, bound by memory).  grid (256 * (F / 256), ceil(M / rows)), local (256, 1).
+extern "C" __global__ __launch_bounds__(256) void swiglu_quant_tile(const float* __restrict__ gu, int F, int M, int M_valid,
+                                                                    signed char* __restrict__ aq, float* __restrict__ asc,
+                                                                    short* __restrict__ absum, int act32, int fused,
+                                                                    int gelu, int rows, int q2_aq, int q2_sc, int q2_ab) {
+  const int s = blockIdx.x;
+  auto load = [&](float (&v)[16], int m) {
+    const float4* g = (const float4*)(gu + (size_t)m * (fused ? F : 2 * F) + s * 256 + 16 * (threadIdx.x & 15));
+    const float4* u = (const float4*)((const float*)g + F);
+    float4 uv[4];
 #pragma unroll
-    for (int u = 0; u < MAXU; ++u) {
-      const int sb = sub + 16 * u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        xv[u][i] = valid && sb < nsb ? *(const float4*)(xr + sb * 256 + 16 * lane16 + 4 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = 0; i < 4; ++i) {
+      const float4 f = g[i];
+      if (!fused) uv[i] = u[i];
+      v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
     }
-  };
-  auto work = [&](const float4 (&xv)[MAXU][4], int r) {
-    const int m = m0 + r;
-    float ss = 0.0f;
-#pragma unroll
-    for (int u = 0; u < MAXU; ++u)
+    if (!fused)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        ss += xv[u][i].x * xv[u][i].x;
-        ss += xv[u][i].y * xv[u][i].y;
-        ss += xv[u][i].z * xv[u][i].z;
-        ss += xv[u][i].w * xv[u][i].w;
+        v[4 * i] = act_gate(v[4 * i], gelu) * uv[i].x;
+        v[4 * i + 1] = act_gate(v[4 * i + 1], gelu) * uv[i].y;
+        v[4 * i + 2] = act_gate(v[4 * i + 2], gelu) * uv[i].z;
+        v[4 * i + 3] = act_gate(v[4 * i + 3], gelu) * uv[i].w;
       }
-    ss = group_sum(ss, red);
-    const float rs = rsqrtf(ss / (float)K + eps);
-#pragma unroll
-    for (int u = 0; u < MAXU; ++u) {
-      const int sb = sub + 16 * u;
-      if (sb >= nsb) break;  // (the same for the 16 threads of a superblock)
-      const int base = sb * 256 + 16 * lane16;
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 f = xv[u][i], g = *(const float4*)(w + base + 4 * i);
-        v[4 * i] = f.x * rs * g.x; v[4 * i + 1] = f.y * rs * g.y; v[4 * i + 2] = f.z * rs * g.z; v[4 * i + 3] = f.w * rs * g.w;
-      }
-      if (write_h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *(float4*)(hout + (size_t)m * K + base + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-      r16_quant(st, v, sb, lane16, r, m, K, act32, aq);
-    }
   };
-  float4 xa[MAXU][4], xb[MAXU][4];
-  load(xa, m0);
-#pragma unroll 1
-  for (int r = 0; r < 16; r += 2) {
-    load(xb, m0 + r + 1);
-    work(xa, r);
-    load(xa, min(m0 + r + 2, m0 + 15));  // (after the last pair: row 15 again, not used)
-    work(xb, r + 1);
-  }
-  r16_flush(st, m0, M, K, act32, asc, absum);
+  quant_tile(load, s, blockIdx.y * rows, rows, F, M, M_valid, aq, asc, absum, act32, q2_aq, q2_sc, q2_ab);
 }
 
-// swiglu_quant over 16 rows a work-group: grid (256, M / 16).
-extern "C" __global__ __launch_bounds__(256, 2) void swiglu_quant_r16(const float* __restrict__ gu, int F, int M, int M_valid,
-                                                                      signed char* __restrict__ aq, float* __restrict__ asc,
-                                                                      short* __restrict__ absum, int act32, int fused,
-                                                                      int gelu) {
-  __shared__ R16Stage<R16_KMAX> st;
-  const int m0 = blockIdx.y * 16;
-  const int lane16 = threadIdx.x & 15, sub = threadIdx.x >> 4, nsb = F >> 8;
-  // (the units of work: superblock s of row r, row-major over the 16 rows, dealt to the 16 groups of threads in turn --
-  //  by rows alone 20 superblocks would keep four groups busy twice and twelve once; the loads of a thread's next unit
-  //  are in flight while it works on the current one)
-  const int units = 16 * nsb, total = (units - sub + 15) / 16;
-  struct Unit { float4 g[4], u[4]; int r, s; };
-  auto load = [&](Unit& t, int j) {
-    const int i = sub + 16 * min(j, total - 1);   // (past the end: the last again, not used)
-    t.r = i / nsb;
-    t.s = i - t.r * nsb;
-    const bool in = m0 + t.r < M_valid;
-    const float* gr = gu + (size_t)(in ? m0 + t.r : 0) * (fused ? F : 2 * F) + t.s * 256 + 16 * lane16;
+// rmsnorm_quant over a chunk: a work-group takes four rows, a wave one row, so that the row's sum is the wave's own and no
+// wave waits for another until the scales and sums, staged in LDS as [block][row], leave in pieces of four tokens.  A lane
+// holds its 16 values of superblocks lane / 16 + 4 u in registers from the sum of squares to the quantization for
+// u < MAXU (rows of up to 6144 values); what a longer row has beyond them is read again, out of the cache.  Bound by
+// memory from about 4096 rows on, below that by one row's chain of loads, sum and stores.  The form before it, 16 rows a
+// work-group one after the other, left most of the chip idle: 384 x 5120 37.9 -> 8.4 us, 1024 x 5120 37.7 -> 9.2, 8192 x
+// 5120 46.6 -> 41.7 (5.3 TB/s); eight rows a work-group (pieces of 32 and 16 bytes) 10.1, 10.7, 50.8.
+// One-pass engines, M a multiple of 4, K <= RW_KMAX.  grid (256, M / 4).
+#define RW_KMAX 16384
+extern "C" __global__ __launch_bounds__(256) void rmsnorm_quant_wave(const float* __restrict__ x, int row_off,
+                                                                     const float* __restrict__ w, int K, int M, int M_valid,
+                                                                     float eps, signed char* __restrict__ aq,
+                                                                     float* __restrict__ asc, short* __restrict__ absum,
+                                                                     float* __restrict__ hout, int write_h, int act32) {
+  __shared__ float st_sc[RW_KMAX / 32 * 4];
+  __shared__ short st_sum[RW_KMAX / 16 * 4];
+  constexpr int MAXU = 6;
+  const int r = threadIdx.x >> 6, lane = threadIdx.x & 63, lane16 = lane & 15, sub = lane >> 4, nsb = K >> 8;
+  // (neighbouring groups of rows on the same chiplet, by the launch order's round over the eight: their pieces of a cache
+  //  line of scales meet in its L2)
+  const int n8 = gridDim.y >> 3, g = blockIdx.y < n8 * 8 ? (blockIdx.y & 7) * n8 + (blockIdx.y >> 3) : blockIdx.y;
+  const int m0 = g * 4, m = m0 + r;
+  const bool valid = m < M_valid;
+  const float* xr = x + (size_t)((valid ? m : 0) + row_off) * K;
+  float4 xv[MAXU][4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      t.g[k] = in ? *(const float4*)(gr + 4 * k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      t.u[k] = in && !fused ? *(const float4*)(gr + F + 4 * k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+  for (int u = 0; u < MAXU; ++u) {
+    const int sb = sub + 4 * u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      xv[u][i] = valid && sb < nsb ? *(const float4*)(xr + sb * 256 + 16 * lane16 + 4 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  float ss = 0.0f;
+  auto square = [&](const float4& f) {
+    ss += f.x * f.x;
+    ss += f.y * f.y;
+    ss += f.z * f.z;
+    ss += f.w * f.w;
   };
-  auto work = [&](const Unit& t) {
+#pragma unroll
+  for (int u = 0; u < MAXU; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) square(xv[u][i]);
+  if (valid)
+    for (int sb = sub + 4 * MAXU; sb < nsb; sb += 4)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) square(*(const float4*)(xr + sb * 256 + 16 * lane16 + 4 * i));
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  const float rs = rsqrtf(ss / (float)K + eps);
+  auto work = [&](const float4* f4, int sb) {
+    const int base = sb * 256 + 16 * lane16;
     float v[16];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      v[4 * k] = t.g[k].x; v[4 * k + 1] = t.g[k].y; v[4 * k + 2] = t.g[k].z; v[4 * k + 3] = t.g[k].w;
+    for (int i = 0; i < 4; ++i) {
+      const float4 f = f4[i], g = *(const float4*)(w + base + 4 * i);
+      v[4 * i] = f.x * rs * g.x; v[4 * i + 1] = f.y * rs * g.y; v[4 * i + 2] = f.z * rs * g.z; v[4 * i + 3] = f.w * rs * g.w;
     }
-    if (m0 + t.r < M_valid && !fused) {
+    if (write_h)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float uv[4] = {t.u[k].x, t.u[k].y, t.u[k].z, t.u[k].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[4 * k + j] = act_gate(v[4 * k + j], gelu) * uv[j];
-      }
+      for (int i = 0; i < 4; ++i)
+        *(float4*)(hout + (size_t)m * K + base + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    const float amax = block_amax(v, act32);
+    uint4 pk;
+    int sum;
+    quant16(v, amax, pk, sum, nullptr);
+    *(uint4*)(aq + (size_t)m * K + base) = pk;
+    st_sum[(sb * 16 + lane16) * 4 + r] = (short)sum;
+    if (act32) {
+      if ((lane16 & 1) == 0) st_sc[(sb * 8 + (lane16 >> 1)) * 4 + r] = amax / 127.0f;
+    } else if (lane16 == 0) {
+      st_sc[sb * 4 + r] = amax / 127.0f;
     }
-    r16_quant(st, v, t.s, lane16, t.r, m0 + t.r, F, act32, aq);
   };
-  if (total > 0) {
-    Unit a, b;
-    load(a, 0);
-#pragma unroll 1
-    for (int j = 0; j < total; j += 2) {
-      load(b, j + 1);
-      work(a);
-      load(a, j + 2);
-      if (j + 1 < total) work(b);
-    }
+#pragma unroll
+  for (int u = 0; u < MAXU; ++u) {
+    if (sub + 4 * u >= nsb) break;  // (the same for the 16 lanes of a superblock)
+    work(xv[u], sub + 4 * u);
   }
-  r16_flush(st, m0, M, F, act32, asc, absum);
+  for (int sb = sub + 4 * MAXU; sb < nsb; sb += 4) {
+    float4 f[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      f[i] = valid ? *(const float4*)(xr + sb * 256 + 16 * lane16 + 4 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    work(f, sb);
+  }
+  __syncthreads();
+  const int nb = act32 ? K >> 5 : K >> 8;
+  for (int i = threadIdx.x; i < nb * 4; i += 256) asc[(size_t)(i >> 2) * M + m0 + (i & 3)] = st_sc[i];
+  for (int i = threadIdx.x; i < (K >> 4) * 2; i += 256)
+    *(uint32_t*)(absum + (size_t)(i >> 1) * M + m0 + 2 * (i & 1)) = *(const uint32_t*)(st_sum + 2 * i);
 }
 
 // softcap_rows: C[t][off + n] = cap * tanh(C[t][off + n] / cap) over N columns of the launch's rows (the output head of

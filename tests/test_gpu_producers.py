@@ -143,6 +143,41 @@ def test_producers_16_rows_a_work_group(rt, T, Mp, K, act32):
         eng.close()
 
 
+@pytest.mark.parametrize("T,Mp,K", [(257, 260, 256), (509, 512, 6400), (300, 304, 16640), (250, 272, 6144), (2047, 2064, 4096),
+                                    (8192, 8192, 2048)])
+def test_producers_tiles_and_waves(rt, T, Mp, K):
+    """The chunk forms at their edges: the RMS norm's wave a row (one superblock, a row longer than a wave's registers
+    hold, one longer than the form takes, numbers of row groups that eight does not divide), tiles of 16 and 64 rows with
+    a ragged last one; all three quantizers give the plain quantizer's bits on the rows that the norm itself wrote out."""
+    print(f"producers tiles T={T} Mp={Mp} K={K}", flush=True)
+    eng = az.Engine(Mp, K)
+    try:
+        def read():
+            return (eng.aq.read(np.int8, Mp * K), eng.asc.read(np.uint32, Mp * K // 32), eng.absum.read(np.int16, Mp * K // 16))
+        x = make_acts(T, K, seed=340 + T, outliers=True)
+        w = (1.0 + 0.1 * az.gen_normal(341, (K,))).astype(np.float32)
+        xb, wb = az.Runtime.from_numpy(x), az.Runtime.from_numpy(w)
+        hb = az.Runtime.alloc(Mp * K * 4).fill(0xFFFFFFFF)
+        poison(eng)
+        eng.rmsnorm_quant(xb, 0, wb, K, Mp, T, 1e-6, hout=hb)
+        got = read()
+        h = hb.read(np.float32, Mp * K).reshape(Mp, K)
+        x64 = x.astype(np.float64)
+        ref = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * w.astype(np.float64)
+        assert np.abs(h[:T] - ref).max() <= 1e-6 * np.abs(ref).max() and not h[T:].any()
+        raq, rasc, rabsum = orc.quantize_act(np.ascontiguousarray(h))
+        want = (raq.reshape(-1), rasc.view(np.uint32).reshape(-1), rabsum.reshape(-1))
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        for step in (lambda: eng.swiglu_quant(hb, K, Mp, T, fused=1), lambda: eng.quantize(hb, K, K, Mp, T)):
+            poison(eng)
+            step()
+            assert all(np.array_equal(a, b) for a, b in zip(read(), want))
+        for b in (xb, wb, hb):
+            b.free()
+    finally:
+        eng.close()
+
+
 def test_producer_feeds_matmul(eng):
     """rmsnorm_quant -> GEMV and GEMM: the matmul of the normalized rows, against the oracle on the GPU's own int8 rows."""
     from common import make_weights, rel_err_rows
