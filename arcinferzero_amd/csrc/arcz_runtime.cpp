@@ -409,7 +409,7 @@ arcz_kernel* arcz_kernel_get(const char* which, const char* defs, const char* na
     }
     const int v = f == dv.end() ? spec->hidden[i].def : (int)f->second;
     if (std::string(spec->hidden[i].name) == "LDS") {
-      if (v < 0 || v > 65536) { fail(ARCZ_E_BUILD, "%s: %d bytes of LDS", nm.c_str(), v); return nullptr; }
+      if (v < 0 || v > 160 * 1024) { fail(ARCZ_E_BUILD, "%s: %d bytes of LDS", nm.c_str(), v); return nullptr; }
       lds = (unsigned)v;
     } else {
       hidden.push_back(v);

@@ -1157,6 +1157,81 @@ class Engine {
     }
   }
 
+  // Passes between the one-slot kernels, whose time goes with the pairs, and the tile GEMM, whose work-groups take about the
+  // same time however few slots a tile has: the matrix-pipe kernels of 16-slot tiles.  us a layer, 128 x 8 experts of 768 x
+  // 2048, one-slot or tile GEMM against these: 8 tokens Q4_K 68 / 70, IQ4_XS 73 / 79; 16: 121 / 83, 131 / 96; 32: 165 / 103,
+  // 315 / 120; 128: 180 / 142, 341 / 153; 256: 182 / 169, 350 / 199; 32 x 4 experts, 8 tokens 45 / 53, 16 tokens 69 / 55.
+  // The upper end is in slots an expert, where the type's tile GEMM overtakes: Q4_K 14 - 19, Q5_K 16, Q6_K 24, the others
+  // 36 - 45.
+  static bool moe_mm_takes(const MoeLayer& L, int T) {
+    const uint32_t t = L.ex[0].type;
+    const int most = t == GGML_Q4_K || t == GGML_Q5_K ? 15 : t == GGML_Q6_K ? 22 : 36;
+    return T > 8 && T * L.NU >= 48 && T * L.NU <= L.NE * most;
+  }
+  // LDS of an expert kernel on the matrix pipe (decode_mm.hip's MmL): tokens of K values, the waves' pieces, the epilogue's
+  // rows, the codebook; 0: K does not fit
+  static size_t moe_mm_lds(uint32_t type, int K, bool gateup) {
+    const bool min = type == GGML_Q4_K || type == GGML_Q5_K;
+    const bool i3 = type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS;
+    const size_t wq = type == GGML_Q8_0 ? 4096 : 2048, wx = type == GGML_Q5_K || i3 ? 2048 : type == GGML_Q6_K ? 4096 : 0;
+    const size_t wd = type == GGML_Q6_K || i3 ? 256 : 0;
+    const size_t grid = type == GGML_IQ3_S ? 2048 : type == GGML_IQ3_XXS ? 1024 : 0;
+    const size_t n = (size_t)(K / 256) * (4096 + 512 + (min ? 512 : 0)) + 8 * (wq + 1024 + wx + wd) + (gateup ? 16 * 132 * 4 : 0) + grid;
+    return n <= 159 * 1024 ? n : 0;
+  }
+  // The experts of a pass through moe_gateup_mm / moe_down_mm, tiles of 16 slots; false: not for this layer
+  bool moe_mm(const MoeLayer& L, cl_mem rl, int ldl, cl_mem x, int T, int Mp, cl_mem sh) {
+    const int E = L.E, F = L.F, NE = L.NE, NU = L.NU, n = T * NU;
+    const size_t lg = moe_mm_lds(L.ex[0].type, E, true), ld = moe_mm_lds(L.ex[2].type, F, false);
+    if (L.ex[0].type != L.ex[1].type || F % 128 || E % 128 || !lg || !ld) return false;
+    route_tiles(L, rl, ldl, T, 16);
+    const size_t tiles_max = (size_t)(n + 15) / 16 + std::min(n, NE);
+    cl_mem tabs = tabs_;
+    const std::string ne = " -DNE=" + std::to_string(NE);
+    {
+      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[0].type) + ne + " -DLDS=" + std::to_string(lg), "moe_gateup_mm");
+      int FF = F, KK = E, MM = Mp, S = slots_;
+      set_args(k, 0, L.ex[0].raw, L.ex[1].raw, FF, KK, tabs, aq_, asc_, MM, mtiles_, stok_, mh_, absum_, S, mhq_, mhsc_, mhbs_);
+      size_t gws[2] = {(size_t)(F / 128) * 512, tiles_max}, lws[2] = {512, 1};
+      run("moe_gateup", k, 2, gws, lws);
+    }
+    {
+      // (groups of 16 rows a wave: K is short, so several behind one staging of the tokens; 40 tokens at 2048 x 768: 138,
+      //  125, 123, 127 us a layer with 1, 2, 4, 8)
+      int gpw = 4;
+      while (E % (128 * gpw)) gpw >>= 1;
+      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[2].type) + ne + " -DLDS=" + std::to_string(ld), "moe_down_mm");
+      int NN = E, KK = F, S = slots_;
+      set_args(k, 0, L.ex[2].raw, NN, KK, tabs, mhq_, mhsc_, S, mtiles_, swt_, my_, mhbs_, gpw);
+      size_t gws[2] = {(size_t)(E / (128 * gpw)) * 512, tiles_max}, lws[2] = {512, 1};
+      run("moe_down", k, 2, gws, lws);
+    }
+    moe_sum(L, x, sh, T);
+    return true;
+  }
+  // x[t] += the token's weighted expert rows in my_, and the shared expert's
+  void moe_sum(const MoeLayer& L, cl_mem x, cl_mem sh, int T) {
+    cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(L.NU), "moe_combine");
+    int EE = L.E;
+    set_args(k, 0, x, sh, sgate_, my_, minv_, EE);
+    size_t gws[2] = {((size_t)L.E + 1023) / 1024 * 256, (size_t)T}, lws[2] = {256, 1};  // (four columns a thread)
+    run("moe_combine", k, 2, gws, lws);
+  }
+  // routing -> slots -> tiles of tm slots; few pairs: the three steps in one work-group (as three launches they took 19 us)
+  void route_tiles(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm) {
+    if (T * L.NU > 1024 || L.NE > 512 || L.variant()) {
+      moe_route(L, rl, ldl, T, tm);
+      return;
+    }
+    if (ldl < L.NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + L.NE) * 4) throw std::runtime_error("layer_moe: router logits do not fit");
+    cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(L.NU) + " -DTM=" + std::to_string(tm),
+                         "moe_route_small");
+    int NR = ldl, TT = T;
+    set_args(k, 0, rl, NR, TT, mids_, mwts_, sgate_, mtiles_, stok_, swt_, minv_);
+    size_t g1 = 1024, l1 = 1024;
+    run("moe_route", k, 1, &g1, &l1);
+  }
+
   // x[t] += sum_k w_k * expert_k(h[t]) for the T tokens whose quantized h is the current activation chunk
   // (zero/engine_moe.h:8-361 layer_moe: standard experts, no shared expert).  x: [T][E] f32.
   // sh (may be null): the shared expert's output rows [T][E] f32, added as sgate[t] * sh[t] (zero/kernels/moe.cl:344-352;
@@ -1170,11 +1245,12 @@ class Engine {
     // A pass of 1-16 tokens (zero/engine_moe.h:86-262 has this form for 1-8): small tiles through the matrix-vector
     // kernels moe_gateup_q / moe_down_q, routed by one launch (moe_route1 for one token, whose NU experts are the tiles;
     // moe_route_small for more) instead of the 64-slot tile GEMMs, which for one token walked K alone in 8 x 6
-    // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings that back).  At 128 x 8 experts
-    // the two forms meet at 24 tokens (170 us); 16 tokens take 112 against 137 us (ARCZ_MOE_DECODE_MAX moves the limit).
+    // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings that back, ARCZ_MOE_DECODE_MAX
+    // moves the limit).
     // (the switches of this function are read when the engine is made: a test sets them before it makes its engine)
     const bool dec_off = moe_dec_off_;
     const int dec_max = moe_dec_max_;
+    if (moe_mm_takes(L, T) && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
     if (!dec_off && T <= dec_max && T * NU <= 512) {
       const int NE = L.NE;
       // (one-slot tiles at every count: eight tokens' 64 pairs hit about 50 experts, so a tile of 8 slots holds 1.3 on
@@ -1201,18 +1277,8 @@ class Engine {
         size_t g1 = 64, l1 = 64;
         run("moe_route", k, 1, &g1, &l1);
         tiles_max = (size_t)NU;
-      } else if (n <= 512 && NE <= 512 && !L.variant()) {
-        // routing, scan and scatter of the few pairs in one work-group (the three launches took 19 us)
-        if (ldl < NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + NE) * 4) throw std::runtime_error("layer_moe: router logits do not fit");
-        cl_kernel k = kernel("moe", "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU) + " -DTM=" + std::to_string(tmd),
-                             "moe_route_small");
-        int NR = ldl, TT = T;
-        set_args(k, 0, rl, NR, TT, mids_, mwts_, sgate_, mtiles_, stok_, swt_, minv_);
-        size_t g1 = 512, l1 = 512;
-        run("moe_route", k, 1, &g1, &l1);
-        tiles_max = (size_t)(n + tmd - 1) / tmd + std::min(n, NE);
       } else {
-        moe_route(L, rl, ldl, T, tmd);
+        route_tiles(L, rl, ldl, T, tmd);
         tiles_max = (size_t)(n + tmd - 1) / tmd + std::min(n, NE);
       }
       cl_mem tabs = tabs_;
@@ -1270,13 +1336,7 @@ class Engine {
           size_t gws[2] = {((size_t)(E + 1) / 2 * 32 + 255) / 256 * 256, tiles_max}, lws[2] = {256, 1};
           run("moe_down", k, 2, gws, lws);
         }
-        {
-          cl_kernel k = kernel("moe", "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU), "moe_combine");
-          int EE = E;
-          set_args(k, 0, x, sh, sgate_, my_, minv_, EE);
-          size_t gws[2] = {((size_t)E + 1023) / 1024 * 256, (size_t)T}, lws[2] = {256, 1};
-          run("moe_combine", k, 2, gws, lws);
-        }
+        moe_sum(L, x, sh, T);
       }
       return;
     }
@@ -1333,13 +1393,7 @@ class Engine {
       run("moe_quant", k, 2, gws, lws);
     }
     moe_gemm(L, 2, Mp, max_tiles, pre_gu ? -1 : n);  // (-1: mhu_ is written already)
-    {
-      cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(NU), "moe_combine");
-      int EE = E;
-      set_args(k, 0, x, sh, sgate_, my_, minv_, EE);
-      size_t gws[2] = {((size_t)E + 1023) / 1024 * 256, (size_t)T}, lws[2] = {256, 1};  // (four columns a thread)
-      run("moe_combine", k, 2, gws, lws);
-    }
+    moe_sum(L, x, sh, T);
   }
 
  private:

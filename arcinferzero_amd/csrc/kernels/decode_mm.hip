@@ -48,22 +48,22 @@ typedef uint32_t mm_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t mm_u4 __attribute__((ext_vector_type(4)));
 
 // Per type: SB, the superblocks of a slice at most; QB, the bytes of a row's superblock in the main plane; D, the
-// superblocks a wave has in flight; XB, the bytes per row and superblock of the second plane that goes through LDS in
-// batches of four; MIN, whether the type has a min term; DPL, whether d is a plane of its own (2 bytes).
+// superblocks a wave has in flight (DX: in the expert kernels, two of whose work-groups share a
+// compute unit); XB, the bytes per row and superblock of the second plane that goes through LDS in batches of four; MIN, whether the type has a min term; DPL, whether d is a plane of its own (2 bytes).
 template <int QT> struct MmT;
-template <> struct MmT<QT_Q4_K> { enum { SB = 24, QB = 128, D = 8, XB = 0, MIN = 1, DPL = 0 }; };
-template <> struct MmT<QT_Q5_K> { enum { SB = 22, QB = 128, D = 4, XB = 32, MIN = 1, DPL = 0 }; };
+template <> struct MmT<QT_Q4_K> { enum { SB = 24, QB = 128, D = 8, DX = 4, XB = 0, MIN = 1, DPL = 0 }; };
+template <> struct MmT<QT_Q5_K> { enum { SB = 22, QB = 128, D = 4, DX = 2, XB = 32, MIN = 1, DPL = 0 }; };
 // (Q6_K: two -- with four the kernel needed 270 registers and kept 14 of them in scratch memory, 60 bytes a lane written
 //  and read back per superblock: 8 tokens at 17408 x 5120 31.1 -> 24.5 us)
-template <> struct MmT<QT_Q6_K> { enum { SB = 20, QB = 128, D = 2, XB = 64, MIN = 0, DPL = 1 }; };
-template <> struct MmT<QT_Q8_0> { enum { SB = 24, QB = 256, D = 4, XB = 0, MIN = 0, DPL = 0 }; };
-template <> struct MmT<QT_Q4_0> { enum { SB = 24, QB = 128, D = 8, XB = 0, MIN = 0, DPL = 0 }; };
+template <> struct MmT<QT_Q6_K> { enum { SB = 20, QB = 128, D = 2, DX = 2, XB = 64, MIN = 0, DPL = 1 }; };
+template <> struct MmT<QT_Q8_0> { enum { SB = 24, QB = 256, D = 4, DX = 2, XB = 0, MIN = 0, DPL = 0 }; };
+template <> struct MmT<QT_Q4_0> { enum { SB = 24, QB = 128, D = 8, DX = 4, XB = 0, MIN = 0, DPL = 0 }; };
 template <> struct MmT<QT_IQ4_NL> : MmT<QT_Q4_0> {};
 template <> struct MmT<QT_MXFP4> : MmT<QT_Q4_0> {};
-template <> struct MmT<QT_IQ4_XS> { enum { SB = 24, QB = 128, D = 8, XB = 0, MIN = 0, DPL = 0 }; };
+template <> struct MmT<QT_IQ4_XS> { enum { SB = 24, QB = 128, D = 8, DX = 4, XB = 0, MIN = 0, DPL = 0 }; };
 // (IQ3_S: the main plane is the 8 index bytes per block, the second the sign bits, the header the ninth bits and scale
 //  nibbles, 12 bytes; the codebook, 2 KiB, sits behind the groups' sums in LDS)
-template <> struct MmT<QT_IQ3_S> { enum { SB = 22, QB = 64, D = 8, XB = 32, MIN = 0, DPL = 1 }; };
+template <> struct MmT<QT_IQ3_S> { enum { SB = 22, QB = 64, D = 8, DX = 2, XB = 32, MIN = 0, DPL = 1 }; };
 // (Q3_K: planes of the same sizes -- 8 bytes of bit pairs per block, the words of third bits, 12 bytes of scales)
 template <> struct MmT<QT_Q3_K> : MmT<QT_IQ3_S> {};
 // (IQ3_XXS: the index bytes and the blocks' words of sign codes and scales likewise; no header plane)
@@ -97,15 +97,26 @@ template <int QT> struct MmSb {
   mm_u4 sg[QT == QT_IQ3_S || QT == QT_Q3_K || QT == QT_IQ3_XXS ? 2 : 1];
 };
 
-// one slice of K, superblocks [s_begin, s_end): at most MmT<QT>::SB of them
-template <int QT>
-__device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, int N, int K,
+// The rows a work-group multiplies, one slice of K at a time: ng groups of 16 rows, group gl at row row0(gl) of the
+// planes at raw(gl), which hold `rows` rows; token t is row tok(t) of the activations.  Here: groups gb0 .. of a matrix.
+struct MmRows {
+  const uint8_t* w;
+  int rows, gb0, ng;
+  __device__ const uint8_t* raw(int) const { return w; }
+  __device__ int row0(int gl) const { return (gb0 + gl) * 16; }
+  __device__ int tok(int t) const { return t; }
+};
+
+// one slice of K, superblocks [s_begin, s_end): at most MmT<QT>::SB of them; store(v, gl): group gl's sums of the slice,
+// lane (n16, g) with tokens 4 g .. 4 g + 3 of its row n16.  LEAN: within 128 registers, so that two work-groups share a
+// compute unit -- fewer superblocks in flight, the tokens' values and scales of two blocks at a time instead of eight
+template <int QT, bool LEAN, class SRC, class STORE>
+__device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& src, int K,
                                 const signed char* __restrict__ aq, const float* __restrict__ asc,
-                                const short* __restrict__ absum, int M, int T, float* C, int ldc, int c_off, int accumulate,
-                                int s_begin, int s_end, float* GA, bool first, bool last) {
+                                const short* __restrict__ absum, int M, int T, int s_begin, int s_end, STORE store) {
   using TT = MmT<QT>;
   using LL = MmL<QT>;
-  constexpr int QB = TT::QB, NQ = QB / 64, D = TT::D, LPRW = QB / 16, RPI = 64 / LPRW;
+  constexpr int QB = TT::QB, NQ = QB / 64, D = LEAN ? TT::DX : TT::D, LPRW = QB / 16, RPI = 64 / LPRW;
   constexpr bool Q45 = QT == QT_Q4_K || QT == QT_Q5_K;
   constexpr bool B16 = qt_nib16(QT) || QT == QT_IQ4_XS;  // a block is 16 bytes: low nibbles values 0..15, high 16..31
   constexpr int HB = QT == QT_IQ3_XXS ? 0 : QT == QT_IQ4_XS || QT == QT_MXFP4 ? 8 : QT == QT_IQ3_S || QT == QT_Q3_K ? 12 : 16;  // bytes of a row's superblock in the header plane
@@ -122,6 +133,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   uint8_t* WH = WQ + LL::WQ;
   uint8_t* WX = WH + LL::WH;
   uint8_t* WD = WX + LL::WX;
+  const int N = src.rows;
   // the planes (all have the main plane first, a row's superblocks together)
   size_t o_hdr, o_x = 0, o_d = 0;
   if constexpr (Q45) {
@@ -143,13 +155,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   } else {
     o_hdr = planes_iq4xs((size_t)N, nsb).hdr;
   }
-  const uint8_t* qs = raw;
-  const uint8_t* hd = raw + o_hdr;
-  const uint8_t* xp = raw + o_x;
-  const uint8_t* dp = raw + o_d;
-  const int groups = (N + 15) >> 4, gd = (int)gridDim.x;
-  const int gb0 = (int)((long)blockIdx.x * groups / gd), gb1 = (int)((long)(blockIdx.x + 1) * groups / gd);
-  const int units = (gb1 - gb0) * sbs;         // >= 1: the grid has at most `groups` work-groups
+  const int units = src.ng * sbs;              // >= 1: the grid has at most as many work-groups as groups
   const int u0 = wave * units / MM_WAVES, u1 = (wave + 1) * units / MM_WAVES;
   const int ulast = max(u1 - 1, 0);            // (a wave without units loads unit 0 and drops it)
   // unit -> group of the run (units below 2^27): the high word of u * ceil(2^32 / sbs)
@@ -161,8 +167,8 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   const uint32_t row_stride = (uint32_t)nsb * QB, piece_off = (uint32_t)(lane % LPRW) * 16;
   auto qload = [&](MmQ<QT>& q, int u) {  // u: the same in the whole wave, within the run
     const int gl = group_of(u), sb = u - gl * sbs;
-    const int g0 = (gb0 + gl) * 16;
-    const uint8_t* base = qs + ((size_t)g0 * nsb + (s_begin + sb)) * QB;
+    const int g0 = src.row0(gl);
+    const uint8_t* base = src.raw(gl) + ((size_t)g0 * nsb + (s_begin + sb)) * QB;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
       const uint32_t rel = (uint32_t)min(i * RPI + lane / LPRW, N - 1 - g0);
@@ -174,7 +180,8 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   auto hload = [&](mm_u4& h, int ub) {  // the headers of units ub .. ub + 3 (past the stretch: its last)
     const int u = min(ub + g, ulast);
     const int gl = group_of(u), sb = u - gl * sbs;
-    const int r = min((gb0 + gl) * 16 + n16, N - 1);
+    const int r = min(src.row0(gl) + n16, N - 1);
+    const uint8_t* hd = src.raw(gl) + o_hdr;
     if constexpr (HB == 0) {
       h = mm_u4{0u, 0u, 0u, 0u};
     } else if constexpr (HB == 16) {
@@ -197,30 +204,45 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
         const int row = i * RX + lane / (4 * PU), j = (lane % (4 * PU)) / PU, p = lane % PU;
         const int u = min(ub + j, ulast);
         const int gl = group_of(u), sb = u - gl * sbs;
-        const int r = min((gb0 + gl) * 16 + row, N - 1);
-        x.r[i] = *(const mm_u4*)(xp + ((size_t)r * nsb + s_begin + sb) * TT::XB + p * 16);
+        const int r = min(src.row0(gl) + row, N - 1);
+        x.r[i] = *(const mm_u4*)(src.raw(gl) + o_x + ((size_t)r * nsb + s_begin + sb) * TT::XB + p * 16);
       }
     }
     if constexpr (TT::DPL) {
       const int u = min(ub + g, ulast);
       const int gl = group_of(u), sb = u - gl * sbs;
-      const int r = min((gb0 + gl) * 16 + n16, N - 1);
-      x.d = *(const unsigned short*)(dp + ((size_t)r * nsb + s_begin + sb) * 2);
+      const int r = min(src.row0(gl) + n16, N - 1);
+      x.d = *(const unsigned short*)(src.raw(gl) + o_d + ((size_t)r * nsb + s_begin + sb) * 2);
     }
   };
 
   // ---- staging.  Loads first: the tokens' int8 rows (wave w: rows 2 w and 2 w + 1, 16-byte pieces lane, lane + 64, ..),
   // their scales and sums (asc [K / 32][M], absum [K / 16][M]), then the wave's first superblocks right behind them:
   // loads come back in order, so the stores below wait for the tokens alone while the weights are on their way.
-  constexpr int NCH = (TT::SB * 16 + 63) / 64;  // pieces per lane and row at most
-  constexpr int NSC = (TT::SB * 8 * 16 + 511) / 512;  // (block, token) pairs per thread at most
+  constexpr int NCH = LEAN ? 1 : (TT::SB * 16 + 63) / 64;  // pieces per lane and row at most
+  constexpr int NSC = LEAN ? 1 : (TT::SB * 8 * 16 + 511) / 512;  // (block, token) pairs per thread at most
   const int cpr = Ks >> 4;
   mm_u4 va[2][NCH];
   float vs[NSC];
   int vu[NSC];
+  if constexpr (LEAN) {  // (the registers are for two work-groups: piece by piece)
+    for (int i = tid; i < 16 * cpr; i += 512) {
+      const int t = i / cpr, k16 = i - t * cpr;
+      mm_u4 v = mm_u4{0, 0, 0, 0};
+      if (t < T) v = *(const mm_u4*)(aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256 + k16 * 16);
+      *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = v;
+    }
+    for (int i = tid; i < nb * 16; i += 512) {
+      const int b = s_begin * 8 + (i >> 4), t = i & 15, tt = src.tok(t < T ? t : 0);
+      const float sa = t < T ? asc[(size_t)b * M + tt] : 0.0f;
+      SA[i] = sa;
+      if constexpr (TT::MIN) U[i] = sa * (float)((int)absum[(size_t)(2 * b) * M + tt] + (int)absum[(size_t)(2 * b + 1) * M + tt]);
+    }
+  }
+  if constexpr (!LEAN) {
 #pragma unroll
   for (int r2 = 0; r2 < 2; ++r2) {
-    const int t = 2 * wave + r2, tt = t < T ? t : 0;
+    const int t = 2 * wave + r2, tt = src.tok(t < T ? t : 0);
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int k16 = min(lane + 64 * i, cpr - 1);
@@ -229,9 +251,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   }
 #pragma unroll
   for (int i = 0; i < NSC; ++i) {
-    const int idx = min(tid + 512 * i, nb * 16 - 1), b = s_begin * 8 + (idx >> 4), t = idx & 15, tt = t < T ? t : 0;
+    const int idx = min(tid + 512 * i, nb * 16 - 1), b = s_begin * 8 + (idx >> 4), t = idx & 15, tt = src.tok(t < T ? t : 0);
     vs[i] = asc[(size_t)b * M + tt];
     if constexpr (TT::MIN) vu[i] = (int)absum[(size_t)(2 * b) * M + tt] + (int)absum[(size_t)(2 * b + 1) * M + tt];
+  }
   }
   __builtin_amdgcn_sched_barrier(0);
   MmQ<QT> q[D];
@@ -243,6 +266,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
 #pragma unroll
   for (int k = 0; k < D; ++k) qload(q[k], min(u0 + k, ulast));
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (!LEAN) {
 #pragma unroll
   for (int r2 = 0; r2 < 2; ++r2) {
     const int t = 2 * wave + r2;
@@ -260,6 +284,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
     const float sa = t < T ? vs[i] : 0.0f;
     SA[idx] = sa;
     if constexpr (TT::MIN) U[idx] = sa * (float)vu[i];
+  }
   }
   __syncthreads();
 
@@ -299,16 +324,26 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
         sa4[b] = *(const float4*)(SA + (b0 + b) * 16 + 4 * g);
       }
     };
-    if constexpr (QT != QT_Q6_K) tokens(0, 8);
+    constexpr int TP = LEAN ? 2 : 8;  // blocks whose tokens are in registers at a time
+    auto ahead = [&](int b) {
+      if (b % TP == 0) {
+        if (LEAN) __builtin_amdgcn_sched_barrier(0);
+        tokens(b, b + TP);
+      }
+    };
     if constexpr (Q45) {
       const float d = f16_bits_to_f32(h.h.x), dmin = f16_bits_to_f32(h.h.x >> 16);
       const float ua = U[(b0 + g) * 16 + n16], ub = U[(b0 + 4 + g) * 16 + n16];
-      int sc[8], mn[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) q4k_scales_pair(h.h.y, h.h.z, h.h.w, j, sc[2 * j], sc[2 * j + 1], mn[2 * j], mn[2 * j + 1]);
-      v4i I[8];
+      int sc[2], m0 = 0, m1 = 0;  // the scales of two blocks; the mins of blocks g and 4 + g
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
+        ahead(b);
+        if ((b & 1) == 0) {
+          int mn[2];
+          q4k_scales_pair(h.h.y, h.h.z, h.h.w, b >> 1, sc[0], sc[1], mn[0], mn[1]);
+          int& m = b < 4 ? m0 : m1;
+          m = g == (b & 3) ? mn[0] : g == (b & 3) + 1 ? mn[1] : m;
+        }
         const mm_u2 cw = h.c[b >> 1];
         uint32_t w0 = ((b & 1) ? cw.x >> 4 : cw.x) & 0x0F0F0F0Fu, w1 = ((b & 1) ? cw.y >> 4 : cw.y) & 0x0F0F0F0Fu;
         if constexpr (QT == QT_Q5_K) {
@@ -327,19 +362,14 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
         }
         const long wv = (long)(((unsigned long)w1 << 32) | w0);
         v4i z = {0, 0, 0, 0};
-        I[b] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[b], wv, z, 0, 0, 0);
-      }
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const float ws = d * (float)sc[b];
-        acc[0] = fmaf((float)I[b][0], sa4[b].x * ws, acc[0]);
-        acc[1] = fmaf((float)I[b][1], sa4[b].y * ws, acc[1]);
-        acc[2] = fmaf((float)I[b][2], sa4[b].z * ws, acc[2]);
-        acc[3] = fmaf((float)I[b][3], sa4[b].w * ws, acc[3]);
+        const v4i I = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[b], wv, z, 0, 0, 0);
+        const float ws = d * (float)sc[b & 1];
+        acc[0] = fmaf((float)I[0], sa4[b].x * ws, acc[0]);
+        acc[1] = fmaf((float)I[1], sa4[b].y * ws, acc[1]);
+        acc[2] = fmaf((float)I[2], sa4[b].z * ws, acc[2]);
+        acc[3] = fmaf((float)I[3], sa4[b].w * ws, acc[3]);
       }
       // the min term of each half's four blocks, - sum_b (sa S)[t][b] (dmin mn)[n][b], as one f32 matrix instruction
-      const int m0 = g == 0 ? mn[0] : g == 1 ? mn[1] : g == 2 ? mn[2] : mn[3];
-      const int m1 = g == 0 ? mn[4] : g == 1 ? mn[5] : g == 2 ? mn[6] : mn[7];
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ua, -(dmin * (float)m0), acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ub, -(dmin * (float)m1), acc, 0, 0, 0);
     } else if constexpr (QT == QT_Q6_K) {
@@ -351,9 +381,9 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       v4f part = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
-        if ((b & 3) == 0) {
+        if ((b & (LEAN ? 1 : 3)) == 0) {
           __builtin_amdgcn_sched_barrier(0);
-          tokens(b, b + 4);
+          tokens(b, b + (LEAN ? 2 : 4));
         }
         const int n2 = b >> 2, hb = b & 3;
         const mm_u2 L = h.c[2 * n2 + (hb & 1)], H = h.x[n2];
@@ -384,10 +414,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       // block b: indices 2 g and 2 g + 1 of its eight (a byte each) name codebook words of four magnitudes; the signs of
       // the lane's eight values are the block's sign code g, the scale the top nibble of that word; d / 4
       // (reference src/quants.h:220-239, zero/kernels/decode.cl:183-478)
-      const uint32_t* grid = (const uint32_t*)(lds + LL::OGRID);
-      const float d3 = 0.25f * f16_bits_to_f32(h.d);
+            const float d3 = 0.25f * f16_bits_to_f32(h.d);
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
+        ahead(b);
         const uint32_t q16 = h.c[b].x;
         const uint32_t a = b < 4 ? h.sg[0][b & 3] : h.sg[1][b & 3];
         const uint32_t s8 = iq3xxs_signs8(a, g);
@@ -410,9 +440,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       const uint32_t keep0 = g < 2 ? 0xFFFFFFFFu : 0u, keep1 = ~keep0;
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
-        const uint32_t D = h.c[b].x;
+        ahead(b);
+        const uint32_t bits = h.c[b].x;
         const uint32_t H = b < 4 ? h.sg[0][b & 3] : h.sg[1][b & 3];
-        const uint32_t w0 = q3k_vals(D, H, 2 * g), w1 = q3k_vals(D, H, 2 * g + 1);
+        const uint32_t w0 = q3k_vals(bits, H, 2 * g), w1 = q3k_vals(bits, H, 2 * g + 1);
         const long wa = (long)(((unsigned long)(w1 & keep0) << 32) | (w0 & keep0));
         const long wb = (long)(((unsigned long)(w1 & keep1) << 32) | (w0 & keep1));
         v4i z = {0, 0, 0, 0};
@@ -431,10 +462,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       // block b: indices 2 g and 2 g + 1 of its eight (a byte each and a ninth bit from byte b of the header) name
       // codebook words of four magnitudes, the signs are bits 8 g .. 8 g + 7 of the block's word; scale 1 + 2 x nibble b
       // of the header's third word, times d (reference src/quants.h IQ3_S, zero/kernels/decode.cl:183-478)
-      const uint32_t* grid = (const uint32_t*)(lds + LL::OGRID);
-      const float d3 = f16_bits_to_f32(h.d);
+            const float d3 = f16_bits_to_f32(h.d);
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
+        ahead(b);
         const uint32_t q16 = h.c[b].x;
         const uint32_t n9 = (b < 4 ? h.h.x : h.h.y) >> (8 * (b & 3) + 2 * g);
         const uint32_t g0 = grid[(q16 & 0xFFu) | ((n9 & 1u) << 8)], g1 = grid[((q16 >> 8) & 0xFFu) | ((n9 & 2u) << 7)];
@@ -459,6 +490,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       const float d4 = f16_bits_to_f32(h.h.x);
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
+        ahead(b);
         const mm_u2 cw = h.c[b];
         uint32_t w0, w1;
         float d;
@@ -489,6 +521,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
       // Q8_0: block b is bytes 32 b .. 32 b + 31 of the row's 256, its f16 scale entry b of the 16-byte header
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
+        ahead(b);
         const mm_u2 cw = h.c[b];
         const long wv = (long)(((unsigned long)cw.y << 32) | cw.x);
         v4i z = {0, 0, 0, 0};
@@ -499,31 +532,6 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
         acc[1] = fmaf((float)I[1], sa4[b].y * d, acc[1]);
         acc[2] = fmaf((float)I[2], sa4[b].z * d, acc[2]);
         acc[3] = fmaf((float)I[3], sa4[b].w * d, acc[3]);
-      }
-    }
-  };
-
-  // lane (n16, g) holds tokens 4 g .. 4 g + 3 of row n16 of a group
-  const int tmax = T > 8 ? 16 : T;  // (9-16 tokens: the chunk has 16 rows, those from T on come out as zeros)
-  // GA: the work-group's groups' sums over the slices so far, in LDS ([group][16 tokens][16 rows]; a load from C at
-  // every group's end would wait for all the weights in flight behind it): C is written by the last slice alone
-  auto store = [&](v4f v, int gl) {
-    const int n = (gb0 + gl) * 16 + n16;
-    if (GA) {
-      float* ga = GA + gl * 256 + 64 * g + n16;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (!first) v[i] += ga[16 * i];
-        if (!last) ga[16 * i] = v[i];
-      }
-      if (!last) return;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 4 * g + i;
-      if (t < tmax && n < N) {
-        float* cp = C + (size_t)t * ldc + c_off + n;
-        *cp = accumulate ? *cp + v[i] : v[i];
       }
     }
   };
@@ -626,6 +634,16 @@ __device__ inline void mm_slice(uint8_t* lds, const uint8_t* __restrict__ raw, i
   }
 }
 
+// The codebook of the types that have one, into LDS (the first slice's meeting orders it): IQ3_S the first 512 words of the
+// tables, IQ3_XXS the 256 behind them.
+template <int QT>
+__device__ inline void mm_grid(uint32_t* grid, const uint32_t* __restrict__ tabs) {
+  if constexpr (QT == QT_IQ3_XXS)
+    for (int i = threadIdx.x; i < 256; i += 512) grid[i] = tabs[512 + i];
+  if constexpr (QT == QT_IQ3_S)
+    for (int i = threadIdx.x; i < 512; i += 512) grid[i] = tabs[i];
+}
+
 // Superblocks [s_begin, s_end) of K, in slices that the work-group takes one after the other.  With more than one slice
 // the sums of a work-group's groups wait in LDS for the last slice (as many groups as the type's LDS leaves room for);
 // with more groups than that a later slice adds to what the work-group itself has stored in C (other waves of it, as
@@ -638,18 +656,42 @@ __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, 
   constexpr int SB = MmT<QT>::SB;
   const int all = s_end - s_begin, slices = (all + SB - 1) / SB;
   const int groups = (N + 15) >> 4, gd = (int)gridDim.x;
-  const int ng = (int)((long)(blockIdx.x + 1) * groups / gd) - (int)((long)blockIdx.x * groups / gd);
-  float* GA = slices > 1 && ng <= MmL<QT>::GA ? (float*)(lds + SB * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ) : nullptr;
-  if constexpr (QT == QT_IQ3_XXS) {  // (its codebook: the 256 words behind IQ3_S's)
-    for (int i = threadIdx.x; i < 256; i += 512) ((uint32_t*)(lds + MmL<QT>::OGRID))[i] = tabs[512 + i];
-  }
-  if constexpr (QT == QT_IQ3_S) {  // (the codebook: the first 512 words of the tables; the first slice's meeting orders it)
-    for (int i = threadIdx.x; i < 512; i += 512) ((uint32_t*)(lds + MmL<QT>::OGRID))[i] = tabs[i];
-  }
+  MmRows src;
+  src.w = raw;
+  src.rows = N;
+  src.gb0 = (int)((long)blockIdx.x * groups / gd);
+  src.ng = (int)((long)(blockIdx.x + 1) * groups / gd) - src.gb0;
+  // GA: the work-group's groups' sums over the slices so far, in LDS ([group][16 tokens][16 rows]; a load from C at
+  // every group's end would wait for all the weights in flight behind it): C is written by the last slice alone
+  float* GA = slices > 1 && src.ng <= MmL<QT>::GA ? (float*)(lds + SB * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ) : nullptr;
+  uint32_t* grid = (uint32_t*)(lds + MmL<QT>::OGRID);
+  mm_grid<QT>(grid, tabs);
+  const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  const int tmax = T > 8 ? 16 : T;  // (9-16 tokens: the chunk has 16 rows, those from T on come out as zeros)
   for (int sl = 0; sl < slices; ++sl) {
     if (sl) __syncthreads();  // (the tokens and partial sums of the slice before have been read)
-    mm_slice<QT>(lds, raw, N, K, aq, asc, absum, M, T, C, ldc, c_off, GA ? accumulate : (accumulate || sl),
-                 s_begin + all * sl / slices, s_begin + all * (sl + 1) / slices, GA, sl == 0, sl == slices - 1);
+    const bool first = sl == 0, last = sl == slices - 1, add = GA ? accumulate : (accumulate || sl);
+    mm_slice<QT, false>(lds, grid, src, K, aq, asc, absum, M, T, s_begin + all * sl / slices,
+                             s_begin + all * (sl + 1) / slices, [&](v4f v, int gl) {
+      const int n = src.row0(gl) + n16;
+      if (GA) {
+        float* ga = GA + gl * 256 + 64 * g + n16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (!first) v[i] += ga[16 * i];
+          if (!last) ga[16 * i] = v[i];
+        }
+        if (!last) return;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 4 * g + i;
+        if (t < tmax && n < N) {
+          float* cp = C + (size_t)t * ldc + c_off + n;
+          *cp = add ? *cp + v[i] : v[i];
+        }
+      }
+    });
   }
 }
 
@@ -689,3 +731,128 @@ extern "C" __global__ __launch_bounds__(256) void gemv_mm_reduce(const float* __
   float* cp = C + (size_t)t * ldc + c_off + n;
   *cp = accumulate ? *cp + v : v;
 }
+
+// ---- the experts of a pass of some tokens each: the same products on the rows of one expert and the slots of one tile
+// (expert, first slot, slots <= 16).  A tile of 2 or 3 slots, what 40 tokens leave an expert of 128, is two orders below
+// the tile GEMM's 64 or 128, whose work-groups then walk K alone; here a work-group takes 128 rows, and a wave reads whole
+// groups of 16 of them in order, so it streams the expert's weights once for all the tile's slots.  Bound by instruction
+// issue (the scale step is taken for 16 slots whatever the tile holds), then by memory: 40 tokens, 128 x 8 experts of 768 x
+// 2048, IQ4_XS: gate / up 61 us (3.2 TB/s), down 35, where the tile GEMM took 3 x 100.  Q6_K and Q3_K, two products a
+// block, need the registers of one work-group a compute unit.
+struct MmExpert {
+  const uint8_t *w0, *w1;  // group 2 i of w0, group 2 i + 1 of w1 (PAIR) or both of w0
+  int rows, r0, ng;
+  bool pair;
+  const int* st;           // the slots' token rows (LDS)
+  __device__ const uint8_t* raw(int gl) const { return pair && (gl & 1) ? w1 : w0; }
+  __device__ int row0(int gl) const { return r0 + 16 * (pair ? gl >> 1 : gl); }
+  __device__ int tok(int t) const { return st[t]; }
+};
+constexpr int MMX_HS = 132;  // floats of a slot's 128 rows in LDS
+
+// moe_gateup_mm: h = silu(gate) * up of the tile's slots for rows 128 x .. 128 x + 127 of the expert, and its int8 form with
+// scales and sums as moe_quant_sums makes them.  Wave w: gate's and up's rows 16 w .. 16 w + 15, so both meet in a lane.
+// grid (F / 128 work-groups of 512, tiles).  LDS: the tokens, the waves' pieces, [16][MMX_HS] floats, the codebook.
+template <int QT>
+__device__ inline void moe_gateup_mm(uint8_t* lds, const uint8_t* __restrict__ rg, const uint8_t* __restrict__ ru, int F, int K,
+                                     const uint32_t* __restrict__ tabs, const signed char* __restrict__ aq,
+                                     const float* __restrict__ asc, const short* __restrict__ absum, int M,
+                                     const int* __restrict__ tiles, const int* __restrict__ stok, float* __restrict__ h, int S,
+                                     signed char* __restrict__ hq, float* __restrict__ hsc, short* __restrict__ hbs, int NE) {
+  __shared__ int st[16];
+  const int ti = blockIdx.y;
+  if (ti >= tiles[0]) return;
+  const int e = tiles[1 + 3 * ti], r0 = tiles[2 + 3 * ti], nr = tiles[3 + 3 * ti];
+  if (threadIdx.x < 16) st[threadIdx.x] = stok[r0 + min((int)threadIdx.x, nr - 1)];
+  float* hs = (float*)(lds + (K >> 8) * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ);
+  uint32_t* grid = (uint32_t*)(hs + 16 * MMX_HS);
+  mm_grid<QT>(grid, tabs);
+  __syncthreads();
+  MmExpert src;
+  src.w0 = rg; src.w1 = ru; src.rows = NE * F; src.r0 = e * F + blockIdx.x * 128; src.ng = 16; src.pair = true; src.st = st;
+  const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  v4f gate = {0.0f, 0.0f, 0.0f, 0.0f};
+  mm_slice<QT, true>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, [&](v4f v, int gl) {
+    if (!(gl & 1)) {
+      gate = v;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) hs[(4 * g + i) * MMX_HS + 8 * (gl & ~1) + n16] = gate[i] / (1.0f + __expf(-gate[i])) * v[i];
+    }
+  });
+  __syncthreads();
+  const int hl = threadIdx.x & 31;
+  for (int b = threadIdx.x >> 5; b < 4 * nr; b += 16) {
+    const int t = b >> 2, fb = blockIdx.x * 128 + (b & 3) * 32;
+    const float v = hs[t * MMX_HS + (b & 3) * 32 + hl];
+    float amax = fabsf(v);
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+    const int q = __float2int_rn(__fmul_rn(v, inv));
+    int sm = q;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) sm += __shfl_xor(sm, o, 64);  // the 16 lanes of a half block
+    const size_t slot = (size_t)(r0 + t);
+    h[slot * F + fb + hl] = v;
+    hq[slot * F + fb + hl] = (signed char)q;
+    if (hl == 0) hsc[(size_t)(fb >> 5) * S + slot] = amax / 127.0f;
+    if ((hl & 15) == 0) hbs[(size_t)((fb >> 4) + (hl >> 4)) * S + slot] = (short)sm;
+  }
+}
+
+// moe_down_mm: y[slot][n] = swt[slot] * (Wd[expert][n] . hq[slot]) for rows RW x .. of the expert, RW = 128 * gpw.
+// grid (N / RW work-groups of 512, tiles).
+template <int QT>
+__device__ inline void moe_down_mm(uint8_t* lds, const uint8_t* __restrict__ raw, int N, int K, const uint32_t* __restrict__ tabs,
+                                   const signed char* __restrict__ hq, const float* __restrict__ hsc,
+                                   const short* __restrict__ hbs, int S, const int* __restrict__ tiles,
+                                   const float* __restrict__ swt, float* __restrict__ y, int gpw, int NE) {
+  __shared__ int st[16];
+  __shared__ float sw[16];
+  const int ti = blockIdx.y;
+  if (ti >= tiles[0]) return;
+  const int e = tiles[1 + 3 * ti], r0 = tiles[2 + 3 * ti], nr = tiles[3 + 3 * ti];
+  if (threadIdx.x < 16) {
+    st[threadIdx.x] = r0 + min((int)threadIdx.x, nr - 1);
+    sw[threadIdx.x] = swt[r0 + min((int)threadIdx.x, nr - 1)];
+  }
+  uint32_t* grid = (uint32_t*)(lds + (K >> 8) * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ);
+  mm_grid<QT>(grid, tabs);
+  __syncthreads();
+  MmExpert src;
+  src.w0 = src.w1 = raw; src.rows = NE * N; src.ng = 8 * gpw; src.r0 = e * N + blockIdx.x * src.ng * 16; src.pair = false; src.st = st;
+  const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  mm_slice<QT, true>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, [&](v4f v, int gl) {
+    const int n = (blockIdx.x * src.ng + gl) * 16 + n16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * g + i < nr) y[(size_t)(r0 + 4 * g + i) * N + n] = sw[4 * g + i] * v[i];
+  });
+}
+
+#define MOE_MM(QTV, WPE)                                                                                                    \
+  extern "C" __global__ __launch_bounds__(512, WPE) void moe_gateup_mm__QT##QTV(                                          \
+      const uint8_t* rg, const uint8_t* ru, int F, int K, const uint32_t* tabs, const signed char* aq, const float* asc, \
+      int M, const int* tiles, const int* stok, float* h, const short* absum, int S, signed char* hq, float* hsc,       \
+      short* hbs, int NE) {                                                                                             \
+    extern __shared__ __attribute__((aligned(16))) uint8_t mm_lds[];                                                    \
+    moe_gateup_mm<QTV>(mm_lds, rg, ru, F, K, tabs, aq, asc, absum, M, tiles, stok, h, S, hq, hsc, hbs, NE);             \
+  }                                                                                                                     \
+  extern "C" __global__ __launch_bounds__(512, WPE) void moe_down_mm__QT##QTV(                                            \
+      const uint8_t* raw, int N, int K, const uint32_t* tabs, const signed char* hq, const float* hsc, int S,           \
+      const int* tiles, const float* swt, float* y, const short* hbs, int gpw, int NE) {                                \
+    extern __shared__ __attribute__((aligned(16))) uint8_t mm_lds[];                                                    \
+    moe_down_mm<QTV>(mm_lds, raw, N, K, tabs, hq, hsc, hbs, S, tiles, swt, y, gpw, NE);                                 \
+  }
+MOE_MM(12, 4)
+MOE_MM(13, 4)
+MOE_MM(14, 2)
+MOE_MM(8, 4)
+MOE_MM(2, 4)
+MOE_MM(18, 4)
+MOE_MM(11, 2)
+MOE_MM(20, 4)
+MOE_MM(39, 4)
+MOE_MM(23, 4)
+MOE_MM(21, 4)

@@ -6,31 +6,22 @@
 
 #define ROUTE_PER_LANE 8
 
-// The better of two (value, expert) candidates: the larger value, the lower expert among equal values.
-__device__ inline void route_better(float& bv, int& bi, float ov, int oi) {
-  if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+// A logit as an unsigned key in the order of the values: 0 for what no round picks (-inf, NaN), both zeros alike.
+__device__ inline uint32_t route_key(float v) {
+  const uint32_t u = __float_as_uint(v + 0.0f);
+  return v > -INFINITY ? ((int)u < 0 ? ~u : u | 0x80000000u) : 0u;
 }
-// Wave arg-max of (bv, bi), the result in every lane: four steps inside each row of 16 lanes in the vector ALU (quad
-// swaps, then the row's mirrors: lanes that have met hold the same candidate, so a mirrored lane brings the other
-// group's), then the four rows' candidates read as scalars.  (Through the LDS crossbar the six dependent exchanges of
-// a round were most of a routing kernel's time.)
-__device__ inline void route_wave_best(float& bv, int& bi) {
-#define ROUTE_STEP(CTRL)                                                                             \
-  route_better(bv, bi, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(bv), CTRL, 0xF, 0xF, true)), \
-               __builtin_amdgcn_mov_dpp(bi, CTRL, 0xF, 0xF, true));
-  ROUTE_STEP(0xB1) ROUTE_STEP(0x4E) ROUTE_STEP(0x141) ROUTE_STEP(0x140)
+__device__ inline float route_unkey(uint32_t k) {
+  return k ? __uint_as_float((int)k < 0 ? k & 0x7FFFFFFFu : ~k) : -INFINITY;
+}
+// The wave's largest key, a scalar: six dependent maxima in the vector ALU (shifts inside the rows of 16 lanes, then each
+// row's last lane into the rows behind it), read from the last lane.
+__device__ inline uint32_t route_wave_max(uint32_t k) {
+#define ROUTE_STEP(CTRL, ROWS) k = max(k, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, CTRL, ROWS, 0xF, false));
+  ROUTE_STEP(0x111, 0xF) ROUTE_STEP(0x112, 0xF) ROUTE_STEP(0x114, 0xF) ROUTE_STEP(0x118, 0xF)  // row_shr 1, 2, 4, 8
+  ROUTE_STEP(0x142, 0xA) ROUTE_STEP(0x143, 0xC)                                                // row_bcast 15, 31
 #undef ROUTE_STEP
-  float rv[4];
-  int ri[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    rv[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bv), 16 * r));
-    ri[r] = __builtin_amdgcn_readlane(bi, 16 * r);
-  }
-  bv = rv[0];
-  bi = ri[0];
-#pragma unroll
-  for (int r = 1; r < 4; ++r) route_better(bv, bi, rv[r], ri[r]);
+  return (uint32_t)__builtin_amdgcn_readlane((int)k, 63);
 }
 
 // The reference's routing variants (zero/kernels/moe.cl:17-46), chosen per launch: escale (its -DESCALE, Gemma 4) -- each
@@ -44,36 +35,42 @@ struct RouteVariant {
 };
 __device__ inline float route_ds_sp(float g) { return sqrtf(g > 20.0f ? g + log1pf(expf(-g)) : log1pf(expf(g))); }
 
+// The choices one after the other: the largest key of the wave, and of the lanes that hold it the lowest expert, by a
+// ballot.  A round is a chain of about ten instructions -- with the (value, expert) pairs compared step by step, which it
+// was, 60 -- and the exponentials are taken once at the end, lane k its own; their sum in the order of the choices.
 template <int PL>
 __device__ inline void route_one_token_pl(const float* __restrict__ lg, int NE, int NU, int lane, int& sel, float& wt,
                                           const RouteVariant rv = RouteVariant()) {
-  float v[PL];
-  float mx = -INFINITY;
+  uint32_t key[PL];
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = i * 64 + lane;
-    v[i] = e < NE ? (rv.ebias ? route_ds_sp(lg[e]) + rv.ebias[e] : lg[e]) : -INFINITY;
-    mx = fmaxf(mx, v[i]);
+    key[i] = e < NE ? route_key(rv.ebias ? route_ds_sp(lg[e]) + rv.ebias[e] : lg[e]) : 0u;
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-  float sum = 0.0f, myp = 0.0f;
+  uint32_t mykey = 0, top = 0;
   int mysel = 0;
   for (int k = 0; k < NU; ++k) {
-    float bv = -INFINITY;
-    int bi = NE;
+    uint32_t mine = key[0];
+#pragma unroll
+    for (int i = 1; i < PL; ++i) mine = max(mine, key[i]);
+    const uint32_t m = route_wave_max(mine);
+    int bi = NE - 1;  // (nothing left to pick: keep the index inside the tables)
+    if (m) {
+#pragma unroll
+      for (int i = PL - 1; i >= 0; --i) {
+        const uint64_t has = __ballot(key[i] == m);
+        if (has) bi = i * 64 + __builtin_ctzll(has);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < PL; ++i)
-      if (v[i] > bv) { bv = v[i]; bi = i * 64 + lane; }
-    route_wave_best(bv, bi);
-#pragma unroll
-    for (int i = 0; i < PL; ++i)
-      if (i * 64 + lane == bi) v[i] = -INFINITY;
-    const int sk = min(bi, NE - 1);  // (a row of NaN picks no lane: keep the index inside the tables)
-    const float p = rv.ebias ? route_ds_sp(lg[sk]) : expf(bv - mx);
-    sum += p;
-    if (lane == k) { mysel = sk; myp = p; }
+      if (i * 64 + lane == bi) key[i] = 0;
+    if (k == 0) top = m;
+    if (lane == k) { mysel = bi; mykey = m; }
   }
+  const float myp = rv.ebias ? (lane < NU ? route_ds_sp(lg[mysel]) : 0.0f) : expf(route_unkey(mykey) - route_unkey(top));
+  float sum = 0.0f;
+  for (int k = 0; k < NU; ++k) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myp), k));
   sel = mysel;
   wt = rv.ebias ? myp / (sum + 1e-20f) * rv.rscale : myp / sum;
   if (rv.escale) wt *= rv.escale[mysel];

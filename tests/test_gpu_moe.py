@@ -113,6 +113,15 @@ def test_moe_small_pass_other_forms(rt, monkeypatch, env, qtype, NE, NU, E, F, T
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 16)
 
 
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q8_0, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q3_K, az.IQ3_S,
+                                   az.IQ3_XXS])
+@pytest.mark.parametrize("NE,NU,E,F,T", [(8, 4, 512, 256, 24), (16, 6, 256, 512, 9), (4, 4, 1280, 256, 12)])
+def test_moe_matrix_pipe_tiles_of_16_slots(rt, qtype, NE, NU, E, F, T):
+    """The passes between the one-slot kernels and the tile GEMM: experts with one slot, a few and more than a tile's 16,
+    rows of one superblock and of several, numbers of row groups that four a wave do not divide."""
+    _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 32)
+
+
 @pytest.mark.parametrize("env", [{}, {"ARCZ_MOE_QFUSE": "0"}, {"ARCZ_MOE_PRE": "0"}, {"ARCZ_MOE_PRE": "0", "ARCZ_MOE_QFUSE": "0"}])
 @pytest.mark.parametrize("NE,NU,E,F,T,Mp", [(16, 4, 512, 256, 300, 304), (8, 2, 256, 512, 70, 80), (8, 3, 256, 768, 90, 96)])
 def test_moe_tile_pass_quantization_forms(rt, monkeypatch, env, NE, NU, E, F, T, Mp):
