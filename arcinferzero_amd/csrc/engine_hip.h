@@ -307,6 +307,19 @@ class Engine {
         wsv_bytes_ = need;
       }
     }
+    if (rows == (size_t)N && digits_take(w.type, max_chunk, N)) {  // (room for its digits and the chunk's, gemm_digits)
+      const DigitForm f = digit_form(w.type);
+      const size_t tile = (size_t)(K / 32) * f.wimg;
+      const size_t need = std::max(tile, std::min((size_t)(N + 127) / 128 * tile, (size_t)512 << 20));
+      if (!xd_) xd_ = buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
+      if (need > wd_bytes_) {
+        if (wd_) release(wd_);
+        wd_ = nullptr;
+        wd_bytes_ = 0;
+        wd_ = buf(need);
+        wd_bytes_ = need;
+      }
+    }
     if (type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS) {  // (room for its GEMM form)
       const size_t need = raw_planes_bytes(QT_Q6_K, rows, K / 256);
       if (need > xw_bytes_) {
@@ -777,7 +790,91 @@ class Engine {
   // 0.401 -> 0.369 ms at 4096 tokens against the same in steps of 128 at two a unit, same bits.  The down projection's
   // kernel in that form -- 121 registers, four work-groups a compute unit -- was built and measured equal to its
   // three-a-unit form in steps of 128: 0.2275 against 0.2255 ms; not kept.)
+  // The GEMM on digits (gemm_d.hip): the chunk's digits, a matrix's (all its rows, or as many tiles of 128 as fit; sized when
+  // such a matrix is uploaded, never in a matmul)
+  cl_mem xd_ = nullptr, wd_ = nullptr;
+  size_t wd_bytes_ = 0;
+  struct DigitForm { int nw, timg, wimg; };  // (nw: digits of a weight, 0: not a type of this GEMM; bytes of the images)
+  static DigitForm digit_form(uint32_t type) {
+    const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS ? 2 : type == GGML_Q4_0 || type == GGML_MXFP4 || type == GGML_IQ3_S ? 1 : 0;
+    return {nw, nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512};
+  }
+  // Where it pays, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
+  // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43.4 / 42.5, 66 / 60, 109 / 79; Q4_0 30 / 35, 42 / 47,
+  // 80 / 64; MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70,
+  // MXFP4 84 / 69, IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows of 4096: Q6_K 98 / 108, 97.5 / 93.8 (of 2048),
+  // 277 / 263; IQ3_XXS 4096 x 4096, 1024 / 2048 tokens 77 / 79, 132 / 124.
+  bool digits_take(uint32_t type, int Mp, int N) const {
+    const double out = (double)Mp * N / (1 << 20);
+    if (Mp < 256) return false;
+    switch (type) {
+      case GGML_Q3_K: return out >= 1.0;
+      case GGML_Q4_0: case GGML_MXFP4: case GGML_IQ3_S: return out >= 3.0;
+      case GGML_Q6_K: return Mp >= 1024 && out >= 7.5;
+      case GGML_IQ3_XXS: return Mp >= 2048 && out >= 8.0;
+      default: return false;
+    }
+  }
+  // Pieces of K (1: none) with the lowest price: the partial tiles are written, read and summed at 5 TB/s; us per 1024 values of K and full round (two work-groups a compute unit) 20, 26, 34
+  // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 133 us.
+  static int digit_pieces(int nw, int Mp, int N, int nsb, size_t ws_bytes) {
+    const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
+    int best = 1;
+    double least = 0.0;
+    for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
+      if (ny > 1 && (size_t)ny * Mp * N * 4 > ws_bytes) break;
+      const size_t full = tiles * ny / (2 * cus), rest = tiles * ny % (2 * cus);
+      const double part = rest == 0 ? 0.0 : rest <= cus ? 0.63 : 1.0;
+      double us = (full + (full ? 0.85 : 1.0) * part) * (nw == 1 ? 20.0 : nw == 2 ? 26.0 : 34.0) * nsb / 4 / ny;
+      if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
+      if (ny == 1 || us < least) {
+        best = ny;
+        least = us;
+      }
+    }
+    return best;
+  }
+  void gemm_digits(const char* name, const GpuWeight& w, int Mp, cl_mem C, int ldc, int c_off, int a) {
+    const DigitForm f = digit_form(w.type);
+    int M = Mp, N = w.N, K = w.K, nsb = K / 256;
+    const int mt = (Mp + 127) / 128, nt_all = (N + 127) / 128;
+    const int panel = (int)std::min<size_t>((size_t)nt_all, wd_bytes_ / ((size_t)(K / 32) * f.wimg));
+    if (panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
+    size_t l[2] = {256, 1}, lg[2] = {512, 1};
+    {
+      cl_kernel k = kernel("gemm", "", "act_digits");
+      int img = f.timg;
+      set_args(k, 0, aq_, asc_, M, K, img, xd_);
+      size_t g[2] = {(size_t)nsb * 256, (size_t)mt * 2};
+      run("act_digits", k, 2, g, l);
+    }
+    for (int t0 = 0; t0 < nt_all; t0 += panel) {
+      int nt = std::min(panel, nt_all - t0), n0 = t0 * 128;
+      cl_kernel kr = kernel("gemm", "-DQTYPE=" + std::to_string(w.type), "row_digits");
+      set_args(kr, 0, w.raw, tabs_, N, nsb, n0, wd_);
+      size_t g[2] = {(size_t)nsb * 256, (size_t)nt * 2};
+      run("row_digits", kr, 2, g, l);
+      cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
+      cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
+      int ny = nt == nt_all ? digit_pieces(f.nw, Mp, N, nsb, noalloc_ ? arcz_mem_size(ws) : sk_ws_bytes_) : 1, zero = 0;
+      size_t gg[2] = {(size_t)mt * nt * 512, (size_t)ny};
+      if (ny > 1) set_args(k, 0, xd_, wd_, ws, M, N, K, N, zero, zero, n0, nt);
+      else set_args(k, 0, xd_, wd_, C, M, N, K, ldc, c_off, a, n0, nt);
+      run(name, k, 2, gg, lg);
+      if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
+    }
+  }
+  void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a) {
+    cl_kernel r = kernel("gemm", "", "splitk_reduce");
+    set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a);
+    size_t g1 = ((size_t)M * N + 255) / 256 * 256, l1 = 256;
+    run(name, r, 1, &g1, &l1);
+  }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
+    if (digits_take(w0.type, Mp, w0.N)) {
+      gemm_digits(name, w0, Mp, C, ldc, c_off, a);
+      return;
+    }
     const GpuWeight w = gemm_form(name, w0);
     int M = Mp, N = w.N, K = w.K;
     // Any type, a chunk so short that its tiles are fewer than two per compute unit: K is shared out over `ny`
@@ -824,11 +921,7 @@ class Engine {
         set_args(k, 0, w.raw, unused, aq_, asc_, absum_, ws, M, N, K, ldw, zero, zero, one, zero, s1);
         size_t gws[2] = {tiles64 * 256, (size_t)ny}, lws[2] = {256, 1};
         run(name, k, 2, gws, lws);
-        cl_kernel r = kernel("gemm", "", "splitk_reduce");
-        int nyy = ny;
-        set_args(r, 0, ws, nyy, C, M, N, ldc, c_off, a);
-        size_t g1 = ((size_t)M * N + 255) / 256 * 256, l1 = 256;
-        run(name, r, 1, &g1, &l1);
+        splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
         return;
       }
     }

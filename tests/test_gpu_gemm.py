@@ -249,6 +249,34 @@ def test_gemm_ready_made_scale_vectors(rt, monkeypatch, qtype, T, Mp, N, K, acc)
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("qtype,T,Mp,N,K,acc", [(az.Q3_K, 256, 256, 4096, 256, 0), (az.Q3_K, 300, 304, 3500, 1280, 1),
+                                                (az.Q4_0, 257, 260, 12289, 256, 0), (az.Q4_0, 1000, 1024, 3200, 768, 2),
+                                                (az.MXFP4, 385, 400, 8190, 512, 1), (az.IQ3_S, 390, 400, 8000, 1024, 0),
+                                                (az.Q6_K, 1030, 1040, 7700, 256, 0), (az.Q6_K, 1024, 1024, 7810, 768, 1),
+                                                (az.IQ3_XXS, 2049, 2052, 4100, 512, 0)])
+def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
+    """The GEMM of long chunks whose tokens and rows are written as digits first: one, two and three digits a weight, K
+    shared out and not, ragged last tiles of tokens and rows, one superblock and odd numbers of them, the three epilogues.
+    Against the oracle, and run to run."""
+    print(f"digits {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc}", flush=True)
+    eng = az.Engine(Mp, K)
+    W = make_weights(qtype, N, K, seed=81)
+    x = make_acts(T, K, seed=82, outliers=True)
+    c0 = np.random.default_rng(83).standard_normal((Mp, N)).astype(np.float32)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp, acc=acc, c_init=c0 if acc else None)[:T]
+    y2 = run_gemm(eng, qtype, W, N, K, x, Mp, acc=acc, c_init=c0 if acc else None)[:T]
+    eng.close()
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32))
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, W, N, K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    if acc == 1:
+        ref = ref + c0[:T]
+    elif acc == 2:
+        g = c0[:T].astype(np.float64)
+        ref = ref * (g / (1.0 + np.exp(-g)))
+    assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
+
+
 @pytest.mark.parametrize("T,Mp,N,K,acc", [(1100, 1104, 392, 512, 0), (1030, 1040, 640, 768, 1), (760, 768, 520, 1024, 2),
                                           (300, 304, 132, 256, 0), (2050, 2064, 136, 256, 1)])
 def test_gemm_tiles_of_256_tokens(rt, monkeypatch, T, Mp, N, K, acc):
