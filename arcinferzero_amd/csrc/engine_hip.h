@@ -815,7 +815,7 @@ class Engine {
       default: return false;
     }
   }
-  // Pieces of K (1: none) with the lowest price: the partial tiles are written, read and summed at 5 TB/s; us per 1024 values of K and full round (two work-groups a compute unit) 20, 26, 34
+  // Pieces of K, priced as in split_pieces: us per 1024 values of K and full round (two work-groups a compute unit) 20, 26, 34
   // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 133 us.
   static int digit_pieces(int nw, int Mp, int N, int nsb, size_t ws_bytes) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
@@ -870,6 +870,31 @@ class Engine {
     size_t g1 = ((size_t)M * N + 255) / 256 * 256, l1 = 256;
     run(name, r, 1, &g1, &l1);
   }
+  // Q8_0 and Q6_K, whose 64 x 128 tiles leave a chunk of some hundred tokens between one and three work-groups a compute
+  // unit: the pieces of K (1: none) with the lowest price.  In us and per 1024 values of K a full round of work-groups
+  // (three a unit for Q8_0, two for Q6_K) takes 21.2 and 24.7; a last round in which a unit has one work-group 0.46 or
+  // 0.62 of that, two of three 0.65, 0.85 of those behind a full round, whose end it overlaps.  The partial tiles are
+  // written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x both types this costs 0.5 % on
+  // average against always knowing (the rule before, three to eight pieces by the tile count alone, 9 %): 300 tokens Q6_K
+  // 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86, 4096 x 4096 x 512 39.3 -> 36.9.
+  static int split_pieces(uint32_t type, int Mp, int N, int nsb, size_t ws_bytes) {
+    const bool q8 = type == GGML_Q8_0;
+    const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)((Mp + 63) / 64) * ((N + 127) / 128);
+    int best = 1;
+    double least = 0.0;
+    for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
+      if (ny > 1 && (size_t)ny * Mp * N * 4 > ws_bytes) break;
+      const size_t full = tiles * ny / slots, rest = tiles * ny % slots;
+      const double part = rest == 0 ? 0.0 : rest <= cus ? (q8 ? 0.46 : 0.62) : rest <= 2 * cus ? (q8 ? 0.65 : 1.0) : 1.0;
+      double us = (full + (full ? 0.85 : 1.0) * part) * (q8 ? 21.2 : 24.7) * nsb / 4 / ny;
+      if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
+      if (ny == 1 || us < least) {
+        best = ny;
+        least = us;
+      }
+    }
+    return best;
+  }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
     if (digits_take(w0.type, Mp, w0.N)) {
       gemm_digits(name, w0, Mp, C, ldc, c_off, a);
@@ -895,9 +920,11 @@ class Engine {
       const int nsb = K / 256;
       const int sk_force = sk_force_;
       int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
+      const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
+      if (priced) ny = split_pieces(w.type, Mp, N, nsb, noalloc_ ? arcz_mem_size(arcz_scratch_mem()) : sk_ws_bytes_);
       if (sk_force >= 2) ny = std::min(sk_force, nsb);
-      // (from three pieces on: with two, 256 tiles of Q8_0 4096 x 4096 x 512 went from 50 to 54 us, the reduce included)
-      if (ny >= 3 || (sk_force >= 2 && ny >= 2)) {
+      // (the others from three pieces on)
+      if (ny >= (priced || sk_force >= 2 ? 2 : 3)) {
         const size_t need = (size_t)ny * Mp * N * 4;
         cl_mem ws = sk_ws_;
         if (noalloc_) {
