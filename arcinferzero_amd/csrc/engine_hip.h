@@ -800,10 +800,10 @@ class Engine {
     return {nw, nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512};
   }
   // Where it pays, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
-  // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43.4 / 42.5, 66 / 60, 109 / 79; Q4_0 30 / 35, 42 / 47,
-  // 80 / 64; MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70,
-  // MXFP4 84 / 69, IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows of 4096: Q6_K 98 / 108, 97.5 / 93.8 (of 2048),
-  // 277 / 263; IQ3_XXS 4096 x 4096, 1024 / 2048 tokens 77 / 79, 132 / 124.
+  // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43 / 42, 66 / 57, 109 / 75; Q4_0 30 / 35, 42 / 47, 80 / 64;
+  // MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70, MXFP4 84 / 69,
+  // IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows: Q6_K 98 / 103, 97.5 / 89 (of 2048), 277 / 234; IQ3_XXS 77 / 76,
+  // -, 193 / 186.
   bool digits_take(uint32_t type, int Mp, int N) const {
     const double out = (double)Mp * N / (1 << 20);
     if (Mp < 256) return false;
@@ -811,12 +811,12 @@ class Engine {
       case GGML_Q3_K: return out >= 1.0;
       case GGML_Q4_0: case GGML_MXFP4: case GGML_IQ3_S: return out >= 3.0;
       case GGML_Q6_K: return Mp >= 1024 && out >= 7.5;
-      case GGML_IQ3_XXS: return Mp >= 2048 && out >= 8.0;
+      case GGML_IQ3_XXS: return Mp >= 1024 && out >= 8.0;
       default: return false;
     }
   }
-  // Pieces of K, priced as in split_pieces: us per 1024 values of K and full round (two work-groups a compute unit) 20, 26, 34
-  // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 133 us.
+  // Pieces of K, priced as in split_pieces: us per 1024 values of K and full round (two work-groups a compute unit) 18, 25, 32
+  // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 123 us.
   static int digit_pieces(int nw, int Mp, int N, int nsb, size_t ws_bytes) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
     int best = 1;
@@ -825,7 +825,7 @@ class Engine {
       if (ny > 1 && (size_t)ny * Mp * N * 4 > ws_bytes) break;
       const size_t full = tiles * ny / (2 * cus), rest = tiles * ny % (2 * cus);
       const double part = rest == 0 ? 0.0 : rest <= cus ? 0.63 : 1.0;
-      double us = (full + (full ? 0.85 : 1.0) * part) * (nw == 1 ? 20.0 : nw == 2 ? 26.0 : 34.0) * nsb / 4 / ny;
+      double us = (full + (full ? 0.85 : 1.0) * part) * (nw == 1 ? 18.0 : nw == 2 ? 25.0 : 32.0) * nsb / 4 / ny;
       if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
       if (ny == 1 || us < least) {
         best = ny;
@@ -840,7 +840,7 @@ class Engine {
     const int mt = (Mp + 127) / 128, nt_all = (N + 127) / 128;
     const int panel = (int)std::min<size_t>((size_t)nt_all, wd_bytes_ / ((size_t)(K / 32) * f.wimg));
     if (panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
-    size_t l[2] = {256, 1}, lg[2] = {512, 1};
+    size_t l[2] = {256, 1};
     {
       cl_kernel k = kernel("gemm", "", "act_digits");
       int img = f.timg;
@@ -857,10 +857,10 @@ class Engine {
       cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
       int ny = nt == nt_all ? digit_pieces(f.nw, Mp, N, nsb, noalloc_ ? arcz_mem_size(ws) : sk_ws_bytes_) : 1, zero = 0;
-      size_t gg[2] = {(size_t)mt * nt * 512, (size_t)ny};
+      size_t gg[2] = {(size_t)mt * nt * 256, (size_t)ny};
       if (ny > 1) set_args(k, 0, xd_, wd_, ws, M, N, K, N, zero, zero, n0, nt);
       else set_args(k, 0, xd_, wd_, C, M, N, K, ldc, c_off, a, n0, nt);
-      run(name, k, 2, gg, lg);
+      run(name, k, 2, gg, l);
       if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
     }
   }

@@ -85,7 +85,7 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "act_digits", nullptr, "ppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits", nullptr, "ppiiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "gemm_d", nullptr, "pppiiiiiiii", {"NW", nullptr}, {{nullptr, 0, false}}, 512},
+    {"gemm", "gemm_d", nullptr, "pppiiiiiiii", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},

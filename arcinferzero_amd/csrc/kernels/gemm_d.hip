@@ -17,13 +17,13 @@
 // Q6_K and Q3_K, whose sub-scales hold for 16 values, have them folded into w ((q - 32) * sc, three digits; (q - 4) * sc, at
 // most 128, two), ws is d; the others' ws is their block scale: Q4_0, MXFP4 and IQ3_S are one digit, IQ3_XXS two.
 //
-// Bound by power: at 17408 x 5120 x 8192 the chip runs this kernel at 1.85 GHz, without its DMA at 2.1, and every part that
-// is taken out -- operand reads from LDS, DMA, multiply-adds -- gives back about its share of the energy, not of the
-// cycles.  Hence few bytes per product (the digits of a row are read once for two tiles, a type of fewer digits is
-// faster), and four waves a SIMD rather than two with twice the tile.  Kernel alone, 17408 x 5120 x 4096: one digit 765 -
-// 800 TOP/s, two 595, three 465 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650 and 375).
-// Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 149, MXFP4 183 / 147, IQ3_S
-// 201 / 160, Q3_K 293 / 203; x 4096: Q6_K 1094 / 901, IQ3_XXS 742 / 671.
+// Bound by power: at 17408 x 5120 x 8192 the chip runs this kernel below 1.9 GHz, without its DMA at 2.1, and every part
+// that is taken out -- operand reads from LDS, DMA, multiply-adds -- gives back about its share of the energy, not of the
+// cycles.  Hence few bytes and few instructions per product: a wave's operands serve 64 x 64 outputs, the addresses of a
+// step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 863 TOP/s, two 651, three
+// 504 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650 and 375).
+// Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 136, MXFP4 183 / 135, IQ3_S
+// 201 / 147, Q3_K 293 / 182, Q6_K 277 / 234; x 4096: Q6_K 1094 / 790, IQ3_XXS 742 / 596.
 #include "common.h"
 #include <type_traits>
 
@@ -266,12 +266,9 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
   }
 ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
 
-// A result leaves for good: stored past the caches, which keep the operands of the neighbouring tiles.
-__device__ inline void st_stream(float* p, float v) { __builtin_nontemporal_store(v, p); }
-
-// ---- gemm_d: 128 tokens x 128 rows in eight waves of 32 x 64, two work-groups a compute unit: four waves a SIMD, in 128
-// registers, so that a wave's waits -- for a product, for the next operands -- lie under the others' work.  Blocks [b0, b1),
-// an even number.
+// ---- gemm_d: 128 tokens x 128 rows in four waves of 64 x 64, two work-groups a compute unit.  Blocks [b0, b1), an even number.
+// (Eight waves of 32 x 64, four a SIMD, hide more waits and read each row digit from LDS twice as often: 5 - 6 % slower, at
+// 17408 x 5120 x 8192 812 against 863 TOP/s with one digit, 632 / 651 with two, 476 / 504 with three.)
 template <int NW>
 __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __restrict__ xt, const uint8_t* __restrict__ wt,
                                             float* __restrict__ C, int M, int N, int ldc, int c_off, int accumulate, int m0,
@@ -279,154 +276,157 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
   // (every access below is by offset; the array itself has to stay)
   asm volatile("" :: "v"((__attribute__((address_space(3))) uint8_t*)lds_base) : "memory");
   using I = DImg<NW>;
-  constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, KB = STAGE / 1024, TKB = NB * I::T / 1024, ND = (KB + 7) / 8;
+  constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, TS = NB * I::T, WS = NB * I::W;
+  constexpr int TKB = TS / 1024, KB = STAGE / 1024, ND = (KB + 3) / 4;
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave & 3, wn = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave & 1, wn = wave >> 1;
   const int steps = (b1 - b0) / NB;
-  const uint8_t* tsrc = xt + ((size_t)(m0 >> 7) * nblk + b0) * I::T;
-  const uint8_t* wsrc = wt + ((size_t)(n0 >> 7) * nblk + b0) * I::W;
+  const uint8_t* tsrc = xt + ((size_t)(m0 >> 7) * nblk + b0) * I::T + wave * 1024;
+  const uint8_t* wsrc = wt + ((size_t)(n0 >> 7) * nblk + b0) * I::W + wave * 1024 - TS;
   uint32_t lane16 = lane * 16;
-  // piece i of a step's DMA for this wave: KiB wave + 8 i of the stage
-  auto dma = [&](int step, uint32_t stage, int i) {
-    const int k = wave + 8 * i;
-    if (8 * i + 8 > KB && k >= KB) return;
-    const size_t off = k < TKB ? (size_t)(tsrc - xt) + (size_t)step * (NB * I::T) + k * 1024 : (size_t)step * (NB * I::W) + (k - TKB) * 1024;
-    const uint8_t* src = (k < TKB ? xt : wsrc) + off;
+  // piece i of a step's DMA for this wave: KiB wave + 4 i of the stage, tokens then rows
+  auto dma = [&](const uint8_t* ts, const uint8_t* ws, uint32_t stage, int i) {
+    if (4 * i + 4 > KB && wave >= (KB & 3)) return;
+    const uint8_t* src = 4 * i + 4 <= TKB || (4 * i < TKB && wave + 4 * i < TKB) ? ts : ws;
     asm volatile("" : "+v"(lane16));
-    dma16(src + lane16, stage + k * 1024);
+    dma16(src + i * 4096 + lane16, stage + wave * 1024 + i * 4096);
   };
   struct F6 { u4v lo; u2v hi; };
-  F6 A, W[NW];
-  float saop, wsop;
-  // (two lane offsets, the others formed where they are used: registers are the scarce thing)
-  auto low16 = [&]() { uint32_t r; asm volatile("v_and_b32 %0, 0x1f0, %1" : "=v"(r) : "v"(lane16)); return r; };  // 16 l32
-  auto shr = [](uint32_t o, auto n) { uint32_t r; asm volatile("v_lshrrev_b32 %0, %1, %2" : "=v"(r) : "i"(decltype(n)::value), "v"(o)); return r; };
-  constexpr std::integral_constant<int, 1> by2{};
-  constexpr std::integral_constant<int, 2> by4{};
-  const uint32_t tw = wm * 1024, rw = wn * 1024;
-  auto ldA = [&](uint32_t tb) {
-    A.lo = *LDS_P(const u4v, lane16 + (tb + tw));
-    A.hi = *LDS_P(const volatile u2v, shr(lane16, by2) + (tb + 4096 + tw / 2));
-    saop = *LDS_P(const float, shr(low16(), by4) + (tb + I::TSA + tw / 8));
+  F6 A[2], W[2][NW];
+  float saop[2], wsop;
+  // addresses of the step the loads are in: token digits, their second part, sa; row digits, second part, ws; the min term's
+  const uint32_t oA16 = wm * 2048 + lane * 16, oA8 = 4096 + wm * 1024 + lane * 8;
+  const uint32_t oW16 = TS + (wn * 64 + l32) * 16, oW8 = TS + 2048 + (wn * 64 + l32) * 8;
+  const uint32_t oSA = I::TSA + (wm * 64 + l32) * 4, oWS = TS + I::WWS + (wn * 64 + lane) * 4;
+  uint32_t pA16, pA8, pW16, pW8, pSA, pWS;
+  auto at = [&](uint32_t stage) {
+    pA16 = oA16 + stage; pA8 = oA8 + stage; pW16 = oW16 + stage; pW8 = oW8 + stage; pSA = oSA + stage; pWS = oWS + stage;
+    asm volatile("" : "+v"(pA16), "+v"(pA8), "+v"(pW16), "+v"(pW8), "+v"(pSA), "+v"(pWS));
   };
-  auto ldW = [&](int ns, uint32_t wb) {
-    const uint32_t l16 = low16(), o8 = shr(l16, by2) + (wb + rw / 2);
+  auto ldA = [&](int ms, int blk) {
+    A[ms].lo = *LDS_P(const u4v, pA16 + (NB == 2 ? blk : 0) * I::T + ms * 1024);
+    A[ms].hi = *LDS_P(const volatile u2v, pA8 + (NB == 2 ? blk : 0) * I::T + ms * 512);
+  };
+  auto ldW = [&](int ns, int blk) {
 #pragma unroll
     for (int d = 0; d < NW; ++d) {
-      W[d].lo = *LDS_P(const u4v, l16 + (wb + rw) + d * 3072 + ns * 512);
-      W[d].hi = *LDS_P(const volatile u2v, o8 + d * 3072 + 2048 + ns * 256);
+      W[ns][d].lo = *LDS_P(const u4v, pW16 + (NB == 2 ? blk : 0) * I::W + d * 3072 + ns * 512);
+      W[ns][d].hi = *LDS_P(const volatile u2v, pW8 + (NB == 2 ? blk : 0) * I::W + d * 3072 + ns * 256);
     }
-    if (ns == 0) wsop = *LDS_P(const float, shr(lane16, by4) + (wb + I::WWS + rw / 4));
   };
+  auto ldSA = [&](int ms, int blk) { saop[ms] = *LDS_P(const float, pSA + (NB == 2 ? blk : 0) * I::T + ms * 128); };
+  auto ldWS = [&](int blk) { wsop = *LDS_P(const float, pWS + (NB == 2 ? blk : 0) * I::W); };
   auto six = [](const F6& f) {
     const i4v a = __builtin_bit_cast(i4v, f.lo);
     const i2v b = __builtin_bit_cast(i2v, f.hi);
     return (i8v){a[0], a[1], a[2], a[3], b[0], b[1], 0, 0};
   };
-  // the scales: token digit g 2^3 or 2^7 (three digits: formed where they are used), row digit d 2^3, 2^7, 2^11, a byte each
-  auto scale_a = [&]() {
-    int v = g ? 134 : 130;
-    if constexpr (NW == 3) asm volatile("v_bfe_u32 %0, %1, 9, 1\n\tv_lshl_or_b32 %0, %0, 2, %2" : "=&v"(v) : "v"(lane16), "s"(130));
-    return v;
-  };
-  auto scale_b = []() {
-    int v = 0x008A8682;
-    if constexpr (NW == 3) asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "i"(0x008A8682));
-    return v;
-  };
-  v16f res[2];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) res[0][e] = res[1][e] = 0.0f;
-  auto product = [&]() {
-    v16f J;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) J[e] = 0.0f;
-    const int sca = scale_a(), scb = scale_b();
-    J = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A), six(W[0]), J, 2, 2, 0, sca, 0, scb);
-    if constexpr (NW > 1) J = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A), six(W[1]), J, 2, 2, 0, sca, 1, scb);
-    if constexpr (NW > 2) J = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A), six(W[2]), J, 2, 2, 0, sca, 2, scb);
-    return J;
-  };
+  const int sca = g ? 134 : 130, scb = 0x008A8682;  // token digit g 2^3 or 2^7; row digit d 2^3, 2^7, 2^11, a byte each
 
+  v16f res[2][2], J[2];
+  v32f P[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) res[i][0][e] = res[i][1][e] = J[i][e] = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 32; ++e) P[0][e] = P[1][e] = 0.0f;
+  auto mfma_p = [&](int ms) {
+    v32f z;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) z[e] = 0.0f;
+    P[ms] = __builtin_amdgcn_mfma_f32_32x32x1f32(saop[ms], wsop, z, 0, 0, 0);
+  };
   // ---- prologue: the first R - 1 steps on their way, the first block's operands
 #pragma unroll
   for (int q = 0; q < R - 1; ++q)
 #pragma unroll
-    for (int i = 0; i < ND; ++i) dma(min(q, steps - 1), q * STAGE, i);
+    for (int i = 0; i < ND; ++i) dma(tsrc + (size_t)min(q, steps - 1) * TS, wsrc + (size_t)min(q, steps - 1) * WS, q * STAGE, i);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  auto tok_of = [&](uint32_t stage, int blk) { return NB == 2 ? stage + blk * I::T : stage; };
-  auto row_of = [&](uint32_t stage, int blk) { return NB == 2 ? stage + NB * I::T + blk * I::W : stage + I::T; };
-  ldA(0); ldW(0, row_of(0, 0));
-  uint32_t st = 0;  // the step's stage
+  at(0);
+  ldA(0, 0); ldSA(0, 0);
+  ldW(0, 0); ldWS(0);
+  mfma_p(0);
+  ldSA(1, 0);
+  uint32_t st = 0;
   int step = 0;
-
+  uint32_t stf = (R - 2) * STAGE;  // (the first turn's first pieces: of a step that the prologue brought, once more)
+  const uint8_t *tf = tsrc + (size_t)min(R - 2, steps - 1) * TS, *wf = wsrc + (size_t)min(R - 2, steps - 1) * WS;
+  // Two blocks a turn, four products a block: tiles (0,0) (0,1) (1,1) (1,0), then (0,1) (0,0) (1,0) (1,1), so that the operands
+  // that come free first are those the next block begins with.  A product's values are added while the next one runs; a
+  // slot also carries a piece of the loads.  The stage of the step R - 1 on is refilled behind the meeting, when no wave
+  // reads the step before any more.
 #pragma unroll 1
   for (int b = b0; b < b1; b += 2) {
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      const uint32_t st1 = st + STAGE == R * STAGE ? 0 : st + STAGE;  // the next step's stage
-      const uint32_t stf = st == 0 ? (R - 1) * STAGE : st - STAGE;    // the stage of step R - 1 from here, which nobody reads any more
-      const bool last = NB == 1 || blk == 1;                          // the step's last block
-      const uint32_t cur_t = tok_of(st, blk), cur_w = row_of(st, blk);
-      const uint32_t nxt_t = last ? st1 : tok_of(st, 1), nxt_w = last ? row_of(st1, 0) : row_of(st, 1);
-      v32f P;
+    for (int p = 0; p < 8; ++p) {
+      const int blk = p >> 2, q = p & 3, ms = q >> 1, ns = blk ? (q == 0 || q == 3) : (q == 1 || q == 2);
+      // -- the product
+      {
+        v16f z;
 #pragma unroll
-      for (int e = 0; e < 32; ++e) P[e] = 0.0f;
-      P = __builtin_amdgcn_mfma_f32_32x32x1f32(saop, wsop, P, 0, 0, 0);
-      v16f J = product();
-      __builtin_amdgcn_sched_barrier(0);
-      ldW(1, cur_w);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) res[0][e] = __builtin_fmaf(P[e], J[e], res[0][e]);
-      asm volatile("" : "+v"(res[0]));
-      __builtin_amdgcn_sched_barrier(0);
-      J = product();
-      __builtin_amdgcn_sched_barrier(0);
-      if (last) {  // the meeting: what the waves brought for the next step lies in LDS, and the step before is read
+        for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+        v16f& j = J[p & 1];
+        j = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A[ms]), six(W[ns][0]), z, 2, 2, 0, sca, 0, scb);
+        if constexpr (NW > 1) j = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A[ms]), six(W[ns][1]), j, 2, 2, 0, sca, 1, scb);
+        if constexpr (NW > 2) j = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(six(A[ms]), six(W[ns][2]), j, 2, 2, 0, sca, 2, scb);
+      }
+      if (q == 1) mfma_p(1);
+      if (q == 3) mfma_p(0);
+      // -- the step's meeting: what the waves brought for the next step lies in LDS, the step before is read
+      if (NB == 2 ? p == 6 : q == 2) {
+        __builtin_amdgcn_sched_barrier(0);
         if (NB == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (ND == 3 && wave < (KB & 7)) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+        else if (wave < (KB & 3)) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        stf = st == 0 ? (R - 1) * STAGE : st - STAGE;
+        st = st + STAGE == R * STAGE ? 0 : st + STAGE;
+        at(st);
+        const int nf = min(step + R - 1, steps - 1);
+        tf = tsrc + (size_t)nf * TS; wf = wsrc + (size_t)nf * WS;
+        ++step;
       }
-      ldA(nxt_t); ldW(0, nxt_w);
-      if (last) {
-#pragma unroll
-        for (int i = 0; i < ND; ++i) dma(min(step + R - 1, steps - 1), stf, i);
+      // -- loads for later
+      const int nb = (p + 2) >> 2 & 1;  // (block of the loads below: from p == 2 the second, from 6 the next step's first)
+      if (q == 0) { ldW(blk ? 0 : 1, blk); ldA(1, blk); }
+      if (q == 2) { ldA(0, nb); ldSA(0, nb); ldWS(nb); }
+      if (q == 3) { ldW(blk ? 0 : 1, nb); ldSA(1, nb); }
+      {
+        // (two blocks a step: two pieces a slot, 6, 7 and, one turn on, 0, 1; one: three and two)
+        const int f = NB == 2 ? (p + 2 & 7) * 2 : q == 2 ? 0 : q == 3 ? 3 : ND;
+        if (f < ND) dma(tf, wf, stf, f);
+        if (f + 1 < ND) dma(tf, wf, stf, f + 1);
+        if (NB == 1 && q == 2) dma(tf, wf, stf, 2);
       }
       __builtin_amdgcn_sched_barrier(0);
+      // -- the values of the product before
+      {
+        const int pb = (p + 7) & 7, blp = pb >> 2, qp = pb & 3, mp = qp >> 1, np = blp ? (qp == 0 || qp == 3) : (qp == 1 || qp == 2);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) res[1][e] = __builtin_fmaf(P[16 + e], J[e], res[1][e]);
-      asm volatile("" : "+v"(res[1]));
+        for (int e = 0; e < 16; ++e) res[mp][np][e] = __builtin_fmaf(P[mp][16 * np + e], J[pb & 1][e], res[mp][np][e]);
+        asm volatile("" : "+v"(res[mp][np]));
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if (last) { st = st1; ++step; }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // the last product: tile (1, 1) of the second block
+#pragma unroll
+  for (int e = 0; e < 16; ++e) res[1][1][e] = __builtin_fmaf(P[1][16 + e], J[1][e], res[1][1][e]);
 
-  // ---- epilogue (its lane index from the one offset that was kept): lane = weight row n, accumulator i = token row 8 * (i / 4) + 4 * g + i % 4
+  // ---- epilogue: lane = weight row n, accumulator i = token row 8 * (i / 4) + 4 * g + i % 4
 #pragma unroll
-  for (int ns = 0; ns < 2; ++ns) {
-    const int el = (int)(lane16 >> 4), n = n0 + wn * 64 + ns * 32 + (el & 31);
-    if (n >= N) continue;
+  for (int ms = 0; ms < 2; ++ms)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = m0 + wm * 32 + 8 * (i >> 2) + 4 * (el >> 5) + (i & 3);
-      if (m >= M) continue;
-      float v = res[ns][i];
-      float* cp = C + (size_t)m * ldc + c_off + n;
-      if (accumulate == 1) {
-        v += *cp;
-      } else if (accumulate == 2) {
-        const float gt = *cp;
-        v *= gt / (1.0f + __expf(-gt));
-      }
-      st_stream(cp, v);
+    for (int ns = 0; ns < 2; ++ns) {
+      const int n = n0 + wn * 64 + ns * 32 + l32, m = m0 + wm * 64 + ms * 32 + 4 * g;
+      if (n >= N || m >= M) continue;
+      store16<true>(res[ms][ns], C + (size_t)m * ldc + c_off + n, ldc, M - m, accumulate, [](float v, int) { return v; });
     }
-  }
 }
 
 // Tile L of mt token tiles x nt row tiles: work-groups go to the eight chiplets in turn, so chiplet x takes the x-th eighth of
@@ -442,7 +442,7 @@ __device__ inline void d_tile_of(int id, int mt, int nt, int& tm, int& tn) {
 // gemm_d__NW: rows [n0, n0 + 128 ..) of an N-row matrix, nt row tiles of them in wt.  grid (ceil(M / 128) * nt, ny); ny > 1:
 // the superblocks shared out, plane y of C (here a workspace [ny][M][ldc]) the y-th piece's sums.
 #define GEMM_D(NWV)                                                                                                     \
-  extern "C" __global__ __launch_bounds__(512, 4) void gemm_d__NW##NWV(                                                 \
+  extern "C" __global__ __launch_bounds__(256, 2) void gemm_d__NW##NWV(                                                 \
       const uint8_t* xt, const uint8_t* wt, float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int n0, int nt) { \
     __shared__ __attribute__((aligned(1024))) uint8_t lds[DImg<NWV>::R * DImg<NWV>::STAGE];                             \
     int tm, tn;                                                                                                         \

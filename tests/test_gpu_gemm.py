@@ -253,7 +253,7 @@ def test_gemm_ready_made_scale_vectors(rt, monkeypatch, qtype, T, Mp, N, K, acc)
                                                 (az.Q4_0, 257, 260, 12289, 256, 0), (az.Q4_0, 1000, 1024, 3200, 768, 2),
                                                 (az.MXFP4, 385, 400, 8190, 512, 1), (az.IQ3_S, 390, 400, 8000, 1024, 0),
                                                 (az.Q6_K, 1030, 1040, 7700, 256, 0), (az.Q6_K, 1024, 1024, 7810, 768, 1),
-                                                (az.IQ3_XXS, 2049, 2052, 4100, 512, 0)])
+                                                (az.IQ3_XXS, 2049, 2052, 4100, 512, 0), (az.IQ3_XXS, 1025, 1040, 8100, 1024, 2)])
 def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
     """The GEMM of long chunks whose tokens and rows are written as digits first: one, two and three digits a weight, K
     shared out and not, ragged last tiles of tokens and rows, one superblock and odd numbers of them, the three epilogues.
