@@ -867,8 +867,8 @@ class Engine {
   void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a) {
     cl_kernel r = kernel("gemm", "", "splitk_reduce");
     set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a);
-    size_t g1 = ((size_t)M * N + 255) / 256 * 256, l1 = 256;
-    run(name, r, 1, &g1, &l1);
+    size_t g[2] = {(size_t)(N + 1023) / 1024 * 256, (size_t)M}, l[2] = {256, 1};
+    run(name, r, 2, g, l);
   }
   // Q8_0 and Q6_K, whose 64 x 128 tiles leave a chunk of some hundred tokens between one and three work-groups a compute
   // unit: the pieces of K (1: none) with the lowest price.  In us and per 1024 values of K a full round of work-groups

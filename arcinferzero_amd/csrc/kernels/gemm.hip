@@ -397,11 +397,6 @@ __device__ inline v8bf as_bf16x8(v4u v) { return __builtin_bit_cast(v8bf, v); }
 #define G3_WS (G3_SA + 4096)
 #define G3_V (G3_SA + 6144)
 
-// A result leaves for good: non-temporal stores keep the output (570 MB for 8192 tokens x 17408 rows, more than every
-// cache) from displacing the operands that the neighbouring tiles still read (8192 tokens: 707 -> 717 TOP/s).  (Not for
-// the expert tiles' y rows, which moe_combine reads right back: 56 -> 62 us there.)
-__device__ inline void st_stream(float* p, float v) { __builtin_nontemporal_store(v, p); }
-
 // (the 4-byte form: lane l's word lands at base + 4 l -- a gather of one value per lane)
 __device__ inline void g3_dma4(const void* src, uint8_t* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -842,21 +837,9 @@ __device__ __forceinline__ void gemm3_body(const uint8_t* __restrict__ raw, cons
     for (int ns = 0; ns < 2; ++ns) {
       const int n = n0 + wn * 64 + ns * 32 + l32;
       if (n >= N) continue;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = wm * 64 + ms * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-        if (r >= rows_valid) continue;
-        float v = res[ms][ns][i];
-        if (TILES && use_scale) v *= rowscale[m0 + r];
-        float* cp = C + (size_t)(m0 + r) * ldc + c_off + n;
-        if (accumulate == 1) {
-          v += *cp;
-        } else if (accumulate == 2) {
-          const float gt = *cp;
-          v *= gt / (1.0f + __expf(-gt));
-        }
-        st_stream(cp, v);
-      }
+      const int r0 = wm * 64 + ms * 32 + 4 * g;
+      store16<true>(res[ms][ns], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+                    [&](float v, int i) { return TILES && use_scale ? v * rowscale[m0 + r0 + 8 * (i >> 2) + (i & 3)] : v; });
     }
 }
 
@@ -1197,21 +1180,11 @@ __device__ __forceinline__ void gemm6_body(const uint8_t* __restrict__ raw, cons
   if (n < N) {
 #pragma unroll
     for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = ms * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-        if (r >= rows_valid) continue;
-        float v = res[ms][i];
-        if (TILES && use_scale) v *= rowscale[m0 + r];
-        float* cp = C + (size_t)(m0 + r) * ldc + c_off + n;
-        if (accumulate == 1) {
-          v += *cp;
-        } else if (accumulate == 2) {
-          const float gt = *cp;
-          v *= gt / (1.0f + __expf(-gt));
-        }
-        *cp = v;
-      }
+    {
+      const int r0 = ms * 32 + 4 * g;
+      store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+                     [&](float v, int i) { return TILES && use_scale ? v * rowscale[m0 + r0 + 8 * (i >> 2) + (i & 3)] : v; });
+    }
   }
 }
 
@@ -1470,21 +1443,11 @@ __device__ __forceinline__ void gemm4_body(const uint8_t* __restrict__ raw, cons
   if (n < N) {
 #pragma unroll
     for (int ms = 0; ms < (TWO ? 2 : 1); ++ms)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = ms * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-        if (r >= rows_valid) continue;
-        float v = res[ms][i];
-        if (use_scale) v *= rowscale[m0 + r];
-        float* cp = C + (size_t)(m0 + r) * ldc + c_off + n;
-        if (accumulate == 1) {
-          v += *cp;
-        } else if (accumulate == 2) {
-          const float gt = *cp;
-          v *= gt / (1.0f + __expf(-gt));
-        }
-        *cp = v;
-      }
+    {
+      const int r0 = ms * 32 + 4 * g;
+      store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+                     [&](float v, int i) { return use_scale ? v * rowscale[m0 + r0 + 8 * (i >> 2) + (i & 3)] : v; });
+    }
   }
 }
 
@@ -1741,20 +1704,11 @@ __device__ __forceinline__ void gemm4gu_body(const uint8_t* __restrict__ rg, con
       if (n >= N) continue;
 #pragma unroll
       for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int r = ms * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-          if (r >= rows_valid) continue;
-          float v = res[x][ms][i];
-          float* cp = H + (size_t)(m0 + r) * ldc + c_off + n;
-          if (accumulate == 1) {
-            v += *cp;
-          } else if (accumulate == 2) {
-            const float gt = *cp;
-            v *= gt / (1.0f + __expf(-gt));
-          }
-          *cp = v;
-        }
+      {
+        const int r0 = ms * 32 + 4 * g;
+        store16<false>(res[x][ms], H + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+                       [](float v, int) { return v; });
+      }
     }
   }
 }
@@ -2106,20 +2060,11 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
   if (n < N) {
 #pragma unroll
     for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = ms * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-        if (r >= rows_valid) continue;
-        float v = res[ms][i];
-        float* cp = C + (size_t)(m0 + r) * ldc + c_off + n;
-        if (accumulate == 1) {
-          v += *cp;
-        } else if (accumulate == 2) {
-          const float gt = *cp;
-          v *= gt / (1.0f + __expf(-gt));
-        }
-        *cp = v;
-      }
+    {
+      const int r0 = ms * 32 + 4 * g;
+      store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+                     [](float v, int) { return v; });
+    }
   }
 }
 
@@ -2355,23 +2300,31 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE13_ACT321_BM128_
   gemm3_body<false, QT_Q5_K>(raw, aq, asc, absum, C + (size_t)y * M * ldc, M, N, K, ldc, 0, 0, s_begin + ns * y / ny,
                              s_begin + ns * (y + 1) / ny, (size_t)N, 0, m0, min(BM, M - m0), n0, nullptr, 0, nullptr, 0);
 }
-// splitk_reduce: C[m][c_off + n] (=, +=, silu(C) *) sum over the ny slices of ws [ny][M][N], slice 0 first.
-// grid: ceil(M * N / 256) work-groups of 256.
+// splitk_reduce: C[m][c_off + n] (=, +=, silu(C) *) sum over the ny slices of ws [ny][M][N], slice 0 first.  A thread takes
+// four columns of a row (whole vectors where the strides allow).  grid (ceil(N / 1024) work-groups of 256, M).
 extern "C" __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ ws, int ny, float* C, int M, int N,
                                                                 int ldc, int c_off, int accumulate) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, total = (size_t)M * N;
-  if (i >= total) return;
-  float v = ws[i];
-  for (int y = 1; y < ny; ++y) v += ws[(size_t)y * total + i];
-  const size_t m = i / (size_t)N, n = i - m * (size_t)N;
-  float* cp = C + m * ldc + c_off + n;
-  if (accumulate == 1) {
-    v += *cp;
-  } else if (accumulate == 2) {
-    const float gt = *cp;
-    v *= gt / (1.0f + __expf(-gt));
+  const int n = (blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+  if (n >= N) return;
+  const float* w = ws + (size_t)m * N + n;
+  float* c = C + (size_t)m * ldc + c_off + n;
+  const size_t plane = (size_t)M * N;
+  auto put = [&](float v, float old) { return accumulate == 1 ? v + old : accumulate == 2 ? v * (old / (1.0f + __expf(-old))) : v; };
+  if (((N | ldc | c_off) & 3) == 0) {
+    const float4 old = accumulate ? *(const float4*)c : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 v = *(const float4*)w;
+    for (int y = 1; y < ny; ++y) {
+      const float4 f = *(const float4*)(w + y * plane);
+      v.x += f.x; v.y += f.y; v.z += f.z; v.w += f.w;
+    }
+    *(float4*)c = make_float4(put(v.x, old.x), put(v.y, old.y), put(v.z, old.z), put(v.w, old.w));
+  } else {
+    for (int k = 0; k < min(4, N - n); ++k) {
+      float v = w[k];
+      for (int y = 1; y < ny; ++y) v += w[y * plane + k];
+      c[k] = put(v, accumulate ? c[k] : 0.0f);
+    }
   }
-  *cp = v;
 }
 // -DBM=64: the 64-token form (grid ceil(N / 128) * ceil(M / 64) work-groups)
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64(
