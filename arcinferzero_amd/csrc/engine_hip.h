@@ -864,8 +864,8 @@ class Engine {
       if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
     }
   }
-  void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a) {
-    cl_kernel r = kernel("gemm", "", "splitk_reduce");
+  void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a, int rows = 0) {
+    cl_kernel r = kernel("gemm", rows ? "-DMV=" + std::to_string(rows) : std::string(), "splitk_reduce");
     set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a);
     size_t g[2] = {(size_t)(N + 1023) / 1024 * 256, (size_t)M}, l[2] = {256, 1};
     run(name, r, 2, g, l);
@@ -877,9 +877,9 @@ class Engine {
   // written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x both types this costs 0.5 % on
   // average against always knowing (the rule before, three to eight pieces by the tile count alone, 9 %): 300 tokens Q6_K
   // 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86, 4096 x 4096 x 512 39.3 -> 36.9.
-  static int split_pieces(uint32_t type, int Mp, int N, int nsb, size_t ws_bytes) {
+  static int split_pieces(uint32_t type, int Mp, int m64, int N, int nsb, size_t ws_bytes) {
     const bool q8 = type == GGML_Q8_0;
-    const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)((Mp + 63) / 64) * ((N + 127) / 128);
+    const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)m64 * ((N + 127) / 128);
     int best = 1;
     double least = 0.0;
     for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
@@ -902,6 +902,8 @@ class Engine {
     }
     const GpuWeight w = gemm_form(name, w0);
     int M = Mp, N = w.N, K = w.K;
+    // (the 64-token tiles that hold a token: the others are padding, whose results are zeros)
+    const int m64 = (std::clamp(cur_T_, 1, Mp) + 63) / 64, M64 = std::min(Mp, m64 * 64);
     // Any type, a chunk so short that its tiles are fewer than two per compute unit: K is shared out over `ny`
     // work-groups per tile, which store partial tiles in a workspace, and splitk_reduce adds the slices in order (the
     // same bits on every run) and applies c_off and the accumulate mode.  One work-group needs 75 us for K = 5120, so
@@ -916,12 +918,12 @@ class Engine {
       const int bm = tm == 64 && q45 && Mp <= 32 ? 32 : tm;  // (Q4_K / Q5_K, at most 32 rows: the one-slot-tile kernel)
       // (the one-slot-tile kernel is light enough for three work-groups a compute unit: 17408 x 5120, 32 tokens, 3 pieces
       //  of K 30.0 us, 5 pieces 28.3)
-      const size_t tiles64 = (size_t)((Mp + tm - 1) / tm) * ((N + 127) / 128), slots = (bm == 32 ? 3 : 2) * (size_t)arcz_device_cus();
+      const size_t tiles64 = (size_t)(tm == 64 && !q45 ? m64 : (Mp + tm - 1) / tm) * ((N + 127) / 128), slots = (bm == 32 ? 3 : 2) * (size_t)arcz_device_cus();
       const int nsb = K / 256;
       const int sk_force = sk_force_;
       int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
       const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
-      if (priced) ny = split_pieces(w.type, Mp, N, nsb, noalloc_ ? arcz_mem_size(arcz_scratch_mem()) : sk_ws_bytes_);
+      if (priced) ny = split_pieces(w.type, Mp, m64, N, nsb, noalloc_ ? arcz_mem_size(arcz_scratch_mem()) : sk_ws_bytes_);
       if (sk_force >= 2) ny = std::min(sk_force, nsb);
       // (the others from three pieces on)
       if (ny >= (priced || sk_force >= 2 ? 2 : 3)) {
@@ -948,7 +950,7 @@ class Engine {
         set_args(k, 0, w.raw, unused, aq_, asc_, absum_, ws, M, N, K, ldw, zero, zero, one, zero, s1);
         size_t gws[2] = {tiles64 * 256, (size_t)ny}, lws[2] = {256, 1};
         run(name, k, 2, gws, lws);
-        splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
+        splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a, priced && M64 < Mp ? M64 : 0);
         return;
       }
     }
@@ -1002,7 +1004,7 @@ class Engine {
     if (t64 && q4_wm_ == 0) {
       const size_t cus = (size_t)arcz_device_cus(), nt = (size_t)(N + 127) / 128;
       const size_t t128 = (size_t)((Mp + 127) / 128) * nt, s128 = 2 * cus, r128 = t128 % s128;
-      const size_t t64n = (size_t)((Mp + 63) / 64) * nt, s64 = 3 * cus, r64 = t64n % s64;
+      const size_t t64n = (size_t)m64 * nt, s64 = 3 * cus, r64 = t64n % s64;
       const double c128 = (double)(t128 / s128) + (r128 == 0 ? 0.0 : 2 * r128 <= s128 ? 0.5 : 1.0);
       const double c64 = 0.8 * (double)(t64n / s64) + (r64 == 0 ? 0.0 : 3 * r64 <= s64 ? 0.30 : 3 * r64 <= 2 * s64 ? 0.48 : 0.8);
       t64 = c64 < 0.97 * c128;
@@ -1021,7 +1023,7 @@ class Engine {
       cl_kernel k = kernel("gemm", "-DQTYPE=12 -DACT32 -DBM=64 -DBN=128 -DPRE64=1", "gemm");
       int rgroup = 1, s0 = 0, s1 = K / 256;
       set_args(k, 0, w.raw, au_, aq_, asc_, wsv_, C, M, N, K, ldc, c_off, a, rgroup, s0, s1);
-      size_t gws[1] = {(size_t)((Mp + 63) / 64) * ((N + 127) / 128) * 256}, lws[1] = {256};
+      size_t gws[1] = {(size_t)m64 * ((N + 127) / 128) * 256}, lws[1] = {256};
       run(name, k, 1, gws, lws);
       return;
     }
@@ -1039,7 +1041,8 @@ class Engine {
     cl_mem unused = nullptr;
     const int bm = wm4 ? 256 : w.type == GGML_Q6_K || q8_small || q4_wide || q4_small ? 64 : 128;  // token rows of a work-group's tile
     const int bn = q4_wide && !q4_small ? 256 : 128;
-    const size_t tiles = (size_t)((Mp + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const bool m64_only = bm == 64 && (w.type == GGML_Q6_K || q8_small);
+    const size_t tiles = (size_t)(m64_only ? m64 : (Mp + bm - 1) / bm) * ((N + bn - 1) / bn);
     const size_t wg = wm4 ? 512 : 256;
     size_t gws[1] = {tiles * wg}, lws[1] = {wg};
     if (au) {

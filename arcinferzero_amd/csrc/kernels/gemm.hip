@@ -2068,6 +2068,15 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
   }
 }
 
+// A chunk laid out for M token rows whose last ones are padding: a launch of the 64-token tiles may leave out the tiles that
+// hold nothing else (their count comes from the grid).  The work-groups of the last tile then write the padding rows'
+// results, zeros where a product is stored or multiplied in; one that is added changes nothing.
+__device__ inline void zero_tail(float* C, int ldc, int c_off, int accumulate, int r0, int M, int n0, int N) {
+  if (accumulate == 1) return;
+  for (int i = threadIdx.x; i < (M - r0) * 128; i += 256)
+    if (n0 + (i & 127) < N) C[(size_t)(r0 + (i >> 7)) * ldc + c_off + n0 + (i & 127)] = 0.0f;
+}
+
 // Tile of work-group `id` out of mt x nt tiles.  XCDs take work-groups in turn (id % 8), each running 64 at a time:
 // those 64 are made an 8 x 8 block of tiles when both tile counts are multiples of 8 and the blocks share out evenly
 // over the 8 XCDs.  Any other shape: the tiles are put in the order "panels of 8 token tiles; within a panel row tile
@@ -2168,10 +2177,11 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE12_ACT321_BM64_B
 extern "C" __global__ __launch_bounds__(256, 3) void gemm__QTYPE12_ACT321_BM64_BN128_PRE641(
     const uint8_t* raw, const float* au, const signed char* aq, const float* asc, const float* wsv, float* C, int M, int N,
     int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
-  const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
+  if (tm == mt - 1) zero_tail(C, ldc, c_off, accumulate, mt * G6_BM, M, n0, N);
   gemm4_body<true, QT_Q4_K, true>(raw, aq, asc, nullptr, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, (size_t)N, 0, m0,
                                   min(G6_BM, M - m0), n0, nullptr, 0, nullptr, 0, au, wsv);
 }
@@ -2236,7 +2246,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE12_ACT321_BM128_
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64_BN128_SPLITK1(
     const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum, float* C,
     int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
-  const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
@@ -2248,7 +2258,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64_BN
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321_BM64_BN128_SPLITK1(
     const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum, float* C,
     int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
-  const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
@@ -2261,7 +2271,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321_BM64_B
   extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321_BM64_BN128_SPLITK1_HDS##HDV(               \
       const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum,      \
       float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {        \
-    const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;                                                   \
+    const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;                                                            \
     int tm, tn;                                                                                                       \
     tile_of(blockIdx.x, mt, nt, tm, tn);                                                                              \
     const int m0 = tm * G6_BM, n0 = tn * BN;                                                                          \
@@ -2301,27 +2311,29 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE13_ACT321_BM128_
                              s_begin + ns * (y + 1) / ny, (size_t)N, 0, m0, min(BM, M - m0), n0, nullptr, 0, nullptr, 0);
 }
 // splitk_reduce: C[m][c_off + n] (=, +=, silu(C) *) sum over the ny slices of ws [ny][M][N], slice 0 first.  A thread takes
-// four columns of a row (whole vectors where the strides allow).  grid (ceil(N / 1024) work-groups of 256, M).
+// four columns of a row (whole vectors where the strides allow).  Rows from MV on (0: none): zero sums, no partial tile
+// holds them.  grid (ceil(N / 1024) work-groups of 256, M).
 extern "C" __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ ws, int ny, float* C, int M, int N,
-                                                                int ldc, int c_off, int accumulate) {
+                                                                int ldc, int c_off, int accumulate, int MV) {
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
   if (n >= N) return;
   const float* w = ws + (size_t)m * N + n;
   float* c = C + (size_t)m * ldc + c_off + n;
   const size_t plane = (size_t)M * N;
+  const bool in = MV == 0 || m < MV;
   auto put = [&](float v, float old) { return accumulate == 1 ? v + old : accumulate == 2 ? v * (old / (1.0f + __expf(-old))) : v; };
   if (((N | ldc | c_off) & 3) == 0) {
     const float4 old = accumulate ? *(const float4*)c : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float4 v = *(const float4*)w;
-    for (int y = 1; y < ny; ++y) {
+    float4 v = in ? *(const float4*)w : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int y = 1; y < ny && in; ++y) {
       const float4 f = *(const float4*)(w + y * plane);
       v.x += f.x; v.y += f.y; v.z += f.z; v.w += f.w;
     }
     *(float4*)c = make_float4(put(v.x, old.x), put(v.y, old.y), put(v.z, old.z), put(v.w, old.w));
   } else {
     for (int k = 0; k < min(4, N - n); ++k) {
-      float v = w[k];
-      for (int y = 1; y < ny; ++y) v += w[y * plane + k];
+      float v = in ? w[k] : 0.0f;
+      for (int y = 1; y < ny && in; ++y) v += w[y * plane + k];
       c[k] = put(v, accumulate ? c[k] : 0.0f);
     }
   }
@@ -2330,10 +2342,11 @@ extern "C" __global__ __launch_bounds__(256) void splitk_reduce(const float* __r
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64(
     const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum, float* C,
     int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
-  const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
+  if (tm == mt - 1) zero_tail(C, ldc, c_off, accumulate, mt * G6_BM, M, n0, N);
   gemm8_body(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0), n0);
 }
 
@@ -2478,10 +2491,11 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE13_ACT321_MOE_TI
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321(
     const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum, float* C,
     int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
-  const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
+  if (tm == mt - 1) zero_tail(C, ldc, c_off, accumulate, mt * G6_BM, M, n0, N);
   gemm6_body<false>(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0), n0);
 }
 // (-DHD=1 / 2, -DHDT=1 / 2: planes written out from IQ3_XXS / IQ3_S, gemm6_body<..., HD>)
@@ -2489,10 +2503,11 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321(
   extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE14_ACT321_HD##HDV(                                   \
       const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum,      \
       float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {        \
-    const int mt = (M + G6_BM - 1) / G6_BM, nt = (N + BN - 1) / BN;                                                   \
+    const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt;                                                            \
     int tm, tn;                                                                                                       \
     tile_of(blockIdx.x, mt, nt, tm, tn);                                                                              \
     const int m0 = tm * G6_BM, n0 = tn * BN;                                                                          \
+    if (tm == mt - 1) zero_tail(C, ldc, c_off, accumulate, mt * G6_BM, M, n0, N);                                     \
     gemm6_body<false, HDV>(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0),   \
                            n0);                                                                                       \
   }                                                                                                                   \

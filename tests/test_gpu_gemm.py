@@ -249,6 +249,30 @@ def test_gemm_ready_made_scale_vectors(rt, monkeypatch, qtype, T, Mp, N, K, acc)
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("qtype,T,Mp,N,K", [(az.Q6_K, 257, 384, 1000, 768), (az.Q6_K, 130, 256, 392, 2048), (az.Q8_0, 300, 384, 520, 4096),
+                                            (az.Q8_0, 129, 256, 3000, 512), (az.Q4_K, 300, 384, 5200, 512), (az.IQ3_S, 257, 384, 1000, 512)])
+@pytest.mark.parametrize("acc", [0, 1, 2])
+def test_gemm_padding_rows(rt, qtype, T, Mp, N, K, acc):
+    """Token tiles that hold padding alone are left out of the launch: the rows from T on come out as the products of zero
+    rows all the same (zeros, or what was there), with K shared out and not."""
+    print(f"padding rows {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc}", flush=True)
+    eng = az.Engine(Mp, K)
+    W = make_weights(qtype, N, K, seed=85)
+    x = make_acts(T, K, seed=86, outliers=True)
+    c0 = np.random.default_rng(87).standard_normal((Mp, N)).astype(np.float32)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp, acc=acc, c_init=c0)
+    eng.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, W, N, K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    if acc == 1:
+        ref = ref + c0[:T]
+    elif acc == 2:
+        g = c0[:T].astype(np.float64)
+        ref = ref * (g / (1.0 + np.exp(-g)))
+    assert np.isfinite(y).all() and mixed_err(y[:T], ref) <= TOL
+    assert np.array_equal(y[T:], c0[T:] if acc == 1 else np.zeros((Mp - T, N), np.float32))
+
+
 @pytest.mark.parametrize("qtype,T,Mp,N,K,acc", [(az.Q3_K, 256, 256, 4096, 256, 0), (az.Q3_K, 300, 304, 3500, 1280, 1),
                                                 (az.Q4_0, 257, 260, 12289, 256, 0), (az.Q4_0, 1000, 1024, 3200, 768, 2),
                                                 (az.MXFP4, 385, 400, 8190, 512, 1), (az.IQ3_S, 390, 400, 8000, 1024, 0),
