@@ -585,12 +585,15 @@ class Engine {
     // A few tokens, any weight type: the matrix-vector form on the matrix pipe (gemv_mm; it
     // takes K in slices of the tokens that fit LDS).  It takes 9-16 tokens in chunks of 16 rows (what the reference pads
     // them to, zero/engine.h:522; the rows from T on come out as zeros, as the GEMM writes them: Q4_K 21 against 95 us at
-    // 17408 x 5120), and 3-8 tokens where it is the faster one: from 5 on always (us at the settled clock, 8 tokens,
-    // against the dot-product kernels, 17408 x 5120: Q4_K 20.8 / 27.6, Q5_K 21.5 / 30.5, Q6_K 31.0 / 33.1, Q8_0 23.7 /
-    // 31.4, Q4_0 20.2 / 27.7, IQ4_XS 23.4 / 31.0, IQ3_S 26.4 / 32.9; with 4 tokens 20.5 / 18.9, 21.4 / 20.7, 30.8 / 23.2, 23.6 / 20.1,
-    // 20.4 / 17.1, 23.3 / 20.0: not taken; ARCZ_GEMV_MM_MIN: the first count it takes), 3 and 4 when the tokens do not
-    // fit the LDS of the dot-product kernels (5120 x 17408, 4 tokens: Q4_K 34 against 88 us, Q5_K 42 against 97).  Not
-    // with two-pass inputs (their second half goes through the kernels below).  ARCZ_GEMV_MM=0: off.
+    // 17408 x 5120), and 3-8 tokens where it is the faster one.  From 5 on, us for 8 tokens against the dot-product kernels:
+    // 17408 x 5120 Q4_K 17.4 / 27.6, Q5_K 19.2 / 30.5, Q6_K 20.8 / 33.1, Q8_0 21.7 / 31.4, Q4_0 16.7 / 27.7, IQ4_XS 20.2 /
+    // 31.0; 8192 x 5120 Q4_K 11.3 / 15.3; 4096 x 4096 Q4_K 8.3 / 10.8, Q6_K 8.7 / 9.1, Q8_0 11.8 / 9.1, IQ4_XS 8.6 / 12.3;
+    // 1024 x 4096 8.0 / 7.5, 8.5 / 6.9, 8.0 / 6.2, 8.4 / 8.9; 2048 x 2048 7.7 / 5.2, 7.7 / 6.0, 7.8 / 5.7, 7.7 / 5.7: not for
+    // matrices of few values (its stagings and meetings take longer than the weights), for Q8_0 not for few rows.  With 3
+    // and 4 tokens when they do not fit the LDS of the dot-product kernels, and, 17408 x 5120, Q4_K 17.3 / 18.2, Q5_K 18.9 /
+    // 20.1, Q6_K 21.1 / 22.0, for large matrices of these types (Q8_0 21.6 / 18.0, IQ4_XS 20.3 / 19.9: not).
+    // ARCZ_GEMV_MM_MIN: the first count it takes.  Not with two-pass inputs (their second half goes through the kernels
+    // below).  ARCZ_GEMV_MM=0: off.
     static const bool mm_off = getenv("ARCZ_GEMV_MM") && atoi(getenv("ARCZ_GEMV_MM")) == 0;
     const bool mm_type = w.type == GGML_Q4_K || w.type == GGML_Q5_K || w.type == GGML_Q6_K || w.type == GGML_Q8_0 ||
                          w.type == GGML_Q4_0 || w.type == GGML_IQ4_XS || w.type == GGML_IQ3_S || w.type == GGML_IQ4_NL ||
@@ -599,7 +602,9 @@ class Engine {
     auto gemv_mm = [&] {
       int N = w.N, K = w.K, M = Mp, T = cur_T_;
       rd_bytes += raw_bytes(w);
-      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(w.type), "gemv_mm");
+      // (the form for at most eight tokens; the three-bit types have the one form)
+      const bool t8 = T <= 8 && w.type != GGML_IQ3_S && w.type != GGML_Q3_K && w.type != GGML_IQ3_XXS;
+      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(w.type) + (t8 ? " -DT8=1" : ""), "gemv_mm");
       const size_t groups = (size_t)(N + 15) / 16, cus = (size_t)arcz_device_cus();
       // Rows longer than the tokens' LDS holds (slices of sb_max superblocks): K is shared out over `ny` work-groups
       // per run of groups, each staging its piece of the tokens once, and gemv_mm_reduce adds the pieces -- inside one
@@ -679,7 +684,11 @@ class Engine {
       // (IQ3_S: 2 KiB of the work-group's LDS hold the codebook)
       const size_t lds_max = w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536;
       const bool fits = !force_v && lpr && lds <= lds_max;
-      static const int mm_min = getenv("ARCZ_GEMV_MM_MIN") ? atoi(getenv("ARCZ_GEMV_MM_MIN")) : 5;
+      static const int mm_env = getenv("ARCZ_GEMV_MM_MIN") ? atoi(getenv("ARCZ_GEMV_MM_MIN")) : 0;
+      const double mvals = (double)N * K / (1 << 20);
+      const bool mm_few = mvals <= 4.5 || (w.type == GGML_Q8_0 && N <= 4096 && mvals <= 17.0);
+      const bool mm_large = mvals >= 64.0 && (w.type == GGML_Q4_K || w.type == GGML_Q5_K || w.type == GGML_Q6_K);
+      const int mm_min = mm_env ? mm_env : mm_few ? 9 : mm_large ? 3 : 5;
       if (mm_ok && T >= 3 && (T >= mm_min || !fits)) {
         rd_bytes -= raw_bytes(w);  // (counted by gemv_mm)
         gemv_mm();

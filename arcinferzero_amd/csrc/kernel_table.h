@@ -52,6 +52,7 @@ static const KernelSpec kKernelTable[] = {
     {"decode", "gemv_mt", nullptr, "piippppiipiii", {"QT", "LPR", "PF", "TB", nullptr},
      {{"LDS", 0, true}, {"Q2_AQ", 0, false}, {"Q2_SC", 0, false}, {"SOFTCAP", 0, false}, {"SCHED", -1, false}, {nullptr, 0, false}}, 256},
     {"decode", "gemv_mm_reduce", nullptr, "pipiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"decode", "gemv_mm", "T8", "piippppiipiiiii", {"QT", "T8", nullptr}, {{nullptr, 0, false}}, 512},
     {"decode", "gemv_mm", nullptr, "piippppiipiiiii", {"QT", nullptr}, {{nullptr, 0, false}}, 512},
     {"decode", "moe_gateup_mm", nullptr, "ppiipppippppippp", {"QT", nullptr}, {{"NE", 0, true}, {"LDS", 0, true}, {nullptr, 0, false}}, 512},
     {"decode", "moe_down_mm", nullptr, "piipppippppi", {"QT", nullptr}, {{"NE", 0, true}, {"LDS", 0, true}, {nullptr, 0, false}}, 512},

@@ -96,6 +96,13 @@ template <int QT> struct MmSb {
   uint32_t d;
   mm_u4 sg[QT == QT_IQ3_S || QT == QT_Q3_K || QT == QT_IQ3_XXS ? 2 : 1];
 };
+// ... and as those of at most eight tokens take it: 16 bytes a lane
+template <int QT> struct MmSb8 {
+  mm_u4 c[4], h, x[2];
+  uint32_t q5[4], d;
+};
+// The types with products of their own for at most eight tokens (mm_slice, T8).
+constexpr bool mm_t8(int qt) { return qt != QT_IQ3_S && qt != QT_Q3_K && qt != QT_IQ3_XXS; }
 
 // The rows a work-group multiplies, one slice of K at a time: ng groups of 16 rows, group gl at row row0(gl) of the
 // planes at raw(gl), which hold `rows` rows; token t is row tok(t) of the activations.  Here: groups gb0 .. of a matrix.
@@ -109,8 +116,13 @@ struct MmRows {
 
 // one slice of K, superblocks [s_begin, s_end): at most MmT<QT>::SB of them; store(v, gl): group gl's sums of the slice,
 // lane (n16, g) with tokens 4 g .. 4 g + 3 of its row n16.  LEAN: within 128 registers, so that two work-groups share a
-// compute unit -- fewer superblocks in flight, the tokens' values and scales of two blocks at a time instead of eight
-template <int QT, bool LEAN, class SRC, class STORE>
+// compute unit -- fewer superblocks in flight, the tokens' values and scales of two blocks at a time instead of eight.
+// T8: at most eight tokens.  Two neighbouring blocks go through one v_mfma_i32_16x16x64_i8: the instruction's rows 0 - 7 are
+// the tokens with the second block's values zero, rows 8 - 15 the tokens with the first one's, so a lane's four sums are of
+// block 2 p + g / 2 and tokens 4 (g & 1) .., and the scale step, a third of the vector instructions and half wasted on
+// eight tokens otherwise, is halved.  Lane (n, g) supplies 16 values of row n: block 2 p + g / 2, half g & 1.  The halves of
+// the lanes meet when a group is stored.
+template <int QT, bool LEAN, bool T8, class SRC, class STORE>
 __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& src, int K,
                                 const signed char* __restrict__ aq, const float* __restrict__ asc,
                                 const short* __restrict__ absum, int M, int T, int s_begin, int s_end, STORE store) {
@@ -312,6 +324,100 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   const uint8_t* arow = A + n16 * Ks + (g & 1) * 8;
 
   // the products of one superblock (sbk: its index within the slice) of the lane's row, into acc
+  // (T8; row8: the token row of the lane's 16 values, or the first of the zero rows)
+  const int row8 = (n16 < 8) == (g < 2) ? (n16 & 7) : 8, hi = g >> 1, lo1 = g & 1;
+  auto products8 = [&](const MmSb8<QT>& h, int sbk, v4f& acc) {
+    const int b0 = sbk * 8;
+    const uint8_t* ar = A + row8 * Ks;
+    float ua = 0.0f, ub = 0.0f, va = 0.0f, vb = 0.0f, d = 0.0f, dmin = 0.0f;
+    uint32_t G[4];
+    v4f part = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (Q45) {
+      d = f16_bits_to_f32(h.h.x);
+      dmin = f16_bits_to_f32(h.h.x >> 16);
+      ua = U[(b0 + g) * 16 + n16];
+      ub = U[(b0 + 4 + g) * 16 + n16];
+      G[0] = h.h.y;
+      G[1] = __builtin_amdgcn_alignbit(h.h.z, h.h.y, 24);
+      G[2] = __builtin_amdgcn_alignbit(h.h.w, h.h.z, 16);
+      G[3] = h.h.w >> 8;
+      va = -(dmin * (float)(((hi ? G[1] : G[0]) >> (12 * lo1 + 6)) & 63u));
+      vb = -(dmin * (float)(((hi ? G[3] : G[2]) >> (12 * lo1 + 6)) & 63u));
+    } else if constexpr (QT == QT_Q6_K) {
+      d = 0.25f * f16_bits_to_f32(h.d);
+    } else if constexpr (QT == QT_IQ4_XS) {
+      d = f16_bits_to_f32(h.h.x);
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      if (LEAN && p) __builtin_amdgcn_sched_barrier(0);
+      const v4i av = *(const v4i*)(ar + (((sbk * 16 + 4 * p + g) ^ row8) << 4));
+      const float4 sa = *(const float4*)(SA + (b0 + 2 * p + hi) * 16 + 4 * lo1);
+      const float sa4[4] = {sa.x, sa.y, sa.z, sa.w};
+      const v4i z = {0, 0, 0, 0};
+      v4i wv;
+      if constexpr (QT == QT_Q6_K) {
+        const mm_u4 L = h.c[p >> 1], H = h.x[p >> 1];
+        const int st = (p & 1 ? 2 : 6) - 2 * hi;  // (the two high bits of block 2 p + g / 2 to the top of the byte)
+        const uint32_t keep = lo1 ? 0u : 0xFCFCFCFCu;
+        v4i wb;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t nib = p & 1 ? L[k] >> 2 : L[k] << 2;
+          const uint32_t w = ((nib & 0x3C3C3C3Cu) | ((H[k] << st) & 0xC0C0C0C0u)) ^ 0x80808080u;
+          wv[k] = (int)(w & keep);
+          wb[k] = (int)(w & ~keep & 0xFCFCFCFCu);
+        }
+        const v4i Ia = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, z, 0, 0, 0);
+        const v4i Ib = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wb, z, 0, 0, 0);
+        const uint32_t sw = (p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi);
+        const int sca = (int)(signed char)sw, scb = (int)(signed char)(sw >> 8);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[i] = fmaf((float)(__mul24(sca, Ia[i]) + __mul24(scb, Ib[i])), sa4[i], part[i]);
+      } else {
+        float ws;
+        const mm_u4 c = h.c[p];
+        if constexpr (Q45) {
+          const uint32_t H5 = QT == QT_Q5_K ? (hi ? h.q5[p] << 4 : h.q5[p]) : 0u;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            wv[k] = (int)((c[k] >> (4 * hi)) & 0x0F0F0F0Fu);
+            if constexpr (QT == QT_Q5_K) wv[k] |= (int)((H5 >> k) & 0x10101010u);
+          }
+          ws = d * (float)((G[p] >> (12 * hi)) & 63u);
+        } else if constexpr (B16) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t q = c[k] >> (4 * lo1);
+            if constexpr (QT == QT_IQ4_XS) wv[k] = (int)iq4_lookup(q);
+            else if constexpr (QT == QT_MXFP4) wv[k] = (int)mxfp4_lookup(q);
+            else wv[k] = (int)nib_vals<QT>(q);
+          }
+          if constexpr (QT == QT_IQ4_XS) {
+            const int b = 2 * p + hi;
+            ws = d * (float)((int)(((h.h.y >> (4 * b)) & 0xFu) | ((((h.h.x >> 16) >> (2 * b)) & 3u) << 4)) - 32);
+          } else if constexpr (QT == QT_MXFP4) {
+            ws = e8m0_half((p < 2 ? h.h.x : h.h.y) >> (16 * (p & 1) + 8 * hi));
+          } else {
+            ws = f16_bits_to_f32((p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi));
+          }
+        } else {  // Q8_0
+          wv = __builtin_bit_cast(v4i, c);
+          ws = f16_bits_to_f32((p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi));
+        }
+        const v4i I = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, z, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = fmaf((float)I[i], sa4[i] * ws, acc[i]);
+      }
+    }
+    if constexpr (Q45) {  // (rows 8 - 15, no tokens, have U = 0)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ua, va, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ub, vb, acc, 0, 0, 0);
+    }
+    if constexpr (QT == QT_Q6_K)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = fmaf(d, part[i], acc[i]);
+  };
   auto products = [&](const MmSb<QT>& h, int sbk, v4f& acc) {
     const int b0 = sbk * 8;
     long av[8];
@@ -536,6 +642,12 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
     }
   };
 
+  auto put = [&](v4f v, int gl) {
+    if constexpr (T8)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += __shfl_xor(v[i], 32, 64);
+    store(v, gl);
+  };
   const int gf = group_of(min(u0, ulast));  // the stretch's first group
   v4f acc = {0.0f, 0.0f, 0.0f, 0.0f}, ph = acc, pt = acc;  // running sums; the cut group at the head, at the tail
   // unit u: its rows out of qq through the wave's LDS, qq refilled with the unit D on (past the stretch the last unit
@@ -547,6 +659,27 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
     }
     qload(qq, min(u + D, ulast));
     if (u < u1) {
+      const int gl = group_of(u), sb = u - gl * sbs;
+      if constexpr (T8) {
+        MmSb8<QT> s;
+        // 16-byte piece of row n16: Q4_K / Q5_K half g & 1 of chunk p, Q8_0 that half of block 2 p + g / 2, the types of
+        // 16-byte blocks that block, Q6_K half g & 1 of chunk 2 n2 + g / 2
+#pragma unroll
+        for (int p = 0; p < (QT == QT_Q6_K ? 2 : 4); ++p) {
+          const int pc = Q45 ? 2 * p + lo1 : B16 ? 2 * p + hi : 4 * p + g;
+          s.c[p] = *(const mm_u4*)(WQ + ((16 * pc + (n16 ^ (LPRW == 8 ? 2 * pc : pc))) << 4));
+        }
+        s.h = *(const mm_u4*)(WH + ((j * 16 + n16) << 4));
+        if constexpr (QT == QT_Q5_K)
+#pragma unroll
+          for (int p = 0; p < 4; ++p) s.q5[p] = *(const uint32_t*)(WX + (j * 16 + n16) * 32 + 4 * (2 * p + lo1));
+        if constexpr (QT == QT_Q6_K) {
+#pragma unroll
+          for (int p = 0; p < 2; ++p) s.x[p] = *(const mm_u4*)(WX + (j * 16 + n16) * 64 + (((2 * p + lo1) ^ (n16 >> 2)) << 4));
+          s.d = *(const uint32_t*)(WD + ((j * 16 + n16) << 2));
+        }
+        products8(s, sb, acc);
+      } else {
       MmSb<QT> s;
       if constexpr (I3) {
 #pragma unroll
@@ -575,10 +708,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
         s.x[1] = *(const mm_u2*)(xr + (((2 + (g >> 1)) ^ (n16 >> 2)) << 4));
         s.d = *(const uint32_t*)(WD + ((j * 16 + n16) << 2));
       }
-      const int gl = group_of(u), sb = u - gl * sbs;
       products(s, sb, acc);
+      }
       if (sb == sbs - 1 || u == u1 - 1) {  // the group ends here, or the stretch does
-        if (gl * sbs >= u0 && (gl + 1) * sbs <= u1) store(acc, gl);
+        if (gl * sbs >= u0 && (gl + 1) * sbs <= u1) put(acc, gl);
         else if (gl == gf) ph = acc;
         else pt = acc;
         acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -630,7 +763,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
         for (int i = 0; i < 4; ++i) v[i] += pw[(4 * g + i) * 16 + n16];
       }
     }
-    store(v, gf);
+    put(v, gf);
   }
 }
 
@@ -648,7 +781,7 @@ __device__ inline void mm_grid(uint32_t* grid, const uint32_t* __restrict__ tabs
 // the sums of a work-group's groups wait in LDS for the last slice (as many groups as the type's LDS leaves room for);
 // with more groups than that a later slice adds to what the work-group itself has stored in C (other waves of it, as
 // the stretches fall: the meetings between the slices order those stores and loads within the work-group).
-template <int QT>
+template <int QT, bool T8>
 __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, int N, int K,
                                  const signed char* __restrict__ aq, const float* __restrict__ asc,
                                  const short* __restrict__ absum, int M, int T, float* C, int ldc, int c_off, int accumulate,
@@ -671,7 +804,7 @@ __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, 
   for (int sl = 0; sl < slices; ++sl) {
     if (sl) __syncthreads();  // (the tokens and partial sums of the slice before have been read)
     const bool first = sl == 0, last = sl == slices - 1, add = GA ? accumulate : (accumulate || sl);
-    mm_slice<QT, false>(lds, grid, src, K, aq, asc, absum, M, T, s_begin + all * sl / slices,
+    mm_slice<QT, false, T8>(lds, grid, src, K, aq, asc, absum, M, T, s_begin + all * sl / slices,
                              s_begin + all * (sl + 1) / slices, [&](v4f v, int gl) {
       const int n = src.row0(gl) + n16;
       if (GA) {
@@ -695,8 +828,8 @@ __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, 
   }
 }
 
-#define MM_KERNEL(QTV)                                                                                                  \
-  extern "C" __global__ __launch_bounds__(512, 1) void gemv_mm__QT##QTV(                                                \
+#define MM_KERNEL(QTV, SUFFIX, T8)                                                                                                  \
+  extern "C" __global__ __launch_bounds__(512, 1) void gemv_mm__QT##QTV##SUFFIX(                                        \
       const uint8_t* __restrict__ raw, int N, int K, const uint32_t* tabs, const signed char* __restrict__ aq,          \
       const float* __restrict__ asc, const short* __restrict__ absum, int M, int T, float* C, int ldc, int c_off,       \
       int accumulate, int s_begin, int s_end) {                                                                         \
@@ -704,20 +837,28 @@ __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, 
     /* gridDim.y > 1: K shared out over the work-groups (x, y), y-th of gridDim.y even pieces of the superblocks, the    \
        partial sums into plane y of C, here a workspace [gridDim.y][16][ldc] that gemv_mm_reduce adds up */              \
     const int ny = (int)gridDim.y, y = (int)blockIdx.y, all = s_end - s_begin;                                          \
-    mm_kernel<QTV>(lds, raw, N, K, aq, asc, absum, M, T, C + (size_t)y * 16 * ldc, ldc, c_off, accumulate,              \
+    mm_kernel<QTV, T8>(lds, raw, N, K, aq, asc, absum, M, T, C + (size_t)y * 16 * ldc, ldc, c_off, accumulate,              \
                    s_begin + all * y / ny, s_begin + all * (y + 1) / ny, tabs);                                         \
   }
-MM_KERNEL(12)
-MM_KERNEL(13)
-MM_KERNEL(14)
-MM_KERNEL(8)
-MM_KERNEL(2)
-MM_KERNEL(18)
-MM_KERNEL(11)
-MM_KERNEL(20)
-MM_KERNEL(39)
-MM_KERNEL(23)
-MM_KERNEL(21)
+MM_KERNEL(12, , false)
+MM_KERNEL(12, _T81, true)
+MM_KERNEL(13, , false)
+MM_KERNEL(13, _T81, true)
+MM_KERNEL(14, , false)
+MM_KERNEL(14, _T81, true)
+MM_KERNEL(8, , false)
+MM_KERNEL(8, _T81, true)
+MM_KERNEL(2, , false)
+MM_KERNEL(2, _T81, true)
+MM_KERNEL(18, , false)
+MM_KERNEL(11, , false)
+MM_KERNEL(20, , false)
+MM_KERNEL(20, _T81, true)
+MM_KERNEL(39, , false)
+MM_KERNEL(39, _T81, true)
+MM_KERNEL(23, , false)
+MM_KERNEL(23, _T81, true)
+MM_KERNEL(21, , false)
 
 // gemv_mm_reduce: C[t][c_off + n] (=, +=) the sum over the ny planes of ws [ny][16][N], plane 0 first, for the `rows`
 // token rows a launch stores.  grid: ceil(rows * N / 256) work-groups of 256.
@@ -772,14 +913,16 @@ __device__ inline void moe_gateup_mm(uint8_t* lds, const uint8_t* __restrict__ r
   src.w0 = rg; src.w1 = ru; src.rows = NE * F; src.r0 = e * F + blockIdx.x * 128; src.ng = 16; src.pair = true; src.st = st;
   const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
   v4f gate = {0.0f, 0.0f, 0.0f, 0.0f};
-  mm_slice<QT, true>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, [&](v4f v, int gl) {
+  auto both = [&](v4f v, int gl) {
     if (!(gl & 1)) {
       gate = v;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) hs[(4 * g + i) * MMX_HS + 8 * (gl & ~1) + n16] = gate[i] / (1.0f + __expf(-gate[i])) * v[i];
     }
-  });
+  };
+  if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT)>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
+  else mm_slice<QT, true, false>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
   __syncthreads();
   const int hl = threadIdx.x & 31;
   for (int b = threadIdx.x >> 5; b < 4 * nr; b += 16) {
@@ -823,12 +966,14 @@ __device__ inline void moe_down_mm(uint8_t* lds, const uint8_t* __restrict__ raw
   MmExpert src;
   src.w0 = src.w1 = raw; src.rows = NE * N; src.ng = 8 * gpw; src.r0 = e * N + blockIdx.x * src.ng * 16; src.pair = false; src.st = st;
   const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-  mm_slice<QT, true>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, [&](v4f v, int gl) {
+  auto rows = [&](v4f v, int gl) {
     const int n = (blockIdx.x * src.ng + gl) * 16 + n16;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (4 * g + i < nr) y[(size_t)(r0 + 4 * g + i) * N + n] = sw[4 * g + i] * v[i];
-  });
+  };
+  if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT)>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
+  else mm_slice<QT, true, false>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
 }
 
 #define MOE_MM(QTV, WPE)                                                                                                    \

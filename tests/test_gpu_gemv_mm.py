@@ -76,6 +76,14 @@ def test_gemv_mm_parity_types(eng, qt, T, N, K):
     _parity(eng, qt, T, N, K)
 
 
+@pytest.mark.parametrize("T,N,K", [(5, 1500, 4096), (8, 4100, 5120), (6, 19000, 256), (7, 700, 17408), (3, 14000, 5120)])
+@pytest.mark.parametrize("qt", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q8_0, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4])
+def test_gemv_mm_at_most_eight_tokens(eng, qt, T, N, K):
+    """The products of at most eight tokens, two blocks an instruction: matrices large enough for the launch rule, one and
+    several superblocks a slice, several slices, a ragged last group."""
+    _parity(eng, qt, T, N, K)
+
+
 @pytest.mark.parametrize("qt,T,N,K", [(az.Q4_K, 7, 200, 1024), (az.Q4_K, 12, 130, 17408), (az.Q6_K, 16, 96, 6400),
                                       (az.Q8_0, 5, 333, 8192)])
 def test_gemv_mm_into_a_wider_output(eng, qt, T, N, K):
