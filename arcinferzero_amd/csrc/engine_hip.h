@@ -1290,15 +1290,18 @@ class Engine {
   }
 
   // Passes between the one-slot kernels, whose time goes with the pairs, and the tile GEMM, whose work-groups take about the
-  // same time however few slots a tile has: the matrix-pipe kernels of 16-slot tiles.  us a layer, 128 x 8 experts of 768 x
-  // 2048, one-slot or tile GEMM against these: 8 tokens Q4_K 68 / 70, IQ4_XS 73 / 79; 16: 121 / 83, 131 / 96; 32: 165 / 103,
-  // 315 / 120; 128: 180 / 142, 341 / 153; 256: 182 / 169, 350 / 199; 32 x 4 experts, 8 tokens 45 / 53, 16 tokens 69 / 55.
-  // The upper end is in slots an expert, where the type's tile GEMM overtakes: Q4_K 14 - 19, Q5_K 16, Q6_K 24, the others
-  // 36 - 45.
+  // same time however few slots a tile has: the matrix-pipe kernels of 16-slot tiles.  us a layer, one-slot or tile GEMM
+  // against these: 128 x 8 experts of 768 x 2048, 4 tokens Q4_K 40 / 49, Q6_K 53 / 60; 6: Q4_K 51 / 51, Q6_K 73 / 62, IQ4_XS
+  // 54 / 58; 8: Q4_K 63 / 61, Q6_K 89 / 84, IQ4_XS 68 / 72; 200: 175 / 148, 291 / 216, 336 / 167; 300: 182 / 192, 301 / 277,
+  // 359 / 221; 64 x 8 of 1536 x 3072, 4 tokens Q4_K 81 / 86, 6: Q4_K 111 / 91, IQ4_NL 102 / 107; 32 x 4, 8 tokens Q4_K 41 /
+  // 47, 12: 54 / 47.  So from 48 pairs on, and 6 tokens for Q4_K - Q6_K, whose one-slot kernels are the heavier, 9 tokens for
+  // the others.  The upper end is in slots an expert, where the type's tile GEMM overtakes: Q4_K 14 - 19, Q5_K 16, Q6_K 24,
+  // the others 36 - 45.
   static bool moe_mm_takes(const MoeLayer& L, int T) {
     const uint32_t t = L.ex[0].type;
     const int most = t == GGML_Q4_K || t == GGML_Q5_K ? 15 : t == GGML_Q6_K ? 22 : 36;
-    return T > 8 && T * L.NU >= 48 && T * L.NU <= L.NE * most;
+    const bool kq = t == GGML_Q4_K || t == GGML_Q5_K || t == GGML_Q6_K;
+    return T > (kq ? 5 : 8) && T * L.NU >= 48 && T * L.NU <= L.NE * most;
   }
   // LDS of an expert kernel on the matrix pipe (decode_mm.hip's MmL): tokens of K values, the waves' pieces, the epilogue's
   // rows, the codebook; 0: K does not fit

@@ -122,6 +122,12 @@ def test_moe_matrix_pipe_tiles_of_16_slots(rt, qtype, NE, NU, E, F, T):
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 32)
 
 
+@pytest.mark.parametrize("qtype,T", [(az.Q4_K, 6), (az.Q5_K, 7), (az.Q6_K, 8), (az.Q4_K, 5), (az.Q8_0, 8)])
+def test_moe_matrix_pipe_tiles_from_six_tokens(rt, qtype, T):
+    """The first token counts that the 16-slot tiles take (48 pairs; Q4_K - Q6_K), and the last that they do not."""
+    _moe_layer_vs_oracle(qtype, 16, 8, 512, 256, T, 16)
+
+
 @pytest.mark.parametrize("env", [{}, {"ARCZ_MOE_QFUSE": "0"}, {"ARCZ_MOE_PRE": "0"}, {"ARCZ_MOE_PRE": "0", "ARCZ_MOE_QFUSE": "0"}])
 @pytest.mark.parametrize("NE,NU,E,F,T,Mp", [(16, 4, 512, 256, 300, 304), (8, 2, 256, 512, 70, 80), (8, 3, 256, 768, 90, 96)])
 def test_moe_tile_pass_quantization_forms(rt, monkeypatch, env, NE, NU, E, F, T, Mp):
