@@ -355,7 +355,7 @@ class Engine {
   }
   // The fused producers of the reference (rmsnorm_quant, zero/engine.h:1256-1267; swiglu_quant via run_rows_quant,
   // zero/engine.h:1404-1440): a work-group per row of the chunk, or -- a pass of 1-8 tokens -- the valid rows only,
-  // their superblocks over several work-groups (the GEMVs read nothing else).
+  // their superblocks a wave each over several work-groups (the GEMVs read nothing else).
   static bool wide_rows(int T) { return T <= 8; }
   // Rows of a quantizer tile: 64 (whole 256-byte runs of scales) once that fills the chip eight work-groups deep, below
   // that 16 (one pass over a thread's loads instead of four).
@@ -373,9 +373,11 @@ class Engine {
     int wh = hout ? 1 : 0;
     set_args(k, 0, x, row_off, w, K, Mp, T, eps, aq_, asc_, absum_, hout, wh, act32);
     size_t gws[2] = {256, (size_t)(wave ? Mp / 4 : Mp)}, lws[2] = {256, 1};
-    if (wide_rows(T)) {
-      gws[0] = 256 * (size_t)((K / 256 + 15) / 16);
-      gws[1] = (size_t)T;
+    // (a wave a superblock up to 64 rows: us at 5120 values, a work-group a row against it: 1 row 3.0 / 3.2, 8 4.0 / 3.3, 16
+    //  4.3 / 3.3, 64 4.5 / 3.8, 128 4.6 / 4.6; 256 x 4096 4.2 / 5.4)
+    if (wide_rows(T) || Mp <= 64) {
+      gws[0] = 256 * (size_t)std::max((K / 256 + 3) / 4, 2);
+      gws[1] = (size_t)(wide_rows(T) ? T : Mp);
     }
     run("rmsnorm_quant", k, 2, gws, lws);
     cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_act32_ = act32 ? 1 : 0;
@@ -389,7 +391,7 @@ class Engine {
     const bool wide = wide_rows(T);
     cl_kernel k = kernel("ops", q2_defs_, wide ? "swiglu_quant" : "swiglu_quant_tile");
     set_args(k, 0, gu, F, Mp, T, aq_, asc_, absum_, act32, fused, gelu);
-    size_t gws[2] = {256 * (size_t)((F / 256 + 15) / 16), (size_t)T}, lws[2] = {256, 1};
+    size_t gws[2] = {256 * (size_t)((F / 256 + 3) / 4), (size_t)T}, lws[2] = {256, 1};
     if (!wide) {
       int rows = tile_rows(F, Mp);
       set_args(k, 10, rows);

@@ -100,9 +100,9 @@ extern "C" __global__ __launch_bounds__(256) void quant_rows(const float* __rest
   quant_tile(load, s, blockIdx.y * rows, rows, K, M, T, aq, asc, absum, act32, q2_aq, q2_sc, q2_ab);
 }
 
-// ---- the two fused producers.  A work-group of 256 threads per row (or several along x, each taking a share of the
-// row's superblocks: the launch for a pass of 1-8 tokens, zero/engine.h:1404-1412); 16 threads per superblock, thread
-// = 16 consecutive values, so a wave works on 4 superblocks at a time.  Scales and sums are stored straight into the
+// ---- the fused producers.  A work-group of 256 threads per row, 16 threads per superblock, thread = 16 consecutive
+// values, so a wave works on 4 superblocks at a time; or several work-groups along x, each taking a share of the row's
+// superblocks (the launch for few rows, zero/engine.h:1404-1412), a wave per superblock.  Scales and sums are stored straight into the
 // token-minor layouts (one element per block and row).
 __device__ inline void store_row_quant1(const float* v, int s, int lane16, int m, int M, int K, int act32,
                                         signed char* __restrict__ aq, float* __restrict__ asc, short* __restrict__ absum,
@@ -132,21 +132,59 @@ __device__ inline void store_row_quant(const float* v, int s, int lane16, int m,
   }
 }
 
+// The same for a wave that holds a whole superblock, four consecutive values a lane: a pass of few rows, whose time is one
+// thread's chain of instructions, has a quarter of it this way, and everything between the lanes of a block is a
+// data-parallel move.
+__device__ inline void store_wave_quant1(const float* v, int s, int lane, int m, int M, int K, int act32,
+                                         signed char* __restrict__ aq, float* __restrict__ asc, short* __restrict__ absum,
+                                         float* res) {
+  float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+  amax = fmaxf(amax, dpp_from<0xB1>(amax));   // neighbour, other pair, other quad: the 8 lanes of a 32-block
+  amax = fmaxf(amax, dpp_from<0x4E>(amax));
+  amax = fmaxf(amax, dpp_from<0x141>(amax));
+  if (!act32) {
+    amax = fmaxf(amax, dpp_from<0x140>(amax));
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+  }
+  uint32_t w[1];
+  int sum;
+  quant_values<4>(v, amax, w, sum, res);
+  sum += __builtin_amdgcn_mov_dpp(sum, 0xB1, 0xF, 0xF, true);
+  sum += __builtin_amdgcn_mov_dpp(sum, 0x4E, 0xF, 0xF, true);
+  *(uint32_t*)(aq + (size_t)m * K + s * 256 + 4 * lane) = w[0];
+  if ((lane & 3) == 0) absum[((size_t)s * 16 + (lane >> 2)) * M + m] = (short)sum;
+  if (act32) {
+    if ((lane & 7) == 0) asc[((size_t)s * 8 + (lane >> 3)) * M + m] = amax / 127.0f;
+  } else if (lane == 0) {
+    asc[(size_t)s * M + m] = amax / 127.0f;
+  }
+}
+__device__ inline void store_wave_quant(const float* v, int s, int lane, int m, int M, int K, int act32,
+                                        signed char* __restrict__ aq, float* __restrict__ asc, short* __restrict__ absum,
+                                        int q2_aq, int q2_sc, int q2_ab) {
+  if (!q2_aq) {
+    store_wave_quant1(v, s, lane, m, M, K, act32, aq, asc, absum, nullptr);
+  } else {
+    float res[4];
+    store_wave_quant1(v, s, lane, m, M, K, act32, aq, asc, absum, res);
+    store_wave_quant1(res, s, lane, m, M, K, act32, aq + q2_aq, asc + q2_sc, absum + q2_ab, nullptr);
+  }
+}
+
 // Sum over the work-group, the same value in every thread, in a fixed order (so every work-group that sums the same
-// row gets the same bits).
+// row gets the same bits).  red: four floats of its own for each sum.
 __device__ inline float group_sum(float v, float* red) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  v = group_sum_last<true>(v);
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  const float r = (red[0] + red[1]) + (red[2] + red[3]);
-  __syncthreads();
-  return r;
+  return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // rmsnorm_quant: y = x[row_off + m] * rsqrt(mean(x^2) + eps) * w, quantized for the next matmul, rows m >= M_valid as
 // zeros; with write_h also stored as f32 in hout [M][K] (reference zero/kernels/ops.cl:107-141, same arguments).
-// grid (256 * G, rows), local (256, 1).
+// grid (256 * G, rows), local (256, 1).  Bound by one thread's chain: loads, sum, norm, quantization.  G > 1, for few rows:
+// a wave a superblock (8 x 5120 4.0 -> 3.3 us against 16 threads a superblock, 16 values each).
 extern "C" __global__ __launch_bounds__(256) void rmsnorm_quant(const float* __restrict__ x, int row_off,
                                                                 const float* __restrict__ w, int K, int M, int M_valid,
                                                                 float eps, signed char* __restrict__ aq,
@@ -202,35 +240,43 @@ extern "C" __global__ __launch_bounds__(256) void rmsnorm_quant(const float* __r
     }
     return;
   }
-  float ss = 0.0f;
-  if (valid)
-    for (int i = threadIdx.x * 4; i < K; i += 1024) {
-      const float4 f = *(const float4*)(xr + i);
-      ss += f.x * f.x;
-      ss += f.y * f.y;
-      ss += f.z * f.z;
-      ss += f.w * f.w;
-    }
-  ss = group_sum(ss, red);
-  const float r = rsqrtf(ss / (float)K + eps);
-  for (int s = blockIdx.x * 16 + sub; s < K / 256; s += 16 * gridDim.x) {
-    const int base = s * 256 + 16 * lane16;
-    float v[16];
-    if (valid) {
+  // Several work-groups per row: each sums the whole row (its loads in flight together with those of the superblock that
+  // the wave is to quantize) and a wave quantizes the superblocks it takes, four values a lane.
+  const int lane = threadIdx.x & 63, nsb = K >> 8;
+  int s = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f), g = f;
+  float r = 0.0f;
+  if (valid) {
+    const int b0 = min(s, nsb - 1) * 256 + 4 * lane;
+    f = *(const float4*)(xr + b0);
+    g = *(const float4*)(w + b0);
+    float4 ss = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i0 = threadIdx.x * 4; i0 < K; i0 += 8 * 1024) {
+      float4 q[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 f = *(const float4*)(xr + base + 4 * i), g = *(const float4*)(w + base + 4 * i);
-        v[4 * i] = f.x * r * g.x; v[4 * i + 1] = f.y * r * g.y; v[4 * i + 2] = f.z * r * g.z; v[4 * i + 3] = f.w * r * g.w;
+      for (int j = 0; j < 8; ++j) q[j] = *(const float4*)(xr + min(i0 + 1024 * j, K - 4));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (i0 + 1024 * j >= K) q[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        ss.x += q[j].x * q[j].x;
+        ss.y += q[j].y * q[j].y;
+        ss.z += q[j].z * q[j].z;
+        ss.w += q[j].w * q[j].w;
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = 0.0f;
     }
-    if (write_h)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *(float4*)(hout + (size_t)m * K + base + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    store_row_quant(v, s, lane16, m, M, K, act32, aq, asc, absum, q2_aq, q2_sc, q2_ab);
+    r = (ss.x + ss.y) + (ss.z + ss.w);
+  }
+  r = group_sum(r, red);
+  r = valid ? rsqrtf(r / (float)K + eps) : 0.0f;
+  for (; s < nsb; s += 4 * gridDim.x) {
+    const int base = s * 256 + 4 * lane;
+    if (valid && s >= 4 * (int)gridDim.x) {
+      f = *(const float4*)(xr + base);
+      g = *(const float4*)(w + base);
+    }
+    float v[4] = {f.x * r * g.x, f.y * r * g.y, f.z * r * g.z, f.w * r * g.w};
+    if (write_h) *(float4*)(hout + (size_t)m * K + base) = make_float4(v[0], v[1], v[2], v[3]);
+    store_wave_quant(v, s, lane, m, M, K, act32, aq, asc, absum, q2_aq, q2_sc, q2_ab);
   }
 }
 
@@ -246,7 +292,7 @@ extern "C" __global__ __launch_bounds__(256) void add_norm_quant(float* __restri
                                                                  signed char* __restrict__ aq, float* __restrict__ asc,
                                                                  short* __restrict__ absum, int act32, int M_valid,
                                                                  int q2_aq, int q2_sc, int q2_ab) {
-  __shared__ float red[4];
+  __shared__ float red[4], red2[4];
   const int m = blockIdx.y;
   const bool valid = m < M_valid;
   const float* tr = t + (size_t)m * K;
@@ -283,7 +329,7 @@ extern "C" __global__ __launch_bounds__(256) void add_norm_quant(float* __restri
         *(float4*)(xr + base + 4 * i) = v;
       }
     }
-  s2 = group_sum(s2, red);
+  s2 = group_sum(s2, red2);
   const float r2 = w2_norm ? rsqrtf(s2 / (float)K + eps) : 1.0f;
   for (int sb = sub; sb < K / 256; sb += 16) {
     const int base = sb * 256 + 16 * lane16;
@@ -389,7 +435,10 @@ __device__ inline float act_gate(float g, int gelu) {
 
 // swiglu_quant: y = silu(gate) * up (or the tanh form of gelu(gate) * up) from rows [gate(F) | up(F)], or the row as it
 // is when the matmul before has fused the product (`fused`), quantized with K = F (reference zero/kernels/ops.cl:
-// 271-315, same arguments; silu(x) = x / (1 + exp(-x)), ops.cl:33).  grid (256 * G, rows), local (256, 1).
+// 271-315, same arguments; silu(x) = x / (1 + exp(-x)), ops.cl:33).  grid (256 * G, rows), local (256, 1).  A wave
+// a superblock, four values a lane: few rows are bound by one thread's chain of instructions, and 16 values a thread made
+// it four times as long (1 x 17408 4.0 -> 3.1 us, 8 x 17408 4.5 -> 3.2; one feed-forward block of one token 40.1 -> 37.3,
+// of eight 73.6 -> 65.7).
 extern "C" __global__ __launch_bounds__(256) void swiglu_quant(const float* __restrict__ gu, int F, int M, int M_valid,
                                                                signed char* __restrict__ aq, float* __restrict__ asc,
                                                                short* __restrict__ absum, int act32, int fused,
@@ -397,43 +446,20 @@ extern "C" __global__ __launch_bounds__(256) void swiglu_quant(const float* __re
   const int m = blockIdx.y;
   const bool valid = m < M_valid;
   const float* gr = gu + (size_t)m * (fused ? F : 2 * F);
-  const int lane16 = threadIdx.x & 15, sub = threadIdx.x >> 4;
-  const int nsb = F >> 8, stride = 16 * gridDim.x;
-  // (a thread's superblocks two at a time: the loads of both are issued before the first is worked on)
-  for (int s0 = blockIdx.x * 16 + sub; s0 < nsb; s0 += 2 * stride) {
-    float4 gv[2][4], uv4[2][4];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int s = s0 + h * stride;
-      const bool in = valid && s < nsb;
-      const int base = (in ? s : 0) * 256 + 16 * lane16;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        gv[h][i] = in ? *(const float4*)(gr + base + 4 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        uv4[h][i] = in && !fused ? *(const float4*)(gr + F + base + 4 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const int lane = threadIdx.x & 63, nsb = F >> 8;
+  for (int s = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); s < nsb; s += 4 * gridDim.x) {
+    const int base = s * 256 + 4 * lane;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (valid) {
+      const float4 f = *(const float4*)(gr + base);
+      v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+      if (!fused) {
+        const float4 u = *(const float4*)(gr + F + base);
+        v[0] = act_gate(f.x, gelu) * u.x; v[1] = act_gate(f.y, gelu) * u.y;
+        v[2] = act_gate(f.z, gelu) * u.z; v[3] = act_gate(f.w, gelu) * u.w;
       }
     }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int s = s0 + h * stride;
-      if (s >= nsb) break;
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[4 * i] = gv[h][i].x; v[4 * i + 1] = gv[h][i].y; v[4 * i + 2] = gv[h][i].z; v[4 * i + 3] = gv[h][i].w;
-      }
-      if (valid && !fused) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float uv[4] = {uv4[h][i].x, uv4[h][i].y, uv4[h][i].z, uv4[h][i].w};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            v[4 * i + j] = act_gate(v[4 * i + j], gelu) * uv[j];
-          }
-        }
-      }
-      store_row_quant(v, s, lane16, m, M, F, act32, aq, asc, absum, q2_aq, q2_sc, q2_ab);
-    }
+    store_wave_quant(v, s, lane, m, M, F, act32, aq, asc, absum, q2_aq, q2_sc, q2_ab);
   }
 }
 

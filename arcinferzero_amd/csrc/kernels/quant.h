@@ -18,17 +18,18 @@ __device__ inline float block_amax(const float* v, int act32) {
   return amax;
 }
 
-// Quantizes v[16] (the 16 values of lane16 in its row's superblock); returns the packed int8 and their sum.  With
+// Quantizes v[N] (N = 16: the 16 values of lane16 in its row's superblock); returns the packed int8 and their sum.  With
 // res, also what the int8 values miss: res[i] = v[i] - (float)q * (amax / 127) (reference zero/kernels/ops.cl:49-59,
 // the two-pass mode's residual; the product and the difference are rounded one after the other).
-__device__ inline void quant16(const float* v, float amax, uint4& pk, int& sum, float* res = nullptr) {
+template <int N> __device__ inline void quant_values(const float* v, float amax, uint32_t (&w)[N / 4], int& sum, float* res = nullptr) {
 #pragma clang fp contract(off)  // (no fused multiply-add below: v * inv and q * scale are rounded on their own)
   const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
   const float sc = amax / 127.0f;
-  uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) w[i] = 0;
   sum = 0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < N; ++i) {
     const float p = __fmul_rn(v[i], inv);
     const int q = __float2int_rn(p);
     sum += q;
@@ -38,6 +39,10 @@ __device__ inline void quant16(const float* v, float amax, uint4& pk, int& sum, 
       res[i] = v[i] - qs;
     }
   }
+}
+__device__ inline void quant16(const float* v, float amax, uint4& pk, int& sum, float* res = nullptr) {
+  uint32_t w[4];
+  quant_values<16>(v, amax, w, sum, res);
   pk = make_uint4(w[0], w[1], w[2], w[3]);
 }
 

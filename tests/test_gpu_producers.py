@@ -143,6 +143,41 @@ def test_producers_16_rows_a_work_group(rt, T, Mp, K, act32):
         eng.close()
 
 
+@pytest.mark.parametrize("T,Mp,K,act32", [(1, 16, 256, 1), (8, 16, 8448, 1), (2, 16, 20736, 0), (40, 48, 2304, 0), (63, 64, 1280, 1),
+                                          (65, 80, 20736, 1)])
+def test_producers_wave_a_superblock(rt, T, Mp, K, act32):
+    """Few rows, a wave a superblock: one superblock, rows longer than a thread's first loads, waves without a superblock,
+    both scale blocks, padding rows; more rows than that with a row too long for one work-group's registers."""
+    print(f"producers few T={T} Mp={Mp} K={K} act32={act32}", flush=True)
+    B, rows = 32 if act32 else 256, T if T <= 8 else Mp
+    eng = az.Engine(Mp, K)
+    try:
+        def read():
+            return (eng.aq.read(np.int8, Mp * K).reshape(Mp, K)[:rows],
+                    np.ascontiguousarray(eng.asc.read(np.float32, Mp * K // B).reshape(K // B, Mp)[:, :rows]).view(np.uint32),
+                    eng.absum.read(np.int16, Mp * K // 16).reshape(K // 16, Mp)[:, :rows])
+        x = make_acts(T, K, seed=350 + T, outliers=True)
+        w = (1.0 + 0.1 * az.gen_normal(351, (K,))).astype(np.float32)
+        xb, wb = az.Runtime.from_numpy(x), az.Runtime.from_numpy(w)
+        hb = az.Runtime.alloc(Mp * K * 4).fill(0xFFFFFFFF)
+        poison(eng)
+        eng.rmsnorm_quant(xb, 0, wb, K, Mp, T, 1e-6, hout=hb, act32=act32)
+        h = hb.read(np.float32, Mp * K).reshape(Mp, K)[:rows]
+        x64 = x.astype(np.float64)
+        ref = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * w.astype(np.float64)
+        assert np.abs(h[:T] - ref).max() <= 1e-6 * np.abs(ref).max() and not h[T:].any()
+        raq, rasc, rabsum = orc.quantize_act(np.ascontiguousarray(h), act32=bool(act32))
+        want = (raq, rasc.view(np.uint32), rabsum)
+        assert all(np.array_equal(a, b) for a, b in zip(read(), want))
+        poison(eng)
+        eng.swiglu_quant(hb, K, Mp, T, fused=1, act32=act32)
+        assert all(np.array_equal(a, b) for a, b in zip(read(), want))
+        for b in (xb, wb, hb):
+            b.free()
+    finally:
+        eng.close()
+
+
 @pytest.mark.parametrize("T,Mp,K", [(257, 260, 256), (509, 512, 6400), (300, 304, 16640), (250, 272, 6144), (2047, 2064, 4096),
                                     (8192, 8192, 2048)])
 def test_producers_tiles_and_waves(rt, T, Mp, K):
