@@ -850,7 +850,7 @@ class Engine {
     int M = Mp, N = w.N, K = w.K, nsb = K / 256;
     const int mt = (Mp + 127) / 128, nt_all = (N + 127) / 128;
     const int panel = (int)std::min<size_t>((size_t)nt_all, wd_bytes_ / ((size_t)(K / 32) * f.wimg));
-    if (panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
+    if (!xd_ || panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
     size_t l[2] = {256, 1};
     {
       cl_kernel k = kernel("gemm", "", "act_digits");
@@ -906,8 +906,11 @@ class Engine {
     }
     return best;
   }
+  // Room for the digits: an engine has it from uploading a weight that the rule takes.  It multiplies with other engines'
+  // weights too, and one that has no room runs those on the int8 kernels.
+  bool digits_room(const GpuWeight& w) const { return xd_ && wd_bytes_ >= (size_t)(w.K / 32) * digit_form(w.type).wimg; }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
-    if (digits_take(w0.type, Mp, w0.N)) {
+    if (digits_take(w0.type, Mp, w0.N) && digits_room(w0)) {
       gemm_digits(name, w0, Mp, C, ldc, c_off, a);
       return;
     }

@@ -301,6 +301,37 @@ def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512)])
+@pytest.mark.parametrize("before", [None, 256, 1024])
+def test_weights_of_another_engine(rt, qtype, T, N, K, before):
+    """Engines share weights: a matrix that an engine for single tokens uploaded, in a long chunk of an engine that
+    uploaded none itself (no room for digits), or one with shorter or longer rows (room for some tiles of this one's rows
+    or for all).  Against the oracle."""
+    print(f"another engine's {TYPE_NAMES[qtype]} T={T} N={N} K={K} before={before}", flush=True)
+    small = az.Engine(16, K)
+    W = make_weights(qtype, N, K, seed=96)
+    w = small.make_weight(qtype, N, K, W)
+    Mp = (T + 127) // 128 * 128
+    eng = az.Engine(Mp, 1024)
+    if before:   # (rows enough for the launch rule of every type)
+        small_n = -(-8 * 1024 * 1024 // Mp)
+        eng.make_weight(qtype, small_n, before, make_weights(qtype, small_n, before, seed=95)).free()
+    x = make_acts(T, K, seed=97, outliers=True)
+    xb = az.Runtime.from_numpy(x)
+    eng.quantize(xb, K, K, Mp, T)
+    cb = az.Runtime.alloc(Mp * N * 4).fill(0xFFFFFFFF)
+    eng.matmul("test", w, Mp, cb, N, 0, 0)
+    y = cb.read(np.float32, Mp * N).reshape(Mp, N)
+    for b in (cb, xb):
+        b.free()
+    w.free()
+    eng.close()
+    small.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, W, N, K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    assert np.isfinite(y).all() and rel_err_rows(y[:T], ref).max() <= TOL and not y[T:].any()
+
+
 @pytest.mark.parametrize("T,Mp,N,K,acc", [(1100, 1104, 392, 512, 0), (1030, 1040, 640, 768, 1), (760, 768, 520, 1024, 2),
                                           (300, 304, 132, 256, 0), (2050, 2064, 136, 256, 1)])
 def test_gemm_tiles_of_256_tokens(rt, monkeypatch, T, Mp, N, K, acc):
