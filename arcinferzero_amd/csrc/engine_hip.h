@@ -193,6 +193,19 @@ class Engine {
     mems_.push_back(m);
     return m;
   }
+  // ... or none, where memory has run out, for what a call can do without
+  cl_mem try_buf(size_t bytes) {
+    struct Throws {
+      bool was = zrt::oom_throws;
+      Throws() { zrt::oom_throws = true; }
+      ~Throws() { zrt::oom_throws = was; }
+    } throws;
+    try {
+      return buf(bytes);
+    } catch (const std::runtime_error&) {
+      return nullptr;
+    }
+  }
   // A recorded launch list keeps the device addresses its kernels were given, the engine's own workspaces among them:
   // a buffer that a live list names is not freed or replaced (the list would read and write freed memory).  The call
   // that wanted to throws, with the engine as it was; free the list first.
@@ -307,19 +320,7 @@ class Engine {
         wsv_bytes_ = need;
       }
     }
-    if (rows == (size_t)N && digits_take(w.type, max_chunk, N)) {  // (room for its digits and the chunk's, gemm_digits)
-      const DigitForm f = digit_form(w.type);
-      const size_t tile = (size_t)(K / 32) * f.wimg;
-      const size_t need = std::max(tile, std::min((size_t)(N + 127) / 128 * tile, (size_t)512 << 20));
-      if (!xd_) xd_ = buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
-      if (need > wd_bytes_) {
-        if (wd_) release(wd_);
-        wd_ = nullptr;
-        wd_bytes_ = 0;
-        wd_ = buf(need);
-        wd_bytes_ = need;
-      }
-    }
+    if (rows == (size_t)N && digits_take(w.type, max_chunk, N)) digits_reserve(w);
     if (type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS) {  // (room for its GEMM form)
       const size_t need = raw_planes_bytes(QT_Q6_K, rows, K / 256);
       if (need > xw_bytes_) {
@@ -906,8 +907,20 @@ class Engine {
     }
     return best;
   }
-  // Room for the digits: an engine has it from uploading a weight that the rule takes.  It multiplies with other engines'
-  // weights too, and one that has no room runs those on the int8 kernels.
+  // Room for the digits: an engine makes it when it uploads a weight that the rule takes.  Without it such a weight runs on
+  // the int8 kernels (it may be another engine's), or in panels of as many rows as there is room for: so an upload is not
+  // refused where memory has run out or where a recorded list names the room that a larger matrix would replace.
+  void digits_reserve(const GpuWeight& w) {
+    const size_t tile = (size_t)(w.K / 32) * digit_form(w.type).wimg;
+    const size_t need = std::max(tile, std::min((size_t)(w.N + 127) / 128 * tile, (size_t)512 << 20));
+    if (!xd_) xd_ = try_buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
+    if (!xd_ || need <= wd_bytes_ || (wd_ && arcz_mem_listed(wd_))) return;
+    if (wd_) release(wd_);
+    wd_ = nullptr;
+    wd_bytes_ = 0;
+    wd_ = try_buf(need);
+    if (wd_) wd_bytes_ = need;
+  }
   bool digits_room(const GpuWeight& w) const { return xd_ && wd_bytes_ >= (size_t)(w.K / 32) * digit_form(w.type).wimg; }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
     if (digits_take(w0.type, Mp, w0.N) && digits_room(w0)) {

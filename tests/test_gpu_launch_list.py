@@ -10,7 +10,8 @@ import numpy as np
 import pytest
 
 import arcinferzero_amd as az
-from common import make_acts, make_weights
+import oracle_lib as orc
+from common import make_acts, make_weights, rel_err_rows
 
 pytestmark = pytest.mark.gpu
 E_RECORDING = -59
@@ -208,3 +209,82 @@ def test_a_list_keeps_the_buffers_it_names(rt):
         if lst is not None:
             lst.free()
         eng.close()
+
+
+def test_a_list_that_names_the_digits_of_rows(rt):
+    """A recorded long chunk of Q4_0 names the engine's room for the digits of the rows.  A larger Q4_0 matrix is uploaded
+    all the same and multiplied in panels of the rows that fit that room, or -- rows longer than it holds a tile of -- on
+    the int8 kernels: against the oracle; the list replays bit for bit behind it."""
+    T = Mp = 256
+    N, K = 12288, 256      # (the fewest rows that the launch rule takes for 256 tokens)
+    eng = az.Engine(Mp, 32768)
+    lst = None
+    try:
+        w = eng.make_weight(az.Q4_0, N, K, make_weights(az.Q4_0, N, K, seed=44))
+        xb = az.Runtime.from_numpy(make_acts(T, K, seed=45))
+        cb = az.Runtime.alloc(Mp * N * 4).fill(0)
+
+        def step():
+            eng.quantize(xb, K, K, Mp, T)
+            eng.matmul("listed", w, Mp, cb, N, 0, 0)
+
+        step()
+        ref = cb.read(np.float32, Mp * N).copy()
+        lst = az.Runtime.record(step)
+        for n2, k2 in ((N, 512), (N, 32768)):
+            print(f"upload while a list names the digits N={n2} K={k2}", flush=True)
+            W2 = make_weights(az.Q4_0, n2, k2, seed=46)
+            w2 = eng.make_weight(az.Q4_0, n2, k2, W2)
+            x2 = make_acts(T, k2, seed=47)
+            b2, c2 = az.Runtime.from_numpy(x2), az.Runtime.alloc(Mp * n2 * 4).fill(0xFFFFFFFF)
+            eng.quantize(b2, k2, k2, Mp, T)
+            eng.matmul("larger", w2, Mp, c2, n2, 0, 0)
+            y = c2.read(np.float32, Mp * n2).reshape(Mp, n2)
+            aq, asc, _ = orc.quantize_act(x2)
+            rows = np.r_[0:200, n2 - 200:n2]          # (the first and last rows: the oracle over all of them takes long)
+            Ws = np.ascontiguousarray(W2.reshape(n2, -1)[rows]).reshape(-1)
+            assert rel_err_rows(y[:16, rows], orc.matmul_ref(az.Q4_0, Ws, len(rows), k2, aq[:16], np.ascontiguousarray(asc[:, :16]))).max() <= 1e-3
+            assert np.isfinite(y).all()
+            cb.fill(0xFFFFFFFF)
+            lst.run()
+            assert np.array_equal(cb.read(np.float32, Mp * N).view(np.uint32), ref.view(np.uint32))
+            for b in (b2, c2):
+                b.free()
+            w2.free()
+        lst.free()
+        lst = None
+        for b in (xb, cb):
+            b.free()
+        w.free()
+    finally:
+        if lst is not None:
+            lst.free()
+        eng.close()
+
+
+@pytest.mark.parametrize("nth", [2, 3])
+def test_an_upload_without_memory_for_digits(rt, nth):
+    """The allocation of the chunk's digits (the second of an upload) or of the rows' (the third) fails: the weight is
+    there all the same and runs on the int8 kernels."""
+    T = Mp = 256
+    N, K = 12288, 512
+    print(f"upload whose allocation {nth} fails", flush=True)
+    W = make_weights(az.Q4_0, N, K, seed=48)
+    x = make_acts(T, K, seed=49)
+    ys = []
+    for n in (0, nth):
+        eng = az.Engine(Mp, K)
+        az.lib.arcz_set_fake_oom(n)
+        try:
+            w = eng.make_weight(az.Q4_0, N, K, W)
+        finally:
+            az.lib.arcz_set_fake_oom(0)
+        xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * N * 4).fill(0xFFFFFFFF)
+        eng.quantize(xb, K, K, Mp, T)
+        eng.matmul("m", w, Mp, cb, N, 0, 0)
+        ys.append(cb.read(np.float32, Mp * N).reshape(Mp, N))
+        for b in (xb, cb):
+            b.free()
+        w.free()
+        eng.close()
+    assert np.isfinite(ys[1]).all() and rel_err_rows(ys[1], ys[0]).max() <= 2e-5      # (the same block sums, f32 from there on)
