@@ -2,8 +2,9 @@
 #pragma once
 #include <stddef.h>
 
-// 32 MiB: the most the short-chunk GEMM's partial tiles can take under the engine's launch rule (pieces x tiles within
-// two work-groups per compute unit of a 256-unit device, tiles of at most 128 x 128 f32: 512 x 128 x 128 x 4 bytes).
+// 32 MiB: the limit that the engine's priced rules for pieces of K and gemv_mm's keep to (SPLIT_BYTES), and the most that
+// the other types' rule asks for on a device of 256 compute units (pieces x tiles within two work-groups a unit, tiles of
+// at most 128 x 128 f32: 512 x 128 x 128 x 4 bytes).
 #define ARCZ_SCRATCH_BYTES (32u << 20)
 
 #ifdef __cplusplus

@@ -85,7 +85,8 @@ class Engine {
     moe_pre_ = getenv("ARCZ_MOE_PRE") ? atoi(getenv("ARCZ_MOE_PRE")) != 0 : true;
     q4_wm_ = getenv("ARCZ_Q4_WM") ? atoi(getenv("ARCZ_Q4_WM")) : 0;
     q4_wm_min_ = getenv("ARCZ_Q4_WM_MIN") ? atoi(getenv("ARCZ_Q4_WM_MIN")) : 2048;
-    sk_ws_bytes_ = (size_t)2 * (size_t)arcz_device_cus() * 128 * 128 * 4;
+    // ... and at least the limit of the launch rules that price the pieces (SPLIT_BYTES)
+    sk_ws_bytes_ = std::max((size_t)2 * (size_t)arcz_device_cus() * 128 * 128 * 4, SPLIT_BYTES);
     sk_ws_ = buf(sk_ws_bytes_);
     // the codebook tables the kernels take as `tabs` (the reference's tabs_, zero/engine_setup.h): IQ3_S's 512 entries
     uint32_t grid[512 + 256];  // (and IQ3_XXS's 256 behind them)
@@ -614,8 +615,7 @@ class Engine {
       // work-group the slices are staged one after the other, and 320 groups on 256 work-groups leave a quarter of them
       // two groups and the rest one (8 tokens, us: 5120 x 17408 Q4_K 34.4 -> 22.6, Q6_K 58.0 -> 32.1, Q8_0 34.4 -> 25.7;
       // 17408 x 17408 Q4_K 60.7 -> 44.9; 40960 x 8192 Q4_K 60.9 -> 46.7, Q8_0 69.1 -> 72.5).  Up to 12 groups a compute
-      // unit (ARCZ_GEMV_MM_SK=n: n, 0: never); beyond that, and when the workspace is not to be had, the kernel walks
-      // the slices itself.
+      // unit (ARCZ_GEMV_MM_SK=n: n, 0: never) and SPLIT_BYTES of pieces; beyond that the kernel walks the slices itself.
       static const int sk_env = getenv("ARCZ_GEMV_MM_SK") ? atoi(getenv("ARCZ_GEMV_MM_SK")) : -1;
       static const bool sk_off = sk_env == 0;
       const size_t sk_groups = (size_t)(sk_env > 0 ? sk_env : 12) * cus;
@@ -624,15 +624,7 @@ class Engine {
       const int ny = (nsb + sb_max - 1) / sb_max;
       const size_t need = (size_t)ny * 16 * N * 4;
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
-      if (!sk_off && ny >= 2 && groups <= sk_groups && (!noalloc_ || need <= arcz_mem_size(ws))) {
-        if (!noalloc_ && need > sk_ws_bytes_) {
-          if (sk_ws_) release(sk_ws_);
-          sk_ws_ = nullptr;
-          sk_ws_bytes_ = 0;
-          sk_ws_ = buf(need);
-          sk_ws_bytes_ = need;
-          ws = sk_ws_;
-        }
+      if (!sk_off && ny >= 2 && groups <= sk_groups && need <= SPLIT_BYTES) {
         int zero = 0, ldw = N, s1 = nsb;
         set_args(k, 0, w.raw, N, K, tabs, aq_, asc_, absum_, M, T, ws, ldw, zero, zero, zero, s1);
         size_t g2[2] = {std::min<size_t>(groups, std::max<size_t>(cus / (size_t)ny, 1)) * 512, (size_t)ny}, l2[2] = {512, 1};
@@ -791,6 +783,10 @@ class Engine {
   // rows from 128 tokens on, :521-522).
   // Workspace of the short-chunk GEMM's partial tiles, [slices][Mp][N] f32: allocated with the engine (only a forced
   // piece count, ARCZ_Q4_SPLITK=n read when the engine is made, can outgrow it; then it is replaced by a larger one).
+  // The rules that choose a number of pieces by its price, and gemv_mm's, stay within SPLIT_BYTES, the size of the static
+  // scratch, whatever the workspace at hand holds: the pieces decide in which order f32 sums are added, and the entry
+  // point that works on the static scratch gives the ordinary one's bits on every device and engine.
+  static constexpr size_t SPLIT_BYTES = ARCZ_SCRATCH_BYTES;
   cl_mem sk_ws_ = nullptr;
   size_t sk_ws_bytes_ = 0;
   int sk_force_ = -1;  // ARCZ_Q4_SPLITK: 0 = never share K out, n >= 2: n pieces, -1 = the rule below
@@ -829,12 +825,12 @@ class Engine {
   }
   // Pieces of K, priced as in split_pieces: us per 1024 values of K and full round (two work-groups a compute unit) 18, 25, 32
   // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 123 us.
-  static int digit_pieces(int nw, int Mp, int N, int nsb, size_t ws_bytes) {
+  static int digit_pieces(int nw, int Mp, int N, int nsb) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
     int best = 1;
     double least = 0.0;
     for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
-      if (ny > 1 && (size_t)ny * Mp * N * 4 > ws_bytes) break;
+      if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const size_t full = tiles * ny / (2 * cus), rest = tiles * ny % (2 * cus);
       const double part = rest == 0 ? 0.0 : rest <= cus ? 0.63 : 1.0;
       double us = (full + (full ? 0.85 : 1.0) * part) * (nw == 1 ? 18.0 : nw == 2 ? 25.0 : 32.0) * nsb / 4 / ny;
@@ -868,7 +864,7 @@ class Engine {
       run("row_digits", kr, 2, g, l);
       cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
-      int ny = nt == nt_all ? digit_pieces(f.nw, Mp, N, nsb, noalloc_ ? arcz_mem_size(ws) : sk_ws_bytes_) : 1, zero = 0;
+      int ny = nt == nt_all ? digit_pieces(f.nw, Mp, N, nsb) : 1, zero = 0;
       size_t gg[2] = {(size_t)mt * nt * 256, (size_t)ny};
       if (ny > 1) set_args(k, 0, xd_, wd_, ws, M, N, K, N, zero, zero, n0, nt);
       else set_args(k, 0, xd_, wd_, C, M, N, K, ldc, c_off, a, n0, nt);
@@ -889,13 +885,13 @@ class Engine {
   // written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x both types this costs 0.5 % on
   // average against always knowing (the rule before, three to eight pieces by the tile count alone, 9 %): 300 tokens Q6_K
   // 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86, 4096 x 4096 x 512 39.3 -> 36.9.
-  static int split_pieces(uint32_t type, int Mp, int m64, int N, int nsb, size_t ws_bytes) {
+  static int split_pieces(uint32_t type, int Mp, int m64, int N, int nsb) {
     const bool q8 = type == GGML_Q8_0;
     const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)m64 * ((N + 127) / 128);
     int best = 1;
     double least = 0.0;
     for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
-      if (ny > 1 && (size_t)ny * Mp * N * 4 > ws_bytes) break;
+      if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const size_t full = tiles * ny / slots, rest = tiles * ny % slots;
       const double part = rest == 0 ? 0.0 : rest <= cus ? (q8 ? 0.46 : 0.62) : rest <= 2 * cus ? (q8 ? 0.65 : 1.0) : 1.0;
       double us = (full + (full ? 0.85 : 1.0) * part) * (q8 ? 21.2 : 24.7) * nsb / 4 / ny;
@@ -950,7 +946,7 @@ class Engine {
       const int sk_force = sk_force_;
       int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
       const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
-      if (priced) ny = split_pieces(w.type, Mp, m64, N, nsb, noalloc_ ? arcz_mem_size(arcz_scratch_mem()) : sk_ws_bytes_);
+      if (priced) ny = split_pieces(w.type, Mp, m64, N, nsb);
       if (sk_force >= 2) ny = std::min(sk_force, nsb);
       // (the others from three pieces on)
       if (ny >= (priced || sk_force >= 2 ? 2 : 3)) {

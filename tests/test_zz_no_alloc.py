@@ -103,6 +103,28 @@ def test_noalloc_as_the_first_call_of_a_fresh_engine(rt, qtype, N, K, T, Mp):
         eng.close()
 
 
+def test_noalloc_equals_matmul_whatever_the_workspace_holds(rt, monkeypatch):
+    """An engine whose own workspace has grown past the static scratch (a chunk with eight pieces forced on it, 71 MB):
+    its GEMM on digits, five pieces of 12.6 MB if the workspace allowed them, takes the pieces that the scratch holds, so
+    both entry points add the same sums in the same order."""
+    monkeypatch.setenv("ARCZ_Q4_SPLITK", "8")   # (read when an engine is made)
+    print("noalloc with a grown workspace", flush=True)
+    eng = az.Engine(768, 17408)
+    try:
+        w = eng.make_weight(az.Q4_K, 4352, 5120, make_weights(az.Q4_K, 4352, 5120, seed=6))
+        xb, cb = az.Runtime.from_numpy(make_acts(512, 5120, seed=7)), az.Runtime.alloc(512 * 4352 * 4)
+        before = az.lib.arcz_device_bytes()
+        eng.quantize(xb, 5120, 5120, 512, 512)
+        eng.matmul("grow", w, 512, cb, 4352, 0, 0)
+        assert az.lib.arcz_device_bytes() > before
+        for b in (xb, cb, w):
+            b.free()
+        ya, yb, _, _ = both(eng, az.Q3_K, 4096, 17408, 768, 768, seed=9)
+        assert np.isfinite(ya.view(np.float32)).all() and np.array_equal(ya, yb)
+    finally:
+        eng.close()
+
+
 def test_noalloc_refuses_what_does_not_fit(rt, monkeypatch):
     """Eight pieces forced on a chunk whose partial tiles take 8 x 512 x 4352 x 4 = 71 MB: past the 32 MiB array."""
     monkeypatch.setenv("ARCZ_Q4_SPLITK", "8")   # (read when an engine is made)
