@@ -2310,19 +2310,21 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE13_ACT321_BM128_
   gemm3_body<false, QT_Q5_K>(raw, aq, asc, absum, C + (size_t)y * M * ldc, M, N, K, ldc, 0, 0, s_begin + ns * y / ny,
                              s_begin + ns * (y + 1) / ny, (size_t)N, 0, m0, min(BM, M - m0), n0, nullptr, 0, nullptr, 0);
 }
-// splitk_reduce: C[m][c_off + n] (=, +=, silu(C) *) sum over the ny slices of ws [ny][M][N], slice 0 first.  A thread takes
-// four columns of a row (whole vectors where the strides allow).  Rows from MV on (0: none): zero sums, no partial tile
-// holds them.  grid (ceil(N / 1024) work-groups of 256, M).
+// splitk_reduce: C[m][c_off + n] (=, +=, silu(C) *) sum over the ny slices of ws [ny][M][N], slice 0 first.  wide: a thread
+// takes four columns of a row in whole vectors, which the launcher asks for where N, ldc, c_off and C's address are whole
+// vectors; else one column, neighbours in neighbouring lanes (four single columns a lane, 16 bytes apart, made a
+// matmul of 64 tokens x 4097 rows of Q4_K, K = 4096, 23.3 us instead of 19.7, of 300 tokens x 1025 IQ4_XS rows 29.6 for 22.9).  Rows from MV on (0: none): zero sums, no partial tile holds them.
+// grid (ceil(N / 1024) or ceil(N / 256) work-groups of 256, M).
 extern "C" __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ ws, int ny, float* C, int M, int N,
-                                                                int ldc, int c_off, int accumulate, int MV) {
-  const int n = (blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+                                                                int ldc, int c_off, int accumulate, int wide, int MV) {
+  const int n = (blockIdx.x * 256 + threadIdx.x) * (wide ? 4 : 1), m = blockIdx.y;
   if (n >= N) return;
   const float* w = ws + (size_t)m * N + n;
   float* c = C + (size_t)m * ldc + c_off + n;
   const size_t plane = (size_t)M * N;
   const bool in = MV == 0 || m < MV;
   auto put = [&](float v, float old) { return accumulate == 1 ? v + old : accumulate == 2 ? v * (old / (1.0f + __expf(-old))) : v; };
-  if (((N | ldc | c_off) & 3) == 0) {
+  if (wide) {
     const float4 old = accumulate ? *(const float4*)c : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float4 v = in ? *(const float4*)w : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int y = 1; y < ny && in; ++y) {
@@ -2331,11 +2333,10 @@ extern "C" __global__ __launch_bounds__(256) void splitk_reduce(const float* __r
     }
     *(float4*)c = make_float4(put(v.x, old.x), put(v.y, old.y), put(v.z, old.z), put(v.w, old.w));
   } else {
-    for (int k = 0; k < min(4, N - n); ++k) {
-      float v = in ? w[k] : 0.0f;
-      for (int y = 1; y < ny && in; ++y) v += w[y * plane + k];
-      c[k] = put(v, accumulate ? c[k] : 0.0f);
-    }
+    const float old = accumulate ? *c : 0.0f;
+    float v = in ? *w : 0.0f;
+    for (int y = 1; y < ny && in; ++y) v += w[y * plane];
+    *c = put(v, old);
   }
 }
 // -DBM=64: the 64-token form (grid ceil(N / 128) * ceil(M / 64) work-groups)

@@ -133,6 +133,39 @@ def test_gemm_split_k(eng, qtype, T, Mp, N, K):
     assert np.array_equal(ys[:, :c_off], c0[:, :c_off])
 
 
+@pytest.mark.parametrize("N,ldc,c_off,skip", [(1, 1, 0, 0), (255, 255, 0, 0), (257, 257, 0, 0), (1025, 1025, 0, 0), (1026, 1028, 2, 0),
+                                              (1023, 1030, 7, 0), (1028, 1028, 0, 1), (1028, 1031, 3, 0), (1028, 1032, 4, 0)])
+@pytest.mark.parametrize("acc", [0, 1, 2])
+def test_gemm_split_k_columns(eng, N, ldc, c_off, skip, acc):
+    """The reduction of the partial tiles where rows of C are whole vectors and where they are not (by N, ldc, c_off, or C
+    itself `skip` floats into its buffer): integer sums, so the same bits whichever way, and nothing beside them touched."""
+    T, Mp, K = 40, 48, 4096
+    print(f"split-K columns N={N} ldc={ldc} c_off={c_off} skip={skip} acc={acc}", flush=True)
+    W, wi = unit_scale_weights(az.Q8_0, N, K, seed=98)
+    x = unit_scale_acts(T, K, seed=99)
+    c0 = np.random.default_rng(100).integers(-50, 51, (Mp, ldc)).astype(np.float32)
+    w = eng.make_weight(az.Q8_0, N, K, W)
+    xb = az.Runtime.from_numpy(x)
+    eng.quantize(xb, K, K, Mp, T)
+    cb = az.Runtime.alloc((Mp * ldc + skip) * 4)
+    cv = cb.view(4 * skip, Mp * ldc * 4)
+    cv.write(c0)
+    eng.matmul("test", w, Mp, cv, ldc, c_off, acc)
+    y = cv.read(np.float32, Mp * ldc).reshape(Mp, ldc)
+    for b in (cv, cb, xb, w):
+        b.free()
+    sums = np.zeros((Mp, N))
+    sums[:T] = x.astype(np.int64) @ wi.T
+    old = c0[:, c_off:c_off + N].astype(np.float64)
+    want = sums if acc == 0 else sums + old if acc == 1 else sums * (old / (1.0 + np.exp(-old)))
+    got = y[:, c_off:c_off + N]
+    # (integers below 2^24 for a store and a sum; silu: the product of three f32 roundings and the exponential's, 2^-21)
+    assert np.abs(sums).max() < 2 ** 24
+    assert np.abs(got - want).max() <= (np.abs(want).max() * 2 ** -21 if acc == 2 else 0.0)
+    y[:, c_off:c_off + N] = c0[:, c_off:c_off + N]
+    assert np.array_equal(y, c0)
+
+
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K])
 @pytest.mark.parametrize("T", [64, 32])
 def test_gemm_split_k_unit_scales_exact(eng, qtype, T):
