@@ -872,11 +872,12 @@ class Engine {
       if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
     }
   }
+  // rows: those that the partial tiles hold, 0: all M
   void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a, int rows = 0) {
-    cl_kernel r = kernel("gemm", rows ? "-DMV=" + std::to_string(rows) : std::string(), "splitk_reduce");
+    cl_kernel r = kernel("gemm", "", "splitk_reduce");
     const bool whole = ((N | ldc | c_off) & 3) == 0 && ((uintptr_t)arcz_mem_ptr(C) & 15) == 0;
     int wide = whole ? 1 : 0;
-    set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a, wide);
+    set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a, wide, rows);
     const size_t cols = whole ? 1024 : 256;
     size_t g[2] = {((size_t)N + cols - 1) / cols * 256, (size_t)M}, l[2] = {256, 1};
     run(name, r, 2, g, l);

@@ -90,7 +90,7 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "splitk_reduce", nullptr, "pipiiiiii", {nullptr}, {{"MV", 0, false}, {nullptr, 0, false}}, 256},
+    {"gemm", "splitk_reduce", nullptr, "pipiiiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "moe_gateup_q", "PRE", "ppiipppippppippppppp", {"QT", "QUANT", "PRE", nullptr}, {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "moe_gateup_q", "QUANT", "ppiipppippppippp", {"QT", "QUANT", nullptr}, {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "moe_gateup_q", nullptr, "ppiipppipppp", {"QT", nullptr}, {{"NE", 0, true}, {nullptr, 0, false}}, 256},
