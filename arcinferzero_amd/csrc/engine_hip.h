@@ -1561,10 +1561,10 @@ class Engine {
   std::vector<cl_mem> mems_;
   std::vector<std::pair<std::string, cl_event>> events_;
 };
-// Start-up check in the pattern of the reference's xmx_check (zero/engine_setup.h:424-520): every tuned GEMM the
-// dispatch can take -- for each weight type, storing, accumulating and with the fused SwiGLU epilogue, in one piece
-// and with K shared out over several work-groups per tile -- against the plain kernel of the same type on the
-// reference's LCG data, with unit scales (weights d = 1, sub-scales 1, Q4_K / Q5_K mins 1; activation scales 1) so that
+// Start-up check in the pattern of the reference's xmx_check (zero/engine_setup.h:424-520): the tuned GEMM that the
+// dispatch takes for a chunk of 128 tokens -- for each weight type, storing, accumulating and with the fused SwiGLU
+// epilogue, in one piece and with K shared out over several work-groups per tile -- and the GEMM on digits (one, two and
+// three digits a weight), against the plain kernel of the same type on the reference's LCG data, with unit scales (weights d = 1, sub-scales 1, Q4_K / Q5_K mins 1; activation scales 1) so that
 // every f32 sum is an integer below 2^24: the two results must be bit-equal to each other and, for store and add, to
 // the integer sums counted on the host.  Returns an empty string, or what differed.
 inline std::string engine_self_check() {
@@ -1625,6 +1625,18 @@ inline std::string engine_self_check() {
           blk[64 * n2 + 32 + l] = (uint8_t)((q[1] & 15) | (q[3] & 15) << 4);
           blk[128 + 32 * n2 + l] = (uint8_t)((q[0] >> 4) | (q[1] >> 4) << 2 | (q[2] >> 4) << 4 | (q[3] >> 4) << 6);
         }
+    } else if (type == GGML_Q3_K) {  // 6-bit scales 33 (- 32 = 1): low nibbles 1, high two bits 2; value = three bits - 4
+      memset(blk, 0, 110);
+      memset(blk + 96, 0x11, 8);
+      memset(blk + 104, 0xAA, 4);
+      blk[108] = 0x00; blk[109] = 0x3C;
+      for (int b = 0; b < 8; ++b)
+        for (int l = 0; l < 32; ++l) {
+          const int q = (int)(next() & 7u);
+          blk[32 + 32 * (b / 4) + l] |= (uint8_t)((q & 3) << (2 * (b % 4)));
+          blk[l] |= (uint8_t)((q >> 2) << b);
+          wq[32 * b + l] = q - 4;
+        }
     } else {  // IQ4_XS: 6-bit scales 33 (- 32 = 1): low nibble 1, high two bits 2
       memset(blk, 0, 136);
       blk[0] = 0x00; blk[1] = 0x3C; blk[2] = 0xAA; blk[3] = 0xAA;
@@ -1656,44 +1668,51 @@ inline std::string engine_self_check() {
     cl_mem c0 = e.buf((size_t)M * N * 4), c1 = e.buf((size_t)M * N * 4);
     std::vector<float> y0((size_t)M * N), y1((size_t)M * N), cinit((size_t)M * N);
     for (auto& v : cinit) v = (float)((int)(next() % 9u) - 4);  // small integers: sums with them stay exact
-    for (uint32_t type : {GGML_Q8_0, GGML_Q4_K, GGML_Q5_K, GGML_Q6_K, GGML_IQ4_XS, GGML_Q4_0, GGML_IQ4_NL, GGML_MXFP4}) {
+    for (uint32_t type : {GGML_Q8_0, GGML_Q4_K, GGML_Q5_K, GGML_Q6_K, GGML_IQ4_XS, GGML_Q4_0, GGML_IQ4_NL, GGML_MXFP4, GGML_Q3_K}) {
       const size_t rb = arcz_gguf_bytes(type, 1, K), sbb = rb / (size_t)(K / 256);
       std::vector<uint8_t> w((size_t)N * rb);
       std::vector<int> wq((size_t)N * K);
       for (int n = 0; n < N; ++n)
         for (int sb = 0; sb < K / 256; ++sb) make_sb(type, &w[n * rb + sb * sbb], &wq[(size_t)n * K + sb * 256]);
       GpuWeight gw = e.make_weight(type, w.data(), w.size(), N, K);
-      for (int mode = 0; mode < 3; ++mode) {
-        CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c0, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
-        CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c1, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
-        e.gemm_dense("self_check", gw, M, c0, N, 0, mode);  // the kernel(s) the engine's dispatch takes for this type
-        {
-          cl_kernel k = e.kernel("gemm", "-DQTYPE=" + std::to_string(type) + " -DACT32", "gemm_simple");
-          cl_mem unused = nullptr;
-          int MM = M, NN = N, KK = K, ldc = N, zero = 0, one = 1, s1 = K / 256, md = mode;
-          set_args(k, 0, gw.raw, unused, e.aq_, e.asc_, e.absum_, c1, MM, NN, KK, ldc, zero, md, one, zero, s1);
-          size_t gws[1] = {(size_t)(M / 128) * (N / 128) * 256}, lws[1] = {256};
-          e.run("self_check", k, 1, gws, lws);
+      std::vector<float> sums((size_t)M * N);
+      for (int m = 0; m < M; ++m)
+        for (int n = 0; n < N; ++n) {
+          long long sm = 0;
+          for (int k2 = 0; k2 < K; ++k2) sm += (long long)aq[(size_t)m * K + k2] * wq[(size_t)n * K + k2];
+          sums[(size_t)m * N + n] = (float)sm;
         }
-        CL_CHECK(clEnqueueReadBuffer(e.cl_.queue, c0, CL_TRUE, 0, y0.size() * 4, y0.data(), 0, nullptr, nullptr));
-        CL_CHECK(clEnqueueReadBuffer(e.cl_.queue, c1, CL_TRUE, 0, y1.size() * 4, y1.data(), 0, nullptr, nullptr));
-        for (int m = 0; m < M; ++m)
-          for (int n = 0; n < N; ++n) {
-            long long sm = 0;
-            for (int k2 = 0; k2 < K; ++k2) sm += (long long)aq[(size_t)m * K + k2] * wq[(size_t)n * K + k2];
-            const float a = y0[(size_t)m * N + n], b = y1[(size_t)m * N + n];
-            const float want = mode == 0 ? (float)sm : mode == 1 ? (float)sm + cinit[(size_t)m * N + n] : a;
+      if (e.digit_form(type).nw) e.digits_reserve(gw);  // (the rule takes longer chunks; the kernels are the same)
+      for (int mode = 0; mode < 3; ++mode)
+        for (int digits = 0; digits < (e.digit_form(type).nw ? 2 : 1); ++digits) {
+          CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c0, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
+          CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c1, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
+          if (digits) e.gemm_digits("self_check", gw, M, c0, N, 0, mode);
+          else e.gemm_dense("self_check", gw, M, c0, N, 0, mode);  // the kernel(s) the engine's dispatch takes for this type
+          {
+            const GpuWeight sw = e.gemm_form("self_check", gw);
+            cl_kernel k = e.kernel("gemm", "-DQTYPE=" + std::to_string(sw.type) + " -DACT32", "gemm_simple");
+            cl_mem unused = nullptr;
+            int MM = M, NN = N, KK = K, ldc = N, zero = 0, one = 1, s1 = K / 256, md = mode;
+            set_args(k, 0, sw.raw, unused, e.aq_, e.asc_, e.absum_, c1, MM, NN, KK, ldc, zero, md, one, zero, s1);
+            size_t gws[1] = {(size_t)(M / 128) * (N / 128) * 256}, lws[1] = {256};
+            e.run("self_check", k, 1, gws, lws);
+          }
+          CL_CHECK(clEnqueueReadBuffer(e.cl_.queue, c0, CL_TRUE, 0, y0.size() * 4, y0.data(), 0, nullptr, nullptr));
+          CL_CHECK(clEnqueueReadBuffer(e.cl_.queue, c1, CL_TRUE, 0, y1.size() * 4, y1.data(), 0, nullptr, nullptr));
+          for (size_t i = 0; i < y0.size(); ++i) {
+            const float a = y0[i], b = y1[i], want = mode == 0 ? sums[i] : mode == 1 ? sums[i] + cinit[i] : a;
             uint32_t ab, bb;
             memcpy(&ab, &a, 4);
             memcpy(&bb, &b, 4);
             if (ab != bb || a != want || !std::isfinite(a)) {
               e.free_weight(gw);
-              return std::string("GEMM self-check ") + ggml_type_name(type) + " K=" + std::to_string(K) + " mode " +
-                     std::to_string(mode) + ": token " + std::to_string(m) + " row " + std::to_string(n) + ": tuned " +
-                     std::to_string(a) + ", simple " + std::to_string(b) + ", integer sum " + std::to_string(sm);
+              return std::string("GEMM self-check ") + ggml_type_name(type) + (digits ? " on digits" : "") + " K=" + std::to_string(K) +
+                     " mode " + std::to_string(mode) + ": token " + std::to_string(i / N) + " row " + std::to_string(i % N) + ": tuned " +
+                     std::to_string(a) + ", simple " + std::to_string(b) + ", integer sum " + std::to_string(sums[i]);
             }
           }
-      }
+        }
       e.free_weight(gw);
     }
   }

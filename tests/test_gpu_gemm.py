@@ -334,6 +334,74 @@ def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+def _extreme_rows(qtype, N, K, rng):
+    """Blocks of random bytes with the superblock's scale set to one (IQ3_XXS: four), so that all values are integers; a
+    fifth of the Q6_K and Q3_K rows at the ends of their ranges: every value -32 or 31 times -128 or 127, -4 or 3 times -32
+    or 31, in runs and alternating."""
+    one = np.frombuffer(np.float16(4.0 if qtype == az.IQ3_XXS else 1.0).tobytes(), np.uint8)
+    nsb = K // 256
+    n = az.gguf_bytes(qtype, 1, 256)
+    if qtype in (az.Q4_0, az.MXFP4):
+        blk = rng.integers(0, 256, (N, nsb * 8, n // 8), dtype=np.uint8)
+        if qtype == az.MXFP4:
+            blk[..., 0] = 128
+        else:
+            blk[..., 0:2] = one
+        return np.ascontiguousarray(blk).reshape(-1)
+    blk = rng.integers(0, 256, (N, nsb, n), dtype=np.uint8)
+    ends = np.arange(N) % 5 == 0
+    fill = np.array([0x00, 0xFF, 0xAA, 0x55], np.uint8)[rng.integers(0, 4, (N, nsb))]
+    if qtype == az.Q6_K:
+        blk[ends, :, :192] = np.where(rng.integers(0, 2, (N, nsb)) == 1, fill, 0)[ends][..., None]
+        blk[ends, :, 192:208] = np.where(rng.integers(0, 2, (N, nsb, 16)) == 1, 128, 127).astype(np.uint8)[ends]
+        blk[..., 208:210] = one
+    elif qtype == az.Q3_K:
+        blk[ends, :, :96] = fill[ends][..., None]
+        blk[ends, :, 96:108] = np.array([0x00, 0xFF], np.uint8)[rng.integers(0, 2, (N, nsb))][ends][..., None]
+        blk[..., 108:110] = one
+    else:
+        blk[..., 0:2] = one
+    return blk.reshape(-1)
+
+
+@pytest.mark.parametrize("qtype,T,N", [(az.Q6_K, 1024, 7808), (az.Q3_K, 256, 4224), (az.IQ3_XXS, 1024, 8192), (az.IQ3_S, 256, 12288),
+                                       (az.Q4_0, 256, 12288), (az.MXFP4, 256, 12288)])
+def test_gemm_on_digits_block_sums_exact(rt, qtype, T, N):
+    """The GEMM on digits keeps every block sum exact, at the ends of the ranges too: a token has one block of values up to
+    -128 (all ends, alternating ends, random ends, random) and zeros elsewhere, unit scales, so an output is one block's
+    sum -- up to 32 x 128 x 4096 = 2^24, with whole and partial cancellation -- and has to be that integer."""
+    print(f"digits, exact block sums {TYPE_NAMES[qtype]} T={T} N={N}", flush=True)
+    K = 512
+    rng = np.random.default_rng(170 + qtype)
+    W = _extreme_rows(qtype, N, K, rng)
+    wi = orc.dequant_rows(qtype, W, N, K).astype(np.float64)
+    assert np.array_equal(wi, np.round(wi))
+    if qtype in (az.Q6_K, az.Q3_K):
+        assert np.abs(wi).max() == (4096 if qtype == az.Q6_K else 128)
+    aq = np.zeros((T, K // 32, 32), np.int8)
+    for t in range(T):
+        i = np.arange(32)
+        v = [np.full(32, 127), np.full(32, -128), np.where(i & 1, 127, -127), np.where(i < 16, -128, 127), np.where(i & 2, -127, 127),
+             np.where(rng.integers(0, 2, 32) == 1, 127, -128), rng.integers(-128, 128, 32), np.where(i & 1, 1, -128)][(t // (K // 32)) % 8]
+        aq[t, t % (K // 32)] = v
+    aq = aq.reshape(T, K)
+    asc = np.ones((K // 32, T), np.float32)
+    absum = np.ascontiguousarray(aq.reshape(T, K // 16, 16).sum(axis=2, dtype=np.int64).astype(np.int16).T)
+    eng = az.Engine(T, K)
+    w = eng.make_weight(qtype, N, K, W)
+    eng.set_activations(aq, asc, absum, K, T, T)
+    cb = az.Runtime.alloc(T * N * 4).fill(0xFFFFFFFF)
+    eng.matmul("test", w, T, cb, N, 0, 0)
+    y = cb.read(np.float32, T * N).reshape(T, N)
+    for b in (cb, w):
+        b.free()
+    eng.close()
+    want = aq.astype(np.float64) @ wi.T
+    assert np.abs(want).max() <= 2 ** 24
+    print(f"  largest sum {np.abs(want).max():.0f}, differing {int((y != want).sum())} of {y.size}", flush=True)
+    assert np.array_equal(y, want.astype(np.float32))
+
+
 @pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512)])
 @pytest.mark.parametrize("before", [None, 256, 1024])
 def test_weights_of_another_engine(rt, qtype, T, N, K, before):
