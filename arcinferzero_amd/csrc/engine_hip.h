@@ -78,7 +78,11 @@ class Engine {
     // the expert layer's launch-rule switches, read when the engine is made (a one-token layer is 16 us: nothing of
     // the environment is looked up per call)
     moe_dec_off_ = getenv("ARCZ_MOE_DECODE") && atoi(getenv("ARCZ_MOE_DECODE")) == 0;
-    moe_dec_max_ = getenv("ARCZ_MOE_DECODE_MAX") ? atoi(getenv("ARCZ_MOE_DECODE_MAX")) : 16;
+    moe_dec_set_ = getenv("ARCZ_MOE_DECODE_MAX") != nullptr;
+    moe_dec_max_ = moe_dec_set_ ? atoi(getenv("ARCZ_MOE_DECODE_MAX")) : 16;
+    moe_mm_off_ = moe_dec_off_ || (getenv("ARCZ_MOE_MM") && atoi(getenv("ARCZ_MOE_MM")) == 0);
+    digits_off_ = getenv("ARCZ_GEMM_DIGITS") && atoi(getenv("ARCZ_GEMM_DIGITS")) == 0;
+    gemm_split_ = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
     moe_fuse_off_ = getenv("ARCZ_MOE_FUSE") && atoi(getenv("ARCZ_MOE_FUSE")) == 0;
     moe_qfuse_off_ = getenv("ARCZ_MOE_QFUSE") && atoi(getenv("ARCZ_MOE_QFUSE")) == 0;
@@ -792,6 +796,9 @@ class Engine {
   int sk_force_ = -1;  // ARCZ_Q4_SPLITK: 0 = never share K out, n >= 2: n pieces, -1 = the rule below
   bool moe_dec_off_ = false, moe_fuse_off_ = false, moe_qfuse_off_ = false;  // ARCZ_MOE_DECODE / _FUSE / _QFUSE = 0
   int moe_dec_max_ = 16, moe_tmd_ = 0;                                      // ARCZ_MOE_DECODE_MAX, ARCZ_MOE_TMD
+  bool moe_dec_set_ = false, moe_mm_off_ = false;                           // ARCZ_MOE_DECODE_MAX given; ARCZ_MOE_MM = 0
+  bool digits_off_ = false;                                                 // ARCZ_GEMM_DIGITS = 0
+  int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
   bool moe_pre_ = true;                                                     // ARCZ_MOE_PRE (0: off)
   // (The gate / up tile kernel on ready-made scale vectors runs in steps of 64 values, three work-groups a compute unit:
@@ -813,8 +820,9 @@ class Engine {
   // IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows: Q6_K 98 / 103, 97.5 / 89 (of 2048), 277 / 234; IQ3_XXS 77 / 76,
   // -, 193 / 186.
   bool digits_take(uint32_t type, int Mp, int N) const {
+    // (ARCZ_GEMM_DIGITS=0: never; nor with ARCZ_GEMM_SPLIT, whose pieces are the int8 kernels')
     const double out = (double)Mp * N / (1 << 20);
-    if (Mp < 256) return false;
+    if (Mp < 256 || digits_off_ || gemm_split_ > 0) return false;
     switch (type) {
       case GGML_Q3_K: return out >= 1.0;
       case GGML_Q4_0: case GGML_MXFP4: case GGML_IQ3_S: return out >= 3.0;
@@ -864,7 +872,10 @@ class Engine {
       run("row_digits", kr, 2, g, l);
       cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
-      int ny = nt == nt_all ? digit_pieces(f.nw, Mp, N, nsb) : 1, zero = 0;
+      // (ARCZ_Q4_SPLITK=0: K in one piece, =n: n pieces, as many as SPLIT_BYTES holds)
+      int ny = nt < nt_all || sk_force_ == 0 ? 1
+               : sk_force_ >= 2 ? std::max(1, (int)std::min<size_t>(std::min(sk_force_, nsb), SPLIT_BYTES / ((size_t)Mp * N * 4)))
+                                : digit_pieces(f.nw, Mp, N, nsb), zero = 0;
       size_t gg[2] = {(size_t)mt * nt * 256, (size_t)ny};
       if (ny > 1) set_args(k, 0, xd_, wd_, ws, M, N, K, N, zero, zero, n0, nt);
       else set_args(k, 0, xd_, wd_, C, M, N, K, ldc, c_off, a, n0, nt);
@@ -1063,8 +1074,7 @@ class Engine {
     // (ARCZ_GEMM_SPLIT: superblocks per split-K piece, 0 = one pass, the default here: a work-group keeps its sums in
     //  registers over the whole of K.  The reference splits rows longer than 8192 into 17-superblock pieces for its
     //  cache, zero/engine.h:1236-1250; pieces after the first accumulate into C and are not bit-identical to one pass.)
-    static const int sk_sb = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
-    const int nsb = K / 256, splits = a != 2 && sk_sb > 0 ? (nsb + sk_sb - 1) / sk_sb : 1, rgroup = 1;
+    const int nsb = K / 256, splits = a != 2 && gemm_split_ > 0 ? (nsb + gemm_split_ - 1) / gemm_split_ : 1, rgroup = 1;
     cl_mem unused = nullptr;
     const int bm = wm4 ? 256 : w.type == GGML_Q6_K || q8_small || q4_wide || q4_small ? 64 : 128;  // token rows of a work-group's tile
     const int bn = q4_wide && !q4_small ? 256 : 128;
@@ -1398,13 +1408,14 @@ class Engine {
     // A pass of 1-16 tokens (zero/engine_moe.h:86-262 has this form for 1-8): small tiles through the matrix-vector
     // kernels moe_gateup_q / moe_down_q, routed by one launch (moe_route1 for one token, whose NU experts are the tiles;
     // moe_route_small for more) instead of the 64-slot tile GEMMs, which for one token walked K alone in 8 x 6
-    // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings that back, ARCZ_MOE_DECODE_MAX
+    // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings those back, ARCZ_MOE_DECODE_MAX
     // moves the limit).
     // (the switches of this function are read when the engine is made: a test sets them before it makes its engine)
-    const bool dec_off = moe_dec_off_;
-    const int dec_max = moe_dec_max_;
-    if (moe_mm_takes(L, T) && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
-    if (!dec_off && T <= dec_max && T * NU <= 512) {
+    // From 6 or 9 tokens on the 16-slot tiles take over (moe_mm_takes) -- not where ARCZ_MOE_DECODE_MAX is given and names
+    // the pass, nor with ARCZ_MOE_DECODE=0 or ARCZ_MOE_MM=0.
+    const bool one_slot = !moe_dec_off_ && T <= moe_dec_max_ && T * NU <= 512;
+    if (!moe_mm_off_ && !(one_slot && moe_dec_set_) && moe_mm_takes(L, T) && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
+    if (one_slot) {
       const int NE = L.NE;
       // (one-slot tiles at every count: eight tokens' 64 pairs hit about 50 experts, so a tile of 8 slots holds 1.3 on
       //  average, and the one-slot kernels are the light ones: 71 us a layer against 113 with 8-slot tiles, 45 against

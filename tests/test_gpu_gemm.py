@@ -334,6 +334,29 @@ def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
+                                                 ({"ARCZ_Q4_SPLITK": "2"}, 1, 2),
+                                                 ({"ARCZ_GEMM_SPLIT": "1", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])
+def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
+    """The launch-rule switches on a chunk that the digits take by rule: off, K in one piece, two pieces forced (the
+    product and its reduction), and the int8 kernels in pieces of superblocks (one expansion and a launch a piece)."""
+    T, N, K = 256, 4224, 768
+    print(f"digits switches {env}", flush=True)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)          # (read when an engine is made)
+    W = make_weights(az.Q3_K, N, K, seed=87)
+    x = make_acts(T, K, seed=88, outliers=True)
+    eng = az.Engine(T, K)
+    eng.profile(True)
+    y = run_gemm(eng, az.Q3_K, W, N, K, x, T)
+    eng.profile_collect()
+    counts = [eng.profile_get(k)[1] for k in ("act_digits", "test")]
+    eng.close()
+    aq, asc, _ = quantize_padded(x, T)
+    assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(az.Q3_K, W, N, K, aq, asc)).max() <= TOL
+    assert counts[0] == digits and products in (None, counts[1]), counts
+
+
 def _extreme_rows(qtype, N, K, rng):
     """Blocks of random bytes with the superblock's scale set to one (IQ3_XXS: four), so that all values are integers; a
     fifth of the Q6_K and Q3_K rows at the ends of their ranges: every value -32 or 31 times -128 or 127, -4 or 3 times -32

@@ -92,8 +92,8 @@ def test_routing_and_sort(rt, NE, NU, T, tm):
                                                    (az.Q3_K, 4, 2, 256, 512, 3, 16), (az.Q3_K, 6, 2, 512, 256, 70, 80),
                                                    # IQ3_S experts (uploaded as Q6_K planes): one token and a tile pass
                                                    (az.IQ3_S, 4, 2, 256, 512, 1, 16), (az.IQ3_S, 6, 2, 512, 256, 40, 48),
-                                                   # 9-16 tokens: still the matrix-vector form, the routing kernel's waves
-                                                   # take two tokens each; 17: the tile GEMMs
+                                                   # 16 tokens on 16-slot tiles, 11 (33 pairs) in the matrix-vector form,
+                                                   # whose routing kernel's waves take two tokens each
                                                    (az.Q4_K, 128, 8, 512, 256, 16, 16), (az.Q6_K, 8, 3, 256, 256, 11, 16),
                                                    (az.Q4_K, 16, 4, 512, 256, 17, 32)])
 def test_moe_layer_vs_oracle(rt, qtype, NE, NU, E, F, T, Mp):
@@ -111,6 +111,22 @@ def test_moe_small_pass_other_forms(rt, monkeypatch, env, qtype, NE, NU, E, F, T
     for k, v in env.items():
         monkeypatch.setenv(k, v)
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 16)
+
+
+@pytest.mark.parametrize("env", [{"ARCZ_MOE_MM": "0"}, {"ARCZ_MOE_DECODE_MAX": "16"}, {"ARCZ_MOE_DECODE": "0"}])
+@pytest.mark.parametrize("qtype,NE,NU,E,F,T", [(az.Q4_K, 16, 8, 512, 256, 6), (az.Q6_K, 16, 8, 512, 256, 16), (az.IQ4_XS, 16, 8, 256, 512, 13),
+                                               (az.Q8_0, 32, 8, 512, 256, 16)])
+def test_moe_forms_in_place_of_the_16_slot_tiles(rt, monkeypatch, env, qtype, NE, NU, E, F, T):
+    """Passes that the 16-slot tiles take by rule, sent back to the one-slot kernels (ARCZ_MOE_MM=0, or
+    ARCZ_MOE_DECODE_MAX naming them: gate / up, down and the combination in one launch each) and to the tile GEMMs
+    (ARCZ_MOE_DECODE=0: routing in three launches)."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    counts = _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 16)
+    if "ARCZ_MOE_DECODE" in env:
+        assert counts["moe_scan"] == 1 and counts["moe_combine"] == 1
+    else:   # (one-slot tiles: the down kernel adds a token's experts up itself)
+        assert counts["moe_scan"] == 0 and counts["moe_gateup"] == 1 and counts["moe_down"] == 1 and counts["moe_combine"] == 0
 
 
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q8_0, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q3_K, az.IQ3_S,
@@ -203,7 +219,10 @@ def _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, Mp):
         lb = az.Runtime.from_numpy(logits)
         x0 = az.gen_normal(9, (T, E))
         ob = az.Runtime.from_numpy(x0)
+        eng.profile(True)
         eng.layer_moe(L, lb, NE, ob, T, Mp)
+        eng.profile_collect()
+        counts = {k: eng.profile_get(k)[1] for k in ("moe_route", "moe_scan", "moe_gateup", "moe_down", "moe_combine")}
         out = ob.read(np.float32, T * E).reshape(T, E)
         aq, asc, _ = quantize_padded(x, Mp)
         ref, href = orc.moe_layer(qtype, Wg, Wu, Wd, NE, NU, E, F, aq[:T], asc, logits)
@@ -264,6 +283,7 @@ def _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, Mp):
         assert np.array_equal(hbs[:, used].T, rq.astype(np.int32).reshape(len(used), F // 16, 16).sum(axis=2))
         for b in (xb, lb, ob):
             b.free()
+        return counts
     finally:
         eng.close()
 
