@@ -159,7 +159,7 @@ class Engine {
       if (*v) { release(*v); *v = nullptr; }
     release(aq_); release(asc_); release(absum_);
     q2mm_ = on;
-    cur_T_ = cur_K_ = cur_Mp_ = 0;
+    cur_T_ = cur_K_ = cur_Mp_ = cur_rows_ = 0;
     alloc_activations();
     q2_defs_.clear();
     q2_aq_ = q2_sc_ = q2_ab_ = 0;
@@ -191,7 +191,12 @@ class Engine {
 
   int max_chunk, max_k;
   cl_mem aq_ = nullptr, asc_ = nullptr, absum_ = nullptr;
-  int cur_T_ = 0, cur_K_ = 0, cur_Mp_ = 0;
+  // The current chunk.  cur_rows_: its first rows, the others being zeros -- T behind the quantizing kernels, which write
+  // the padding as zeros, all Mp behind set_activations, whose rows are the caller's.
+  int cur_T_ = 0, cur_K_ = 0, cur_Mp_ = 0, cur_rows_ = 0;
+  void chunk_is(int K, int Mp, int T, int rows, int act32) {
+    cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_rows_ = rows; cur_act32_ = act32 ? 1 : 0;
+  }
 
   cl_mem buf(size_t bytes, const void* host = nullptr) {
     cl_mem m = cl_.buffer(CL_MEM_READ_WRITE, bytes, host);
@@ -357,7 +362,7 @@ class Engine {
     set_args(k, 0, x, ldx, K, Mp, T, aq_, asc_, absum_, act32, rows);
     size_t gws[2] = {(size_t)256 * (K / 256), (size_t)((Mp + rows - 1) / rows)}, lws[2] = {256, 1};
     run("quant_rows", k, 2, gws, lws);
-    cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_act32_ = act32 ? 1 : 0;
+    chunk_is(K, Mp, T, T, act32);
   }
   // The fused producers of the reference (rmsnorm_quant, zero/engine.h:1256-1267; swiglu_quant via run_rows_quant,
   // zero/engine.h:1404-1440): a work-group per row of the chunk, or -- a pass of 1-8 tokens -- the valid rows only,
@@ -386,7 +391,7 @@ class Engine {
       gws[1] = (size_t)(wide_rows(T) ? T : Mp);
     }
     run("rmsnorm_quant", k, 2, gws, lws);
-    cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_act32_ = act32 ? 1 : 0;
+    chunk_is(K, Mp, T, T, act32);
   }
   // gu: rows [gate(F) | up(F)] f32, or rows of F values when the matmul before has fused the product
   void swiglu_quant(cl_mem gu, int F, int Mp, int T, int act32, int fused, int gelu) {
@@ -405,7 +410,7 @@ class Engine {
       gws[1] = (size_t)((Mp + rows - 1) / rows);
     }
     run("swiglu_quant", k, 2, gws, lws);
-    cur_T_ = T; cur_K_ = F; cur_Mp_ = Mp; cur_act32_ = act32 ? 1 : 0;
+    chunk_is(F, Mp, T, T, act32);
   }
   // x = (x + rmsnorm(t) * w) * s over the first T rows ([T][K] f32 each), then the next matmul's input from the new x:
   // rmsnorm(x) * w2, or x itself with norm2 = false (zero/engine.h:1393-1403 add_norm_quant, whose x_ and big_ are the
@@ -423,16 +428,17 @@ class Engine {
     // (a pass of 1-8 tokens: the valid rows only, as the reference; a longer chunk: all Mp rows, the padding as zeros)
     size_t gws[2] = {256, (size_t)(wide_rows(T) ? T : Mp)}, lws[2] = {256, 1};
     run("add_rmsnorm", k, 2, gws, lws);
-    cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_act32_ = act32 ? 1 : 0;
+    chunk_is(K, Mp, T, T, act32);
   }
-  // Activations quantized elsewhere (the reference's benches quantize on the host, bench/gemv_bench.cpp:103-129).
+  // Activations quantized elsewhere (the reference's benches quantize on the host, bench/gemv_bench.cpp:103-129).  All Mp
+  // rows are the caller's: with more than 8 tokens every row is multiplied as it is given, the padding too.
   void set_activations(const int8_t* aq, const float* asc, const int16_t* absum, int K, int Mp, int T) {
     check_chunk(K, Mp, T);
     if (q2mm_) throw std::runtime_error("set_activations: a two-pass engine takes its inputs from the quantizing kernels");
     CL_CHECK(clEnqueueWriteBuffer(cl_.queue, aq_, CL_TRUE, 0, (size_t)Mp * K, aq, 0, nullptr, nullptr));
     CL_CHECK(clEnqueueWriteBuffer(cl_.queue, asc_, CL_TRUE, 0, (size_t)Mp * (K / 32) * 4, asc, 0, nullptr, nullptr));
     CL_CHECK(clEnqueueWriteBuffer(cl_.queue, absum_, CL_TRUE, 0, (size_t)Mp * (K / 16) * 2, absum, 0, nullptr, nullptr));
-    cur_T_ = T; cur_K_ = K; cur_Mp_ = Mp; cur_act32_ = 1;
+    chunk_is(K, Mp, T, Mp, 1);
   }
 
   // ---- matmul (zero/engine.h:1080-1112): C[:, c_off : c_off+N] (+)= act * W^T for the current chunk.  acc: 0 = store,
@@ -608,7 +614,7 @@ class Engine {
                          w.type == GGML_MXFP4 || w.type == GGML_Q3_K || w.type == GGML_IQ3_XXS;
     const bool mm_ok = !mm_off && !q2mm_ && mm_type && a <= 1 && w.softcap <= 0.0f;  // (gemv_mm has no soft cap)
     auto gemv_mm = [&] {
-      int N = w.N, K = w.K, M = Mp, T = cur_T_;
+      int N = w.N, K = w.K, M = Mp, T = cur_T_ > 8 ? cur_rows_ : cur_T_;
       rd_bytes += raw_bytes(w);
       // (the form for at most eight tokens; the three-bit types have the one form)
       const bool t8 = T <= 8 && w.type != GGML_IQ3_S && w.type != GGML_Q3_K && w.type != GGML_IQ3_XXS;
@@ -940,8 +946,8 @@ class Engine {
     }
     const GpuWeight w = gemm_form(name, w0);
     int M = Mp, N = w.N, K = w.K;
-    // (the 64-token tiles that hold a token: the others are padding, whose results are zeros)
-    const int m64 = (std::clamp(cur_T_, 1, Mp) + 63) / 64, M64 = std::min(Mp, m64 * 64);
+    // (the 64-token tiles that hold more than zeros: the others are padding, whose results are zeros)
+    const int m64 = (std::clamp(cur_rows_, 1, Mp) + 63) / 64, M64 = std::min(Mp, m64 * 64);
     // Any type, a chunk so short that its tiles are fewer than two per compute unit: K is shared out over `ny`
     // work-groups per tile, which store partial tiles in a workspace, and splitk_reduce adds the slices in order (the
     // same bits on every run) and applies c_off and the accumulate mode.  One work-group needs 75 us for K = 5120, so

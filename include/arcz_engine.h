@@ -89,7 +89,8 @@ int arcz_engine_two_pass(arcz_engine* e, int on);
 /* The second halves (0 = int8 values, 1 = scales, 2 = 16-sums) as views, NULL in one-pass mode. */
 arcz_mem* arcz_engine_residual(arcz_engine* e, int which);
 /* Activations quantized by the caller, as the reference's benches do (bench/gemv_bench.cpp:103-129).  One-pass engines
- * only. */
+ * only.  All Mp rows are taken as they are given: a matmul of more than 8 tokens multiplies the rows from T on too (rows
+ * of zeros give zeros, as the quantizing calls above write them), one of 1-8 tokens reads and writes the first T alone. */
 int arcz_engine_set_activations(arcz_engine* e, const int8_t* aq, const float* asc, const int16_t* absum, int K, int Mp,
                                 int T);
 /* The engine's activation buffers (Engine::aq_, asc_, absum_; zero/engine_sessions.h:571). */

@@ -334,6 +334,27 @@ def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
     assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("qtype,T,Mp,N,K", [(az.Q6_K, 20, 256, 1000, 768), (az.Q8_0, 20, 256, 3000, 512), (az.Q8_0, 60, 384, 256, 4096),
+                                            (az.Q4_K, 20, 384, 5200, 512), (az.Q4_K, 130, 256, 392, 2048), (az.Q3_K, 100, 256, 4224, 256),
+                                            (az.Q4_K, 10, 16, 264, 1024), (az.Q5_K, 12, 16, 264, 6400), (az.IQ4_XS, 40, 256, 300, 512)])
+def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
+    """set_activations takes all Mp rows from the caller: in a chunk of more than 8 tokens the rows from T on are multiplied
+    like the others, whatever form the launch rule takes (tiles left out, K in pieces, digits, gemv_mm)."""
+    print(f"caller's rows {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=89)
+    aq, asc, absum = orc.quantize_act(make_acts(Mp, K, seed=90, outliers=True))
+    eng = az.Engine(Mp, K)
+    w = eng.make_weight(qtype, N, K, W)
+    cb = az.Runtime.alloc(Mp * N * 4).fill(0xFFFFFFFF)
+    eng.set_activations(aq, asc, absum, K, Mp, T)
+    eng.matmul("test", w, Mp, cb, N, 0, 0)
+    y = cb.read(np.float32, Mp * N).reshape(Mp, N)
+    for b in (cb, w):
+        b.free()
+    eng.close()
+    assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
+
+
 @pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
                                                  ({"ARCZ_Q4_SPLITK": "2"}, 1, 2),
                                                  ({"ARCZ_GEMM_SPLIT": "1", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])
