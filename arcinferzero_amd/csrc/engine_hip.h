@@ -1324,18 +1324,46 @@ class Engine {
   }
 
   // Passes between the one-slot kernels, whose time goes with the pairs, and the tile GEMM, whose work-groups take about the
-  // same time however few slots a tile has: the matrix-pipe kernels of 16-slot tiles.  us a layer, one-slot or tile GEMM
-  // against these: 128 x 8 experts of 768 x 2048, 4 tokens Q4_K 40 / 49, Q6_K 53 / 60; 6: Q4_K 51 / 51, Q6_K 73 / 62, IQ4_XS
-  // 54 / 58; 8: Q4_K 63 / 61, Q6_K 89 / 84, IQ4_XS 68 / 72; 200: 175 / 148, 291 / 216, 336 / 167; 300: 182 / 192, 301 / 277,
-  // 359 / 221; 64 x 8 of 1536 x 3072, 4 tokens Q4_K 81 / 86, 6: Q4_K 111 / 91, IQ4_NL 102 / 107; 32 x 4, 8 tokens Q4_K 41 /
-  // 47, 12: 54 / 47.  So from 48 pairs on, and 6 tokens for Q4_K - Q6_K, whose one-slot kernels are the heavier, 9 tokens for
-  // the others.  The upper end is in slots an expert, where the type's tile GEMM overtakes: Q4_K 14 - 19, Q5_K 16, Q6_K 24,
-  // the others 36 - 45.
+  // same time however few slots a tile has: the matrix-pipe kernels of 16-slot tiles.  From 48 pairs on, and 6 tokens for
+  // Q4_K - Q6_K, whose one-slot kernels are the heavier, 9 tokens for the others.  The upper end is in slots an expert, where
+  // the type's tile GEMM overtakes (Q4_K 14 - 19, Q5_K 16, Q6_K 24, the others 36 - 45; 128 x 8 experts of 768 x 2048, us a
+  // layer, tile GEMM against these, 200 tokens: Q4_K 175 / 148, Q6_K 291 / 216, IQ4_XS 336 / 167; 300: Q4_K 182 / 192).
   static bool moe_mm_takes(const MoeLayer& L, int T) {
     const uint32_t t = L.ex[0].type;
     const int most = t == GGML_Q4_K || t == GGML_Q5_K ? 15 : t == GGML_Q6_K ? 22 : 36;
     const bool kq = t == GGML_Q4_K || t == GGML_Q5_K || t == GGML_Q6_K;
     return T > (kq ? 5 : 8) && T * L.NU >= 48 && T * L.NU <= L.NE * most;
+  }
+  // Against the one-slot kernels, where those take the pass too (up to 16 tokens): they go with the pairs' values, in 2^20;
+  // the 16-slot kernels with what a compute unit is given, a work-group's rows of K values -- its length where the tiles
+  // make fewer work-groups than there are compute units -- of the gate / up kernel and, 0.37 as heavy, the down kernel, times
+  // the type's price.  Fitted to a sweep of six layers x eleven types x 6 - 16 tokens (411 passes): 0.4 % lost on average
+  // against always knowing, where 48 pairs alone lost 6.8 %.  us a layer, one-slot / 16-slot, 128 x 8 of 768 x 2048, 9 tokens:
+  // Q4_K 56 / 52, IQ4_XS 62 / 61, Q8_0 64 / 70, Q4_0 44 / 51, Q3_K 60 / 89, IQ3_XXS 52 / 81, 16 tokens: Q4_K 91 / 63, Q4_0
+  // 65 / 63, Q3_K 94 / 111; 64 x 8 of 1536 x 3072, 12 tokens: Q4_K 177 / 115, Q8_0 188 / 156, Q3_K 212 / 207; 64 x 4 of 512 x
+  // 1024, 16 tokens: Q4_K 30 / 29, Q4_0 23 / 28, IQ3_S 40 / 41; 16 x 8 of 256 x 512, 8: Q4_K 16 / 25 (rows of fewer than 1024
+  // values cost as much).
+  static bool moe_mm_cheaper(const MoeLayer& L, int T) {
+    double price = 30.0;
+    switch (L.ex[0].type) {
+      case GGML_Q5_K: case GGML_Q6_K: price = 27.0; break;
+      case GGML_IQ3_S: price = 38.0; break;
+      case GGML_IQ4_NL: case GGML_MXFP4: case GGML_Q8_0: price = 39.0; break;
+      case GGML_Q4_0: price = 43.0; break;
+      case GGML_Q3_K: case GGML_IQ3_XXS: price = 47.0; break;
+    }
+    const double cus = arcz_device_cus(), tiles = L.NE * (1.0 - std::pow(1.0 - (double)L.NU / L.NE, T));
+    const int gpw = moe_down_groups(L.E);
+    const double gu = std::max(L.E, 1024) / 1024.0 * std::max(1.0, tiles * (L.F / 128) / cus);
+    const double dn = gpw * L.F / 1024.0 * std::max(1.0, tiles * (L.E / (128 * gpw)) / cus);
+    return price * (gu + 0.37 * dn) < (double)T * L.NU * L.E * L.F / (1 << 20) + 20.0;
+  }
+  // (groups of 16 rows a wave of the down kernel: K is short, so several behind one staging of the tokens; 40 tokens at
+  //  2048 x 768: 138, 125, 123, 127 us a layer with 1, 2, 4, 8)
+  static int moe_down_groups(int E) {
+    int gpw = 4;
+    while (E % (128 * gpw)) gpw >>= 1;
+    return gpw;
   }
   // LDS of an expert kernel on the matrix pipe (decode_mm.hip's MmL): tokens of K values, the waves' pieces, the epilogue's
   // rows, the codebook; 0: K does not fit
@@ -1365,10 +1393,7 @@ class Engine {
       run("moe_gateup", k, 2, gws, lws);
     }
     {
-      // (groups of 16 rows a wave: K is short, so several behind one staging of the tokens; 40 tokens at 2048 x 768: 138,
-      //  125, 123, 127 us a layer with 1, 2, 4, 8)
-      int gpw = 4;
-      while (E % (128 * gpw)) gpw >>= 1;
+      const int gpw = moe_down_groups(E);
       cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[2].type) + ne + " -DLDS=" + std::to_string(ld), "moe_down_mm");
       int NN = E, KK = F, S = slots_;
       set_args(k, 0, L.ex[2].raw, NN, KK, tabs, mhq_, mhsc_, S, mtiles_, swt_, my_, mhbs_, gpw);
@@ -1417,10 +1442,11 @@ class Engine {
     // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings those back, ARCZ_MOE_DECODE_MAX
     // moves the limit).
     // (the switches of this function are read when the engine is made: a test sets them before it makes its engine)
-    // From 6 or 9 tokens on the 16-slot tiles take over (moe_mm_takes) -- not where ARCZ_MOE_DECODE_MAX is given and names
+    // From 6 or 9 tokens on the 16-slot tiles take over where they are cheaper (moe_mm_takes, moe_mm_cheaper) -- not where ARCZ_MOE_DECODE_MAX is given and names
     // the pass, nor with ARCZ_MOE_DECODE=0 or ARCZ_MOE_MM=0.
     const bool one_slot = !moe_dec_off_ && T <= moe_dec_max_ && T * NU <= 512;
-    if (!moe_mm_off_ && !(one_slot && moe_dec_set_) && moe_mm_takes(L, T) && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
+    const bool mm = !moe_mm_off_ && moe_mm_takes(L, T) && (!one_slot || (!moe_dec_set_ && moe_mm_cheaper(L, T)));
+    if (mm && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
     if (one_slot) {
       const int NE = L.NE;
       // (one-slot tiles at every count: eight tokens' 64 pairs hit about 50 experts, so a tile of 8 slots holds 1.3 on

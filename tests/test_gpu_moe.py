@@ -92,8 +92,8 @@ def test_routing_and_sort(rt, NE, NU, T, tm):
                                                    (az.Q3_K, 4, 2, 256, 512, 3, 16), (az.Q3_K, 6, 2, 512, 256, 70, 80),
                                                    # IQ3_S experts (uploaded as Q6_K planes): one token and a tile pass
                                                    (az.IQ3_S, 4, 2, 256, 512, 1, 16), (az.IQ3_S, 6, 2, 512, 256, 40, 48),
-                                                   # 16 tokens on 16-slot tiles, 11 (33 pairs) in the matrix-vector form,
-                                                   # whose routing kernel's waves take two tokens each
+                                                   # 9-16 tokens: the matrix-vector form, the routing kernel's waves take
+                                                   # two tokens each, or 16-slot tiles; 17: these or the tile GEMMs
                                                    (az.Q4_K, 128, 8, 512, 256, 16, 16), (az.Q6_K, 8, 3, 256, 256, 11, 16),
                                                    (az.Q4_K, 16, 4, 512, 256, 17, 32)])
 def test_moe_layer_vs_oracle(rt, qtype, NE, NU, E, F, T, Mp):
@@ -111,6 +111,33 @@ def test_moe_small_pass_other_forms(rt, monkeypatch, env, qtype, NE, NU, E, F, T
     for k, v in env.items():
         monkeypatch.setenv(k, v)
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 16)
+
+
+@pytest.mark.parametrize("qtype,NE,NU,E,F,T,mm", [(az.Q3_K, 128, 8, 2048, 768, 9, False), (az.IQ3_XXS, 128, 8, 2048, 768, 9, False),
+                                                  (az.Q4_0, 64, 4, 1024, 512, 16, False), (az.Q4_K, 128, 8, 2048, 768, 9, True),
+                                                  (az.IQ3_S, 32, 4, 2816, 1024, 13, True), (az.Q8_0, 32, 8, 1024, 1536, 10, False),
+                                                  (az.Q8_0, 32, 8, 1024, 1536, 15, True), (az.Q3_K, 64, 4, 1024, 512, 17, True),
+                                                  (az.Q4_K, 16, 8, 512, 256, 8, False)])
+def test_moe_16_slot_tiles_where_they_are_cheaper(rt, qtype, NE, NU, E, F, T, mm):
+    """Which of the two forms a pass of at most 16 tokens takes (each measured faster at its passes here by 5 % and more);
+    from 17 on there is no one-slot form.  The 16-slot tiles combine a token's experts in a launch of its own."""
+    print(f"moe form {TYPE_NAMES[qtype]} NE={NE} NU={NU} E={E} F={F} T={T}", flush=True)
+    eng = az.Engine(32, max(E, F))
+    try:
+        W = make_weights(qtype, NE * F, E, seed=1)
+        L = eng.make_moe_layer(qtype, W, W, make_weights(qtype, NE * E, F, seed=3), NE, NU, E, F)
+        xb, lb = az.Runtime.from_numpy(make_acts(T, E, seed=4)), az.Runtime.from_numpy(az.gen_normal(5, (T, NE)))
+        ob = az.Runtime.alloc(T * E * 4).fill(0)
+        eng.quantize(xb, E, E, 32, T)
+        eng.profile(True)
+        eng.layer_moe(L, lb, NE, ob, T, 32)
+        eng.profile_collect()
+        assert eng.profile_get("moe_combine")[1] == (1 if mm else 0) and eng.profile_get("moe_scan")[1] == 0
+        assert np.isfinite(ob.read(np.float32, T * E)).all()
+        for b in (xb, lb, ob):
+            b.free()
+    finally:
+        eng.close()
 
 
 @pytest.mark.parametrize("env", [{"ARCZ_MOE_MM": "0"}, {"ARCZ_MOE_DECODE_MAX": "16"}, {"ARCZ_MOE_DECODE": "0"}])
@@ -132,15 +159,18 @@ def test_moe_forms_in_place_of_the_16_slot_tiles(rt, monkeypatch, env, qtype, NE
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q8_0, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q3_K, az.IQ3_S,
                                    az.IQ3_XXS])
 @pytest.mark.parametrize("NE,NU,E,F,T", [(8, 4, 512, 256, 24), (16, 6, 256, 512, 9), (4, 4, 1280, 256, 12)])
-def test_moe_matrix_pipe_tiles_of_16_slots(rt, qtype, NE, NU, E, F, T):
+def test_moe_matrix_pipe_tiles_of_16_slots(rt, monkeypatch, qtype, NE, NU, E, F, T):
     """The passes between the one-slot kernels and the tile GEMM: experts with one slot, a few and more than a tile's 16,
-    rows of one superblock and of several, numbers of row groups that four a wave do not divide."""
+    rows of one superblock and of several, numbers of row groups that four a wave do not divide.  (No one-slot form: its
+    price against these is another matter.)"""
+    monkeypatch.setenv("ARCZ_MOE_DECODE_MAX", "0")
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 32)
 
 
 @pytest.mark.parametrize("qtype,T", [(az.Q4_K, 6), (az.Q5_K, 7), (az.Q6_K, 8), (az.Q4_K, 5), (az.Q8_0, 8)])
-def test_moe_matrix_pipe_tiles_from_six_tokens(rt, qtype, T):
+def test_moe_matrix_pipe_tiles_from_six_tokens(rt, monkeypatch, qtype, T):
     """The first token counts that the 16-slot tiles take (48 pairs; Q4_K - Q6_K), and the last that they do not."""
+    monkeypatch.setenv("ARCZ_MOE_DECODE_MAX", "0")
     _moe_layer_vs_oracle(qtype, 16, 8, 512, 256, T, 16)
 
 
