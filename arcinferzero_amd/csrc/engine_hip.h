@@ -385,8 +385,10 @@ class Engine {
     set_args(k, 0, x, row_off, w, K, Mp, T, eps, aq_, asc_, absum_, hout, wh, act32);
     size_t gws[2] = {256, (size_t)(wave ? Mp / 4 : Mp)}, lws[2] = {256, 1};
     // (a wave a superblock up to 64 rows: us at 5120 values, a work-group a row against it: 1 row 3.0 / 3.2, 8 4.0 / 3.3, 16
-    //  4.3 / 3.3, 64 4.5 / 3.8, 128 4.6 / 4.6; 256 x 4096 4.2 / 5.4)
-    if (wide_rows(T) || Mp <= 64) {
+    //  4.3 / 3.3, 64 4.5 / 3.8, 128 4.6 / 4.6; 256 x 4096 4.2 / 5.4 -- and 64 rows of 6144 values or 384 Ki values in all, since
+    //  each of a row's work-groups sums the whole row: 64 x 8192 4.5 / 5.1, 64 x 17408 6.9 / 9.9, 48 x 17408 6.8 / 8.9, 32 x
+    //  12288 5.2 / 4.8, 16 x 17408 6.5 / 4.4)
+    if (wide_rows(T) || (Mp <= 64 && (size_t)Mp * K <= 384 << 10)) {
       gws[0] = 256 * (size_t)std::max((K / 256 + 3) / 4, 2);
       gws[1] = (size_t)(wide_rows(T) ? T : Mp);
     }
