@@ -81,7 +81,7 @@ class Engine {
     moe_dec_set_ = getenv("ARCZ_MOE_DECODE_MAX") != nullptr;
     moe_dec_max_ = moe_dec_set_ ? atoi(getenv("ARCZ_MOE_DECODE_MAX")) : 16;
     moe_mm_off_ = moe_dec_off_ || (getenv("ARCZ_MOE_MM") && atoi(getenv("ARCZ_MOE_MM")) == 0);
-    digits_off_ = getenv("ARCZ_GEMM_DIGITS") && atoi(getenv("ARCZ_GEMM_DIGITS")) == 0;
+    digits_env_ = getenv("ARCZ_GEMM_DIGITS") ? atoi(getenv("ARCZ_GEMM_DIGITS")) : -1;
     gemm_split_ = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
     moe_fuse_off_ = getenv("ARCZ_MOE_FUSE") && atoi(getenv("ARCZ_MOE_FUSE")) == 0;
@@ -330,7 +330,7 @@ class Engine {
         wsv_bytes_ = need;
       }
     }
-    if (rows == (size_t)N && digits_take(w.type, max_chunk, N)) digits_reserve(w);
+    if (rows == (size_t)N && digits_take(w.type, max_chunk, N, K)) digits_reserve(w);
     if (type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS) {  // (room for its GEMM form)
       const size_t need = raw_planes_bytes(QT_Q6_K, rows, K / 256);
       if (need > xw_bytes_) {
@@ -805,7 +805,7 @@ class Engine {
   bool moe_dec_off_ = false, moe_fuse_off_ = false, moe_qfuse_off_ = false;  // ARCZ_MOE_DECODE / _FUSE / _QFUSE = 0
   int moe_dec_max_ = 16, moe_tmd_ = 0;                                      // ARCZ_MOE_DECODE_MAX, ARCZ_MOE_TMD
   bool moe_dec_set_ = false, moe_mm_off_ = false;                           // ARCZ_MOE_DECODE_MAX given; ARCZ_MOE_MM = 0
-  bool digits_off_ = false;                                                 // ARCZ_GEMM_DIGITS = 0
+  int digits_env_ = -1;                                                     // ARCZ_GEMM_DIGITS (-1: by rule)
   int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
   bool moe_pre_ = true;                                                     // ARCZ_MOE_PRE (0: off)
@@ -826,13 +826,15 @@ class Engine {
   // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43 / 42, 66 / 57, 109 / 75; Q4_0 30 / 35, 42 / 47, 80 / 64;
   // MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70, MXFP4 84 / 69,
   // IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows: Q6_K 98 / 103, 97.5 / 89 (of 2048), 277 / 234; IQ3_XXS 77 / 76,
-  // -, 193 / 186.
-  bool digits_take(uint32_t type, int Mp, int N) const {
-    // (ARCZ_GEMM_DIGITS=0: never; nor with ARCZ_GEMM_SPLIT, whose pieces are the int8 kernels')
+  // -, 193 / 186; 4096 rows, K = 1024, 256 / 512 / 768 tokens: Q3_K 22 / 26, 23 / 27, 34 / 28.
+  bool digits_take(uint32_t type, int Mp, int N, int K) const {
+    // (ARCZ_GEMM_DIGITS=0: never, =1: always; not with ARCZ_GEMM_SPLIT, whose pieces are the int8 kernels')
     const double out = (double)Mp * N / (1 << 20);
-    if (Mp < 256 || digits_off_ || gemm_split_ > 0) return false;
+    if (digits_env_ == 0 || gemm_split_ > 0) return false;
+    if (digits_env_ > 0) return digit_form(type).nw != 0;
+    if (Mp < 256) return false;
     switch (type) {
-      case GGML_Q3_K: return out >= 1.0;
+      case GGML_Q3_K: return out >= (K >= 2048 ? 1.0 : 3.0);
       case GGML_Q4_0: case GGML_MXFP4: case GGML_IQ3_S: return out >= 3.0;
       case GGML_Q6_K: return Mp >= 1024 && out >= 7.5;
       case GGML_IQ3_XXS: return Mp >= 1024 && out >= 8.0;
@@ -903,13 +905,16 @@ class Engine {
   }
   // Q8_0 and Q6_K, whose 64 x 128 tiles leave a chunk of some hundred tokens between one and three work-groups a compute
   // unit: the pieces of K (1: none) with the lowest price.  In us and per 1024 values of K a full round of work-groups
-  // (three a unit for Q8_0, two for Q6_K) takes 21.2 and 24.7; a last round in which a unit has one work-group 0.46 or
+  // (three a unit for Q8_0, two for Q6_K) takes 21.2 and 24.7 (Q6_K planes of IQ3_S and IQ3_XXS: 20.4); a last round in which a unit has one work-group 0.46 or
   // 0.62 of that, two of three 0.65, 0.85 of those behind a full round, whose end it overlaps.  The partial tiles are
   // written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x both types this costs 0.5 % on
   // average against always knowing (the rule before, three to eight pieces by the tile count alone, 9 %): 300 tokens Q6_K
   // 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86, 4096 x 4096 x 512 39.3 -> 36.9.
-  static int split_pieces(uint32_t type, int Mp, int m64, int N, int nsb) {
+  // IQ3_S and IQ3_XXS over six matrices x 40 - 900 tokens: 1.0 % (1.2 % at Q6_K's price, 10 % at 256 x 4096 rows, K = 1024,
+  // which two pieces make 19.4 instead of 17.7 us).
+  static int split_pieces(uint32_t type, int half_d, int Mp, int m64, int N, int nsb) {
     const bool q8 = type == GGML_Q8_0;
+    const double round = q8 ? 21.2 : half_d ? 20.4 : 24.7;
     const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)m64 * ((N + 127) / 128);
     int best = 1;
     double least = 0.0;
@@ -917,7 +922,7 @@ class Engine {
       if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const size_t full = tiles * ny / slots, rest = tiles * ny % slots;
       const double part = rest == 0 ? 0.0 : rest <= cus ? (q8 ? 0.46 : 0.62) : rest <= 2 * cus ? (q8 ? 0.65 : 1.0) : 1.0;
-      double us = (full + (full ? 0.85 : 1.0) * part) * (q8 ? 21.2 : 24.7) * nsb / 4 / ny;
+      double us = (full + (full ? 0.85 : 1.0) * part) * round * nsb / 4 / ny;
       if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
       if (ny == 1 || us < least) {
         best = ny;
@@ -942,7 +947,7 @@ class Engine {
   }
   bool digits_room(const GpuWeight& w) const { return xd_ && wd_bytes_ >= (size_t)(w.K / 32) * digit_form(w.type).wimg; }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
-    if (digits_take(w0.type, Mp, w0.N) && digits_room(w0)) {
+    if (digits_take(w0.type, Mp, w0.N, w0.K) && digits_room(w0)) {
       gemm_digits(name, w0, Mp, C, ldc, c_off, a);
       return;
     }
@@ -969,7 +974,7 @@ class Engine {
       const int sk_force = sk_force_;
       int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
       const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
-      if (priced) ny = split_pieces(w.type, Mp, m64, N, nsb);
+      if (priced) ny = split_pieces(w.type, w.half_d, Mp, m64, N, nsb);
       if (sk_force >= 2) ny = std::min(sk_force, nsb);
       // (the others from three pieces on)
       if (ny >= (priced || sk_force >= 2 ? 2 : 3)) {

@@ -311,10 +311,11 @@ def test_gemm_padding_rows(rt, qtype, T, Mp, N, K, acc):
                                                 (az.MXFP4, 385, 400, 8190, 512, 1), (az.IQ3_S, 390, 400, 8000, 1024, 0),
                                                 (az.Q6_K, 1030, 1040, 7700, 256, 0), (az.Q6_K, 1024, 1024, 7810, 768, 1),
                                                 (az.IQ3_XXS, 2049, 2052, 4100, 512, 0), (az.IQ3_XXS, 1025, 1040, 8100, 1024, 2)])
-def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
+def test_gemm_on_digits(rt, monkeypatch, qtype, T, Mp, N, K, acc):
     """The GEMM of long chunks whose tokens and rows are written as digits first: one, two and three digits a weight, K
     shared out and not, ragged last tiles of tokens and rows, one superblock and odd numbers of them, the three epilogues.
     Against the oracle, and run to run."""
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")   # (read when an engine is made; the rule leaves the smallest to the int8 kernels)
     print(f"digits {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc}", flush=True)
     eng = az.Engine(Mp, K)
     W = make_weights(qtype, N, K, seed=81)
@@ -335,7 +336,7 @@ def test_gemm_on_digits(rt, qtype, T, Mp, N, K, acc):
 
 
 @pytest.mark.parametrize("qtype,T,Mp,N,K", [(az.Q6_K, 20, 256, 1000, 768), (az.Q8_0, 20, 256, 3000, 512), (az.Q8_0, 60, 384, 256, 4096),
-                                            (az.Q4_K, 20, 384, 5200, 512), (az.Q4_K, 130, 256, 392, 2048), (az.Q3_K, 100, 256, 4224, 256),
+                                            (az.Q4_K, 20, 384, 5200, 512), (az.Q4_K, 130, 256, 392, 2048), (az.Q3_K, 100, 256, 4224, 2048),
                                             (az.Q4_K, 10, 16, 264, 1024), (az.Q5_K, 12, 16, 264, 6400), (az.IQ4_XS, 40, 256, 300, 512)])
 def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     """set_activations takes all Mp rows from the caller: in a chunk of more than 8 tokens the rows from T on are multiplied
@@ -355,13 +356,13 @@ def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
 
 
-@pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
+@pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "1", "ARCZ_Q4_SPLITK": "2"}, 1, 2), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
                                                  ({"ARCZ_Q4_SPLITK": "2"}, 1, 2),
-                                                 ({"ARCZ_GEMM_SPLIT": "1", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])
+                                                 ({"ARCZ_GEMM_SPLIT": "3", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])
 def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
     """The launch-rule switches on a chunk that the digits take by rule: off, K in one piece, two pieces forced (the
     product and its reduction), and the int8 kernels in pieces of superblocks (one expansion and a launch a piece)."""
-    T, N, K = 256, 4224, 768
+    T, N, K = 256, 4224, 2048
     print(f"digits switches {env}", flush=True)
     for k, v in env.items():
         monkeypatch.setenv(k, v)          # (read when an engine is made)
@@ -372,6 +373,13 @@ def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
     y = run_gemm(eng, az.Q3_K, W, N, K, x, T)
     eng.profile_collect()
     counts = [eng.profile_get(k)[1] for k in ("act_digits", "test")]
+    eng.close()
+    # (where the rule ends: the same outputs over shorter rows)
+    eng = az.Engine(T, K)
+    eng.profile(True)
+    run_gemm(eng, az.Q3_K, make_weights(az.Q3_K, N, 1024, seed=86), N, 1024, x[:, :1024].copy(), T)
+    eng.profile_collect()
+    assert eng.profile_get("act_digits")[1] == (1 if env.get("ARCZ_GEMM_DIGITS") == "1" else 0)
     eng.close()
     aq, asc, _ = quantize_padded(x, T)
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(az.Q3_K, W, N, K, aq, asc)).max() <= TOL
@@ -410,10 +418,11 @@ def _extreme_rows(qtype, N, K, rng):
 
 @pytest.mark.parametrize("qtype,T,N", [(az.Q6_K, 1024, 7808), (az.Q3_K, 256, 4224), (az.IQ3_XXS, 1024, 8192), (az.IQ3_S, 256, 12288),
                                        (az.Q4_0, 256, 12288), (az.MXFP4, 256, 12288)])
-def test_gemm_on_digits_block_sums_exact(rt, qtype, T, N):
+def test_gemm_on_digits_block_sums_exact(rt, monkeypatch, qtype, T, N):
     """The GEMM on digits keeps every block sum exact, at the ends of the ranges too: a token has one block of values up to
     -128 (all ends, alternating ends, random ends, random) and zeros elsewhere, unit scales, so an output is one block's
     sum -- up to 32 x 128 x 4096 = 2^24, with whole and partial cancellation -- and has to be that integer."""
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")   # (read when an engine is made; the rule leaves the smallest to the int8 kernels)
     print(f"digits, exact block sums {TYPE_NAMES[qtype]} T={T} N={N}", flush=True)
     K = 512
     rng = np.random.default_rng(170 + qtype)
