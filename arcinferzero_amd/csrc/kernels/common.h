@@ -268,13 +268,13 @@ __device__ inline int dot4_first(uint32_t a, uint32_t b) {
 // A lane's 16 sums of a 32 x 32 tile (rows 8 (i / 4) + i % 4 from c on, those below `rows`) out to one column of C with
 // stride ldc: stored, added to what is there, or times silu of it.  What is there is loaded for all of them before the
 // first is used: one memory latency instead of sixteen (the up projection's epilogue, 64 outputs a lane, took 30 - 50 us
-// more than the gate's).  A plain store forms each address on its own: with the sixteen rows' offsets shared, as the
+// more than the gate's).  A plain store forms each address on its own (EACH): with the sixteen rows' offsets shared, as the
 // compiler would have them, 17408 x 5120 x 8192 took 2.03 ms instead of 1.99 (Q4_K; 2048 tokens 0.538 / 0.527, Q5_K 2.22 /
 // 2.19, Q8_0 x 4096 1.09 / 1.064), the loop before it being the same instructions.  scale(v, i): the row's factor, if any.
 // STREAM: stored past the caches, so that an output larger than every cache does not displace the operands that the
 // neighbouring tiles still read (Q4_K, 8192 tokens x 17408 rows: 707 -> 717 TOP/s; not for the expert tiles' y rows, which
 // moe_combine reads right back: 56 -> 62 us there).
-template <bool STREAM, class SCALE>
+template <bool STREAM, bool EACH = true, class SCALE>
 __device__ __forceinline__ void store16(const v16f& res, float* c, int ldc, int rows, int accumulate, SCALE scale) {
   auto put = [&](int r, float v) {
     float* cp = c + (size_t)r * ldc;
@@ -286,7 +286,7 @@ __device__ __forceinline__ void store16(const v16f& res, float* c, int ldc, int 
     for (int i = 0; i < 16; ++i) {
       int r = 8 * (i >> 2) + (i & 3);
       if (r >= rows) continue;
-      asm volatile("" : "+v"(r));
+      if (EACH) asm volatile("" : "+v"(r));
       put(r, scale(res[i], i));
     }
     return;

@@ -1923,6 +1923,8 @@ extern "C" __global__ __launch_bounds__(256, 2) void moe_gateup_q__QT12_QUANT1(
 #define G8_SA 24576
 #define G8_WS 25600
 
+// (PART: partial tiles, whose plain stores share their rows' offsets: 512 tokens x 4096 rows, K = 4096, 35.25 -> 34.95 us)
+template <bool PART>
 __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, const signed char* __restrict__ aq,
                                   const float* __restrict__ asc, float* __restrict__ C, int M, int N, int K, int ldc,
                                   int c_off, int accumulate, int s_begin, int s_end, int m0, int rows_valid, int n0) {
@@ -2062,7 +2064,7 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
     for (int ms = 0; ms < 2; ++ms)
     {
       const int r0 = ms * 32 + 4 * g;
-      store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
+      store16<false, !PART>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
                      [](float v, int) { return v; });
     }
   }
@@ -2253,7 +2255,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64_BN
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
   const int ns = s_end - s_begin, y = blockIdx.y, ny = gridDim.y;
-  gemm8_body(raw, aq, asc, C + (size_t)y * M * ldc, M, N, K, ldc, 0, 0, s_begin + ns * y / ny, s_begin + ns * (y + 1) / ny,
+  gemm8_body<true>(raw, aq, asc, C + (size_t)y * M * ldc, M, N, K, ldc, 0, 0, s_begin + ns * y / ny, s_begin + ns * (y + 1) / ny,
              m0, min(G6_BM, M - m0), n0);
 }
 // (Q6_K -DBM=64 -DBN=128 -DSPLITK: its dense kernel's tiles)
@@ -2349,7 +2351,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64(
   int tm, tn;
   tile_of(blockIdx.x, mt, nt, tm, tn);
   const int m0 = tm * G6_BM, n0 = tn * BN;
-  gemm8_body(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0), n0);
+  gemm8_body<false>(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0), n0);
   zero_tail(C, ldc, c_off, accumulate, tm, mt, M, n0, N);
 }
 
