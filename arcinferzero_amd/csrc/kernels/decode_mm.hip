@@ -520,7 +520,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
       // block b: indices 2 g and 2 g + 1 of its eight (a byte each) name codebook words of four magnitudes; the signs of
       // the lane's eight values are the block's sign code g, the scale the top nibble of that word; d / 4
       // (reference src/quants.h:220-239, zero/kernels/decode.cl:183-478)
-            const float d3 = 0.25f * f16_bits_to_f32(h.d);
+      const float d3 = 0.25f * f16_bits_to_f32(h.d);
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
         ahead(b);
@@ -568,7 +568,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
       // block b: indices 2 g and 2 g + 1 of its eight (a byte each and a ninth bit from byte b of the header) name
       // codebook words of four magnitudes, the signs are bits 8 g .. 8 g + 7 of the block's word; scale 1 + 2 x nibble b
       // of the header's third word, times d (reference src/quants.h IQ3_S, zero/kernels/decode.cl:183-478)
-            const float d3 = f16_bits_to_f32(h.d);
+      const float d3 = f16_bits_to_f32(h.d);
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
         ahead(b);
@@ -976,6 +976,12 @@ __device__ inline void moe_down_mm(uint8_t* lds, const uint8_t* __restrict__ raw
   else mm_slice<QT, true, false>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
 }
 
+// WPE: waves a SIMD the registers are kept to.  4 (128 registers: two work-groups a compute unit, where LDS holds two -- not
+// for rows of K >= 2816 values, nor, from K = 2048 on, for Q5_K, Q8_0 and the three-bit types), 2 for Q6_K and Q3_K, which
+// need 200 and more.  At 128 the compiler keeps some in scratch: bytes a lane, gate / up and down, Q5_K 40 and 44, IQ3_S 8
+// and 20, Q8_0 and IQ4_NL 0 and 20.  us a layer with 4 / 2, 128 x 8 of 768 x 2048, 16, 40 and 100 tokens: IQ4_NL 71 / 80, 91 /
+// 106, 116 / 130; IQ3_S 103 / 107, 135 / 139, 152 / 158; Q8_0 91 / 90, 121 / 121, 149 / 146; Q5_K 80 / 81, 105 / 106, 143 /
+// 131: from 100 tokens on Q5_K and Q8_0 would be ahead without.
 #define MOE_MM(QTV, WPE)                                                                                                    \
   extern "C" __global__ __launch_bounds__(512, WPE) void moe_gateup_mm__QT##QTV(                                          \
       const uint8_t* rg, const uint8_t* ru, int F, int K, const uint32_t* tabs, const signed char* aq, const float* asc, \

@@ -1179,8 +1179,7 @@ __device__ __forceinline__ void gemm6_body(const uint8_t* __restrict__ raw, cons
   const int n = n0 + wave * 32 + l32;
   if (n < N) {
 #pragma unroll
-    for (int ms = 0; ms < 2; ++ms)
-    {
+    for (int ms = 0; ms < 2; ++ms) {
       const int r0 = ms * 32 + 4 * g;
       store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
                      [&](float v, int i) { return TILES && use_scale ? v * rowscale[m0 + r0 + 8 * (i >> 2) + (i & 3)] : v; });
@@ -1442,8 +1441,7 @@ __device__ __forceinline__ void gemm4_body(const uint8_t* __restrict__ raw, cons
   const int n = n0 + wave * 32 + l32;
   if (n < N) {
 #pragma unroll
-    for (int ms = 0; ms < (TWO ? 2 : 1); ++ms)
-    {
+    for (int ms = 0; ms < (TWO ? 2 : 1); ++ms) {
       const int r0 = ms * 32 + 4 * g;
       store16<false>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
                      [&](float v, int i) { return use_scale ? v * rowscale[m0 + r0 + 8 * (i >> 2) + (i & 3)] : v; });
@@ -1703,8 +1701,7 @@ __device__ __forceinline__ void gemm4gu_body(const uint8_t* __restrict__ rg, con
       const int n = nx[x] + wave * 32 + l32;
       if (n >= N) continue;
 #pragma unroll
-      for (int ms = 0; ms < 2; ++ms)
-      {
+      for (int ms = 0; ms < 2; ++ms) {
         const int r0 = ms * 32 + 4 * g;
         store16<false>(res[x][ms], H + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
                        [](float v, int) { return v; });
@@ -2061,11 +2058,10 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
   const int n = n0 + wave * 32 + l32;
   if (n < N) {
 #pragma unroll
-    for (int ms = 0; ms < 2; ++ms)
-    {
+    for (int ms = 0; ms < 2; ++ms) {
       const int r0 = ms * 32 + 4 * g;
       store16<false, !PART>(res[ms], C + (size_t)(m0 + r0) * ldc + c_off + n, ldc, rows_valid - r0, accumulate,
-                     [](float v, int) { return v; });
+                            [](float v, int) { return v; });
     }
   }
 }
@@ -2073,8 +2069,8 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
 // A chunk laid out for M token rows whose last ones are padding: a launch of the 64-token tiles may leave out the tiles that
 // hold nothing else (their count comes from the grid).  The padding rows' results are zeros where a product is stored or
 // multiplied in (one that is added changes nothing): the mt work-groups of a row tile write a share of them each, behind
-// their own results (Q8_0, 300 tokens x 4096 rows, K = 1024: 12.8 us; by the last
-// tile's alone, in front of its loads, 14.4; no tile left out 13.6).
+// their own results (Q8_0, 300 tokens x 4096 rows, K = 1024: 12.8 us; by the last tile's alone, in front of its loads, 14.4;
+// no tile left out 13.6).
 __device__ inline void zero_tail(float* C, int ldc, int c_off, int accumulate, int tm, int mt, int M, int n0, int N) {
   const int n = n0 + (threadIdx.x & 127);
   if (accumulate == 1 || n >= N) return;

@@ -492,7 +492,8 @@ extern "C" __global__ __launch_bounds__(256) void q4k_wscales_int(const uint8_t*
 
 // swiglu_quant over a chunk: no value depends on another superblock of its row, so the tiles of quant_rows do (rows, 16
 // or 64, the launcher's choice), and every size fills the chip; 16 whole rows a work-group, the form before, took 123 us
-// at 384 x 17408, now 13.2 (1024: 125 -> 28, 4096 x 5120: 43.5 -> 33, 8192 x 5120: 91.4 -> 90.9, bound by memory).  grid (256 * (F / 256), ceil(M / rows)), local (256, 1).
+// at 384 x 17408, now 13.4 (three inputs in turn; 1024: 133 -> 38, 4096 x 5120: 47.7 -> 45.4; four in turn, 8192 x 5120: 90.2 -> 89.8, bound by
+// memory).  grid (256 * (F / 256), ceil(M / rows)), local (256, 1).
 extern "C" __global__ __launch_bounds__(256) void swiglu_quant_tile(const float* __restrict__ gu, int F, int M, int M_valid,
                                                                     signed char* __restrict__ aq, float* __restrict__ asc,
                                                                     short* __restrict__ absum, int act32, int fused,
@@ -525,8 +526,9 @@ extern "C" __global__ __launch_bounds__(256) void swiglu_quant_tile(const float*
 // holds its 16 values of superblocks lane / 16 + 4 u in registers from the sum of squares to the quantization for
 // u < MAXU (rows of up to 6144 values); what a longer row has beyond them is read again, out of the cache.  Bound by
 // memory from about 4096 rows on, below that by one row's chain of loads, sum and stores.  The form before it, 16 rows a
-// work-group one after the other, left most of the chip idle: 384 x 5120 37.9 -> 8.4 us, 1024 x 5120 37.7 -> 9.2, 8192 x
-// 5120 46.6 -> 41.7 (5.3 TB/s); eight rows a work-group (pieces of 32 and 16 bytes) 10.1, 10.7, 50.8.
+// work-group one after the other, left most of the chip idle: 384 x 5120 35.4 -> 6.8 us, 1024 x 5120 37.1 -> 9.4, 8192 x
+// 5120 56.2 -> 53.8 (4.1 TB/s, four inputs in turn, more than the caches hold; one input again and again 44.4 -> 39.4);
+// eight rows a work-group (pieces of 32 and 16 bytes) lost a fifth against four.
 // One-pass engines, M a multiple of 4, K <= RW_KMAX.  grid (256, M / 4).
 #define RW_KMAX 16384
 extern "C" __global__ __launch_bounds__(256) void rmsnorm_quant_wave(const float* __restrict__ x, int row_off,

@@ -90,12 +90,14 @@ def test_swiglu_quant(eng, T, Mp, F, gelu):
     gb.free(); vb.free()
 
 
-@pytest.mark.parametrize("T,Mp,K,act32", [(256, 256, 16384, 1), (300, 320, 5120, 1), (250, 256, 4096, 0), (1000, 1024, 256, 0)])
-def test_producers_16_rows_a_work_group(rt, T, Mp, K, act32):
-    """Chunks of at least 256 rows go through the forms that take 16 rows a work-group and write scales and sums in
-    pieces of 16 rows: the same bits as the plain quantizer on the f32 rows (RMS norm: on the rows the kernel itself
-    wrote out), per-32 and per-256 scales, rows past T as zeros, the longest rows each form takes."""
-    print(f"producers r16 T={T} Mp={Mp} K={K} act32={act32}", flush=True)
+@pytest.mark.parametrize("T,Mp,K,act32", [(256, 256, 16384, 1), (300, 320, 5120, 1), (250, 256, 4096, 0), (1000, 1024, 256, 0),
+                                          (60, 64, 6144, 1), (60, 64, 6400, 1), (40, 48, 8448, 0), (20, 32, 12288, 1)])
+def test_producers_of_chunks(rt, T, Mp, K, act32):
+    """The chunk producers by their launch rules: the RMS norm of up to 64 rows a wave a superblock, or, where these are too
+    many values, a work-group a row as up to 256 rows have, a wave a row beyond; SwiGLU in the quantizer's tiles of 16 or
+    64 rows.  The same bits as the plain quantizer on the f32 rows (RMS norm: on the rows the kernel itself wrote out),
+    per-32 and per-256 scales, rows past T as zeros, the longest rows each form takes."""
+    print(f"producers of chunks T={T} Mp={Mp} K={K} act32={act32}", flush=True)
     eng = az.Engine(Mp, max(K, 256))
     try:
         B = 32 if act32 else 256
