@@ -945,9 +945,18 @@ class Engine {
     wd_ = try_buf(need);
     if (wd_) wd_bytes_ = need;
   }
-  bool digits_room(const GpuWeight& w) const { return xd_ && wd_bytes_ >= (size_t)(w.K / 32) * digit_form(w.type).wimg; }
+  // All the rows at once, or panels that give every compute unit a work-group: a launch of fewer takes as long as one that
+  // fills the chip (Q4_0 17408 x 5120 x 1024 in panels of 2, 8, 32, 64 row tiles and at once 4111, 1060, 335, 288, 260 us, on
+  // the int8 kernels 335; x 256 in panels of 64 212, at once 113, int8 138).  A three-bit weight that the int8 kernels have no
+  // room for either (xw_): any panel.
+  bool digits_room(const GpuWeight& w, int Mp) const {
+    const size_t panel = wd_bytes_ / ((size_t)(w.K / 32) * digit_form(w.type).wimg), all = (size_t)(w.N + 127) / 128;
+    const bool expanded = w.type == GGML_IQ3_S || w.type == GGML_Q3_K || w.type == GGML_IQ3_XXS;
+    if (expanded && raw_planes_bytes(QT_Q6_K, w.rows, w.K / 256) > xw_bytes_) return xd_ && panel >= 1;
+    return xd_ && (panel >= all || panel * ((Mp + 127) / 128) >= (size_t)arcz_device_cus());
+  }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
-    if (digits_take(w0.type, Mp, w0.N, w0.K) && digits_room(w0)) {
+    if (digits_take(w0.type, Mp, w0.N, w0.K) && digits_room(w0, Mp)) {
       gemm_digits(name, w0, Mp, C, ldc, c_off, a);
       return;
     }

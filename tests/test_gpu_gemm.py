@@ -455,35 +455,49 @@ def test_gemm_on_digits_block_sums_exact(rt, monkeypatch, qtype, T, N):
     assert np.array_equal(y, want.astype(np.float32))
 
 
-@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512)])
+@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512), (az.Q3_K, 300, 4224, 2560)])
 @pytest.mark.parametrize("before", [None, 256, 1024])
 def test_weights_of_another_engine(rt, qtype, T, N, K, before):
     """Engines share weights: a matrix that an engine for single tokens uploaded, in a long chunk of an engine that
-    uploaded none itself (no room for digits), or one with shorter or longer rows (room for some tiles of this one's rows
-    or for all).  Against the oracle."""
+    uploaded none itself (no room for digits: the int8 kernels), or one with shorter or longer rows (room for panels of
+    this one's rows, where these fill the chip, or for all).  Against the oracle."""
     print(f"another engine's {TYPE_NAMES[qtype]} T={T} N={N} K={K} before={before}", flush=True)
     small = az.Engine(16, K)
     W = make_weights(qtype, N, K, seed=96)
     w = small.make_weight(qtype, N, K, W)
     Mp = (T + 127) // 128 * 128
-    eng = az.Engine(Mp, 1024)
+    eng = az.Engine(Mp, max(K, 1024))
     if before:   # (rows enough for the launch rule of every type)
-        small_n = -(-8 * 1024 * 1024 // Mp)
+        small_n = -(-8 * 1024 * 1024 // Mp) if qtype != az.Q3_K else -(-3 * 1024 * 1024 // Mp)
         eng.make_weight(qtype, small_n, before, make_weights(qtype, small_n, before, seed=95)).free()
     x = make_acts(T, K, seed=97, outliers=True)
     xb = az.Runtime.from_numpy(x)
     eng.quantize(xb, K, K, Mp, T)
+    eng.profile(True)
     cb = az.Runtime.alloc(Mp * N * 4).fill(0xFFFFFFFF)
+    if qtype == az.Q3_K and before is None:
+        with pytest.raises(az.ArczError):   # (no room for the expansion that the int8 kernels take either)
+            eng.matmul("test", w, Mp, cb, N, 0, 0)
+        for b in (cb, xb, w, eng, small):
+            b.close() if isinstance(b, az.Engine) else b.free()
+        return
     eng.matmul("test", w, Mp, cb, N, 0, 0)
     y = cb.read(np.float32, Mp * N).reshape(Mp, N)
     for b in (cb, xb):
         b.free()
     w.free()
+    eng.profile_collect()
+    launches = eng.profile_get("row_digits")[1]
     eng.close()
     small.close()
     aq, asc, _ = quantize_padded(x, Mp)
     ref = orc.matmul_ref(qtype, W, N, K, aq[:T], np.ascontiguousarray(asc[:, :T]))
     assert np.isfinite(y).all() and rel_err_rows(y[:T], ref).max() <= TOL and not y[T:].any()
+    # (256: half the room that rows of 512 values need, 32 row tiles x 8 token tiles for Q6_K, 85 x 3 for Q4_0; Q3_K, whose
+    #  expansion has no room: 6 row tiles a panel, or 25)
+    want = {None: 0, 256: {az.Q4_0: 0, az.MXFP4: 1, az.Q6_K: 2}, 1024: {az.Q4_0: 1, az.MXFP4: 1, az.Q6_K: 1}}[before]
+    assert qtype == az.Q3_K or launches == (want[qtype] if before else 0)
+    assert launches > 1 or qtype != az.Q3_K
 
 
 @pytest.mark.parametrize("T,Mp,N,K,acc", [(1100, 1104, 392, 512, 0), (1030, 1040, 640, 768, 1), (760, 768, 520, 1024, 2),

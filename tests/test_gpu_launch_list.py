@@ -213,11 +213,11 @@ def test_a_list_keeps_the_buffers_it_names(rt):
 
 def test_a_list_that_names_the_digits_of_rows(rt):
     """A recorded long chunk of Q4_0 names the engine's room for the digits of the rows.  A larger Q4_0 matrix is uploaded
-    all the same and multiplied in panels of the rows that fit that room, or -- rows longer than it holds a tile of -- on
-    the int8 kernels: against the oracle; the list replays bit for bit behind it."""
-    T = Mp = 256
-    N, K = 12288, 256      # (the fewest rows that the launch rule takes for 256 tokens)
-    eng = az.Engine(Mp, 32768)
+    all the same and multiplied in panels of the rows that fit that room (48 of 96 row tiles, two launches), or -- rows so
+    long that it holds one tile of them -- on the int8 kernels: against the oracle; the list replays bit for bit behind."""
+    T = Mp = 768
+    N, K = 12288, 256
+    eng = az.Engine(Mp, 16384)
     lst = None
     try:
         w = eng.make_weight(az.Q4_0, N, K, make_weights(az.Q4_0, N, K, seed=44))
@@ -231,7 +231,9 @@ def test_a_list_that_names_the_digits_of_rows(rt):
         step()
         ref = cb.read(np.float32, Mp * N).copy()
         lst = az.Runtime.record(step)
-        for n2, k2 in ((N, 512), (N, 32768)):
+        eng.profile(True)
+        for n2, k2, panels in ((N, 512, 2), (N, 16384, 0)):
+            eng.profile_reset()
             print(f"upload while a list names the digits N={n2} K={k2}", flush=True)
             W2 = make_weights(az.Q4_0, n2, k2, seed=46)
             w2 = eng.make_weight(az.Q4_0, n2, k2, W2)
@@ -245,6 +247,8 @@ def test_a_list_that_names_the_digits_of_rows(rt):
             Ws = np.ascontiguousarray(W2.reshape(n2, -1)[rows]).reshape(-1)
             assert rel_err_rows(y[:16, rows], orc.matmul_ref(az.Q4_0, Ws, len(rows), k2, aq[:16], np.ascontiguousarray(asc[:, :16]))).max() <= 1e-3
             assert np.isfinite(y).all()
+            eng.profile_collect()
+            assert eng.profile_get("row_digits")[1] == panels
             cb.fill(0xFFFFFFFF)
             lst.run()
             assert np.array_equal(cb.read(np.float32, Mp * N).view(np.uint32), ref.view(np.uint32))
