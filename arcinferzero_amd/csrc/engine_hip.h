@@ -905,13 +905,13 @@ class Engine {
   }
   // Q8_0 and Q6_K, whose 64 x 128 tiles leave a chunk of some hundred tokens between one and three work-groups a compute
   // unit: the pieces of K (1: none) with the lowest price.  In us and per 1024 values of K a full round of work-groups
-  // (three a unit for Q8_0, two for Q6_K) takes 21.2 and 24.7 (Q6_K planes of IQ3_S and IQ3_XXS: 20.4); a last round in which a unit has one work-group 0.46 or
-  // 0.62 of that, two of three 0.65, 0.85 of those behind a full round, whose end it overlaps.  The partial tiles are
-  // written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x both types this costs 0.5 % on
-  // average against always knowing (the rule before, three to eight pieces by the tile count alone, 9 %): 300 tokens Q6_K
-  // 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86, 4096 x 4096 x 512 39.3 -> 36.9.
-  // IQ3_S and IQ3_XXS over six matrices x 40 - 900 tokens: 1.0 % (1.2 % at Q6_K's price, 10 % at 256 x 4096 rows, K = 1024,
-  // which two pieces make 19.4 instead of 17.7 us).
+  // (three a unit for Q8_0, two for Q6_K) takes 21.2 and 24.7 (Q6_K planes of IQ3_S and IQ3_XXS: 20.4); a last round in
+  // which a unit has one work-group 0.46 or 0.62 of that, two of three 0.65, 0.85 of those behind a full round, whose end it
+  // overlaps.  The partial tiles are written, read and summed at 5 TB/s.  Over a sweep of six matrices x 64 - 1024 tokens x
+  // both types this costs 0.5 % on average against always knowing (the rule before, three to eight pieces by the tile count
+  // alone, 9 %): 300 tokens Q6_K 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86,
+  // 4096 x 4096 x 512 39.3 -> 36.9.  IQ3_S and IQ3_XXS over six matrices x 40 - 900 tokens: 1.0 % (1.2 % at Q6_K's price, 10 %
+  // at 256 x 4096 rows, K = 1024, which two pieces make 19.4 instead of 17.7 us).
   static int split_pieces(uint32_t type, int half_d, int Mp, int m64, int N, int nsb) {
     const bool q8 = type == GGML_Q8_0;
     const double round = q8 ? 21.2 : half_d ? 20.4 : 24.7;
@@ -1466,8 +1466,8 @@ class Engine {
     // work-groups (128 us a layer at 128 experts x 768 x 2048; ARCZ_MOE_DECODE=0 brings those back, ARCZ_MOE_DECODE_MAX
     // moves the limit).
     // (the switches of this function are read when the engine is made: a test sets them before it makes its engine)
-    // From 6 or 9 tokens on the 16-slot tiles take over where they are cheaper (moe_mm_takes, moe_mm_cheaper) -- not where ARCZ_MOE_DECODE_MAX is given and names
-    // the pass, nor with ARCZ_MOE_DECODE=0 or ARCZ_MOE_MM=0.
+    // From 6 or 9 tokens on the 16-slot tiles take over where they are cheaper (moe_mm_takes, moe_mm_cheaper) -- not where
+    // ARCZ_MOE_DECODE_MAX is given and names the pass, nor with ARCZ_MOE_DECODE=0 or ARCZ_MOE_MM=0.
     const bool one_slot = !moe_dec_off_ && T <= moe_dec_max_ && T * NU <= 512;
     const bool mm = !moe_mm_off_ && moe_mm_takes(L, T) && (!one_slot || (!moe_dec_set_ && moe_mm_cheaper(L, T)));
     if (mm && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;
@@ -1631,9 +1631,10 @@ class Engine {
 // Start-up check in the pattern of the reference's xmx_check (zero/engine_setup.h:424-520): the tuned GEMM that the
 // dispatch takes for a chunk of 128 tokens -- for each weight type, storing, accumulating and with the fused SwiGLU
 // epilogue, in one piece and with K shared out over several work-groups per tile -- and the GEMM on digits (one, two and
-// three digits a weight), against the plain kernel of the same type on the reference's LCG data, with unit scales (weights d = 1, sub-scales 1, Q4_K / Q5_K mins 1; activation scales 1) so that
-// every f32 sum is an integer below 2^24: the two results must be bit-equal to each other and, for store and add, to
-// the integer sums counted on the host.  Returns an empty string, or what differed.
+// three digits a weight), against the plain kernel of the same type on the reference's LCG data, with unit scales (weights
+// d = 1, sub-scales 1, Q4_K / Q5_K mins 1; activation scales 1) so that every f32 sum is an integer below 2^24: the two
+// results must be bit-equal to each other and, for store and add, to the integer sums counted on the host.  Returns an
+// empty string, or what differed.
 inline std::string engine_self_check() {
   const int M = 128, N = 128;
   uint32_t lcg = 12345u;
@@ -1749,9 +1750,10 @@ inline std::string engine_self_check() {
           for (int k2 = 0; k2 < K; ++k2) sm += (long long)aq[(size_t)m * K + k2] * wq[(size_t)n * K + k2];
           sums[(size_t)m * N + n] = (float)sm;
         }
-      if (e.digit_form(type).nw) e.digits_reserve(gw);  // (the rule takes longer chunks; the kernels are the same)
+      const bool on_digits = e.digit_form(type).nw != 0;  // (the rule takes longer chunks; the kernels are the same)
+      if (on_digits) e.digits_reserve(gw);
       for (int mode = 0; mode < 3; ++mode)
-        for (int digits = 0; digits < (e.digit_form(type).nw ? 2 : 1); ++digits) {
+        for (int digits = 0; digits < (on_digits && e.digits_room(gw, M) ? 2 : 1); ++digits) {
           CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c0, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
           CL_CHECK(clEnqueueWriteBuffer(e.cl_.queue, c1, CL_TRUE, 0, cinit.size() * 4, cinit.data(), 0, nullptr, nullptr));
           if (digits) e.gemm_digits("self_check", gw, M, c0, N, 0, mode);
@@ -1774,8 +1776,8 @@ inline std::string engine_self_check() {
             memcpy(&bb, &b, 4);
             if (ab != bb || a != want || !std::isfinite(a)) {
               e.free_weight(gw);
-              return std::string("GEMM self-check ") + ggml_type_name(type) + (digits ? " on digits" : "") + " K=" + std::to_string(K) +
-                     " mode " + std::to_string(mode) + ": token " + std::to_string(i / N) + " row " + std::to_string(i % N) + ": tuned " +
+              return std::string("GEMM self-check ") + ggml_type_name(type) + (digits ? " on digits" : "") + " K=" +
+                     std::to_string(K) + " mode " + std::to_string(mode) + ": token " + std::to_string(i / N) + " row " + std::to_string(i % N) + ": tuned " +
                      std::to_string(a) + ", simple " + std::to_string(b) + ", integer sum " + std::to_string(sums[i]);
             }
           }
