@@ -41,6 +41,7 @@ _sig("arcz_device_name", C.c_char_p)
 _sig("arcz_device_cus", _i)
 _sig("arcz_device_mem", _z)
 _sig("arcz_device_bytes", _z)
+_sig("arcz_spare_bytes", _z)
 _sig("arcz_alloc", _p, _z)
 _sig("arcz_view", _p, _p, _z, _z)
 _sig("arcz_free", _i, _p)

@@ -22,6 +22,7 @@ struct arcz_mem {
   size_t size;
   bool owner;
   arcz_mem* parent = nullptr;  // a view's owner (the root of a chain of views)
+  bool spare = false;          // its contents can be done without: given back when memory runs out (arcz_mem_spare)
 };
 struct arcz_kernel {
   hipFunction_t fn;
@@ -49,7 +50,7 @@ struct Runtime {
   hipDeviceProp_t prop;
   std::string name;
   std::set<arcz_mem*> mems;
-  size_t device_bytes = 0;
+  size_t device_bytes = 0, spare_bytes = 0;
   std::map<std::string, std::vector<hipModule_t>> modules;  // a module may be several code objects
   std::map<std::string, arcz_kernel*> kernels;
   int (*oom_hook)(void) = nullptr;
@@ -185,7 +186,7 @@ void arcz_shutdown(void) {
   }
   R.mems.clear();
   R.scratch = nullptr;  // (its handle went with the others; the array itself stays with the device)
-  R.device_bytes = 0;
+  R.device_bytes = R.spare_bytes = 0;
   hipStreamDestroy(R.stream);
   R.stream = nullptr;
   R.up = false;
@@ -196,6 +197,22 @@ const char* arcz_device_name(void) { return R.name.c_str(); }
 int arcz_device_cus(void) { return R.up ? R.prop.multiProcessorCount : 0; }
 size_t arcz_device_mem(void) { return R.up ? R.prop.totalGlobalMem : 0; }
 size_t arcz_device_bytes(void) { return R.device_bytes; }
+
+// Frees the spare buffers that no recorded list names; their handles stay, of size 0.
+static bool give_back_spares() {
+  bool any = false;
+  for (arcz_mem* m : R.mems) {
+    if (!m->spare || !m->ptr || arcz_mem_listed(m)) continue;
+    if (!any && hipStreamSynchronize(R.stream) != hipSuccess) return false;
+    if (hipFree(m->ptr) != hipSuccess) return any;
+    R.device_bytes -= m->size;
+    R.spare_bytes -= m->size;
+    m->ptr = nullptr;
+    m->size = 0;
+    any = true;
+  }
+  return any;
+}
 
 arcz_mem* arcz_alloc(size_t bytes) {
   if (!R.up) { fail(ARCZ_E_DEVICE, "arcz_alloc before arcz_init"); return nullptr; }
@@ -210,6 +227,7 @@ arcz_mem* arcz_alloc(size_t bytes) {
     if (e == hipSuccess) break;
     if (!fake) (void)hipGetLastError();
     if (e != hipErrorOutOfMemory) break;
+    if (give_back_spares()) continue;
     if (!(R.oom_hook && R.oom_hook())) break;  // nothing was freed: give up (clrt.h:474-487)
   }
   if (e != hipSuccess || !p) {
@@ -248,12 +266,24 @@ int arcz_free(arcz_mem* m) {
     HIP_TRY(hipStreamSynchronize(R.stream));
     HIP_TRY(hipFree(m->ptr));
     R.device_bytes -= m->size;
+    if (m->spare) R.spare_bytes -= m->size;
   }
   R.mems.erase(m);
   delete m;
   return ARCZ_OK;
 }
 
+int arcz_mem_spare(arcz_mem* m) {
+  if (!m || !R.mems.count(m) || !m->owner || m == R.scratch) return fail(ARCZ_E_ARG_VALUE, "arcz_mem_spare of a handle that owns no buffer");
+  if (!m->spare) R.spare_bytes += m->size;
+  m->spare = true;
+  return ARCZ_OK;
+}
+size_t arcz_spare_bytes(void) { return R.spare_bytes; }
+size_t arcz_device_mem_free(void) {
+  size_t free = 0, total = 0;
+  return R.up && hipMemGetInfo(&free, &total) == hipSuccess ? free : 0;
+}
 int arcz_mem_listed(const arcz_mem* m) {
   if (!m || !R.mems.count(const_cast<arcz_mem*>(m))) return 0;
   arcz_mem* o = m->owner ? const_cast<arcz_mem*>(m) : m->parent;

@@ -47,6 +47,8 @@ struct GpuWeight {
   // Q6_K planes written out from a type with one scale per 32 values, for the GEMM forms (the kernels' -DHD forms):
   // 2 = the two sub-scales of a block are equal (IQ3_S), 1 = moreover the planes hold half the values (IQ3_XXS)
   int half_d = 0;
+  // the rows as digits for the prefill GEMM, kept with the weight (Engine::digits_keep); none, or given back: size 0
+  cl_mem digits = nullptr;
 };
 
 inline const char* ggml_type_name(uint32_t t) {
@@ -82,6 +84,7 @@ class Engine {
     moe_dec_max_ = moe_dec_set_ ? atoi(getenv("ARCZ_MOE_DECODE_MAX")) : 16;
     moe_mm_off_ = moe_dec_off_ || (getenv("ARCZ_MOE_MM") && atoi(getenv("ARCZ_MOE_MM")) == 0);
     digits_env_ = getenv("ARCZ_GEMM_DIGITS") ? atoi(getenv("ARCZ_GEMM_DIGITS")) : -1;
+    digits_keep_ = !(getenv("ARCZ_DIGITS_KEEP") && atoi(getenv("ARCZ_DIGITS_KEEP")) == 0);
     gemm_split_ = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
     moe_fuse_off_ = getenv("ARCZ_MOE_FUSE") && atoi(getenv("ARCZ_MOE_FUSE")) == 0;
@@ -330,7 +333,12 @@ class Engine {
         wsv_bytes_ = need;
       }
     }
-    if (rows == (size_t)N && digits_take(w.type, max_chunk, N, K)) digits_reserve(w);
+    if (rows == (size_t)N) {
+      if (digits_take(w.type, max_chunk, N, K, false, max_chunk)) digits_reserve(w);
+      bool keep = false;  // (whether a chunk of this engine would take them)
+      for (int m = 128; !keep && m < 2 * max_chunk; m *= 2) keep = digits_take(w.type, std::min(m, max_chunk), N, K, true, std::min(m, max_chunk));
+      if (keep) digits_keep(w);
+    }
     if (type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS) {  // (room for its GEMM form)
       const size_t need = raw_planes_bytes(QT_Q6_K, rows, K / 256);
       if (need > xw_bytes_) {
@@ -344,8 +352,11 @@ class Engine {
     return w;
   }
   void free_weight(GpuWeight& w) {
+    not_listed(w.digits, "free_weight");
     if (w.raw) release(w.raw);
     w.raw = nullptr;
+    if (w.digits) release(w.digits);
+    w.digits = nullptr;
   }
   static uint64_t raw_bytes(const GpuWeight& w) { return arcz_gguf_bytes(w.type, w.rows, w.K); }  // (zero/engine.h:209)
 
@@ -806,6 +817,7 @@ class Engine {
   int moe_dec_max_ = 16, moe_tmd_ = 0;                                      // ARCZ_MOE_DECODE_MAX, ARCZ_MOE_TMD
   bool moe_dec_set_ = false, moe_mm_off_ = false;                           // ARCZ_MOE_DECODE_MAX given; ARCZ_MOE_MM = 0
   int digits_env_ = -1;                                                     // ARCZ_GEMM_DIGITS (-1: by rule)
+  bool digits_keep_ = true;                                                 // ARCZ_DIGITS_KEEP (0: off)
   int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
   bool moe_pre_ = true;                                                     // ARCZ_MOE_PRE (0: off)
@@ -817,21 +829,36 @@ class Engine {
   // such a matrix is uploaded, never in a matmul)
   cl_mem xd_ = nullptr, wd_ = nullptr;
   size_t wd_bytes_ = 0;
-  struct DigitForm { int nw, timg, wimg; };  // (nw: digits of a weight, 0: not a type of this GEMM; bytes of the images)
+  // (nw: digits of a weight, 0: not a type of this GEMM; bytes of the images)
+  struct DigitForm { int nw, timg, wimg; };
   static DigitForm digit_form(uint32_t type) {
     const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS ? 2 : type == GGML_Q4_0 || type == GGML_MXFP4 || type == GGML_IQ3_S ? 1 : 0;
     return {nw, nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512};
   }
-  // Where it pays, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
+  // Where it pays.  With the rows' digits kept (digits_keep) from more than 64 token rows on, against the int8 kernels: us, 128
+  // / 300 / 1024 tokens, 4096 x 4096: Q4_0 23 / 24, 31 / 40, 54 / 80, Q3_K 22 / 35, 36 / 52, 63 / 109, IQ3_XXS 22 / 31, 36 / 41,
+  // 62 / 76; 17408 x 5120: Q4_0 44 / 58, 87 / 139, 222 / 337, MXFP4 45 / 61, 86 / 146, 219 / 349, IQ3_S 44 / 93, 89 / 146, 223 /
+  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362; Q6_K (three digits) and IQ3_XXS where it is
+  // priced cheaper: Q6_K 17408 x 5120 75 / 90, 154 / 179, 391 / 518, but 2048 x 5120 28 / 22, 33 / 35, 59 / 70, 12288 x 4096, 300
+  // tokens, 109 / 99.
+  // Without, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
   // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43 / 42, 66 / 57, 109 / 75; Q4_0 30 / 35, 42 / 47, 80 / 64;
   // MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70, MXFP4 84 / 69,
   // IQ3_S 79 / 81; 1024 tokens x 4096 / 8192 / 12288 rows: Q6_K 98 / 103, 97.5 / 89 (of 2048), 277 / 234; IQ3_XXS 77 / 76,
   // -, 193 / 186; 4096 rows, K = 1024, 256 / 512 / 768 tokens: Q3_K 22 / 26, 23 / 27, 34 / 28.
-  bool digits_take(uint32_t type, int Mp, int N, int K) const {
+  bool digits_take(uint32_t type, int Mp, int N, int K, bool kept, int rows) const {
     // (ARCZ_GEMM_DIGITS=0: never, =1: always; not with ARCZ_GEMM_SPLIT, whose pieces are the int8 kernels')
     const double out = (double)Mp * N / (1 << 20);
     if (digits_env_ == 0 || gemm_split_ > 0) return false;
     if (digits_env_ > 0) return digit_form(type).nw != 0;
+    if (kept && Mp > 64 && digit_form(type).nw) {
+      if (type != GGML_Q6_K && type != GGML_IQ3_XXS) return true;
+      double d = 0.0, i8 = 0.0;
+      digit_pieces(digit_form(type), Mp, N, K / 256, &d);
+      split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
+      if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes: 128 tokens x
+      return d < i8;                                                 //  4096 x 4096 22 / 31, 300 x 12288 x 4096 88 / 82)
+    }
     if (Mp < 256) return false;
     switch (type) {
       case GGML_Q3_K: return out >= (K >= 2048 ? 1.0 : 3.0);
@@ -841,30 +868,44 @@ class Engine {
       default: return false;
     }
   }
-  // Pieces of K, priced as in split_pieces: us per 1024 values of K and full round (two work-groups a compute unit) 18, 25, 32
-  // with one, two, three digits; a last round of one work-group a unit 0.63.  Q3_K 4096 x 12288, 512 tokens: 195 -> 123 us.
-  static int digit_pieces(int nw, int Mp, int N, int nsb) {
+  // Pieces of K, priced as in split_pieces: a full round (two work-groups a compute unit) takes 15, 19.5, 28 us per 1024 values
+  // of K with one, two, three digits and 8 us for its ends, a last round of one work-group a unit 0.65 of
+  // that; the partial tiles cost 4 us and 12 TB/s.  Over 507 products of four types and six matrices, 100 - 1024 tokens in 1 - 8
+  // pieces, this is 5 % off on average and its choice loses 0.2 %.  Q3_K 4096 x 12288, 512 tokens: 195 -> 93 us.
+  static int digit_pieces(const DigitForm& f, int Mp, int N, int nsb, double* price = nullptr) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
+    const double k1024 = f.nw == 1 ? 15.0 : f.nw == 2 ? 19.5 : 28.0;
     int best = 1;
     double least = 0.0;
-    for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
+    for (int ny = 1; ny <= 16 && (ny == 1 || ny <= nsb / 2); ++ny) {
       if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const size_t full = tiles * ny / (2 * cus), rest = tiles * ny % (2 * cus);
-      const double part = rest == 0 ? 0.0 : rest <= cus ? 0.63 : 1.0;
-      double us = (full + (full ? 0.85 : 1.0) * part) * (nw == 1 ? 18.0 : nw == 2 ? 25.0 : 32.0) * nsb / 4 / ny;
-      if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
+      const double part = rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0;
+      double us = (full + part) * (k1024 * nsb / 4 / ny + 8.0);
+      if (ny > 1) us += 4.0 + 2.0 * ny * Mp * N * 4 / 12.0e6;
       if (ny == 1 || us < least) {
         best = ny;
         least = us;
       }
     }
+    if (price) *price = least + 3.0 + Mp * (nsb * 256) / 1.7e6;  // (with the tokens' digits)
     return best;
+  }
+  // rows [n0, n0 + 128 nt) of w as digits, into out
+  void row_digits(const char* name, const GpuWeight& w, int n0, int nt, cl_mem out) {
+    cl_kernel k = kernel("gemm", "-DQTYPE=" + std::to_string(w.type), "row_digits");
+    int N = w.N, nsb = w.K / 256;
+    set_args(k, 0, w.raw, tabs_, N, nsb, n0, out);
+    size_t g[2] = {(size_t)nsb * 256, (size_t)nt * 2}, l[2] = {256, 1};
+    run(name, k, 2, g, l);
   }
   void gemm_digits(const char* name, const GpuWeight& w, int Mp, cl_mem C, int ldc, int c_off, int a) {
     const DigitForm f = digit_form(w.type);
     int M = Mp, N = w.N, K = w.K, nsb = K / 256;
+    const bool kept = digits_kept(w);
+    cl_mem wd = kept ? w.digits : wd_;
     const int mt = (Mp + 127) / 128, nt_all = (N + 127) / 128;
-    const int panel = (int)std::min<size_t>((size_t)nt_all, wd_bytes_ / ((size_t)(K / 32) * f.wimg));
+    const int panel = kept ? nt_all : (int)std::min<size_t>((size_t)nt_all, wd_bytes_ / ((size_t)(K / 32) * f.wimg));
     if (!xd_ || panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
     size_t l[2] = {256, 1};
     {
@@ -876,19 +917,16 @@ class Engine {
     }
     for (int t0 = 0; t0 < nt_all; t0 += panel) {
       int nt = std::min(panel, nt_all - t0), n0 = t0 * 128;
-      cl_kernel kr = kernel("gemm", "-DQTYPE=" + std::to_string(w.type), "row_digits");
-      set_args(kr, 0, w.raw, tabs_, N, nsb, n0, wd_);
-      size_t g[2] = {(size_t)nsb * 256, (size_t)nt * 2};
-      run("row_digits", kr, 2, g, l);
+      if (!kept) row_digits("row_digits", w, n0, nt, wd_);
       cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
       // (ARCZ_Q4_SPLITK=0: K in one piece, =n: n pieces, as many as SPLIT_BYTES holds)
       int ny = nt < nt_all || sk_force_ == 0 ? 1
                : sk_force_ >= 2 ? std::max(1, (int)std::min<size_t>(std::min(sk_force_, nsb), SPLIT_BYTES / ((size_t)Mp * N * 4)))
-                                : digit_pieces(f.nw, Mp, N, nsb), zero = 0;
+                                : digit_pieces(f, Mp, N, nsb), zero = 0;
       size_t gg[2] = {(size_t)mt * nt * 256, (size_t)ny};
-      if (ny > 1) set_args(k, 0, xd_, wd_, ws, M, N, K, N, zero, zero, n0, nt);
-      else set_args(k, 0, xd_, wd_, C, M, N, K, ldc, c_off, a, n0, nt);
+      if (ny > 1) set_args(k, 0, xd_, wd, ws, M, N, K, N, zero, zero, n0, nt);
+      else set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, n0, nt);
       run(name, k, 2, gg, l);
       if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
     }
@@ -912,7 +950,7 @@ class Engine {
   // alone, 9 %): 300 tokens Q6_K 5120 x 17408 248 -> 209 us, 4096 x 12288 176 -> 125; Q8_0 4096 x 12288 x 512 107 -> 86,
   // 4096 x 4096 x 512 39.3 -> 36.9.  IQ3_S and IQ3_XXS over six matrices x 40 - 900 tokens: 1.0 % (1.2 % at Q6_K's price, 10 %
   // at 256 x 4096 rows, K = 1024, which two pieces make 19.4 instead of 17.7 us).
-  static int split_pieces(uint32_t type, int half_d, int Mp, int m64, int N, int nsb) {
+  static int split_pieces(uint32_t type, int half_d, int Mp, int m64, int N, int nsb, double* price = nullptr) {
     const bool q8 = type == GGML_Q8_0;
     const double round = q8 ? 21.2 : half_d ? 20.4 : 24.7;
     const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)m64 * ((N + 127) / 128);
@@ -929,6 +967,7 @@ class Engine {
         least = us;
       }
     }
+    if (price) *price = least;
     return best;
   }
   // Room for the digits: an engine makes it when it uploads a weight that the rule takes.  Without it such a weight runs on
@@ -937,7 +976,7 @@ class Engine {
   void digits_reserve(const GpuWeight& w) {
     const size_t tile = (size_t)(w.K / 32) * digit_form(w.type).wimg;
     const size_t need = std::max(tile, std::min((size_t)(w.N + 127) / 128 * tile, (size_t)512 << 20));
-    if (!xd_) xd_ = try_buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
+    digits_tokens();
     if (!xd_ || need <= wd_bytes_ || (wd_ && arcz_mem_listed(wd_))) return;
     if (wd_) release(wd_);
     wd_ = nullptr;
@@ -945,18 +984,38 @@ class Engine {
     wd_ = try_buf(need);
     if (wd_) wd_bytes_ = need;
   }
+  void digits_tokens() {
+    if (!xd_) xd_ = try_buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
+  }
+  // The rows' digits kept with the weight, so that no matmul writes them: 5 us of 4096 x 4096, 33 us of 17408 x 5120 with one
+  // digit (512 tokens Q4_0 169 -> 140 us, 300 118 -> 87).  1 - 2.5 bytes a weight beside
+  // the 0.4 - 0.8 of its planes: from 2^23 values on -- smaller ones are written in about a launch's time --, while such
+  // copies hold less than an eighth of the device's memory and a quarter of it stays free behind them; where an allocation
+  // finds no memory later they are given back (arcz_mem_spare) and the matmul writes digits again or takes the int8 kernels.
+  // ARCZ_DIGITS_KEEP=0 when the engine is made: never.
+  void digits_keep(GpuWeight& w) {
+    const size_t bytes = (size_t)(w.N + 127) / 128 * (w.K / 32) * digit_form(w.type).wimg, total = arcz_device_mem();
+    if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << 23)) return;
+    if (arcz_spare_bytes() + bytes > total / 8 || arcz_device_mem_free() < bytes + total / 4) return;
+    digits_tokens();
+    if (!xd_ || !(w.digits = try_buf(bytes))) return;
+    CL_CHECK(arcz_mem_spare(w.digits));
+    row_digits("keep_digits", w, 0, (w.N + 127) / 128, w.digits);
+  }
+  static bool digits_kept(const GpuWeight& w) { return w.digits && arcz_mem_size(w.digits) != 0; }
   // All the rows at once, or panels that give every compute unit a work-group: a launch of fewer takes as long as one that
   // fills the chip (Q4_0 17408 x 5120 x 1024 in panels of 2, 8, 32, 64 row tiles and at once 4111, 1060, 335, 288, 260 us, on
   // the int8 kernels 335; x 256 in panels of 64 212, at once 113, int8 138).  A three-bit weight that the int8 kernels have no
   // room for either (xw_): any panel.
   bool digits_room(const GpuWeight& w, int Mp) const {
+    if (digits_kept(w)) return xd_ != nullptr;
     const size_t panel = wd_bytes_ / ((size_t)(w.K / 32) * digit_form(w.type).wimg), all = (size_t)(w.N + 127) / 128;
     const bool expanded = w.type == GGML_IQ3_S || w.type == GGML_Q3_K || w.type == GGML_IQ3_XXS;
     if (expanded && raw_planes_bytes(QT_Q6_K, w.rows, w.K / 256) > xw_bytes_) return xd_ && panel >= 1;
     return xd_ && (panel >= all || panel * ((Mp + 127) / 128) >= (size_t)arcz_device_cus());
   }
   void gemm_dense(const char* name, const GpuWeight& w0, int Mp, cl_mem C, int ldc, int c_off, int a) {
-    if (digits_take(w0.type, Mp, w0.N, w0.K) && digits_room(w0, Mp)) {
+    if (digits_take(w0.type, Mp, w0.N, w0.K, digits_kept(w0), std::clamp(cur_rows_, 1, Mp)) && digits_room(w0, Mp)) {
       gemm_digits(name, w0, Mp, C, ldc, c_off, a);
       return;
     }

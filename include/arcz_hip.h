@@ -44,6 +44,8 @@ const char* arcz_last_error(void);
 const char* arcz_device_name(void);
 int arcz_device_cus(void);
 size_t arcz_device_mem(void);
+/* Bytes of it that are free now. */
+size_t arcz_device_mem_free(void);
 
 /* clCreateBuffer (clrt.h:744-751): device memory, at least 64 bytes, 256-byte aligned; NULL + error text on failure.
  * An allocation that fails calls the out-of-memory hook and is retried up to 8 times (clrt.h:474-487). */
@@ -54,6 +56,12 @@ arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes);
  * caller frees views before their parents (zero/engine.h:251-252): an owner that still has live views is refused
  * (ARCZ_E_ARG_VALUE, nothing freed). */
 int arcz_free(arcz_mem* m);
+/* Marks a buffer whose contents the caller can do without (weights laid out a second time for one of the kernels): where an
+ * allocation finds no memory, all such buffers that no launch list names are freed before the out-of-memory hook is asked;
+ * their handles stay live, of size 0, until arcz_free. */
+int arcz_mem_spare(arcz_mem* m);
+/* Bytes of such buffers held now. */
+size_t arcz_spare_bytes(void);
 size_t arcz_mem_size(const arcz_mem* m);
 /* The device address of a buffer (for interop with another runtime on the same device; not used by the engine). */
 void* arcz_mem_ptr(const arcz_mem* m);

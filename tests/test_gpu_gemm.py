@@ -386,6 +386,65 @@ def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
     assert counts[0] == digits and products in (None, counts[1]), counts
 
 
+@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 128, 4096, 2048), (az.Q3_K, 200, 4099, 2304), (az.Q6_K, 256, 4100, 4096), (az.IQ3_XXS, 200, 12300, 2048),
+                                         (az.MXFP4, 65, 4225, 2048)])
+def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
+    """Matrices of 2^23 values and more keep their rows' digits: no matmul writes them, and shorter chunks are multiplied on
+    digits.  Given back where an allocation finds no memory -- not while a recorded list names them --, the weight is
+    multiplied all the same.  Against the oracle."""
+    print(f"kept digits {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    Mp = (T + 15) // 16 * 16 if T < 128 else (T + 127) // 128 * 128
+    W = make_weights(qtype, N, K, seed=61)
+    x = make_acts(T, K, seed=62, outliers=True)
+    aq, asc, _ = quantize_padded(x, Mp)
+    rows = np.r_[0:300, N - 300:N]
+    Ws = np.ascontiguousarray(W.reshape(N, -1)[rows]).reshape(-1)
+    ref = orc.matmul_ref(qtype, Ws, len(rows), K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    eng = az.Engine(512, K)
+    spare0 = az.lib.arcz_spare_bytes()
+    w = eng.make_weight(qtype, N, K, W)
+    spare1 = az.lib.arcz_spare_bytes()
+    assert spare1 > spare0
+    xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * N * 4)
+
+    def step():
+        eng.quantize(xb, K, K, Mp, T)
+        eng.matmul("test", w, Mp, cb, N, 0, 0)
+
+    def out(f):
+        cb.fill(0xFFFFFFFF)
+        f()
+        y = cb.read(np.float32, Mp * N).reshape(Mp, N)
+        assert np.isfinite(y).all() and not y[T:].any() and rel_err_rows(y[:T, rows], ref).max() <= TOL
+        return y.view(np.uint32)
+
+    eng.profile(True)
+    y = out(step)
+    eng.profile_collect()
+    assert eng.profile_get("act_digits")[1] == 1 and eng.profile_get("row_digits")[1] == 0
+    eng.profile(False)
+    lst = az.Runtime.record(step)
+    try:
+        az.lib.arcz_set_fake_oom(1)
+        with pytest.raises(az.ArczError):
+            az.Runtime.alloc(1024)                      # (every allocation fails once; what the list names stays)
+        assert az.lib.arcz_spare_bytes() == spare1
+        assert np.array_equal(out(lst.run), y)
+        lst.free()
+        lst = None
+        az.Runtime.alloc(1024).free()
+        assert az.lib.arcz_spare_bytes() == spare0
+    finally:
+        az.lib.arcz_set_fake_oom(0)
+        if lst is not None:
+            lst.free()
+    out(step)
+    for b in (xb, cb, w):
+        b.free()
+    eng.close()
+    assert az.lib.arcz_spare_bytes() == spare0
+
+
 def _extreme_rows(qtype, N, K, rng):
     """Blocks of random bytes with the superblock's scale set to one (IQ3_XXS: four), so that all values are integers; a
     fifth of the Q6_K and Q3_K rows at the ends of their ranges: every value -32 or 31 times -128 or 127, -4 or 3 times -32
