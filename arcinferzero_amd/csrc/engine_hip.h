@@ -829,18 +829,20 @@ class Engine {
   // such a matrix is uploaded, never in a matmul)
   cl_mem xd_ = nullptr, wd_ = nullptr;
   size_t wd_bytes_ = 0;
-  // (nw: digits of a weight, 0: not a type of this GEMM; bytes of the images)
-  struct DigitForm { int nw, timg, wimg; };
+  // (nw: digits of a weight, 0: not a type of this GEMM; mn: with a minimum; bytes of the images: gemm_d.hip's DImg)
+  struct DigitForm { int nw, mn, timg, wimg; };
   static DigitForm digit_form(uint32_t type) {
-    const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS ? 2 : type == GGML_Q4_0 || type == GGML_MXFP4 || type == GGML_IQ3_S ? 1 : 0;
-    return {nw, nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512};
+    const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS ? 2
+                   : type == GGML_Q4_0 || type == GGML_MXFP4 || type == GGML_IQ3_S || type == GGML_Q4_K || type == GGML_Q5_K ? 1 : 0;
+    const int mn = type == GGML_Q4_K || type == GGML_Q5_K ? 1 : 0;
+    return {nw, mn, mn ? 7680 : nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512 + 1024 * mn};
   }
   // Where it pays.  With the rows' digits kept (digits_keep) from more than 64 token rows on, against the int8 kernels: us, 128
   // / 300 / 1024 tokens, 4096 x 4096: Q4_0 23 / 24, 31 / 40, 54 / 80, Q3_K 22 / 35, 36 / 52, 63 / 109, IQ3_XXS 22 / 31, 36 / 41,
   // 62 / 76; 17408 x 5120: Q4_0 44 / 58, 87 / 139, 222 / 337, MXFP4 45 / 61, 86 / 146, 219 / 349, IQ3_S 44 / 93, 89 / 146, 223 /
-  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362; Q6_K (three digits) and IQ3_XXS where it is
-  // priced cheaper: Q6_K 17408 x 5120 75 / 90, 154 / 179, 391 / 518, but 2048 x 5120 28 / 22, 33 / 35, 59 / 70, 12288 x 4096, 300
-  // tokens, 109 / 99.
+  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362, Q5_K 51 / 68, 102 / 143, 268 / 336; Q4_K,
+  // Q6_K (three digits) and IQ3_XXS where it is priced cheaper: Q4_K 17408 x 5120 50 / 61, 101 / 110, 262 / 295, but 12288 x
+  // 4096, 300 tokens, 82 / 69; Q6_K 17408 x 5120 75 / 90, 154 / 179, 391 / 518, but 2048 x 5120 28 / 22, 33 / 35, 59 / 70.
   // Without, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
   // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43 / 42, 66 / 57, 109 / 75; Q4_0 30 / 35, 42 / 47, 80 / 64;
   // MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70, MXFP4 84 / 69,
@@ -851,11 +853,16 @@ class Engine {
     const double out = (double)Mp * N / (1 << 20);
     if (digits_env_ == 0 || gemm_split_ > 0) return false;
     if (digits_env_ > 0) return digit_form(type).nw != 0;
+    // (Q4_K, Q5_K: not with a switch that names one of the int8 forms, the number of their pieces among them; per-256 activation
+    //  scales have Q4_K's form that adds a superblock's block sums as integers)
+    static const bool q4_forms = getenv("ARCZ_Q4_BM") || getenv("ARCZ_Q4_BN") || getenv("ARCZ_Q4_SMALL") || getenv("ARCZ_Q4_AU");
+    if ((type == GGML_Q4_K || type == GGML_Q5_K) && (sk_force_ >= 2 || q4_wm_ != 0 || q4_forms || (a256_ && type == GGML_Q4_K))) return false;
     if (kept && Mp > 64 && digit_form(type).nw) {
-      if (type != GGML_Q6_K && type != GGML_IQ3_XXS) return true;
+      if (type != GGML_Q6_K && type != GGML_IQ3_XXS && type != GGML_Q4_K) return true;
       double d = 0.0, i8 = 0.0;
       digit_pieces(digit_form(type), Mp, N, K / 256, &d);
-      split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
+      if (type == GGML_Q4_K) i8 = q4k_price(Mp, rows, N, K / 256);
+      else split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
       if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes: 128 tokens x
       return d < i8;                                                 //  4096 x 4096 22 / 31, 300 x 12288 x 4096 88 / 82)
     }
@@ -868,13 +875,24 @@ class Engine {
       default: return false;
     }
   }
+  // us of a Q4_K product on the int8 kernels as gemm_dense launches them: pieces of K, 64 x 128 tiles (three work-groups a compute
+  // unit) or 128 x 128 (two).  Fitted to seven matrices x 128 - 2048 tokens, 4.6 % off on average.
+  static double q4k_price(int Mp, int rows, int N, int nsb) {
+    const double cus = arcz_device_cus(), nt = (N + 127) / 128, t128 = (Mp + 127) / 128 * nt, t64 = (rows + 63) / 64 * nt;
+    const int ny = (int)std::min({8.0, nsb / 2.0, 2 * cus / t128});
+    if (ny >= 3) return 8.0 + (t128 * ny <= cus ? 0.71 : 1.0) * (24.6 * nsb / 4 / ny + 2.7) + 2.0 * ny * Mp * N * 4 / 8.0e6;
+    const double r128 = std::fmod(t128, 2 * cus), r64 = std::fmod(t64, 3 * cus), f128 = std::floor(t128 / (2 * cus)), f64 = std::floor(t64 / (3 * cus));
+    const double c128 = f128 + (r128 == 0 ? 0.0 : r128 <= cus ? 0.5 : 1.0), c64 = 0.8 * f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.30 : r64 <= 2 * cus ? 0.48 : 0.8);
+    if (c64 < 0.97 * c128) return 8.3 + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.63 : r64 <= 2 * cus ? 0.73 : 1.0)) * (19.1 * nsb / 4 + 2.7);
+    return 8.3 + (f128 + (r128 == 0 ? 0.0 : r128 <= cus ? 0.71 : 1.0)) * (24.6 * nsb / 4 + 2.7);
+  }
   // Pieces of K, priced as in split_pieces: a full round (two work-groups a compute unit) takes 15, 19.5, 28 us per 1024 values
-  // of K with one, two, three digits and 8 us for its ends, a last round of one work-group a unit 0.65 of
+  // of K with one, two, three digits (Q4_K, Q5_K: 18.5) and 8 us for its ends, a last round of one work-group a unit 0.65 of
   // that; the partial tiles cost 4 us and 12 TB/s.  Over 507 products of four types and six matrices, 100 - 1024 tokens in 1 - 8
   // pieces, this is 5 % off on average and its choice loses 0.2 %.  Q3_K 4096 x 12288, 512 tokens: 195 -> 93 us.
   static int digit_pieces(const DigitForm& f, int Mp, int N, int nsb, double* price = nullptr) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
-    const double k1024 = f.nw == 1 ? 15.0 : f.nw == 2 ? 19.5 : 28.0;
+    const double k1024 = f.nw == 1 ? (f.mn ? 18.5 : 15.0) : f.nw == 2 ? 19.5 : 28.0;
     int best = 1;
     double least = 0.0;
     for (int ny = 1; ny <= 16 && (ny == 1 || ny <= nsb / 2); ++ny) {
@@ -911,14 +929,14 @@ class Engine {
     {
       cl_kernel k = kernel("gemm", "", "act_digits");
       int img = f.timg;
-      set_args(k, 0, aq_, asc_, M, K, img, xd_);
+      set_args(k, 0, aq_, asc_, absum_, M, K, img, xd_);
       size_t g[2] = {(size_t)nsb * 256, (size_t)mt * 2};
       run("act_digits", k, 2, g, l);
     }
     for (int t0 = 0; t0 < nt_all; t0 += panel) {
       int nt = std::min(panel, nt_all - t0), n0 = t0 * 128;
       if (!kept) row_digits("row_digits", w, n0, nt, wd_);
-      cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw), "gemm_d");
+      cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw) + (f.mn ? " -DMN=1" : ""), "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
       // (ARCZ_Q4_SPLITK=0: K in one piece, =n: n pieces, as many as SPLIT_BYTES holds)
       int ny = nt < nt_all || sk_force_ == 0 ? 1
@@ -985,7 +1003,7 @@ class Engine {
     if (wd_) wd_bytes_ = need;
   }
   void digits_tokens() {
-    if (!xd_) xd_ = try_buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7168);
+    if (!xd_) xd_ = try_buf(((size_t)max_chunk + 127) / 128 * (max_k / 32) * 7680);
   }
   // The rows' digits kept with the weight, so that no matmul writes them: 5 us of 4096 x 4096, 33 us of 17408 x 5120 with one
   // digit (512 tokens Q4_0 169 -> 140 us, 300 118 -> 87).  1 - 2.5 bytes a weight beside

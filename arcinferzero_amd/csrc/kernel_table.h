@@ -84,8 +84,9 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm", "AU", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "AU", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm", "BM", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "BM", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "act_digits", nullptr, "ppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "act_digits", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits", nullptr, "ppiiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm_d", "MN", "pppiiiiiiii", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_d", nullptr, "pppiiiiiiii", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},

@@ -1,4 +1,4 @@
-// "gemm" module, second file: the prefill GEMM on digits (Q4_0, MXFP4, IQ3_S, IQ3_XXS, Q3_K, Q6_K; long chunks).
+// "gemm" module, second file: the prefill GEMM on digits (Q4_K, Q5_K, Q4_0, MXFP4, IQ3_S, IQ3_XXS, Q3_K, Q6_K).
 //
 //   C[m][c_off + n] (=, +=, silu(C) *)  sum over 32-blocks b of  (sa[m][b] * ws[n][b]) * J[m][n][b]
 //   J[m][n][b] = sum over the block's 32 k of x[m][k] * w[n][k], integers
@@ -22,6 +22,8 @@
 // cycles.  Hence few bytes and few instructions per product: a wave's operands serve 64 x 64 outputs, the addresses of a
 // step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 863 TOP/s, two 651, three
 // 504 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650 and 375).
+// Q4_K and Q5_K with the min term, 17408 x 5120, us, int8 kernels and this: 8192 tokens Q4_K 2020 / 1850, 2048 544 / 470, Q5_K
+// 593 / 472, 300 110 / 100, 143 / 100.
 // Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 136, MXFP4 183 / 135, IQ3_S
 // 201 / 147, Q3_K 293 / 182, Q6_K 277 / 234; x 4096: Q6_K 1094 / 790, IQ3_XXS 742 / 596.
 #include "common.h"
@@ -45,12 +47,14 @@ __device__ inline void dma16(const void* src, uint32_t lds_wave_base) {
 // and 128 weight rows x one block
 //   per digit [128][16 bytes], [128][8 bytes]; then [128] f32 ws
 // A tile's blocks follow each other.  NB: blocks a step of the GEMM takes; steps are whole KiB.
-template <int NW> struct DImg {
+// Types with a minimum (MN: Q4_K, Q5_K) have behind sa [128][8 bytes] u = sa * S, and behind ws v, of the min term: bf16 pieces
+// x1 | x2 << 16, x3 | x3 << 16.
+template <int NW, int MN = 0> struct DImg {
   static constexpr int NB = NW == 3 ? 1 : 2;
   static constexpr int R = NB == 2 ? 3 : 4;  // stages in LDS
-  static constexpr int T = NB == 2 ? 6656 : 7168, W = NB == 2 ? NW * 3072 + 512 : 10240;
+  static constexpr int T = MN ? 7680 : NB == 2 ? 6656 : 7168, W = NB == 2 ? NW * 3072 + 512 + 1024 * MN : 10240;
   static constexpr int STAGE = NB * (T + W);
-  static constexpr int TSA = 6144, WWS = NW * 3072;
+  static constexpr int TSA = 6144, TU = 6656, WWS = NW * 3072, WV = WWS + 512;
 };
 
 // 16 codes, a byte each, to 96 bits
@@ -78,10 +82,11 @@ __device__ inline void sign_mag(uint32_t v, uint32_t& s, uint32_t& a) {
   a = (v ^ ((s << 8) - s)) + s;
 }
 
-// act_digits: aq [M][K], asc [K/32][M] -> token images xt of img bytes.  Rows past M are zeros.  A thread: two blocks of a
-// row.  grid (K / 256, 2 * token tiles), local 256.
+// act_digits: aq [M][K], asc [K/32][M], absum [K/16][M] -> token images xt of img bytes, 7680: with u.  Rows past M are
+// zeros.  A thread: two blocks of a row.  grid (K / 256, 2 * token tiles), local 256.
 extern "C" __global__ __launch_bounds__(256) void act_digits(const signed char* __restrict__ aq, const float* __restrict__ asc,
-                                                             int M, int K, int img, uint8_t* __restrict__ xt) {
+                                                             const short* __restrict__ absum, int M, int K, int img,
+                                                             uint8_t* __restrict__ xt) {
   const int s = blockIdx.x, r = (blockIdx.y & 1) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6, m = (blockIdx.y >> 1) * 128 + r;
   uint8_t* dst = xt + ((size_t)(blockIdx.y >> 1) * (K >> 5) + s * 8 + 2 * q) * img;
   u4v x[4] = {};
@@ -105,18 +110,22 @@ extern "C" __global__ __launch_bounds__(256) void act_digits(const signed char* 
     const int b = s * 8 + 2 * q + i;
     const float sa = m < M ? asc[(size_t)b * M + m] : 0.0f;
     *(float*)(dst + i * img + 6144 + r * 4) = sa;
+    if (img == DImg<1, 1>::T) {
+      uint32_t w0, w1;
+      split3(m < M ? sa * (float)((int)absum[(size_t)(2 * b) * M + m] + (int)absum[(size_t)(2 * b + 1) * M + m]) : 0.0f, w0, w1);
+      *(u2v*)(dst + i * img + DImg<1, 1>::TU + r * 8) = (u2v){w0, w1 | w1 << 16};
+    }
   }
 }
 
 // ---- the rows.  A thread: two blocks b[0], b[1] of row n; v[i]: their values as int8, four a word, or, with the sub-scales
 // folded in (Q6_K, Q3_K), signs and the products of the magnitudes.
-template <int QT> struct DType;
-template <> struct DType<QT_Q6_K> { enum { NW = 3 }; };
-template <> struct DType<QT_Q4_0> { enum { NW = 1 }; };
-template <> struct DType<QT_MXFP4> { enum { NW = 1 }; };
-template <> struct DType<QT_Q3_K> { enum { NW = 2 }; };
-template <> struct DType<QT_IQ3_S> { enum { NW = 1 }; };
-template <> struct DType<QT_IQ3_XXS> { enum { NW = 2 }; };
+template <int QT> struct DType { enum { NW = 1, MN = 0 }; };
+template <> struct DType<QT_Q6_K> { enum { NW = 3, MN = 0 }; };
+template <> struct DType<QT_Q3_K> { enum { NW = 2, MN = 0 }; };
+template <> struct DType<QT_IQ3_XXS> { enum { NW = 2, MN = 0 }; };
+template <> struct DType<QT_Q4_K> { enum { NW = 1, MN = 1 }; };
+template <> struct DType<QT_Q5_K> { enum { NW = 1, MN = 1 }; };
 
 // int8 values of eight words -> NW digits' codes
 template <int NW> __device__ inline void codes_i8(const uint32_t* v, uint32_t (*c)[8]) {
@@ -154,14 +163,14 @@ template <int NW> __device__ inline void codes_scaled(const uint32_t* v, int sc0
 template <int QT>
 __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_t* __restrict__ tabs, int N, int nsb, int n0,
                                   uint8_t* __restrict__ wt) {
-  constexpr int NW = DType<QT>::NW;
-  using I = DImg<NW>;
+  constexpr int NW = DType<QT>::NW, MN = DType<QT>::MN;
+  using I = DImg<NW, MN>;
   const int s = blockIdx.x, r = (blockIdx.y & 1) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6, n = n0 + (blockIdx.y >> 1) * 128 + r;
   const bool in = n < N;
   const size_t u = (size_t)(in ? n : 0) * nsb + s;  // the row's superblock in every plane
   int b[2] = {2 * q, 2 * q + 1};
   uint32_t c[2][NW][8];
-  float ws[2];
+  float ws[2], mv[2] = {};  // (mv: the min term's row factor)
   if constexpr (QT == QT_Q6_K) {
     // blocks 4 n2 + c and 4 n2 + c + 2: low and high nibbles of ql bytes 64 n2 + 32 c + 0..31, bits 2 c + 4 i of qh bytes 32 n2 + 0..31
     const PlanesQ6K pl = planes_q6k((size_t)N, nsb);
@@ -181,6 +190,33 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
         v[k] = ((l | h << 4) + 0x60606060u) ^ 0x80808080u;  // q - 32
       }
       codes_scaled<3>(v, sc[2 * b[i]], sc[2 * b[i] + 1], c[i]);
+    }
+  } else if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
+    // blocks 2 q and 2 q + 1: the low and high nibbles of bytes 32 q .. 32 q + 31.  The values are taken around their middle
+    // h = 8 or 16, which makes Q5_K's one digit (-16 is one) and leaves less to cancel between products and min term, v: d sc
+    // q - dmin mn = d sc (q - h) + (h d sc - dmin mn).  Off by, against 64 bits, K = 5120 and 17408, of the result's norm: Q4_K
+    // 1.2e-7 and 1.7e-7 (int8 kernels 1.6e-7, 2.4e-7), tokens with a mean of half their deviation 2.3e-7 and 3.8e-7 (2.8e-7,
+    // 3.3e-7; with the values as they are 9.7e-7, 1.8e-6), Q5_K 1.6e-7 and 2.5e-7.
+    const PlanesQ4K pl = planes_q4k((size_t)N, nsb);
+    const u4v L[2] = {*(const u4v*)(raw + pl.qs + u * 128 + 32 * q), *(const u4v*)(raw + pl.qs + u * 128 + 32 * q + 16)};
+    const u4v h = *(const u4v*)(raw + pl.hdr + u * 16);
+    u2v H = {0, 0};
+    if constexpr (QT == QT_Q5_K) H = *(const u2v*)(raw + pl.qh + u * 32 + 8 * q);
+    const float d = f16_bits_to_f32(h[0]), dmin = f16_bits_to_f32(h[0] >> 16);
+    int sc[2], mn[2];
+    q4k_scales_pair(h[1], h[2], h[3], q, sc[0], sc[1], mn[0], mn[1]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t w = L[k >> 2][k & 3];
+        if constexpr (QT == QT_Q4_K) v[k] = q40_vals(w >> (4 * i));  // q - 8
+        else v[k] = ((i ? q5k_hi(w, H[k >> 2], k & 3) : q5k_lo(w, H[k >> 2], k & 3)) + 0x70707070u) ^ 0x80808080u;  // q - 16
+      }
+      codes_i8<1>(v, c[i]);
+      ws[i] = d * (float)sc[i];
+      mv[i] = (QT == QT_Q4_K ? 8.0f : 16.0f) * ws[i] - dmin * (float)mn[i];
     }
   } else if constexpr (QT == QT_Q3_K) {
     const PlanesIQ3S pl = planes_iq3s((size_t)N, nsb);
@@ -257,6 +293,12 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
       put_digit(img + d * 3072 + r * 16, img + d * 3072 + 2048 + r * 8, c[i][d]);
     }
     *(float*)(img + I::WWS + r * 4) = in ? ws[i] : 0.0f;
+    if (!in) mv[i] = 0.0f;
+    if constexpr (MN) {
+      uint32_t w0, w1;
+      split3(mv[i], w0, w1);
+      *(u2v*)(img + I::WV + r * 8) = (u2v){w0, w1 | w1 << 16};
+    }
   }
 }
 #define ROW_DIGITS(QT)                                                                                                  \
@@ -264,18 +306,18 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
                                                                           int nsb, int n0, uint8_t* wt) {               \
     row_digits<QT>(raw, tabs, N, nsb, n0, wt);                                                                          \
   }
-ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
+ROW_DIGITS(12) ROW_DIGITS(13) ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
 
 // ---- gemm_d: 128 tokens x 128 rows in four waves of 64 x 64, two work-groups a compute unit.  Blocks [b0, b1), an even number.
 // (Eight waves of 32 x 64, four a SIMD, hide more waits and read each row digit from LDS twice as often: 5 - 6 % slower, at
 // 17408 x 5120 x 8192 812 against 863 TOP/s with one digit, 632 / 651 with two, 476 / 504 with three.)
-template <int NW>
+template <int NW, int MN>
 __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __restrict__ xt, const uint8_t* __restrict__ wt,
                                             float* __restrict__ C, int M, int N, int ldc, int c_off, int accumulate, int m0,
                                             int n0, int nblk, int b0, int b1) {
   // (every access below is by offset; the array itself has to stay)
   asm volatile("" :: "v"((__attribute__((address_space(3))) uint8_t*)lds_base) : "memory");
-  using I = DImg<NW>;
+  using I = DImg<NW, MN>;
   constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, TS = NB * I::T, WS = NB * I::W;
   constexpr int TKB = TS / 1024, KB = STAGE / 1024, ND = (KB + 3) / 4;
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
@@ -298,10 +340,15 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
   const uint32_t oA16 = wm * 2048 + lane * 16, oA8 = 4096 + wm * 1024 + lane * 8;
   const uint32_t oW16 = TS + (wn * 64 + l32) * 16, oW8 = TS + 2048 + (wn * 64 + l32) * 8;
   const uint32_t oSA = I::TSA + (wm * 64 + l32) * 4, oWS = TS + I::WWS + (wn * 64 + lane) * 4;
-  uint32_t pA16, pA8, pW16, pW8, pSA, pWS;
+  const uint32_t oU = I::TU + g * I::T + (wm * 64 + l32) * 8, oV = TS + I::WV + g * I::W + (wn * 64 + l32) * 8;
+  uint32_t pA16, pA8, pW16, pW8, pSA, pWS, pU = 0, pV = 0;
   auto at = [&](uint32_t stage) {
     pA16 = oA16 + stage; pA8 = oA8 + stage; pW16 = oW16 + stage; pW8 = oW8 + stage; pSA = oSA + stage; pWS = oWS + stage;
     asm volatile("" : "+v"(pA16), "+v"(pA8), "+v"(pW16), "+v"(pW8), "+v"(pSA), "+v"(pWS));
+    if constexpr (MN) {
+      pU = oU + stage; pV = oV + stage;
+      asm volatile("" : "+v"(pU), "+v"(pV));
+    }
   };
   auto ldA = [&](int ms, int blk) {
     A[ms].lo = *LDS_P(const u4v, pA16 + (NB == 2 ? blk : 0) * I::T + ms * 1024);
@@ -336,6 +383,17 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
 #pragma unroll
     for (int e = 0; e < 32; ++e) z[e] = 0.0f;
     P[ms] = __builtin_amdgcn_mfma_f32_32x32x1f32(saop[ms], wsop, z, 0, 0, 0);
+  };
+  // The min term, u x v of both blocks of a step in one bf16 instruction, added straight to the results: a lane half takes a
+  // block, its eight k are the products of the pieces but u3 v3 (2^-32 of the whole).
+  u2v U[2], V[2];
+  auto ldU = [&](int ms) { U[ms] = *LDS_P(const u2v, pU + ms * 256); };
+  auto ldV = [&](int ns) { V[ns] = *LDS_P(const u2v, pV + ns * 256); };
+  auto mfma_min = [&](int ms, int ns) {
+    typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+    const uint32_t v11 = __builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x01000100u), v22 = __builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x03020302u);
+    const u4v a = {U[ms][0], U[ms][0], U[ms][0], U[ms][1]}, b = {v11, v22, V[ns][1], V[ns][0]};
+    res[ms][ns] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), res[ms][ns], 0, 0, 0);
   };
   // ---- prologue: the first R - 1 steps on their way, the first block's operands
 #pragma unroll
@@ -374,6 +432,12 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
       }
       if (q == 1) mfma_p(1);
       if (q == 3) mfma_p(0);
+      if constexpr (MN) {  // (each tile between two of its multiply-adds)
+        if (p == 2) mfma_min(0, 0);
+        if (p == 3) mfma_min(0, 1);
+        if (p == 4) mfma_min(1, 1);
+        if (p == 5) mfma_min(1, 0);
+      }
       // -- the step's meeting: what the waves brought for the next step lies in LDS, the step before is read
       if (NB == 2 ? p == 6 : q == 2) {
         __builtin_amdgcn_sched_barrier(0);
@@ -395,6 +459,10 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
       if (q == 0) { ldW(blk ? 0 : 1, blk); ldA(1, blk); }
       if (q == 2) { ldA(0, nb); ldSA(0, nb); ldWS(nb); }
       if (q == 3) { ldW(blk ? 0 : 1, nb); ldSA(1, nb); }
+      if constexpr (MN) {
+        if (p == 0) { ldU(0); ldV(0); ldV(1); }
+        if (p == 1) ldU(1);
+      }
       {
         // (two blocks a step: two pieces a slot, 6, 7 and, one turn on, 0, 1; one: three and two)
         const int f = NB == 2 ? (p + 2 & 7) * 2 : q == 2 ? 0 : q == 3 ? 3 : ND;
@@ -441,14 +509,15 @@ __device__ inline void d_tile_of(int id, int mt, int nt, int& tm, int& tn) {
 
 // gemm_d__NW: rows [n0, n0 + 128 ..) of an N-row matrix, nt row tiles of them in wt.  grid (ceil(M / 128) * nt, ny); ny > 1:
 // the superblocks shared out, plane y of C (here a workspace [ny][M][ldc]) the y-th piece's sums.
-#define GEMM_D(NWV)                                                                                                     \
-  extern "C" __global__ __launch_bounds__(256, 2) void gemm_d__NW##NWV(                                                 \
+#define GEMM_D(NAME, ...)                                                                                               \
+  extern "C" __global__ __launch_bounds__(256, 2) void gemm_d__##NAME(                                                  \
       const uint8_t* xt, const uint8_t* wt, float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int n0, int nt) { \
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[DImg<NWV>::R * DImg<NWV>::STAGE];                             \
+    using I = DImg<__VA_ARGS__>;                                                                                        \
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[I::R * I::STAGE];                                             \
     int tm, tn;                                                                                                         \
     d_tile_of(blockIdx.x, (M + 127) / 128, nt, tm, tn);                                                                 \
     const int y = blockIdx.y, ny = gridDim.y, nsb = K >> 8;                                                             \
-    gemm_d_body<NWV>(lds, xt, wt - (size_t)(n0 >> 7) * (K >> 5) * DImg<NWV>::W, C + (size_t)y * M * ldc, M, N, ldc, c_off, \
-                     accumulate, tm * 128, n0 + tn * 128, K >> 5, nsb * y / ny * 8, nsb * (y + 1) / ny * 8);            \
+    gemm_d_body<__VA_ARGS__>(lds, xt, wt - (size_t)(n0 >> 7) * (K >> 5) * I::W, C + (size_t)y * M * ldc, M, N, ldc, c_off, \
+                             accumulate, tm * 128, n0 + tn * 128, K >> 5, nsb * y / ny * 8, nsb * (y + 1) / ny * 8);    \
   }
-GEMM_D(1) GEMM_D(2) GEMM_D(3)
+GEMM_D(NW1, 1, 0) GEMM_D(NW2, 2, 0) GEMM_D(NW3, 3, 0) GEMM_D(NW1_MN1, 1, 1)

@@ -514,6 +514,59 @@ def test_gemm_on_digits_block_sums_exact(rt, monkeypatch, qtype, T, N):
     assert np.array_equal(y, want.astype(np.float32))
 
 
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K])
+@pytest.mark.parametrize("T,Mp,N,K,acc", [(130, 144, 392, 512, 0), (257, 260, 390, 768, 1), (300, 384, 1029, 256, 2), (100, 112, 136, 5120, 0)])
+def test_gemm_on_digits_with_a_minimum(rt, monkeypatch, qtype, T, Mp, N, K, acc):
+    """Q4_K and Q5_K on digits: the values around their middle in one digit, the min term with what that leaves on the bf16
+    instruction; K shared out and not, ragged last tiles, the three epilogues.  Tokens with a mean, where products and min
+    term are both large: against 64 bits the result is no further off than the int8 kernels' (measured 1.1 - 2.3e-7 of its
+    norm, theirs 1.6 - 2.9e-7)."""
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")
+    print(f"digits with a minimum {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc}", flush=True)
+    W = make_weights(qtype, N, K, seed=63)
+    x = make_acts(T, K, seed=64, outliers=True) + np.float32(0.5)
+    c0 = np.random.default_rng(65).standard_normal((Mp, N)).astype(np.float32)
+    eng = az.Engine(Mp, K)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp, acc=acc, c_init=c0 if acc else None)
+    eng.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = (aq * np.repeat(asc.astype(np.float64).T, 32, axis=1)) @ orc.dequant_rows(qtype, W, N, K).astype(np.float64).T
+    c64 = c0.astype(np.float64)
+    ref = ref + c64 if acc == 1 else ref * (c64 / (1.0 + np.exp(-c64))) if acc == 2 else ref
+    assert np.isfinite(y).all() and mixed_err(y, ref) <= TOL
+    if acc == 0:
+        assert np.linalg.norm(y - ref) <= 4e-7 * np.linalg.norm(ref) and not y[T:].any()
+
+
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K])
+def test_gemm_on_digits_with_a_minimum_exact(rt, monkeypatch, qtype):
+    """... and exact where all is whole: scale and minimum one, random sub-scales and values, a token one block of values at
+    the ends of the range; the largest products are 63 x 31 x 32 x 128 < 2^23."""
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")
+    T, N, K = 256, 640, 512
+    rng = np.random.default_rng(180 + qtype)
+    blk = rng.integers(0, 256, (N, K // 256, az.gguf_bytes(qtype, 1, 256)), dtype=np.uint8)
+    blk[..., 0:4] = np.frombuffer(np.array([1.0, 1.0], np.float16).tobytes(), np.uint8)
+    W = blk.reshape(-1)
+    wi = orc.dequant_rows(qtype, W, N, K).astype(np.float64)
+    aq = np.zeros((T, K // 32, 32), np.int8)
+    for t in range(T):
+        i = np.arange(32)
+        aq[t, t % (K // 32)] = [np.full(32, 127), np.full(32, -128), np.where(i & 1, 127, -127), rng.integers(-128, 128, 32)][(t // (K // 32)) % 4]
+    aq = aq.reshape(T, K)
+    absum = np.ascontiguousarray(aq.reshape(T, K // 16, 16).sum(axis=2, dtype=np.int64).astype(np.int16).T)
+    eng = az.Engine(T, K)
+    w = eng.make_weight(qtype, N, K, W)
+    eng.set_activations(aq, np.ones((K // 32, T), np.float32), absum, K, T, T)
+    cb = az.Runtime.alloc(T * N * 4).fill(0xFFFFFFFF)
+    eng.matmul("test", w, T, cb, N, 0, 0)
+    y = cb.read(np.float32, T * N).reshape(T, N)
+    for b in (cb, w):
+        b.free()
+    eng.close()
+    assert np.array_equal(y, (aq.astype(np.float64) @ wi.T).astype(np.float32))
+
+
 @pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512), (az.Q3_K, 300, 4224, 2560)])
 @pytest.mark.parametrize("before", [None, 256, 1024])
 def test_weights_of_another_engine(rt, qtype, T, N, K, before):
