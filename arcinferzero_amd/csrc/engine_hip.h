@@ -832,7 +832,7 @@ class Engine {
   // (nw: digits of a weight, 0: not a type of this GEMM; mn: with a minimum; bytes of the images: gemm_d.hip's DImg)
   struct DigitForm { int nw, mn, timg, wimg; };
   static DigitForm digit_form(uint32_t type) {
-    const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS ? 2
+    const int nw = type == GGML_Q6_K ? 3 : type == GGML_Q3_K || type == GGML_IQ3_XXS || type == GGML_IQ4_XS || type == GGML_IQ4_NL ? 2
                    : type == GGML_Q4_0 || type == GGML_MXFP4 || type == GGML_IQ3_S || type == GGML_Q4_K || type == GGML_Q5_K ? 1 : 0;
     const int mn = type == GGML_Q4_K || type == GGML_Q5_K ? 1 : 0;
     return {nw, mn, mn ? 7680 : nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512 + 1024 * mn};
@@ -840,7 +840,8 @@ class Engine {
   // Where it pays.  With the rows' digits kept (digits_keep) from more than 64 token rows on, against the int8 kernels: us, 128
   // / 300 / 1024 tokens, 4096 x 4096: Q4_0 23 / 24, 31 / 40, 54 / 80, Q3_K 22 / 35, 36 / 52, 63 / 109, IQ3_XXS 22 / 31, 36 / 41,
   // 62 / 76; 17408 x 5120: Q4_0 44 / 58, 87 / 139, 222 / 337, MXFP4 45 / 61, 86 / 146, 219 / 349, IQ3_S 44 / 93, 89 / 146, 223 /
-  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362, Q5_K 51 / 68, 102 / 143, 268 / 336; Q4_K,
+  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362, Q5_K 51 / 68, 102 / 143, 268 / 336,
+  // IQ4_XS 61 / 59, 118 / 142, 298 / 346 (4096 x 4096 22 / 25, 36 / 41, 62 / 85); Q4_K,
   // Q6_K (three digits) and IQ3_XXS where it is priced cheaper: Q4_K 17408 x 5120 50 / 61, 101 / 110, 262 / 295, but 12288 x
   // 4096, 300 tokens, 82 / 69; Q6_K 17408 x 5120 75 / 90, 154 / 179, 391 / 518, but 2048 x 5120 28 / 22, 33 / 35, 59 / 70.
   // Without, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us

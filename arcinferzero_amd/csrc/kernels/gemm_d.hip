@@ -1,4 +1,5 @@
-// "gemm" module, second file: the prefill GEMM on digits (Q4_K, Q5_K, Q4_0, MXFP4, IQ3_S, IQ3_XXS, Q3_K, Q6_K).
+// "gemm" module, second file: the prefill GEMM on digits, every weight type but Q8_0 (whose int8 kernels
+// decode nothing: 4096 x 4096, 300 and 2048 tokens, 28 and 105 us, in two digits 36 and 108).
 //
 //   C[m][c_off + n] (=, +=, silu(C) *)  sum over 32-blocks b of  (sa[m][b] * ws[n][b]) * J[m][n][b]
 //   J[m][n][b] = sum over the block's 32 k of x[m][k] * w[n][k], integers
@@ -15,7 +16,8 @@
 // (v_mfma_f32_32x32x1_2b_f32: both row tiles at once).
 //
 // Q6_K and Q3_K, whose sub-scales hold for 16 values, have them folded into w ((q - 32) * sc, three digits; (q - 4) * sc, at
-// most 128, two), ws is d; the others' ws is their block scale: Q4_0, MXFP4 and IQ3_S are one digit, IQ3_XXS two.
+// most 128, two), ws is d; the others' ws is their block scale: Q4_0, MXFP4, IQ3_S, Q4_K and
+// Q5_K are one digit, IQ3_XXS, IQ4_XS and IQ4_NL two.
 //
 // Bound by power: at 17408 x 5120 x 8192 the chip runs this kernel below 1.9 GHz, without its DMA at 2.1, and every part
 // that is taken out -- operand reads from LDS, DMA, multiply-adds -- gives back about its share of the energy, not of the
@@ -124,6 +126,8 @@ template <int QT> struct DType { enum { NW = 1, MN = 0 }; };
 template <> struct DType<QT_Q6_K> { enum { NW = 3, MN = 0 }; };
 template <> struct DType<QT_Q3_K> { enum { NW = 2, MN = 0 }; };
 template <> struct DType<QT_IQ3_XXS> { enum { NW = 2, MN = 0 }; };
+template <> struct DType<QT_IQ4_XS> { enum { NW = 2, MN = 0 }; };
+template <> struct DType<QT_IQ4_NL> { enum { NW = 2, MN = 0 }; };
 template <> struct DType<QT_Q4_K> { enum { NW = 1, MN = 1 }; };
 template <> struct DType<QT_Q5_K> { enum { NW = 1, MN = 1 }; };
 
@@ -233,7 +237,18 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
       q3k_scales(h[0], h[1], h[2], b[i], sc0, sc1);
       codes_scaled<2>(v, sc0, sc1, c[i]);
     }
-  } else if constexpr (QT == QT_Q4_0 || QT == QT_MXFP4) {
+  } else if constexpr (QT == QT_IQ4_XS) {
+    const u2v h = *(const u2v*)(raw + planes_iq4xs((size_t)N, nsb).hdr + u * 8);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const u4v w = *(const u4v*)(raw + u * 128 + 16 * b[i]);
+      uint32_t v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = iq4_lookup(k < 4 ? w[k] : w[k - 4] >> 4);
+      codes_i8<2>(v, c[i]);
+      ws[i] = f16_bits_to_f32(h[0]) * (float)((int)(((h[1] >> (4 * b[i])) & 15u) | ((h[0] >> (16 + 2 * b[i])) & 3u) << 4) - 32);
+    }
+  } else if constexpr (QT == QT_Q4_0 || QT == QT_MXFP4 || QT == QT_IQ4_NL) {
     // block b: 16 bytes, low nibbles values 0..15, high nibbles 16..31
     const uint32_t h = QT == QT_MXFP4 ? *(const unsigned short*)(raw + planes_mxfp4((size_t)N, nsb).e + u * 8 + 2 * q)
                                       : *(const uint32_t*)(raw + planes_q40((size_t)N, nsb).d + u * 16 + 4 * q);
@@ -244,7 +259,7 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const uint32_t x = k < 4 ? w[k] : w[k - 4] >> 4;
-        v[k] = QT == QT_MXFP4 ? mxfp4_lookup(x) : nib_vals<QT>(x);
+        v[k] = nib_vals<QT>(x);
       }
       codes_i8<NW>(v, c[i]);
       ws[i] = QT == QT_MXFP4 ? e8m0_half(h >> (8 * i)) : f16_bits_to_f32(i ? h >> 16 : h);
@@ -306,7 +321,7 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
                                                                           int nsb, int n0, uint8_t* wt) {               \
     row_digits<QT>(raw, tabs, N, nsb, n0, wt);                                                                          \
   }
-ROW_DIGITS(12) ROW_DIGITS(13) ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
+ROW_DIGITS(12) ROW_DIGITS(13) ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(20) ROW_DIGITS(23) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
 
 // ---- gemm_d: 128 tokens x 128 rows in four waves of 64 x 64, two work-groups a compute unit.  Blocks [b0, b1), an even number.
 // (Eight waves of 32 x 64, four a SIMD, hide more waits and read each row digit from LDS twice as often: 5 - 6 % slower, at

@@ -387,7 +387,7 @@ def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
 
 
 @pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 128, 4096, 2048), (az.Q3_K, 200, 4099, 2304), (az.Q6_K, 256, 4100, 4096), (az.IQ3_XXS, 200, 12300, 2048),
-                                         (az.MXFP4, 65, 4225, 2048)])
+                                         (az.MXFP4, 65, 4225, 2048), (az.IQ4_XS, 90, 4200, 2048), (az.IQ4_NL, 300, 4097, 2304)])
 def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     """Matrices of 2^23 values and more keep their rows' digits: no matmul writes them, and shorter chunks are multiplied on
     digits.  Given back where an allocation finds no memory -- not while a recorded list names them --, the weight is
