@@ -134,6 +134,16 @@ _sig("arcz_gen_normal", None, _u64, _z, C.c_float, C.c_float, _p)
 _sig("arcz_gen_weights", _i, _u32, _u64, _z, _i, C.c_float, _p)
 
 
+# The calls of a forward pass: through the extension next to the library (csrc/pycall.c: the same functions, converted
+# faster), or through ctypes where it was not built for this interpreter.
+try:
+    from ._pycall import gemv_gu as _gemv_gu, layer_moe as _layer_moe, matmul as _matmul, quantize as _quantize
+    from ._pycall import rmsnorm_quant as _rmsnorm_quant, swiglu_quant as _swiglu_quant
+except ImportError:
+    _quantize, _rmsnorm_quant, _swiglu_quant = lib.arcz_engine_quantize, lib.arcz_engine_rmsnorm_quant, lib.arcz_engine_swiglu_quant
+    _matmul, _gemv_gu, _layer_moe = lib.arcz_engine_matmul, lib.arcz_engine_gemv_gu, lib.arcz_engine_layer_moe
+
+
 def _check(code, engine=False):
     if code != 0:
         msg = (lib.arcz_engine_error() if engine and code == -100 else lib.arcz_last_error()) or b""
@@ -485,18 +495,23 @@ class Engine:
         return MoeLayer(self, h, t["dims"][2], NU, Ep.value, Fp.value)
 
     def quantize(self, x, ldx, K, Mp, T, act32=1):
-        _check(lib.arcz_engine_quantize(self.h, x.h, ldx, K, Mp, T, act32), engine=True)
+        r = _quantize(self.h, x.h, ldx, K, Mp, T, act32)
+        if r:
+            _check(r, engine=True)
 
     def add_norm_quant(self, x, t, w, K, T, Mp, s, w2, norm2, eps, act32=1):
         _check(lib.arcz_engine_add_norm_quant(self.h, x.h, t.h, w.h, K, T, Mp, s, w2.h if w2 else None, 1 if norm2 else 0,
                                               act32, eps), "add_norm_quant")
 
     def rmsnorm_quant(self, x, row_off, w, K, Mp, T, eps, hout=None, act32=1):
-        _check(lib.arcz_engine_rmsnorm_quant(self.h, x.h, row_off, w.h, K, Mp, T, act32, eps, hout.h if hout else None),
-               engine=True)
+        r = _rmsnorm_quant(self.h, x.h, row_off, w.h, K, Mp, T, act32, eps, hout.h if hout else None)
+        if r:
+            _check(r, engine=True)
 
     def swiglu_quant(self, gu, F, Mp, T, fused=0, gelu=0, act32=1):
-        _check(lib.arcz_engine_swiglu_quant(self.h, gu.h, F, Mp, T, act32, fused, gelu), engine=True)
+        r = _swiglu_quant(self.h, gu.h, F, Mp, T, act32, fused, gelu)
+        if r:
+            _check(r, engine=True)
 
     def set_activations(self, aq, asc, absum, K, Mp, T):
         aq = np.ascontiguousarray(aq, dtype=np.int8)
@@ -532,11 +547,13 @@ class Engine:
                 self.absum.read(np.int16, Mp * K // 16).reshape(K // 16, Mp))
 
     def matmul(self, name, w, Mp, Cbuf, ldc, c_off=0, acc=0, act32=True):
-        _check(lib.arcz_engine_matmul(self.h, name.encode(), w.h, Mp, Cbuf.h, ldc, c_off, acc, 1 if act32 else 0), engine=True)
+        r = _matmul(self.h, name.encode(), w.h, Mp, Cbuf.h, ldc, c_off, acc, 1 if act32 else 0)
+        if r:
+            _check(r, engine=True)
 
     def gemv_gu(self, g, u, Mp, Cbuf):
         """Gate and up of one token in one launch: True if taken, False if the caller must run the two matmuls."""
-        r = lib.arcz_engine_gemv_gu(self.h, g.h, u.h, Mp, Cbuf.h)
+        r = _gemv_gu(self.h, g.h, u.h, Mp, Cbuf.h)
         if r < 0:
             _check(r, engine=True)
         return r == 1
@@ -558,7 +575,9 @@ class Engine:
 
     def layer_moe(self, L, logits, ldl, x, T, Mp, sh=None):
         if sh is None:
-            _check(lib.arcz_engine_layer_moe(self.h, L.h, logits.h, ldl, x.h, T, Mp), engine=True)
+            r = _layer_moe(self.h, L.h, logits.h, ldl, x.h, T, Mp)
+            if r:
+                _check(r, engine=True)
         else:
             _check(lib.arcz_engine_layer_moe_sh(self.h, L.h, logits.h, ldl, x.h, T, Mp, sh.h), engine=True)
 

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <map>
 #include <set>
+#include <unordered_set>
 #include <string>
 #include <vector>
 
@@ -49,7 +50,7 @@ struct Runtime {
   hipStream_t stream = nullptr;
   hipDeviceProp_t prop;
   std::string name;
-  std::set<arcz_mem*> mems;
+  std::unordered_set<arcz_mem*> mems;  // (looked up for every buffer argument of a launch)
   size_t device_bytes = 0, spare_bytes = 0;
   std::map<std::string, std::vector<hipModule_t>> modules;  // a module may be several code objects
   std::map<std::string, arcz_kernel*> kernels;

@@ -150,7 +150,10 @@ class Engine {
   // three buffers, and every matmul runs a second time over that half, accumulating (matmul below).
   bool q2mm_ = false;
   size_t q2_aq_ = 0, q2_sc_ = 0, q2_ab_ = 0;  // bytes
-  std::string q2_defs_;
+  cl_kernel producer(const char* name) {
+    return q2mm_ ? variant("ops", {{"Q2_AQ", (long)q2_aq_}, {"Q2_SC", (long)(q2_sc_ / 4)}, {"Q2_AB", (long)(q2_ab_ / 2)}}, name)
+                 : variant("ops", {}, name);
+  }
   cl_mem aq2_ = nullptr, asc2_ = nullptr, absum2_ = nullptr;  // views of the second halves
   void set_two_pass(bool on) {
     if (on == q2mm_) return;
@@ -164,15 +167,12 @@ class Engine {
     q2mm_ = on;
     cur_T_ = cur_K_ = cur_Mp_ = cur_rows_ = 0;
     alloc_activations();
-    q2_defs_.clear();
     q2_aq_ = q2_sc_ = q2_ab_ = 0;
     if (!on) return;
     const size_t M = (size_t)max_chunk;
     q2_aq_ = M * max_k;
     q2_sc_ = M * (max_k / 32) * 4;
     q2_ab_ = M * (max_k / 16) * 2;
-    q2_defs_ = " -DQ2_AQ=" + std::to_string(q2_aq_) + " -DQ2_SC=" + std::to_string(q2_sc_ / 4) + " -DQ2_AB=" +
-               std::to_string(q2_ab_ / 2);
     aq2_ = view(aq_, q2_aq_, q2_aq_);
     asc2_ = view(asc_, q2_sc_, q2_sc_);
     absum2_ = view(absum_, q2_ab_, q2_ab_);
@@ -243,6 +243,44 @@ class Engine {
     cl_kernel k = cl_.kernel(p, name.c_str());
     kernels_[key] = k;
     return k;
+  }
+  // The same by the -D names and values as they are, for launches that a pass makes for each layer: no string is put together
+  // or compared, which took as long as submitting the launch (quantize + matmul of one token, 2048 x 2048, from C, one after the other: 5.5 - 6.5 us, now
+  // 5.05, of which the runtime's own submissions are 4.5).  A name of nullptr: left out.
+  struct Def { const char* name; long value; };
+  cl_kernel variant(const char* which, std::initializer_list<Def> defs, const char* name) {
+    struct Mix {
+      uint64_t h = 0xcbf29ce484222325ull;
+      void operator()(uint64_t v) { h = (h ^ v) * 0x9E3779B97F4A7C15ull; h ^= h >> 29; }
+    } mix;
+    Variant v;
+    v.which = which;
+    v.name = name;
+    mix((uintptr_t)which);
+    mix((uintptr_t)name);
+    for (const Def& d : defs) {
+      if (!d.name) continue;
+      if (v.n == MAX_DEFS) throw std::logic_error("variant: too many definitions");
+      v.defs[v.n++] = d;
+      mix((uintptr_t)d.name);
+      mix((uint64_t)d.value);
+    }
+    v.hash = mix.h;
+    if (variants_.empty()) variants_.resize(256);
+    size_t i = v.hash & (variants_.size() - 1);
+    for (; variants_[i].k; i = (i + 1) & (variants_.size() - 1))
+      if (variants_[i].same(v)) return variants_[i].k;
+    std::string opts;
+    for (int j = 0; j < v.n; ++j) opts += std::string(j ? " -D" : "-D") + v.defs[j].name + "=" + std::to_string(v.defs[j].value);
+    v.k = kernel(which, opts, name);
+    if (++variants_used_ * 2 > variants_.size()) {
+      std::vector<Variant> old(variants_.size() * 2);
+      old.swap(variants_);
+      for (const Variant& o : old)
+        if (o.k) put_variant(o);
+    }
+    put_variant(v);
+    return v.k;
   }
   // (zero/engine.h:936-950)
   void run(const char* name, cl_kernel k, int dims, const size_t* gws, const size_t* lws) {
@@ -368,7 +406,7 @@ class Engine {
     check_chunk(K, Mp, T);
     if (!act32 && q2mm_) throw std::runtime_error("quantize_rows: two-pass inputs take per-32 activation scales (act32)");
     if (ldx < K || arcz_mem_size(x) < ((size_t)(T - 1) * ldx + K) * 4) throw std::runtime_error("quantize_rows: x is too small");
-    cl_kernel k = kernel("ops", q2_defs_, "quant_rows");
+    cl_kernel k = producer("quant_rows");
     int rows = tile_rows(K, Mp);
     set_args(k, 0, x, ldx, K, Mp, T, aq_, asc_, absum_, act32, rows);
     size_t gws[2] = {(size_t)256 * (K / 256), (size_t)((Mp + rows - 1) / rows)}, lws[2] = {256, 1};
@@ -391,7 +429,7 @@ class Engine {
     // A wave a row for chunks of more rows than compute units; a work-group a row below that (its 256 threads are through
     // the row sooner: 128 x 5120 6.7 against 8.7 us), for longer rows than the wave form stages and on two-pass engines.
     const bool wave = !q2mm_ && Mp > 256 && Mp % 4 == 0 && K <= 16384 && !wide_rows(T);
-    cl_kernel k = wave ? kernel("ops", "", "rmsnorm_quant_wave") : kernel("ops", q2_defs_, "rmsnorm_quant");
+    cl_kernel k = wave ? variant("ops", {}, "rmsnorm_quant_wave") : producer("rmsnorm_quant");
     int wh = hout ? 1 : 0;
     set_args(k, 0, x, row_off, w, K, Mp, T, eps, aq_, asc_, absum_, hout, wh, act32);
     size_t gws[2] = {256, (size_t)(wave ? Mp / 4 : Mp)}, lws[2] = {256, 1};
@@ -413,7 +451,7 @@ class Engine {
     if (arcz_mem_size(gu) < (size_t)T * F * (fused ? 1 : 2) * 4) throw std::runtime_error("swiglu_quant: gu is too small");
     // (a pass of 1-8 tokens: the valid rows only, their superblocks over several work-groups; a chunk: quant_rows' tiles)
     const bool wide = wide_rows(T);
-    cl_kernel k = kernel("ops", q2_defs_, wide ? "swiglu_quant" : "swiglu_quant_tile");
+    cl_kernel k = wide ? producer("swiglu_quant") : producer("swiglu_quant_tile");
     set_args(k, 0, gu, F, Mp, T, aq_, asc_, absum_, act32, fused, gelu);
     size_t gws[2] = {256 * (size_t)((F / 256 + 3) / 4), (size_t)T}, lws[2] = {256, 1};
     if (!wide) {
@@ -435,7 +473,7 @@ class Engine {
     if (arcz_mem_size(x) < (size_t)T * K * 4 || arcz_mem_size(t) < (size_t)T * K * 4 || arcz_mem_size(w) < (size_t)K * 4 ||
         (norm2 && (!w2 || arcz_mem_size(w2) < (size_t)K * 4)))
       throw std::runtime_error("add_norm_quant: a buffer is too small for " + std::to_string(T) + " rows of " + std::to_string(K));
-    cl_kernel k = kernel("ops", q2_defs_, "add_norm_quant");
+    cl_kernel k = producer("add_norm_quant");
     int nrm = norm2 ? 1 : 0, MM = Mp, TT = T, KK = K;
     set_args(k, 0, x, t, w, KK, eps, s, w2, nrm, MM, aq_, asc_, absum_, act32, TT);
     // (a pass of 1-8 tokens: the valid rows only, as the reference; a longer chunk: all Mp rows, the padding as zeros)
@@ -631,7 +669,7 @@ class Engine {
       rd_bytes += raw_bytes(w);
       // (the form for at most eight tokens; the three-bit types have the one form)
       const bool t8 = T <= 8 && w.type != GGML_IQ3_S && w.type != GGML_Q3_K && w.type != GGML_IQ3_XXS;
-      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(w.type) + (t8 ? " -DT8=1" : ""), "gemv_mm");
+      cl_kernel k = variant("decode", {{"QT", w.type}, {t8 ? "T8" : nullptr, 1}}, "gemv_mm");
       const size_t groups = (size_t)(N + 15) / 16, cus = (size_t)arcz_device_cus();
       // Rows longer than the tokens' LDS holds (slices of sb_max superblocks): K is shared out over `ny` work-groups
       // per run of groups, each staging its piece of the tokens once, and gemv_mm_reduce adds the pieces -- inside one
@@ -652,7 +690,7 @@ class Engine {
         set_args(k, 0, w.raw, N, K, tabs, aq_, asc_, absum_, M, T, ws, ldw, zero, zero, zero, s1);
         size_t g2[2] = {std::min<size_t>(groups, std::max<size_t>(cus / (size_t)ny, 1)) * 512, (size_t)ny}, l2[2] = {512, 1};
         run(name, k, 2, g2, l2);
-        cl_kernel kr = kernel("decode", "", "gemv_mm_reduce");
+        cl_kernel kr = variant("decode", {}, "gemv_mm_reduce");
         int rows = T > 8 ? 16 : T, nyy = ny;
         set_args(kr, 0, ws, nyy, C, rows, N, ldc, c_off, a);
         size_t g3 = ((size_t)rows * N + 255) / 256 * 256, l3 = 256;
@@ -734,13 +772,15 @@ class Engine {
         const int wpc = wpc_env > 0 ? wpc_env : bt == 512 || (tb == 1 && !codebook && !q6_mid) ? 1 : 2;
         size_t wgs = std::min<size_t>((size_t)(N + g - 1) / g, (size_t)arcz_device_cus() * wpc);
         if (wgs_env > 0) wgs = std::min<size_t>((size_t)(N + g - 1) / g, (size_t)wgs_env);
-        const std::string defs = "-DQT=" + std::to_string(w.type) + " -DLPR=" + std::to_string(lpr) + " -DPF=" +
-                                 std::to_string(pf) + (tb > 1 ? " -DTB=" + std::to_string(tb) : std::string()) +
-                                 (bt == 512 ? " -DBT=512" : "") + " -DLDS=" +
-                                 std::to_string(lds) +
-                                 (q2f ? " -DQ2_AQ=" + std::to_string(q2_aq_) + " -DQ2_SC=" + std::to_string(q2_sc_ / 4) : std::string()) +
-                                 head_defs(w) + " -DSCHED=" + std::to_string(gemv_sched(N, g, wgs, false, raw_bytes(w), lpr >= 128 && tb == 1 && bt == 256, !codebook && tb <= 2));
-        cl_kernel k = kernel("decode", defs, tb == 1 ? "gemv" : "gemv_mt");
+        const int sched = gemv_sched(N, g, wgs, false, raw_bytes(w), lpr >= 128 && tb == 1 && bt == 256, !codebook && tb <= 2);
+        const std::string cap = head_defs(w);
+        cl_kernel k = cap.empty() ? variant("decode", {{"QT", w.type}, {"LPR", lpr}, {"PF", pf}, {tb > 1 ? "TB" : nullptr, tb}, {bt == 512 ? "BT" : nullptr, 512},
+                                                       {"LDS", (long)lds}, {q2f ? "Q2_AQ" : nullptr, (long)q2_aq_}, {q2f ? "Q2_SC" : nullptr, (long)(q2_sc_ / 4)},
+                                                       {"SCHED", sched}}, tb == 1 ? "gemv" : "gemv_mt")
+                                  : kernel("decode", "-DQT=" + std::to_string(w.type) + " -DLPR=" + std::to_string(lpr) + " -DPF=" + std::to_string(pf) +
+                                                         (tb > 1 ? " -DTB=" + std::to_string(tb) : std::string()) + (bt == 512 ? " -DBT=512" : "") + " -DLDS=" + std::to_string(lds) +
+                                                         (q2f ? " -DQ2_AQ=" + std::to_string(q2_aq_) + " -DQ2_SC=" + std::to_string(q2_sc_ / 4) : std::string()) +
+                                                         cap + " -DSCHED=" + std::to_string(sched), tb == 1 ? "gemv" : "gemv_mt");
         int ld1 = T == 1 ? 0 : ldc;  // (one token: C is the row itself)
         if (tb == 1) set_args(k, 0, w.raw, N, K, tabs, aq_, asc_, absum_, M, C, c_off, a);
         else set_args(k, 0, w.raw, N, K, tabs, aq_, asc_, absum_, M, T, C, ld1, c_off, a);
@@ -790,10 +830,8 @@ class Engine {
     const int pf = (units + lpr - 1) / lpr;
     static const int gu_wpc = getenv("ARCZ_GEMV_GU_WPC") ? atoi(getenv("ARCZ_GEMV_GU_WPC")) : 1;  // (17.6 against 18.2 us with two)
     const size_t wgs = std::min<size_t>((size_t)2 * N / gr, (size_t)arcz_device_cus() * gu_wpc);
-    const std::string defs = "-DQT=" + std::to_string(g.type) + " -DLPR=" + std::to_string(lpr) + " -DPF=" + std::to_string(pf) +
-                             " -DLDS=" + std::to_string(lds) + " -DGU2 -DSCHED=" +
-                             std::to_string(gemv_sched(2 * N, gr, wgs, true, raw_bytes(g) + raw_bytes(u), lpr >= 128));
-    cl_kernel k = kernel("decode", defs, "gemv");
+    cl_kernel k = variant("decode", {{"QT", g.type}, {"LPR", lpr}, {"PF", pf}, {"LDS", (long)lds}, {"GU2", 1},
+                                     {"SCHED", gemv_sched(2 * N, gr, wgs, true, raw_bytes(g) + raw_bytes(u), lpr >= 128)}}, "gemv");
     cl_mem tabs = tabs_;
     int NN = N, KK = K, M = Mp, c_off = 0, a = 0;
     set_args(k, 0, g.raw, NN, KK, tabs, aq_, asc_, absum_, M, C, c_off, a, u.raw);
@@ -912,7 +950,7 @@ class Engine {
   }
   // rows [n0, n0 + 128 nt) of w as digits, into out
   void row_digits(const char* name, const GpuWeight& w, int n0, int nt, cl_mem out) {
-    cl_kernel k = kernel("gemm", "-DQTYPE=" + std::to_string(w.type), "row_digits");
+    cl_kernel k = variant("gemm", {{"QTYPE", w.type}}, "row_digits");
     int N = w.N, nsb = w.K / 256;
     set_args(k, 0, w.raw, tabs_, N, nsb, n0, out);
     size_t g[2] = {(size_t)nsb * 256, (size_t)nt * 2}, l[2] = {256, 1};
@@ -928,7 +966,7 @@ class Engine {
     if (!xd_ || panel < 1) throw std::logic_error("gemm_digits: no room for a tile of rows");
     size_t l[2] = {256, 1};
     {
-      cl_kernel k = kernel("gemm", "", "act_digits");
+      cl_kernel k = variant("gemm", {}, "act_digits");
       int img = f.timg;
       set_args(k, 0, aq_, asc_, absum_, M, K, img, xd_);
       size_t g[2] = {(size_t)nsb * 256, (size_t)mt * 2};
@@ -937,7 +975,7 @@ class Engine {
     for (int t0 = 0; t0 < nt_all; t0 += panel) {
       int nt = std::min(panel, nt_all - t0), n0 = t0 * 128;
       if (!kept) row_digits("row_digits", w, n0, nt, wd_);
-      cl_kernel k = kernel("gemm", "-DNW=" + std::to_string(f.nw) + (f.mn ? " -DMN=1" : ""), "gemm_d");
+      cl_kernel k = variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
       // (ARCZ_Q4_SPLITK=0: K in one piece, =n: n pieces, as many as SPLIT_BYTES holds)
       int ny = nt < nt_all || sk_force_ == 0 ? 1
@@ -952,7 +990,7 @@ class Engine {
   }
   // rows: those that the partial tiles hold, 0: all M
   void splitk_reduce(const char* name, cl_mem ws, int ny, cl_mem C, int M, int N, int ldc, int c_off, int a, int rows = 0) {
-    cl_kernel r = kernel("gemm", "", "splitk_reduce");
+    cl_kernel r = variant("gemm", {}, "splitk_reduce");
     const bool whole = ((N | ldc | c_off) & 3) == 0 && ((uintptr_t)arcz_mem_ptr(C) & 15) == 0;
     int wide = whole ? 1 : 0;
     set_args(r, 0, ws, ny, C, M, N, ldc, c_off, a, wide, rows);
@@ -1089,8 +1127,7 @@ class Engine {
           sk_ws_bytes_ = need;
           ws = sk_ws_;
         }
-        cl_kernel k = kernel("gemm", std::string("-DQTYPE=") + std::to_string(w.type) + " -DACT32 -DBM=" + std::to_string(bm) +
-                                         " -DBN=128 -DSPLITK" + (w.half_d ? " -DHDS=" + std::to_string(w.half_d) : std::string()), "gemm");
+        cl_kernel k = variant("gemm", {{"QTYPE", w.type}, {"ACT32", 1}, {"BM", bm}, {"BN", 128}, {"SPLITK", 1}, {w.half_d ? "HDS" : nullptr, w.half_d}}, "gemm");
         cl_mem unused = nullptr;
         int zero = 0, one = 1, ldw = N, s1 = nsb;
         set_args(k, 0, w.raw, unused, aq_, asc_, absum_, ws, M, N, K, ldw, zero, zero, one, zero, s1);
@@ -1486,9 +1523,8 @@ class Engine {
     route_tiles(L, rl, ldl, T, 16);
     const size_t tiles_max = (size_t)(n + 15) / 16 + std::min(n, NE);
     cl_mem tabs = tabs_;
-    const std::string ne = " -DNE=" + std::to_string(NE);
     {
-      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[0].type) + ne + " -DLDS=" + std::to_string(lg), "moe_gateup_mm");
+      cl_kernel k = variant("decode", {{"QT", L.ex[0].type}, {"NE", NE}, {"LDS", (long)lg}}, "moe_gateup_mm");
       int FF = F, KK = E, MM = Mp, S = slots_;
       set_args(k, 0, L.ex[0].raw, L.ex[1].raw, FF, KK, tabs, aq_, asc_, MM, mtiles_, stok_, mh_, absum_, S, mhq_, mhsc_, mhbs_);
       size_t gws[2] = {(size_t)(F / 128) * 512, tiles_max}, lws[2] = {512, 1};
@@ -1496,7 +1532,7 @@ class Engine {
     }
     {
       const int gpw = moe_down_groups(E);
-      cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[2].type) + ne + " -DLDS=" + std::to_string(ld), "moe_down_mm");
+      cl_kernel k = variant("decode", {{"QT", L.ex[2].type}, {"NE", NE}, {"LDS", (long)ld}}, "moe_down_mm");
       int NN = E, KK = F, S = slots_;
       set_args(k, 0, L.ex[2].raw, NN, KK, tabs, mhq_, mhsc_, S, mtiles_, swt_, my_, mhbs_, gpw);
       size_t gws[2] = {(size_t)(E / (128 * gpw)) * 512, tiles_max}, lws[2] = {512, 1};
@@ -1507,7 +1543,7 @@ class Engine {
   }
   // x[t] += the token's weighted expert rows in my_, and the shared expert's
   void moe_sum(const MoeLayer& L, cl_mem x, cl_mem sh, int T) {
-    cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(L.NU), "moe_combine");
+    cl_kernel k = variant("moe", {{"NE", L.NE}, {"NU", L.NU}}, "moe_combine");
     int EE = L.E;
     set_args(k, 0, x, sh, sgate_, my_, minv_, EE);
     size_t gws[2] = {((size_t)L.E + 1023) / 1024 * 256, (size_t)T}, lws[2] = {256, 1};  // (four columns a thread)
@@ -1520,8 +1556,7 @@ class Engine {
       return;
     }
     if (ldl < L.NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + L.NE) * 4) throw std::runtime_error("layer_moe: router logits do not fit");
-    cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(L.NU) + " -DTM=" + std::to_string(tm),
-                         "moe_route_small");
+    cl_kernel k = variant("moe", {{"NE", L.NE}, {"NU", L.NU}, {"TM", tm}}, "moe_route_small");
     int NR = ldl, TT = T;
     set_args(k, 0, rl, NR, TT, mids_, mwts_, sgate_, mtiles_, stok_, swt_, minv_);
     size_t g1 = 1024, l1 = 1024;
@@ -1580,23 +1615,20 @@ class Engine {
         tiles_max = (size_t)(n + tmd - 1) / tmd + std::min(n, NE);
       }
       cl_mem tabs = tabs_;
-      const std::string dd = " -DGROWS=2 -DTM=" + std::to_string(tmd) + " -DNE=" + std::to_string(NE);
       if (L.ex[0].type != L.ex[1].type) throw std::runtime_error("layer_moe: gate and up experts of different types");
       // Tiles of one or two slots: the gate/up kernel quantizes its own output (32 rows a work-group: one block per
       // slot); one-slot tiles: the down kernel sums a token's experts into x itself.  3 launches instead of 5
       // (ARCZ_MOE_FUSE=0: the 5).
       const bool fq = !fuse_off && tmd <= 2 && F % 32 == 0, fc = !fuse_off && tmd == 1 && NU <= 64 && !sh;
       if (froute) {
-        cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[0].type) + " -DGROWS=4 -DTM=1 -DQUANT=1 -DROUTE=1 -DNE=" +
-                                           std::to_string(NE), "moe_gateup_q");
+        cl_kernel k = variant("decode", {{"QT", L.ex[0].type}, {"GROWS", 4}, {"TM", 1}, {"QUANT", 1}, {"ROUTE", 1}, {"NE", NE}}, "moe_gateup_q");
         int FF = F, KK = E, MM = Mp, S = slots_, NUU = NU, NR = ldl, TT = T;
         set_args(k, 0, L.ex[0].raw, L.ex[1].raw, FF, KK, tabs, aq_, asc_, MM, mtiles_, stok_, mh_, absum_, S, mhq_, mhsc_,
                  mhbs_, rl, sgate_, swt_, minv_, NUU, NR, TT, mids_, mwts_);
         size_t gws[2] = {(size_t)(F / 32) * 512, tiles_max}, lws[2] = {512, 1};
         run("moe_gateup", k, 2, gws, lws);
       } else if (fq) {
-        cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[0].type) + " -DGROWS=4 -DTM=" + std::to_string(tmd) +
-                                           " -DQUANT=1 -DNE=" + std::to_string(NE), "moe_gateup_q");
+        cl_kernel k = variant("decode", {{"QT", L.ex[0].type}, {"GROWS", 4}, {"TM", tmd}, {"QUANT", 1}, {"NE", NE}}, "moe_gateup_q");
         int FF = F, KK = E, MM = Mp, S = slots_;
         set_args(k, 0, L.ex[0].raw, L.ex[1].raw, FF, KK, tabs, aq_, asc_, MM, mtiles_, stok_, mh_, absum_, S, mhq_, mhsc_,
                  mhbs_);
@@ -1604,14 +1636,14 @@ class Engine {
         run("moe_gateup", k, 2, gws, lws);
       } else {
         {
-          cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[0].type) + dd, "moe_gateup_q");
+          cl_kernel k = variant("decode", {{"QT", L.ex[0].type}, {"GROWS", 2}, {"TM", tmd}, {"NE", NE}}, "moe_gateup_q");
           int FF = F, KK = E, MM = Mp;
           set_args(k, 0, L.ex[0].raw, L.ex[1].raw, FF, KK, tabs, aq_, asc_, MM, mtiles_, stok_, mh_, absum_);
           size_t gws[2] = {((size_t)(F + 1) / 2 * 32 + 255) / 256 * 256, tiles_max}, lws[2] = {256, 1};
           run("moe_gateup", k, 2, gws, lws);
         }
         {
-          cl_kernel k = kernel("moe", "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU), "moe_quant_sums");
+          cl_kernel k = variant("moe", {{"NE", NE}, {"NU", NU}}, "moe_quant_sums");
           int FF = F, S = slots_;
           set_args(k, 0, mh_, FF, S, mhq_, mhsc_, mhbs_);
           size_t gws[2] = {(size_t)256 * (F / 256), (size_t)(n + 63) / 64}, lws[2] = {256, 1};
@@ -1619,8 +1651,7 @@ class Engine {
         }
       }
       if (fc) {
-        cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[2].type) + " -DGROWS=4 -DNE=" + std::to_string(NE),
-                             "moe_down1_q");
+        cl_kernel k = variant("decode", {{"QT", L.ex[2].type}, {"GROWS", 4}, {"NE", NE}}, "moe_down1_q");
         int NN = E, KK = F, S = slots_;
         int NUU = NU;
         set_args(k, 0, L.ex[2].raw, NN, KK, tabs, mhq_, mhsc_, S, mtiles_, swt_, x, mhbs_, minv_, NUU);
@@ -1628,7 +1659,7 @@ class Engine {
         run("moe_down", k, 2, gws, lws);
       } else {
         {
-          cl_kernel k = kernel("decode", "-DQT=" + std::to_string(L.ex[2].type) + dd, "moe_down_q");
+          cl_kernel k = variant("decode", {{"QT", L.ex[2].type}, {"GROWS", 2}, {"TM", tmd}, {"NE", NE}}, "moe_down_q");
           int NN = E, KK = F, S = slots_;
           set_args(k, 0, L.ex[2].raw, NN, KK, tabs, mhq_, mhsc_, S, mtiles_, swt_, my_, mhbs_);
           size_t gws[2] = {((size_t)(E + 1) / 2 * 32 + 255) / 256 * 256, tiles_max}, lws[2] = {256, 1};
@@ -1684,7 +1715,7 @@ class Engine {
     }
     if (!quant_fused) {
       // (the reference's moe_quant writes no sums; the Q4_K tile GEMM here takes them for its min term)
-      cl_kernel k = kernel("moe", "-DNE=" + std::to_string(L.NE) + " -DNU=" + std::to_string(NU), "moe_quant_sums");
+      cl_kernel k = variant("moe", {{"NE", L.NE}, {"NU", NU}}, "moe_quant_sums");
       int FF = F, S = slots_;
       set_args(k, 0, mh_, FF, S, mhq_, mhsc_, mhbs_);
       size_t gws[2] = {(size_t)256 * (F / 256), (size_t)(n + 63) / 64}, lws[2] = {256, 1};
@@ -1702,6 +1733,28 @@ class Engine {
                                std::to_string(max_k) + ")");
   }
   std::map<std::string, cl_kernel> kernels_;
+  // variant()'s lookups, open addressing: a name is told apart by where its text lies, so one kernel may have several entries
+  static constexpr int MAX_DEFS = 9;
+  struct Variant {
+    cl_kernel k = nullptr;
+    uint64_t hash = 0;
+    const char *which = nullptr, *name = nullptr;
+    int n = 0;
+    Def defs[MAX_DEFS] = {};
+    bool same(const Variant& o) const {
+      if (hash != o.hash || which != o.which || name != o.name || n != o.n) return false;
+      for (int i = 0; i < n; ++i)
+        if (defs[i].name != o.defs[i].name || defs[i].value != o.defs[i].value) return false;
+      return true;
+    }
+  };
+  std::vector<Variant> variants_;
+  size_t variants_used_ = 0;
+  void put_variant(const Variant& v) {
+    size_t i = v.hash & (variants_.size() - 1);
+    while (variants_[i].k) i = (i + 1) & (variants_.size() - 1);
+    variants_[i] = v;
+  }
   std::vector<cl_program> progs_;
   std::vector<cl_mem> mems_;
   std::vector<std::pair<std::string, cl_event>> events_;

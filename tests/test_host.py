@@ -188,3 +188,20 @@ def test_byte_counts_match_the_formats():
     assert az.gguf_bytes(az.Q8_0, 4096, 4096) == 17825792
     assert az.gguf_bytes(az.Q4_K, 128 * 768, 2048) * 2 + az.gguf_bytes(az.Q4_K, 128 * 2048, 768) == 339738624
     assert az.gguf_bytes(5, 1, 256) == 0
+
+
+@pytest.mark.parametrize("via", ["ctypes", "extension"])
+def test_calls_of_a_pass_convert_their_arguments_alike(via):
+    """The extension that the forward pass's calls go through takes and refuses what the ctypes functions do: handles as
+    addresses or None, integers by their low 32 bits, a missing weight as the library's own status."""
+    import ctypes
+    f = az.lib.arcz_engine_matmul
+    if via == "extension":
+        f = pytest.importorskip("arcinferzero_amd._pycall").matmul
+    good = (None, b"m", None, 16, None, 4, 0, True, 2 ** 32 + 1)
+    assert f(*good) == -100 and b"no weight" in az.lib.arcz_engine_error()
+    for i, wrong in ((0, 1.5), (1, "m"), (3, 2.0), (4, "x")):
+        with pytest.raises(ctypes.ArgumentError):
+            f(*good[:i], wrong, *good[i + 1:])
+    with pytest.raises(TypeError):
+        f(*good[:3])
