@@ -200,7 +200,7 @@ def test_calls_of_a_pass_convert_their_arguments_alike(via):
         f = pytest.importorskip("arcinferzero_amd._pycall").matmul
     good = (None, b"m", None, 16, None, 4, 0, True, 2 ** 32 + 1)
     assert f(*good) == -100 and b"no weight" in az.lib.arcz_engine_error()
-    for i, wrong in ((0, 1.5), (1, "m"), (3, 2.0), (4, "x")):
+    for i, wrong in ((0, 1.5), (1, "m"), (3, 2.0), (4, 2.5)):
         with pytest.raises(ctypes.ArgumentError):
             f(*good[:i], wrong, *good[i + 1:])
     with pytest.raises(TypeError):
