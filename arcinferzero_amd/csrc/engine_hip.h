@@ -245,8 +245,8 @@ class Engine {
     return k;
   }
   // The same by the -D names and values as they are, for launches that a pass makes for each layer: no string is put together
-  // or compared, which took as long as submitting the launch (quantize + matmul of one token, 2048 x 2048, from C, one after the other: 5.5 - 6.5 us, now
-  // 5.05, of which the runtime's own submissions are 4.5).  A name of nullptr: left out.
+  // or compared (quantize + matmul of one token, 2048 x 2048, from C, one after the other: 5.5 - 6.5 us, now 5.05, of which the
+  // runtime's own submissions are 4.5).  A name of nullptr: left out.
   struct Def { const char* name; long value; };
   cl_kernel variant(const char* which, std::initializer_list<Def> defs, const char* name) {
     struct Mix {
@@ -898,8 +898,8 @@ class Engine {
     if ((type == GGML_Q4_K || type == GGML_Q5_K) && (sk_force_ >= 2 || q4_wm_ != 0 || q4_forms || (a256_ && type == GGML_Q4_K))) return false;
     if (kept && Mp > 64 && digit_form(type).nw) {
       if (type != GGML_Q6_K && type != GGML_IQ3_XXS && type != GGML_Q4_K) return true;
-      double d = 0.0, i8 = 0.0;
-      digit_pieces(digit_form(type), Mp, N, K / 256, &d);
+      const double d = digit_plan(digit_form(type), Mp, N, K / 256).us;
+      double i8 = 0.0;
       if (type == GGML_Q4_K) i8 = q4k_price(Mp, rows, N, K / 256);
       else split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
       if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes: 128 tokens x
@@ -925,27 +925,32 @@ class Engine {
     if (c64 < 0.97 * c128) return 8.3 + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.63 : r64 <= 2 * cus ? 0.73 : 1.0)) * (19.1 * nsb / 4 + 2.7);
     return 8.3 + (f128 + (r128 == 0 ? 0.0 : r128 <= cus ? 0.71 : 1.0)) * (24.6 * nsb / 4 + 2.7);
   }
-  // Pieces of K, priced as in split_pieces: a full round (two work-groups a compute unit) takes 15, 19.5, 28 us per 1024 values
-  // of K with one, two, three digits (Q4_K, Q5_K: 18.5) and 8 us for its ends, a last round of one work-group a unit 0.65 of
-  // that; the partial tiles cost 4 us and 12 TB/s.  Over 507 products of four types and six matrices, 100 - 1024 tokens in 1 - 8
-  // pieces, this is 5 % off on average and its choice loses 0.2 %.  Q3_K 4096 x 12288, 512 tokens: 195 -> 93 us.
-  static int digit_pieces(const DigitForm& f, int Mp, int N, int nsb, double* price = nullptr) {
-    const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)((Mp + 127) / 128) * ((N + 127) / 128);
+  // How a product on digits is launched: the first `whole` tiles a work-group each, the others in `pieces` of K.  Priced, in us: a
+  // full round (two work-groups a compute unit) takes 15, 19.5, 28 per 1024 values of K with one, two, three digits (Q4_K, Q5_K:
+  // 18.5) and 8 for its ends, a last round of one work-group a unit 0.65 of that; the pieces' sums cost 4 us and 12 TB/s.  (Over
+  // 507 products of four types and six matrices, 100 - 1024 tokens, all tiles in 1 - 8 pieces: 5 % off on average, 0.2 % lost
+  // by the choice.)  Either all tiles go in pieces -- 512 tokens x 4096 rows of Q3_K, K = 12288, 195 -> 93 us --, or those that
+  // full rounds leave over, at most 512 pieces in all (SPLIT_BYTES).
+  struct DigitPlan { int whole, pieces; double us; };
+  static DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb) {
+    const int cus = arcz_device_cus(), n = ((Mp + 127) / 128) * ((N + 127) / 128), slots = 2 * cus;
     const double k1024 = f.nw == 1 ? (f.mn ? 18.5 : 15.0) : f.nw == 2 ? 19.5 : 28.0;
-    int best = 1;
-    double least = 0.0;
-    for (int ny = 1; ny <= 16 && (ny == 1 || ny <= nsb / 2); ++ny) {
-      if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
-      const size_t full = tiles * ny / (2 * cus), rest = tiles * ny % (2 * cus);
-      const double part = rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0;
-      double us = (full + part) * (k1024 * nsb / 4 / ny + 8.0);
-      if (ny > 1) us += 4.0 + 2.0 * ny * Mp * N * 4 / 12.0e6;
-      if (ny == 1 || us < least) {
-        best = ny;
-        least = us;
-      }
+    const int most = (int)std::min<size_t>(slots, SPLIT_BYTES / 65536);
+    auto tile = [&](int p) { return k1024 * nsb / 4 / p + 8.0; };
+    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? 0.65 : 1.0; };
+    const int full = n / slots, rest = n % slots;
+    DigitPlan best = {n, 1, (full + part(rest)) * tile(1)};
+    auto take = [&](int whole, int p, double us) {
+      us += 4.0 + (n - whole) * p * 0.131 / 12.0;
+      if (us < best.us) best = {whole, p, us};
+    };
+    for (int p = 2; p <= 16 && p <= nsb / 2; ++p) {
+      if (n * p <= most) take(0, p, part(n * p) * tile(p));
+      if (full && rest && rest * p <= most) take(n - rest, p, full * tile(1) + part(rest * p) * tile(p));
+      // (the second places of a round of one work-group a unit: beside it a piece runs as in a full round)
+      if (rest > cus && (rest - cus) * p <= std::min(cus, most)) take(n - rest + cus, p, (full + 0.65 + 0.35 / p) * tile(1) + 4.0);
     }
-    if (price) *price = least + 3.0 + Mp * (nsb * 256) / 1.7e6;  // (with the tokens' digits)
+    best.us += 3.0 + Mp * (nsb * 256) / 1.7e6;  // (the tokens' digits)
     return best;
   }
   // rows [n0, n0 + 128 nt) of w as digits, into out
@@ -977,15 +982,23 @@ class Engine {
       if (!kept) row_digits("row_digits", w, n0, nt, wd_);
       cl_kernel k = variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
-      // (ARCZ_Q4_SPLITK=0: K in one piece, =n: n pieces, as many as SPLIT_BYTES holds)
-      int ny = nt < nt_all || sk_force_ == 0 ? 1
-               : sk_force_ >= 2 ? std::max(1, (int)std::min<size_t>(std::min(sk_force_, nsb), SPLIT_BYTES / ((size_t)Mp * N * 4)))
-                                : digit_pieces(f, Mp, N, nsb), zero = 0;
-      size_t gg[2] = {(size_t)mt * nt * 256, (size_t)ny};
-      if (ny > 1) set_args(k, 0, xd_, wd, ws, M, N, K, N, zero, zero, n0, nt);
-      else set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, n0, nt);
-      run(name, k, 2, gg, l);
-      if (ny > 1) splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a);
+      // (ARCZ_Q4_SPLITK=0: K in one piece, =n: all tiles in n pieces, as many as SPLIT_BYTES holds)
+      const int tiles = mt * nt;
+      DigitPlan pl = {tiles, 1, 0.0};
+      if (sk_force_ >= 2 && nt == nt_all) pl = {0, std::min({sk_force_, nsb, (int)(SPLIT_BYTES / 65536) / tiles}), 0.0};
+      else if (sk_force_ != 0 && nt == nt_all) pl = digit_plan(f, Mp, N, nsb);
+      if (pl.pieces < 2) pl = {tiles, 1, 0.0};
+      const int tail = tiles - pl.whole;
+      set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, n0, nt, pl.whole, pl.pieces, ws);
+      size_t gg = (size_t)(pl.whole + tail * pl.pieces) * 256, l1 = 256;
+      run(name, k, 1, &gg, &l1);
+      if (tail) {
+        cl_kernel kr = variant("gemm", {}, "d_reduce");
+        int wide = ((N | ldc | c_off) & 3) == 0 && ((uintptr_t)arcz_mem_ptr(C) & 15) == 0 ? 1 : 0;
+        set_args(kr, 0, ws, C, M, N, ldc, c_off, a, wide, n0, nt, pl.whole, pl.pieces);
+        size_t g[2] = {(size_t)tail * 256, 16};
+        run(name, kr, 2, g, l);
+      }
     }
   }
   // rows: those that the partial tiles hold, 0: all M

@@ -86,8 +86,9 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "act_digits", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits", nullptr, "ppiiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "gemm_d", "MN", "pppiiiiiiii", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "gemm_d", nullptr, "pppiiiiiiii", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm_d", "MN", "pppiiiiiiiiiip", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "d_reduce", nullptr, "ppiiiiiiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm_d", nullptr, "pppiiiiiiiiiip", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},

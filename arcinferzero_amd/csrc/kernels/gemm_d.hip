@@ -512,27 +512,90 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
     }
 }
 
-// Tile L of mt token tiles x nt row tiles: work-groups go to the eight chiplets in turn, so chiplet x takes the x-th eighth of
-// a list of tiles in panels of eight token tiles, row tile by row tile -- neighbours in one L2 share rows and tokens.
-__device__ inline void d_tile_of(int id, int mt, int nt, int& tm, int& tn) {
-  const int total = mt * nt, x = id & 7, j = id >> 3;
-  const int L = x * (total >> 3) + min(x, total & 7) + j;  // (chiplet y has total / 8 tiles, one more if y < total % 8)
+// Work-groups go to the eight chiplets in turn: chiplet x takes the x-th eighth of a list of n, so that neighbours in it
+// share an L2 (chiplet y has n / 8, one more if y < n % 8).
+__device__ inline int d_list_of(int id, int n) {
+  const int x = id & 7;
+  return x * (n >> 3) + min(x, n & 7) + (id >> 3);
+}
+// Tile L of the list of mt token tiles x nt row tiles: panels of eight token tiles, row tile by row tile.
+__device__ inline void d_tile_of(int L, int mt, int nt, int& tm, int& tn) {
   const int panel = L / (8 * nt), rem = L - panel * 8 * nt, pw = min(8, mt - panel * 8);
   tn = rem / pw;
   tm = panel * 8 + rem - tn * pw;
 }
 
-// gemm_d__NW: rows [n0, n0 + 128 ..) of an N-row matrix, nt row tiles of them in wt.  grid (ceil(M / 128) * nt, ny); ny > 1:
-// the superblocks shared out, plane y of C (here a workspace [ny][M][ldc]) the y-th piece's sums.
+// gemm_d__NW: rows [n0, n0 + 128 ..) of an N-row matrix, nt row tiles of them in wt.  The list's first `whole` tiles take a
+// work-group each; each of the others is shared out over `pieces`, superblocks by superblocks, which leave their sums in ws
+// [tile][piece][128][128] for d_reduce: a launch's last round, of a few tiles, would take as long as a full one (17408 x 5120,
+// Q4_0: 512 tokens are 544 tiles on 512 places, 139 us, with the last 32 in 10 pieces 109).  grid (whole + (tiles - whole) *
+// pieces).
 #define GEMM_D(NAME, ...)                                                                                               \
   extern "C" __global__ __launch_bounds__(256, 2) void gemm_d__##NAME(                                                  \
-      const uint8_t* xt, const uint8_t* wt, float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int n0, int nt) { \
+      const uint8_t* xt, const uint8_t* wt, float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int n0, int nt, \
+      int whole, int pieces, float* ws) {                                                                               \
     using I = DImg<__VA_ARGS__>;                                                                                        \
     __shared__ __attribute__((aligned(1024))) uint8_t lds[I::R * I::STAGE];                                             \
+    const int mt = (M + 127) / 128, tail = mt * nt - whole, nsb = K >> 8;                                               \
+    int L, y = 0, ny = 1;                                                                                               \
+    if ((int)blockIdx.x < whole) {                                                                                      \
+      L = d_list_of(blockIdx.x, whole);                                                                                 \
+    } else {                                                                                                            \
+      const int q = blockIdx.x - whole;                                                                                 \
+      y = q / tail;                                                                                                     \
+      ny = pieces;                                                                                                      \
+      L = whole + d_list_of(q - y * tail, tail);                                                                        \
+    }                                                                                                                   \
     int tm, tn;                                                                                                         \
-    d_tile_of(blockIdx.x, (M + 127) / 128, nt, tm, tn);                                                                 \
-    const int y = blockIdx.y, ny = gridDim.y, nsb = K >> 8;                                                             \
-    gemm_d_body<__VA_ARGS__>(lds, xt, wt - (size_t)(n0 >> 7) * (K >> 5) * I::W, C + (size_t)y * M * ldc, M, N, ldc, c_off, \
-                             accumulate, tm * 128, n0 + tn * 128, K >> 5, nsb * y / ny * 8, nsb * (y + 1) / ny * 8);    \
+    d_tile_of(L, mt, nt, tm, tn);                                                                                       \
+    const int m0 = tm * 128, r0 = n0 + tn * 128;                                                                        \
+    if (ny > 1) {                                                                                                       \
+      C = ws + (ptrdiff_t)((L - whole) * ny + y) * 16384 - (ptrdiff_t)(m0 * 128 + r0);                                  \
+      ldc = 128;                                                                                                        \
+      c_off = accumulate = 0;                                                                                           \
+    }                                                                                                                   \
+    gemm_d_body<__VA_ARGS__>(lds, xt, wt - (size_t)(n0 >> 7) * (K >> 5) * I::W, C, M, N, ldc, c_off, accumulate, m0, r0, \
+                             K >> 5, nsb * y / ny * 8, nsb * (y + 1) / ny * 8);                                         \
   }
 GEMM_D(NW1, 1, 0) GEMM_D(NW2, 2, 0) GEMM_D(NW3, 3, 0) GEMM_D(NW1_MN1, 1, 1)
+
+// d_reduce: the pieces' sums of the tiles from `whole` on, added in their order, out to C.  wide: rows of whole vectors.
+// grid (tiles, 16), local 256: eight rows of a tile; eight planes are loaded before the first is added.
+extern "C" __global__ __launch_bounds__(256) void d_reduce(const float* __restrict__ ws, float* __restrict__ C, int M, int N, int ldc,
+                                                           int c_off, int accumulate, int wide, int n0, int nt, int whole,
+                                                           int pieces) {
+  int tm, tn;
+  d_tile_of(whole + blockIdx.x, (M + 127) / 128, nt, tm, tn);
+  const int r = blockIdx.y * 8 + (threadIdx.x >> 5), m = tm * 128 + r, c = threadIdx.x & 31;
+  if (m >= M) return;
+  // (a thread: four columns next to each other, or, where a row's vectors would not be whole, 32 apart)
+  const float* p = ws + (size_t)blockIdx.x * pieces * 16384 + r * 128;
+  const int nb = n0 + tn * 128;
+  v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto plane = [&](int y) {
+    const float* q = p + (size_t)y * 16384;
+    return wide ? *(const v4f*)(q + 4 * c) : (v4f){q[c], q[c + 32], q[c + 64], q[c + 96]};
+  };
+  for (int y = 0; y < pieces; y += 8) {
+    v4f a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = plane(min(y + i, pieces - 1));
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (y + i < pieces) s += a[i];
+  }
+  float* cr = C + (size_t)m * ldc + c_off + nb;
+  auto out = [&](float v, float old) { return accumulate == 1 ? v + old : accumulate == 2 ? v * (old / (1.0f + __expf(-old))) : v; };
+  if (wide) {
+    if (nb + 4 * c >= N) return;
+    v4f* o = (v4f*)(cr + 4 * c);
+    const v4f old = accumulate ? *o : s;
+    *o = (v4f){out(s[0], old[0]), out(s[1], old[1]), out(s[2], old[2]), out(s[3], old[3])};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int n = c + 32 * i;
+    if (nb + n < N) cr[n] = out(s[i], accumulate ? cr[n] : 0.0f);
+  }
+}

@@ -445,6 +445,43 @@ def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     assert az.lib.arcz_spare_bytes() == spare0
 
 
+@pytest.mark.parametrize("qtype,T,N,K,ldc,acc", [(az.Q4_0, 300, 11653, 4096, 11660, 1), (az.Q4_K, 640, 13308, 2560, 13312, 2), (az.Q6_K, 130, 17501, 4096, 17501, 0)])
+def test_gemm_on_digits_in_pieces_of_the_last_tiles(rt, qtype, T, N, K, ldc, acc):
+    """Tiles that full rounds of work-groups leave over go in pieces of K, the others whole (273, 520 and 274 tiles on a chip
+    of 256 compute units): ragged rows and whole vectors, the three epilogues, run to run, the columns beside C's untouched.
+    Against the oracle on the first and last rows."""
+    print(f"last tiles in pieces {TYPE_NAMES[qtype]} T={T} N={N} K={K} acc={acc}", flush=True)
+    Mp = (T + 127) // 128 * 128
+    W = make_weights(qtype, N, K, seed=51)
+    x = make_acts(T, K, seed=52, outliers=True)
+    c0 = np.random.default_rng(53).standard_normal((Mp, ldc)).astype(np.float32)
+    eng = az.Engine(Mp, K)
+    w = eng.make_weight(qtype, N, K, W)
+    xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * ldc * 4)
+    eng.quantize(xb, K, K, Mp, T)
+    ys = []
+    for i in range(2):
+        cb.write(c0)
+        eng.profile(i == 0)
+        eng.matmul("test", w, Mp, cb, ldc, 0, acc)
+        ys.append(cb.read(np.float32, Mp * ldc).reshape(Mp, ldc))
+        if i == 0:
+            eng.profile_collect()
+            assert eng.profile_get("test")[1] == 2 and eng.profile_get("act_digits")[1] == 1
+    for b in (xb, cb, w):
+        b.free()
+    eng.close()
+    assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32)) and np.array_equal(ys[0][:, N:], c0[:, N:])
+    rows = np.r_[0:200, N - 400:N]
+    Ws = np.ascontiguousarray(W.reshape(N, -1)[rows]).reshape(-1)
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, Ws, len(rows), K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    g = c0[:T, rows].astype(np.float64)
+    ref = ref + g if acc == 1 else ref * (g / (1.0 + np.exp(-g))) if acc == 2 else ref
+    y = ys[0][:T, rows]
+    assert np.isfinite(ys[0]).all() and mixed_err(y, ref) <= TOL
+
+
 def _extreme_rows(qtype, N, K, rng):
     """Blocks of random bytes with the superblock's scale set to one (IQ3_XXS: four), so that all values are integers; a
     fifth of the Q6_K and Q3_K rows at the ends of their ranges: every value -32 or 31 times -128 or 127, -4 or 3 times -32
