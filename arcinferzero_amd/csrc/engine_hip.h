@@ -89,6 +89,7 @@ class Engine {
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
     moe_fuse_off_ = getenv("ARCZ_MOE_FUSE") && atoi(getenv("ARCZ_MOE_FUSE")) == 0;
     moe_qfuse_off_ = getenv("ARCZ_MOE_QFUSE") && atoi(getenv("ARCZ_MOE_QFUSE")) == 0;
+    moe_digits_ = getenv("ARCZ_MOE_DIGITS") ? atoi(getenv("ARCZ_MOE_DIGITS")) : 1;
     moe_pre_ = getenv("ARCZ_MOE_PRE") ? atoi(getenv("ARCZ_MOE_PRE")) != 0 : true;
     q4_wm_ = getenv("ARCZ_Q4_WM") ? atoi(getenv("ARCZ_Q4_WM")) : 0;
     q4_wm_min_ = getenv("ARCZ_Q4_WM_MIN") ? atoi(getenv("ARCZ_Q4_WM_MIN")) : 2048;
@@ -858,6 +859,7 @@ class Engine {
   bool digits_keep_ = true;                                                 // ARCZ_DIGITS_KEEP (0: off)
   int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
+  int moe_digits_ = 1;                                                      // ARCZ_MOE_DIGITS (0: off)
   bool moe_pre_ = true;                                                     // ARCZ_MOE_PRE (0: off)
   // (The gate / up tile kernel on ready-made scale vectors runs in steps of 64 values, three work-groups a compute unit:
   // 0.401 -> 0.369 ms at 4096 tokens against the same in steps of 128 at two a unit, same bits.  The down projection's
@@ -1286,6 +1288,8 @@ class Engine {
     // 128 experts x 768 x 2048 at 4096 tokens: 0.80 -> 0.70 ms (gate / up 0.430 -> 0.375, down 0.256 -> 0.212: without
     // the scale registers both tile kernels fit three work-groups a compute unit) for 151 MB on top of the layer's 340.
     cl_mem wsv[3] = {nullptr, nullptr, nullptr};
+    // gate's and up's rows as digits, in the expert tiles' images (moe_d.hip), and down's; none, or given back: size 0
+    cl_mem digits[2] = {nullptr, nullptr};
     bool variant() const { return escale || ebias; }
     std::string route_defs() const {
       if (ebias) {
@@ -1391,13 +1395,123 @@ class Engine {
         size_t g2[2] = {(rows + 255) / 256 * 256, (size_t)nsb}, l2[2] = {256, 1};
         run("q4k_wscales", kw, 2, g2, l2);
       }
+    moe_digits_keep(L);
     return L;
   }
+  // The experts' rows as digits, kept with the layer as digits_keep keeps a matrix's, in the same limits; and the records of the
+  // chunk's tokens and of the experts' inputs, sized for the engine's longest chunk.  ARCZ_MOE_DIGITS=0 when the engine is made:
+  // never (nor with a switch that names a form of the int8 tiles).
+  cl_mem xr_ = nullptr, sr_ = nullptr;
+  static size_t moe_digit_bytes(uint32_t type, size_t rows, int K) {
+    const DigitForm f = digit_form(type);
+    return rows / 256 * (K / 32) * (size_t)(f.nw * 6144 + 1024 + 2048 * f.mn);
+  }
+  void moe_digits_keep(MoeLayer& L) {
+    const size_t NE = L.NE, E = L.E, F = L.F, total = arcz_device_mem();
+    if (!digits_keep_ || !moe_digits_ || digits_env_ == 0 || moe_qfuse_off_ || !moe_pre_ || max_chunk < 32) return;
+    if (L.ex[0].type != L.ex[1].type || !digit_form(L.ex[0].type).nw || !digit_form(L.ex[2].type).nw || NE * E * F < ((size_t)1 << 23)) return;
+    // (32-bit offsets of the records, two bytes a value; the writing launches' grids)
+    if ((size_t)max_chunk * E >= (1ull << 31) || (size_t)slots_ * F >= (1ull << 31) || NE * std::max(F / 128, E / 256) * 4 > 65535) return;
+    const size_t bytes[2] = {moe_digit_bytes(L.ex[0].type, 2 * NE * F, L.E), moe_digit_bytes(L.ex[2].type, NE * E, L.F)};
+    if (arcz_spare_bytes() + bytes[0] + bytes[1] > total / 8 || arcz_device_mem_free() < bytes[0] + bytes[1] + total / 4) return;
+    if (!xr_) xr_ = try_buf((size_t)max_chunk * E * 2);
+    if (!sr_) sr_ = try_buf((size_t)slots_ * F * 2);
+    if (!xr_ || !sr_) return;
+    for (int i = 0; i < 2; ++i) {
+      if (!(L.digits[i] = try_buf(bytes[i]))) return;
+      CL_CHECK(arcz_mem_spare(L.digits[i]));
+      const GpuWeight &a = L.ex[i ? 2 : 0], &b = L.ex[i ? 2 : 1];
+      const size_t tiles = i ? a.rows / 256 : a.rows / 128;
+      cl_kernel k = variant("gemm", {{"QTYPE", a.type}}, "row_digits_e");
+      int nsb = a.K / 256, step = i ? 256 : 128, second = i ? 128 : 0;
+      size_t rows = a.rows, g[2] = {(size_t)nsb * 256, tiles * 4}, l[2] = {256, 1};
+      set_args(k, 0, a.raw, b.raw, tabs_, rows, nsb, step, second, L.digits[i]);
+      run("keep_digits", k, 2, g, l);
+    }
+  }
+  // Which passes: by slots an expert, from where the type's other forms are slower (us a layer, these forms / digits, 128 x 8 experts of
+  // 768 x 2048 at 200, 400, 1000, 4096 tokens: Q5_K 193 / 173, 229 / 188, 339 / 257, 923 / 640; Q4_0 128 / 150, 197 / 164, 366 / 226,
+  // 876 / 570; Q3_K 205 / 219, 331 / 239, 630 / 310; IQ4_XS 146 / 219, 220 / 238, 374 / 312; IQ3_S 191 / 150, 303 / 164; Q6_K 191 /
+  // 298, 279 / 316, 415 / 413, 1129 / 900): below it the pass is the images' bytes, 1.6 - 3 times the planes'.  Q4_K by price:
+  // 382 / 368 at 2000, 254 / 257 at 1000, 184 / 202 at 600; 32 x 8 of 1536 x 3072, 1000 461 / 433; 64 x 4 of 1024 x 1024 96 / 103.
+  bool moe_on_digits(const MoeLayer& L, int T) const {
+    if (!L.digits[1] || arcz_mem_size(L.digits[0]) == 0 || arcz_mem_size(L.digits[1]) == 0) return false;
+    if (moe_digits_ > 1) return true;
+    if (moe_dec_off_ || moe_mm_off_ || (moe_dec_set_ && T <= moe_dec_max_)) return false;  // (switches that name another form)
+    const double slots = (double)T * L.NU / L.NE;
+    const bool large = (size_t)L.E * L.F >= ((size_t)1 << 22);
+    auto least = [&](uint32_t t) {
+      return t == GGML_IQ3_S ? 5.0 : t == GGML_IQ3_XXS ? 10.0 : t == GGML_Q5_K ? 11.0 : t == GGML_Q3_K ? 14.0 : t == GGML_Q4_0 || t == GGML_MXFP4 ? 15.0
+             : t == GGML_Q6_K ? (large ? 25.0 : 70.0) : t == GGML_Q4_K ? 100.0 : 26.0;
+    };
+    const uint32_t gu = L.ex[0].type, dn = L.ex[2].type;
+    if (gu != GGML_Q4_K || dn != GGML_Q4_K) return slots >= std::max(least(gu), least(dn));
+    return slots > 15.0 && moe_q4k_digits_cheaper(L, T);
+  }
+  // Tiles of 64 slots, on average: the experts that more than 0, 64, 128, ... of the tokens choose.
+  static double moe_tiles(const MoeLayer& L, int T) {
+    const double p = (double)L.NU / L.NE, mean = T * p, dev = std::sqrt(2.0 * mean * (1.0 - p)) + 1e-9;
+    double t = 1.0 - std::pow(1.0 - p, T);
+    for (int k = 64; k <= T; k += 64) {
+      const double more = 0.5 * std::erfc((k + 0.5 - mean) / dev);
+      if (more < 1e-4 && k > mean) break;
+      t += more;
+    }
+    return t * L.NE;
+  }
+  // Both kernels of both forms in rounds of work-groups: 512 places on digits, or the images' bytes, 768 for the int8 tiles.  Fitted to
+  // 25 passes of four layers (5 and 8 % off on average).
+  static bool moe_q4k_digits_cheaper(const MoeLayer& L, int T) {
+    const double cus = arcz_device_cus(), t = moe_tiles(L, T), E = L.E, F = L.F, hit = 1.0 - std::pow(1.0 - (double)L.NU / L.NE, T);
+    auto rounds = [](double f, double half, double over) { return f <= 0.5 ? half : f <= 1.0 ? 1.0 : f + over; };
+    const double bytes = hit * L.NE * E * F * 1.125 / 4.28e6;
+    const double d = 5.0 + std::max(2.0 * bytes, rounds(t * F / 128 / (2 * cus), 0.35, 0.31) * (20.5 * E / 1024 + 8.3)) +
+                     std::max(bytes, rounds(t * E / 256 / (2 * cus), 0.35, 0.31) * (20.5 * F / 1024 + 8.3));
+    const double i8 = rounds(t * F / 128 / (3 * cus), 0.76, 0.25) * (39.4 * E / 1024 + 3.1) + rounds(t * E / 128 / (3 * cus), 0.76, 0.25) * (19.7 * F / 1024 + 3.1);
+    return d < 0.97 * i8;
+  }
+  void moe_digits(const MoeLayer& L, cl_mem rl, int ldl, cl_mem x, int T, int Mp, cl_mem sh) {
+    const int E = L.E, F = L.F, n = T * L.NU;
+    route_tiles(L, rl, ldl, T, 64);
+    const size_t tiles = ((size_t)(n + 63) / 64 + std::min(n, L.NE) + 7) / 8 * 8;
+    auto tile_kernel = [&](const char* name, uint32_t type) {
+      const DigitForm f = digit_form(type);
+      return variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, name);
+    };
+    size_t l[2] = {256, 1};
+    {
+      cl_kernel k = variant("gemm", {}, "act_records");
+      int MM = Mp, KK = E, TT = T;
+      set_args(k, 0, aq_, asc_, absum_, MM, KK, TT, xr_);
+      size_t g[2] = {(size_t)E, (size_t)(T + 63) / 64};
+      run("act_records", k, 2, g, l);
+    }
+    {
+      cl_kernel k = tile_kernel("moe_gu_d", L.ex[0].type);
+      int FF = F, KK = E, S = slots_;
+      set_args(k, 0, xr_, L.digits[0], FF, KK, mtiles_, stok_, mh_, S, mhq_, mhsc_, mhbs_, sr_);
+      size_t g[2] = {(size_t)F / 128 * 256, tiles};
+      run("moe_gateup", k, 2, g, l);
+    }
+    {
+      cl_kernel k = tile_kernel("moe_down_d", L.ex[2].type);
+      int NN = E, KK = F;
+      set_args(k, 0, sr_, L.digits[1], NN, KK, mtiles_, swt_, my_);
+      size_t g[2] = {(size_t)E, tiles};
+      run("moe_down", k, 2, g, l);
+    }
+    moe_sum(L, x, sh, T);
+  }
   void free_moe_layer(MoeLayer& L) {
+    for (cl_mem m : L.digits) not_listed(m, "free_moe_layer");
     for (int i = 0; i < 3; ++i) {
       free_weight(L.ex[i]);
       if (L.wsv[i]) release(L.wsv[i]);
       L.wsv[i] = nullptr;
+    }
+    for (cl_mem& m : L.digits) {
+      if (m) release(m);
+      m = nullptr;
     }
     set_moe_routing(L, nullptr, nullptr, 1.0f);
   }
@@ -1594,6 +1708,10 @@ class Engine {
     // (the switches of this function are read when the engine is made: a test sets them before it makes its engine)
     // From 6 or 9 tokens on the 16-slot tiles take over where they are cheaper (moe_mm_takes, moe_mm_cheaper) -- not where
     // ARCZ_MOE_DECODE_MAX is given and names the pass, nor with ARCZ_MOE_DECODE=0 or ARCZ_MOE_MM=0.
+    if (moe_on_digits(L, T)) {
+      moe_digits(L, rl, ldl, x, T, Mp, sh);
+      return;
+    }
     const bool one_slot = !moe_dec_off_ && T <= moe_dec_max_ && T * NU <= 512;
     const bool mm = !moe_mm_off_ && moe_mm_takes(L, T) && (!one_slot || (!moe_dec_set_ && moe_mm_cheaper(L, T)));
     if (mm && moe_mm(L, rl, ldl, x, T, Mp, sh)) return;

@@ -24,5 +24,6 @@
     BLOB arcz_blob_decode_mm, "decode_mm.hsaco"
     BLOB arcz_blob_gemm, "gemm.hsaco"
     BLOB arcz_blob_gemm_d, "gemm_d.hsaco"
+    BLOB arcz_blob_moe_d, "moe_d.hsaco"
     BLOB arcz_blob_moe, "moe.hsaco"
     .section .note.GNU-stack,"",@progbits

@@ -87,6 +87,12 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "act_digits", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits", nullptr, "ppiiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_d", "MN", "pppiiiiiiiiiip", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "act_records", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "row_digits_e", nullptr, "pppziiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "moe_gu_d", "MN", "ppiipppipppp", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "moe_gu_d", nullptr, "ppiipppipppp", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "moe_down_d", "MN", "ppiippp", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "moe_down_d", nullptr, "ppiippp", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "d_reduce", nullptr, "ppiiiiiiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_d", nullptr, "pppiiiiiiiiiip", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},

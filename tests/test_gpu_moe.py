@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import arcinferzero_amd as az
+import gguf_writer as gw
 import oracle_lib as orc
 from common import TYPE_NAMES, make_acts, make_weights, quantize_padded, rel_err_rows
 
@@ -489,3 +490,79 @@ def test_moe_layer_upload_checks_the_tensors_byte_counts(rt):
             L.free()
         finally:
             eng.close()
+
+
+@pytest.mark.parametrize("qtype,qdown,NE,NU,E,F,T,Mp", [(az.Q4_K, az.Q6_K, 16, 4, 1024, 768, 33, 48), (az.Q5_K, az.Q5_K, 128, 2, 256, 256, 130, 256),
+                                                        (az.Q4_0, az.Q3_K, 9, 3, 1280, 768, 200, 256), (az.Q6_K, az.Q4_K, 33, 8, 512, 512, 65, 80),
+                                                        (az.IQ4_XS, az.IQ3_XXS, 8, 2, 1024, 1024, 1, 16), (az.IQ3_S, az.MXFP4, 16, 8, 768, 768, 300, 304)])
+def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E, F, T, Mp):
+    """The expert tiles on digits against the int8 forms of the same layer, one to three digits a weight, with a minimum and
+    without, gate / up and down of different types; tiles of 1 to 64 slots, experts without a token.  h to f32 rounding,
+    its int8 form bit for bit the quantizer's on that h, the down projection's rows on that int8 form against the
+    oracle's sums, the layer run to run; digits given back: the other forms again."""
+    print(f"moe digits {TYPE_NAMES[qtype]} {TYPE_NAMES[qdown]} NE={NE} NU={NU} E={E} F={F} T={T}", flush=True)
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "2")            # (read when the engine is made: whatever the rule says)
+    Wg, Wu, Wd = make_weights(qtype, NE * F, E, seed=1), make_weights(qtype, NE * F, E, seed=2), make_weights(qdown, NE * E, F, seed=3)
+    x = make_acts(T, E, seed=4)
+    logits = np.random.default_rng(5).standard_normal((T, NE)).astype(np.float32)
+    logits[:, NE - 1] = -50.0                             # (an expert that no token chooses)
+    p, names = tmp_path / "layer.gguf", ("gate", "up", "down")
+    gw.write_gguf(p, [], [(names[0], qtype, [E, F, NE], Wg), (names[1], qtype, [E, F, NE], Wu), (names[2], qdown, [F, E, NE], Wd)])
+    eng = az.Engine(max(Mp, 48), max(E, F))
+    spare0 = az.lib.arcz_spare_bytes()
+    with az.GgufFile(p) as gf:
+        L = eng.make_moe_layer_gguf(gf, *names, NU)
+    assert az.lib.arcz_spare_bytes() > spare0
+    xb, lb = az.Runtime.from_numpy(x), az.Runtime.from_numpy(logits)
+    S, n = eng.moe_slots, T * NU
+
+    def run():
+        ob = az.Runtime.alloc(T * E * 4).fill(0)
+        eng.quantize(xb, E, E, Mp, T)
+        eng.layer_moe(L, lb, NE, ob, T, Mp)
+        y = ob.read(np.float32, T * E).reshape(T, E)
+        ob.free()
+        return y
+
+    eng.profile(True)
+    y1 = run()
+    eng.profile_collect()
+    assert eng.profile_get("act_records")[1] == 1
+    eng.profile(False)
+    assert np.array_equal(y1.view(np.uint32), run().view(np.uint32))
+    inv = eng.moe_buffer("inv").read(np.int32, n).reshape(T, NU)
+    h = eng.moe_buffer("h").read(np.float32, S * F).reshape(S, F)
+    hq, hsc = eng.moe_buffer("hq").read(np.int8, S * F).reshape(S, F), eng.moe_buffer("hsc").read(np.float32, S * F // 32).reshape(F // 32, S)
+    yr = eng.moe_buffer("y").read(np.float32, S * E).reshape(S, E)
+    used = np.sort(inv.reshape(-1))
+    raq, rasc, _ = orc.quantize_act(np.ascontiguousarray(h[used]))
+    assert np.array_equal(hq[used], raq) and np.array_equal(hsc[:, used].view(np.uint32), rasc.view(np.uint32))
+    aq, asc, _ = orc.quantize_act(x)
+    ids, wts = np.zeros((T, NU), int), np.zeros((T, NU))
+    for t in range(T):
+        ids[t] = np.argsort(-logits[t], kind="stable")[:NU]
+        e = np.exp(logits[t, ids[t]].astype(np.float64) - logits[t].max())
+        wts[t] = e / e.sum()
+    rbg, rbd = len(Wg) // NE, len(Wd) // NE
+    for t in sorted({0, T // 2, T - 1}):
+        for k in range(NU):
+            s, e = inv[t, k], ids[t, k]
+            a1, s1 = np.ascontiguousarray(aq[t:t + 1]), np.ascontiguousarray(asc[:, t:t + 1])
+            g = orc.matmul_ref(qtype, Wg[e * rbg:(e + 1) * rbg], F, E, a1, s1)[0]
+            u = orc.matmul_ref(qtype, Wu[e * rbg:(e + 1) * rbg], F, E, a1, s1)[0]
+            want = u * (g / (1.0 + np.exp(-g.astype(np.float64))))
+            assert np.abs(h[s] - want).max() <= 1e-3 * np.abs(want).max()
+            d = orc.matmul_ref(qdown, Wd[e * rbd:(e + 1) * rbd], E, F, np.ascontiguousarray(hq[s:s + 1]), np.ascontiguousarray(hsc[:, s:s + 1]))[0] * wts[t, k]
+            assert np.abs(yr[s] - d).max() <= 1e-3 * np.abs(d).max()
+    az.lib.arcz_set_fake_oom(1)
+    try:
+        az.Runtime.alloc(64).free()                       # (an allocation that fails once takes the digits back)
+    finally:
+        az.lib.arcz_set_fake_oom(0)
+    assert az.lib.arcz_spare_bytes() == spare0
+    y2 = run()
+    assert np.linalg.norm(y2 - y1) <= 5e-4 * np.linalg.norm(y1)   # (values on a rounding boundary of the int8 grid may fall either way)
+    L.free()
+    for b in (xb, lb):
+        b.free()
+    eng.close()
