@@ -85,6 +85,7 @@ class Engine {
     moe_mm_off_ = moe_dec_off_ || (getenv("ARCZ_MOE_MM") && atoi(getenv("ARCZ_MOE_MM")) == 0);
     digits_env_ = getenv("ARCZ_GEMM_DIGITS") ? atoi(getenv("ARCZ_GEMM_DIGITS")) : -1;
     digits_keep_ = !(getenv("ARCZ_DIGITS_KEEP") && atoi(getenv("ARCZ_DIGITS_KEEP")) == 0);
+    digits64_ = getenv("ARCZ_GEMM_D64") ? atoi(getenv("ARCZ_GEMM_D64")) : -1;
     gemm_split_ = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
     moe_fuse_off_ = getenv("ARCZ_MOE_FUSE") && atoi(getenv("ARCZ_MOE_FUSE")) == 0;
@@ -375,7 +376,7 @@ class Engine {
     if (rows == (size_t)N) {
       if (digits_take(w.type, max_chunk, N, K, false, max_chunk)) digits_reserve(w);
       bool keep = false;  // (whether a chunk of this engine would take them)
-      for (int m = 128; !keep && m < 2 * max_chunk; m *= 2) keep = digits_take(w.type, std::min(m, max_chunk), N, K, true, std::min(m, max_chunk));
+      for (int m = 32; !keep && m < 2 * max_chunk; m *= 2) keep = digits_take(w.type, std::min(m, max_chunk), N, K, true, std::min(m, max_chunk));
       if (keep) digits_keep(w);
     }
     if (type == GGML_IQ3_S || type == GGML_Q3_K || type == GGML_IQ3_XXS) {  // (room for its GEMM form)
@@ -857,6 +858,7 @@ class Engine {
   bool moe_dec_set_ = false, moe_mm_off_ = false;                           // ARCZ_MOE_DECODE_MAX given; ARCZ_MOE_MM = 0
   int digits_env_ = -1;                                                     // ARCZ_GEMM_DIGITS (-1: by rule)
   bool digits_keep_ = true;                                                 // ARCZ_DIGITS_KEEP (0: off)
+  int digits64_ = -1;                                                       // ARCZ_GEMM_D64 (-1: by price, 0: never, 1: always)
   int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
   int moe_digits_ = 1;                                                      // ARCZ_MOE_DIGITS (0: off)
@@ -877,13 +879,11 @@ class Engine {
     const int mn = type == GGML_Q4_K || type == GGML_Q5_K ? 1 : 0;
     return {nw, mn, mn ? 7680 : nw == 3 ? 7168 : 6656, nw == 3 ? 10240 : nw * 3072 + 512 + 1024 * mn};
   }
-  // Where it pays.  With the rows' digits kept (digits_keep) from more than 64 token rows on, against the int8 kernels: us, 128
-  // / 300 / 1024 tokens, 4096 x 4096: Q4_0 23 / 24, 31 / 40, 54 / 80, Q3_K 22 / 35, 36 / 52, 63 / 109, IQ3_XXS 22 / 31, 36 / 41,
-  // 62 / 76; 17408 x 5120: Q4_0 44 / 58, 87 / 139, 222 / 337, MXFP4 45 / 61, 86 / 146, 219 / 349, IQ3_S 44 / 93, 89 / 146, 223 /
-  // 367, Q3_K 61 / 113, 117 / 201, 304 / 550, IQ3_XXS 60 / 89, 116 / 145, 296 / 362, Q5_K 51 / 68, 102 / 143, 268 / 336,
-  // IQ4_XS 61 / 59, 118 / 142, 298 / 346 (4096 x 4096 22 / 25, 36 / 41, 62 / 85); Q4_K,
-  // Q6_K (three digits) and IQ3_XXS where it is priced cheaper: Q4_K 17408 x 5120 50 / 61, 101 / 110, 262 / 295, but 12288 x
-  // 4096, 300 tokens, 82 / 69; Q6_K 17408 x 5120 75 / 90, 154 / 179, 391 / 518, but 2048 x 5120 28 / 22, 33 / 35, 59 / 70.
+  // Where it pays.  With the rows' digits kept (digits_keep) from more than 16 or 64 token rows on, where the prices below say so:
+  // over eight matrices (2048 x 5120 - 17408 x 5120, among them 1500 x 8192 and 9000 x 1024) x 17 - 1500 tokens, 666 products with
+  // weights from memory, the time against the int8 kernels': Q3_K 0.74, IQ3_S 0.72, Q4_0 0.82, MXFP4 0.79, IQ3_XXS 0.82, Q5_K
+  // 0.87, IQ4_XS 0.88, Q6_K 0.93, Q4_K 0.95 on average.  (us at 17408 x 5120, 128 / 300 / 1000 tokens: Q3_K 61 / 113, 101 / 201,
+  // 296 / 550; Q4_0 50 / 59, 87 / 139, 214 / 337; Q4_K 57 / 61, 104 / 115, 256 / 295.)
   // Without, in outputs (token rows x weight rows), since the digits of the rows are written for every matmul.  us
   // before and now, 4096 x 4096, 256 / 512 / 1024 tokens: Q3_K 43 / 42, 66 / 57, 109 / 75; Q4_0 30 / 35, 42 / 47, 80 / 64;
   // MXFP4 32 / 35, 44 / 47, 85 / 64; IQ3_S 36 / 39, 51 / 52, 77 / 68; 12288 x 4096, 256 tokens: Q4_0 79 / 70, MXFP4 84 / 69,
@@ -898,14 +898,22 @@ class Engine {
     //  scales have Q4_K's form that adds a superblock's block sums as integers)
     static const bool q4_forms = getenv("ARCZ_Q4_BM") || getenv("ARCZ_Q4_BN") || getenv("ARCZ_Q4_SMALL") || getenv("ARCZ_Q4_AU");
     if ((type == GGML_Q4_K || type == GGML_Q5_K) && (sk_force_ >= 2 || q4_wm_ != 0 || q4_forms || (a256_ && type == GGML_Q4_K))) return false;
-    if (kept && Mp > 64 && digit_form(type).nw) {
-      if (type != GGML_Q6_K && type != GGML_IQ3_XXS && type != GGML_Q4_K) return true;
-      const double d = digit_plan(digit_form(type), Mp, N, K / 256).us;
+    if (kept && Mp > 16 && digit_form(type).nw) {
+      // (17 - 64 rows: us at 17408 x 5120, 40 tokens, Q4_0 33 / 54, Q3_K 45 / 72, IQ4_XS 45 / 56, 5120 x 17408 34 / 67, 46 / 75, 46 /
+      //  69; Q4_K 40 / 37, Q5_K 40 / 41, Q6_K 59 / 50: not)
+      if (Mp <= 64 && (type == GGML_Q4_K || type == GGML_Q5_K || type == GGML_Q6_K)) return false;
+      // (these always: of 267 products, with digits 0.42 - 1.02 of the time without; IQ3_XXS 0.67 - 1.00, Q5_K 0.50 - 1.00)
+      if (type == GGML_Q3_K || type == GGML_IQ3_S || type == GGML_Q4_0 || type == GGML_MXFP4) return true;
+      if (type == GGML_IQ3_XXS ? Mp <= 128 : type == GGML_Q5_K && Mp >= 256) return true;
+      // (the others where they are priced cheaper by more than the prices' own error)
+      const double d = digit_plan(digit_form(type), Mp, N, K / 256, true, rows).us;
       double i8 = 0.0;
-      if (type == GGML_Q4_K) i8 = q4k_price(Mp, rows, N, K / 256);
-      else split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
-      if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes: 128 tokens x
-      return d < i8;                                                 //  4096 x 4096 22 / 31, 300 x 12288 x 4096 88 / 82)
+      if (type == GGML_Q6_K || type == GGML_IQ3_XXS)
+        split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
+      else i8 = i8_price(type, Mp, rows, N, K / 256);
+      if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes)
+      const double less = type == GGML_IQ3_XXS || type == GGML_Q6_K ? 1.0 : type == GGML_Q4_K ? (K <= 1024 ? 0.9 : 0.94) : type == GGML_Q5_K ? 0.95 : 0.93;
+      return d < less * i8;  // (Q4_K 9000 x 1024, 1500 tokens: 65 / 60 us)
     }
     if (Mp < 256) return false;
     switch (type) {
@@ -916,43 +924,58 @@ class Engine {
       default: return false;
     }
   }
-  // us of a Q4_K product on the int8 kernels as gemm_dense launches them: pieces of K, 64 x 128 tiles (three work-groups a compute
-  // unit) or 128 x 128 (two).  Fitted to seven matrices x 128 - 2048 tokens, 4.6 % off on average.
-  static double q4k_price(int Mp, int rows, int N, int nsb) {
-    const double cus = arcz_device_cus(), nt = (N + 127) / 128, t128 = (Mp + 127) / 128 * nt, t64 = (rows + 63) / 64 * nt;
-    const int ny = (int)std::min({8.0, nsb / 2.0, 2 * cus / t128});
-    if (ny >= 3) return 8.0 + (t128 * ny <= cus ? 0.71 : 1.0) * (24.6 * nsb / 4 / ny + 2.7) + 2.0 * ny * Mp * N * 4 / 8.0e6;
-    const double r128 = std::fmod(t128, 2 * cus), r64 = std::fmod(t64, 3 * cus), f128 = std::floor(t128 / (2 * cus)), f64 = std::floor(t64 / (3 * cus));
-    const double c128 = f128 + (r128 == 0 ? 0.0 : r128 <= cus ? 0.5 : 1.0), c64 = 0.8 * f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.30 : r64 <= 2 * cus ? 0.48 : 0.8);
-    if (c64 < 0.97 * c128) return 8.3 + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.63 : r64 <= 2 * cus ? 0.73 : 1.0)) * (19.1 * nsb / 4 + 2.7);
-    return 8.3 + (f128 + (r128 == 0 ? 0.0 : r128 <= cus ? 0.71 : 1.0)) * (24.6 * nsb / 4 + 2.7);
+  // us of a product of Q4_K, Q5_K, IQ4_XS or IQ4_NL on the int8 kernels as gemm_dense launches them: pieces of K, 128 x 128 tiles
+  // (two work-groups a compute unit) or, Q4_K, 64 x 128 (three).  Fitted to eight matrices x 80 - 1500 tokens, 4 - 6 % off.
+  static double i8_price(uint32_t type, int Mp, int rows, int N, int nsb) {
+    struct P { double base, pieces, round, ends, one, sums, out; };
+    const P p = type == GGML_Q4_K ? P{9.0, 11.6, 26.0, 2.1, 0.62, 13.3e6, 14.6e6}
+                : type == GGML_Q5_K ? P{7.2, 11.7, 26.7, 3.1, 0.61, 11.3e6, 10.1e6} : P{7.2, 9.8, 26.1, 2.9, 0.69, 13.4e6, 12.6e6};
+    const int cus = arcz_device_cus(), nt = (N + 127) / 128, t = (Mp + 127) / 128 * nt, ny = std::min({8, nsb / 2, 2 * cus / t});
+    const double out = rows * (double)N * 4 / p.out;
+    if (ny >= 3) return p.pieces + (t * ny <= cus ? p.one : 1.0) * (p.round * nsb / 4 / ny + p.ends) + 2.0 * ny * Mp * N * 4 / p.sums + out;
+    const int full = t / (2 * cus), rest = t % (2 * cus), t64 = (rows + 63) / 64 * nt, f64 = t64 / (3 * cus), r64 = t64 % (3 * cus);
+    const double c128 = full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : 1.0), c64 = 0.8 * f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.30 : r64 <= 2 * cus ? 0.48 : 0.8);
+    if (type == GGML_Q4_K && c64 < 0.97 * c128)  // (gemm_dense's choice)
+      return p.base + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.5 : 0.63 + 0.37 * (r64 - cus) / (2.0 * cus))) * (19.9 * nsb / 4 + p.ends) + out;
+    return p.base + (full + (rest == 0 ? 0.0 : rest <= cus ? p.one : 1.0)) * (p.round * nsb / 4 + p.ends) + out;
   }
-  // How a product on digits is launched: the first `whole` tiles a work-group each, the others in `pieces` of K.  Priced, in us: a
-  // full round (two work-groups a compute unit) takes 15, 19.5, 28 per 1024 values of K with one, two, three digits (Q4_K, Q5_K:
-  // 18.5) and 8 for its ends, a last round of one work-group a unit 0.65 of that; the pieces' sums cost 4 us and 12 TB/s.  (Over
-  // 507 products of four types and six matrices, 100 - 1024 tokens, all tiles in 1 - 8 pieces: 5 % off on average, 0.2 % lost
-  // by the choice.)  Either all tiles go in pieces -- 512 tokens x 4096 rows of Q3_K, K = 12288, 195 -> 93 us --, or those that
-  // full rounds leave over, at most 512 pieces in all (SPLIT_BYTES).
-  struct DigitPlan { int whole, pieces; double us; };
-  static DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb) {
-    const int cus = arcz_device_cus(), n = ((Mp + 127) / 128) * ((N + 127) / 128), slots = 2 * cus;
-    const double k1024 = f.nw == 1 ? (f.mn ? 18.5 : 15.0) : f.nw == 2 ? 19.5 : 28.0;
-    const int most = (int)std::min<size_t>(slots, SPLIT_BYTES / 65536);
-    auto tile = [&](int p) { return k1024 * nsb / 4 / p + 8.0; };
-    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? 0.65 : 1.0; };
-    const int full = n / slots, rest = n % slots;
-    DigitPlan best = {n, 1, (full + part(rest)) * tile(1)};
-    auto take = [&](int whole, int p, double us) {
-      us += 4.0 + (n - whole) * p * 0.131 / 12.0;
-      if (us < best.us) best = {whole, p, us};
-    };
-    for (int p = 2; p <= 16 && p <= nsb / 2; ++p) {
-      if (n * p <= most) take(0, p, part(n * p) * tile(p));
-      if (full && rest && rest * p <= most) take(n - rest, p, full * tile(1) + part(rest * p) * tile(p));
-      // (the second places of a round of one work-group a unit: beside it a piece runs as in a full round)
-      if (rest > cus && (rest - cus) * p <= std::min(cus, most)) take(n - rest + cus, p, (full + 0.65 + 0.35 / p) * tile(1) + 4.0);
+  // How a product on digits is launched: in tiles of 128 x 128 or, of a matrix whose rows' digits are kept, 64 tokens x 256 rows;
+  // the first `whole` tiles a work-group each, the others in `pieces` of K -- all of them (512 tokens x 4096 rows of Q3_K, K =
+  // 12288, 195 -> 93 us), or those that full rounds leave over, at most 512 pieces (SPLIT_BYTES).  Priced, in us: a full round
+  // (two work-groups a compute unit) by 1024 values of K and for its ends, a last round of one work-group a unit 0.64 of that
+  // and from there on by its work-groups, the pieces' sums 4 us and 12 TB/s, 3 % of
+  // a product of more than a round (at the power limit of the chip their traffic costs more).  Fitted to 666 products of nine
+  // types and eight matrices, 17 - 1500 tokens, weights from memory: 5 - 6 % off.
+  struct DigitPlan { int th, whole, pieces; double us; };
+  DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb, bool kept, int rows) const {
+    const int cus = arcz_device_cus(), slots = 2 * cus, most = (int)std::min<size_t>(slots, SPLIT_BYTES / 65536);
+    const double k1024 = f.mn ? 21.3 : f.nw == 1 ? 17.4 : f.nw == 2 ? 23.7 : 30.7, ends = f.mn ? 5.6 : f.nw == 1 ? 4.4 : 8.0;
+    const double two = f.nw == 1 && !f.mn ? 0.84 : 0.76;
+    // (tiles of 64 tokens: fewer stages in flight with two and three digits; at most 32 tokens: half the products)
+    const double k64 = (f.nw == 1 ? 1.02 : f.nw == 2 ? 1.10 : 1.12) * (rows <= 32 && f.nw < 3 ? 0.7 : 1.0), e64 = ends + (f.nw == 1 ? 0.7 : f.nw == 2 ? 1.5 : 2.0);
+    int th = 128;
+    auto tile = [&](int p) { return (th == 128 ? k1024 : k64 * k1024) * ((nsb + p - 1) / p) / 4 + (th == 128 ? ends : e64); };
+    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? 0.64 : two + (1.0 - two) * (wgs - cus) / cus; };
+    DigitPlan best = {128, 0, 1, 1e30};
+    for (th = 128; th >= 64; th -= 64) {
+      if (th == 64 ? !kept || digits64_ == 0 : kept && digits64_ == 1) continue;
+      const int n = th == 64 ? (rows + 63) / 64 * ((N + 255) / 256) : (Mp + 127) / 128 * ((N + 127) / 128);
+      const int full = n / slots, rest = n % slots;
+      auto take = [&](int whole, int p, double us) {
+        if (p > 1) us += 4.0 + (n - whole) * p * 0.131 / 12.0;
+        if (us < best.us) best = {th, whole, p, us};
+      };
+      take(n, 1, (full + part(rest)) * tile(1));
+      for (int p = 2; p <= 16 && p <= nsb / 2; ++p) {
+        if (n * p <= most) take(0, p, part(n * p) * tile(p));
+        if (full && rest && rest * p <= most) take(n - rest, p, 1.03 * (full * tile(1) + part(rest * p) * tile(p)));
+        // (the second places of a round of one work-group a unit: beside it a piece runs as in a full round)
+        if (rest > cus && (rest - cus) * p <= std::min(cus, most)) take(n - rest + cus, p, (full + 0.64 + 0.36 / p) * tile(1) + 4.0);
+      }
     }
-    best.us += 3.0 + Mp * (nsb * 256) / 1.7e6;  // (the tokens' digits)
+    // (the tokens' digits and the launches; the rows' digits from memory)
+    best.us += (f.mn ? 5.4 : f.nw == 1 ? 6.2 : f.nw == 2 ? 2.5 : 1.9) + Mp * (nsb * 256) / 1.7e6 +
+               (double)((N + 127) / 128) * nsb * 8 * f.wimg / (f.nw == 3 ? 18.0e6 : 40.0e6) + rows * (double)N * 4 / 9.0e6;
     return best;
   }
   // rows [n0, n0 + 128 nt) of w as digits, into out
@@ -982,22 +1005,28 @@ class Engine {
     for (int t0 = 0; t0 < nt_all; t0 += panel) {
       int nt = std::min(panel, nt_all - t0), n0 = t0 * 128;
       if (!kept) row_digits("row_digits", w, n0, nt, wd_);
-      cl_kernel k = variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, "gemm_d");
       cl_mem ws = noalloc_ ? arcz_scratch_mem() : sk_ws_;
       // (ARCZ_Q4_SPLITK=0: K in one piece, =n: all tiles in n pieces, as many as SPLIT_BYTES holds)
-      const int tiles = mt * nt;
-      DigitPlan pl = {tiles, 1, 0.0};
-      if (sk_force_ >= 2 && nt == nt_all) pl = {0, std::min({sk_force_, nsb, (int)(SPLIT_BYTES / 65536) / tiles}), 0.0};
-      else if (sk_force_ != 0 && nt == nt_all) pl = digit_plan(f, Mp, N, nsb);
-      if (pl.pieces < 2) pl = {tiles, 1, 0.0};
+      int valid = std::clamp(cur_rows_, 1, Mp);
+      const bool all = nt == nt_all;
+      DigitPlan pl = {128, mt * nt, 1, 0.0};
+      if (all && sk_force_ < 0) pl = digit_plan(f, Mp, N, nsb, kept, valid);
+      else if (kept && digits64_ == 1) pl = {64, (valid + 63) / 64 * ((N + 255) / 256), 1, 0.0};
+      const int tiles = pl.th == 64 ? (valid + 63) / 64 * ((N + 255) / 256) : mt * nt;
+      if (all && sk_force_ >= 2) {
+        pl.pieces = std::min({sk_force_, nsb, (int)(SPLIT_BYTES / 65536) / tiles});
+        pl.whole = pl.pieces >= 2 ? 0 : tiles;
+      }
       const int tail = tiles - pl.whole;
-      set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, n0, nt, pl.whole, pl.pieces, ws);
+      cl_kernel k = variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, pl.th == 64 ? "gemm_d64" : "gemm_d");
+      if (pl.th == 64) set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, valid, pl.whole, pl.pieces, ws);
+      else set_args(k, 0, xd_, wd, C, M, N, K, ldc, c_off, a, n0, nt, pl.whole, pl.pieces, ws);
       size_t gg = (size_t)(pl.whole + tail * pl.pieces) * 256, l1 = 256;
       run(name, k, 1, &gg, &l1);
       if (tail) {
         cl_kernel kr = variant("gemm", {}, "d_reduce");
-        int wide = ((N | ldc | c_off) & 3) == 0 && ((uintptr_t)arcz_mem_ptr(C) & 15) == 0 ? 1 : 0;
-        set_args(kr, 0, ws, C, M, N, ldc, c_off, a, wide, n0, nt, pl.whole, pl.pieces);
+        int wide = ((N | ldc | c_off) & 3) == 0 && ((uintptr_t)arcz_mem_ptr(C) & 15) == 0 ? 1 : 0, nr = pl.th == 64 ? (N + 255) / 256 : nt;
+        set_args(kr, 0, ws, C, M, N, ldc, c_off, a, wide, n0, nr, pl.whole, pl.pieces, pl.th, valid);
         size_t g[2] = {(size_t)tail * 256, 16};
         run(name, kr, 2, g, l);
       }
@@ -1066,13 +1095,14 @@ class Engine {
   // finds no memory later they are given back (arcz_mem_spare) and the matmul writes digits again or takes the int8 kernels.
   // ARCZ_DIGITS_KEEP=0 when the engine is made: never.
   void digits_keep(GpuWeight& w) {
-    const size_t bytes = (size_t)(w.N + 127) / 128 * (w.K / 32) * digit_form(w.type).wimg, total = arcz_device_mem();
+    const int tiles = (w.N + 255) / 256 * 2;  // (whole pairs, for tiles of 256 rows)
+    const size_t bytes = (size_t)tiles * (w.K / 32) * digit_form(w.type).wimg, total = arcz_device_mem();
     if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << 23)) return;
     if (arcz_spare_bytes() + bytes > total / 8 || arcz_device_mem_free() < bytes + total / 4) return;
     digits_tokens();
     if (!xd_ || !(w.digits = try_buf(bytes))) return;
     CL_CHECK(arcz_mem_spare(w.digits));
-    row_digits("keep_digits", w, 0, (w.N + 127) / 128, w.digits);
+    row_digits("keep_digits", w, 0, tiles, w.digits);
   }
   static bool digits_kept(const GpuWeight& w) { return w.digits && arcz_mem_size(w.digits) != 0; }
   // All the rows at once, or panels that give every compute unit a work-group: a launch of fewer takes as long as one that

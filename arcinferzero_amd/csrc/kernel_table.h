@@ -86,6 +86,8 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm", nullptr, "ppppppiiiiiiiii", {"QTYPE", "ACT32", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "act_digits", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits", nullptr, "ppiiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm_d64", "MN", "pppiiiiiiiiip", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm_d64", nullptr, "pppiiiiiiiiip", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_d", "MN", "pppiiiiiiiiiip", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "act_records", nullptr, "pppiiip", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "row_digits_e", nullptr, "pppziiip", {"QTYPE", nullptr}, {{nullptr, 0, false}}, 256},
@@ -93,7 +95,7 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "moe_gu_d", nullptr, "ppiipppipppp", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "moe_down_d", "MN", "ppiippp", {"NW", "MN", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "moe_down_d", nullptr, "ppiippp", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
-    {"gemm", "d_reduce", nullptr, "ppiiiiiiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "d_reduce", nullptr, "ppiiiiiiiiiiii", {nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_d", nullptr, "pppiiiiiiiiiip", {"NW", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm_simple", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},

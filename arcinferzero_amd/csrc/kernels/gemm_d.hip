@@ -208,22 +208,125 @@ __device__ inline void d_tile_of(int L, int mt, int nt, int& tm, int& tn) {
   }
 GEMM_D(NW1, 1, 0) GEMM_D(NW2, 2, 0) GEMM_D(NW3, 3, 0) GEMM_D(NW1_MN1, 1, 1)
 
-// d_reduce: the pieces' sums of the tiles from `whole` on, added in their order, out to C.  wide: rows of whole vectors.
-// grid (tiles, 16), local 256: eight rows of a tile; eight planes are loaded before the first is added.
+// ---- gemm_d64: 64 tokens x 256 rows, the same loop and the same images: half a token tile's, two row tiles'.  Where its tiles are
+// fewer: 300 tokens are five token tiles of 64 instead of three of 128, with 17408 rows 340 tiles of the same work instead of
+// 408 (Q4_K, K = 5120, 101 -> 95 us).  A tile of at most 32 tokens takes the loop for those.
+template <int NW, int MN> struct HImg {
+  using D = DImg<NW, MN>;
+  static constexpr int NB = NW == 1 ? 2 : 1, R = NW == 2 ? 4 : 3;
+  static constexpr int T = 4096, W = D::W, STAGE = NB * (T + 2 * W);  // (a block's tokens: 2 KiB, 1 KiB; sa, u)
+  static constexpr int A_MS = 1024, A8_MS = 512, S_MS = 128, U_MS = 256, DIG = 3072;
+};
+template <int NW, int MN>
+__device__ __forceinline__ void gemm_d64_body(uint8_t* lds_base, const uint8_t* __restrict__ xt, const uint8_t* __restrict__ wt,
+                                              float* __restrict__ C, int M, int N, int ldc, int c_off, int accumulate, int m0,
+                                              int n0, int valid, int nblk, int b0, int b1) {
+  asm volatile("" :: "v"((__attribute__((address_space(3))) uint8_t*)lds_base) : "memory");
+  using I = HImg<NW, MN>;
+  using D = DImg<NW, MN>;
+  static constexpr int TS = I::NB * I::T, WS = I::NB * I::W, KB = I::STAGE / 1024;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = (m0 >> 6) & 1;
+  struct {
+    const uint8_t *t0, *w0, *ts, *ws;
+    uint32_t toff, lane16, gap;  // (gap: from a step's end in the first row tile's image to its start in the second's)
+    int wave;
+    __device__ void at(int step) {
+      ts = t0 + (size_t)step * I::NB * D::T;
+      ws = w0 + (size_t)step * WS;
+    }
+    __device__ void operator()(uint32_t stage, int i) {
+      if (4 * i + 4 > KB && wave >= (KB & 3)) return;
+      asm volatile("" : "+v"(toff), "+v"(lane16));
+      if (i < I::NB) {
+        dma16(ts + i * D::T + toff, stage + wave * 1024 + i * 4096);
+      } else {
+        const uint32_t off = (wave + 4 * (i - I::NB)) * 1024 + lane16;
+        dma16(ws + (off < WS ? off : off + gap), stage + wave * 1024 + i * 4096);
+      }
+    }
+  } dma = {xt + ((size_t)(m0 >> 7) * nblk + b0) * D::T, wt + ((size_t)(n0 >> 7) * nblk + b0) * D::W, nullptr, nullptr,
+           // a wave's KiB of a block's tokens: both groups of 32's first 16 bytes, their other 8, sa and u
+           wave < 2 ? half * 2048 + wave * 1024 + lane * 16u : wave == 2 ? 4096 + half * 1024 + lane * 16u
+           : MN && lane >= 16 && lane < 48 ? D::TU + half * 512 + (lane - 16) * 16u : D::TSA + half * 256 + (lane & 15) * 16u,
+           (uint32_t)lane * 16, (uint32_t)(nblk * D::W - WS), wave};
+  const uint32_t row = TS + (wave >> 1) * WS, r = (wave & 1) * 64;
+  const DAddr o = {lane * 16u, 2048u + lane * 8u, 3072u + l32 * 4u, 3328u + g * I::T + l32 * 8u, row + (r + l32) * 16u, row + 2048u + (r + l32) * 8u,
+                   row + D::WWS + (r + lane) * 4u, row + D::WV + g * I::W + (r + l32) * 8u};
+  v16f res[2][2];
+  if (valid - m0 <= 32) {
+    d_loop32<NW, MN, I>(o, dma, wave, b1 - b0, res[0]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) res[1][0][i] = res[1][1][i] = 0.0f;
+  } else {
+    d_loop<NW, MN, I>(o, dma, wave, b1 - b0, res);
+  }
+#pragma unroll
+  for (int ms = 0; ms < 2; ++ms)
+#pragma unroll
+    for (int ns = 0; ns < 2; ++ns) {
+      const int n = n0 + wave * 64 + ns * 32 + l32, m = m0 + ms * 32 + 4 * g;
+      if (n >= N || m >= M) continue;
+      store16<true>(res[ms][ns], C + (size_t)m * ldc + c_off + n, ldc, M - m, accumulate, [](float v, int) { return v; });
+    }
+}
+// The padding rows [m, M) of 256 columns: products of zeros
+__device__ inline void d_zero_rows(float* C, int m, int M, int N, int ldc, int c_off, int accumulate, int n0) {
+  const int n = n0 + threadIdx.x;
+  if (accumulate == 1 || n >= N) return;
+  for (; m < M; ++m) C[(size_t)m * ldc + c_off + n] = 0.0f;
+}
+// gemm_d64__NW: arguments as gemm_d's, and the rows that are not padding; token tiles that hold padding alone are left out, the last
+// one's work-groups write their zeros.
+#define GEMM_D64(NAME, ...)                                                                                             \
+  extern "C" __global__ __launch_bounds__(256, 2) void gemm_d64__##NAME(                                                \
+      const uint8_t* xt, const uint8_t* wt, float* C, int M, int N, int K, int ldc, int c_off, int accumulate, int valid, \
+      int whole, int pieces, float* ws) {                                                                               \
+    using I = HImg<__VA_ARGS__>;                                                                                        \
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[I::R * I::STAGE];                                             \
+    const int mt = (valid + 63) / 64, nt = (N + 255) / 256, tail = mt * nt - whole, nsb = K >> 8;                       \
+    int L, y = 0, ny = 1;                                                                                               \
+    if ((int)blockIdx.x < whole) {                                                                                      \
+      L = d_list_of(blockIdx.x, whole);                                                                                 \
+    } else {                                                                                                            \
+      const int q = blockIdx.x - whole;                                                                                 \
+      y = q / tail;                                                                                                     \
+      ny = pieces;                                                                                                      \
+      L = whole + d_list_of(q - y * tail, tail);                                                                        \
+    }                                                                                                                   \
+    int tm, tn;                                                                                                         \
+    d_tile_of(L, mt, nt, tm, tn);                                                                                       \
+    const int m0 = tm * 64, r0 = tn * 256;                                                                              \
+    if (ny == 1 && tm == mt - 1) d_zero_rows(C, mt * 64, M, N, ldc, c_off, accumulate, r0);                             \
+    if (ny > 1) {                                                                                                       \
+      C = ws + (ptrdiff_t)((L - whole) * ny + y) * 16384 - (ptrdiff_t)(m0 * 256 + r0);                                  \
+      ldc = 256;                                                                                                        \
+      c_off = accumulate = 0;                                                                                           \
+    }                                                                                                                   \
+    gemm_d64_body<__VA_ARGS__>(lds, xt, wt, C, M, N, ldc, c_off, accumulate, m0, r0, valid, K >> 5, nsb * y / ny * 8,   \
+                               nsb * (y + 1) / ny * 8);                                                                 \
+  }
+GEMM_D64(NW1, 1, 0) GEMM_D64(NW2, 2, 0) GEMM_D64(NW3, 3, 0) GEMM_D64(NW1_MN1, 1, 1)
+
+// d_reduce: the pieces' sums of the tiles from `whole` on, added in their order, out to C.  wide: rows of whole vectors.  th: a
+// tile's token rows, 128 or 64 (of `valid` rows, padding rows as gemm_d64 writes them).  grid (tiles, 16), local 256: a sixteenth of a
+// tile; eight planes are loaded before the first is added.
 extern "C" __global__ __launch_bounds__(256) void d_reduce(const float* __restrict__ ws, float* __restrict__ C, int M, int N, int ldc,
                                                            int c_off, int accumulate, int wide, int n0, int nt, int whole,
-                                                           int pieces) {
+                                                           int pieces, int th, int valid) {
+  const int cols = 16384 / th, vecs = cols >> 2, mt = th == 64 ? (valid + 63) / 64 : (M + 127) / 128;
   int tm, tn;
-  d_tile_of(whole + blockIdx.x, (M + 127) / 128, nt, tm, tn);
-  const int r = blockIdx.y * 8 + (threadIdx.x >> 5), m = tm * 128 + r, c = threadIdx.x & 31;
+  d_tile_of(whole + blockIdx.x, mt, nt, tm, tn);
+  const int nb = n0 + tn * cols;
+  if (th == 64 && blockIdx.y == 0 && tm == mt - 1) d_zero_rows(C, mt * 64, M, N, ldc, c_off, accumulate, nb);
+  const int r = blockIdx.y * (th >> 4) + (threadIdx.x / vecs), m = tm * th + r, c = threadIdx.x & (vecs - 1);
   if (m >= M) return;
-  // (a thread: four columns next to each other, or, where a row's vectors would not be whole, 32 apart)
-  const float* p = ws + (size_t)blockIdx.x * pieces * 16384 + r * 128;
-  const int nb = n0 + tn * 128;
+  // (a thread: four columns next to each other, or, where a row's vectors would not be whole, a quarter of the row apart)
+  const float* p = ws + (size_t)blockIdx.x * pieces * 16384 + r * cols;
   v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
   auto plane = [&](int y) {
     const float* q = p + (size_t)y * 16384;
-    return wide ? *(const v4f*)(q + 4 * c) : (v4f){q[c], q[c + 32], q[c + 64], q[c + 96]};
+    return wide ? *(const v4f*)(q + 4 * c) : (v4f){q[c], q[c + vecs], q[c + 2 * vecs], q[c + 3 * vecs]};
   };
   for (int y = 0; y < pieces; y += 8) {
     v4f a[8];
@@ -244,7 +347,7 @@ extern "C" __global__ __launch_bounds__(256) void d_reduce(const float* __restri
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int n = c + 32 * i;
+    const int n = c + vecs * i;
     if (nb + n < N) cr[n] = out(s[i], accumulate ? cr[n] : 0.0f);
   }
 }

@@ -386,8 +386,8 @@ def test_switches_of_the_gemm_on_digits(rt, monkeypatch, env, digits, products):
     assert counts[0] == digits and products in (None, counts[1]), counts
 
 
-@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 128, 4096, 2048), (az.Q3_K, 200, 4099, 2304), (az.Q6_K, 256, 4100, 4096), (az.IQ3_XXS, 200, 12300, 2048),
-                                         (az.MXFP4, 65, 4225, 2048), (az.IQ4_XS, 90, 4200, 2048), (az.IQ4_NL, 300, 4097, 2304)])
+@pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 128, 4096, 2048), (az.Q3_K, 200, 4099, 2304), (az.Q6_K, 400, 4100, 4096), (az.IQ3_XXS, 200, 12300, 2048),
+                                         (az.MXFP4, 65, 4225, 2048), (az.IQ4_XS, 90, 9001, 1024), (az.IQ4_NL, 300, 16500, 1024)])
 def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     """Matrices of 2^23 values and more keep their rows' digits: no matmul writes them, and shorter chunks are multiplied on
     digits.  Given back where an allocation finds no memory -- not while a recorded list names them --, the weight is
@@ -445,11 +445,54 @@ def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     assert az.lib.arcz_spare_bytes() == spare0
 
 
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q4_0, az.Q3_K, az.Q6_K])
+@pytest.mark.parametrize("T,Mp,N,K,acc,pieces", [(17, 32, 8200, 1024, 0, 1), (33, 128, 4099, 2304, 2, 4), (150, 256, 4228, 2048, 1, 1), (193, 208, 33000, 256, 0, 1), (260, 384, 4096, 2560, 2, 3)])
+def test_gemm_on_digits_tiles_of_64_tokens(rt, monkeypatch, qtype, T, Mp, N, K, acc, pieces):
+    """Tiles of 64 tokens x 256 rows on the images of 128 and 128: at most 32 tokens and more in the last one, the second half of
+    an image of tokens, an odd number of row tiles, K in pieces and not, padding rows and the columns beside C's, the three
+    epilogues.  Against the oracle on the first and last rows, and run to run."""
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")
+    monkeypatch.setenv("ARCZ_GEMM_D64", "1")
+    if pieces > 1:
+        monkeypatch.setenv("ARCZ_Q4_SPLITK", str(pieces))
+    else:
+        monkeypatch.setenv("ARCZ_Q4_SPLITK", "0")
+    print(f"64-token tiles on digits {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc} pieces={pieces}", flush=True)
+    ldc = N + 5
+    W = make_weights(qtype, N, K, seed=41)
+    x = make_acts(T, K, seed=42, outliers=True)
+    c0 = np.random.default_rng(43).standard_normal((Mp, ldc)).astype(np.float32)
+    eng = az.Engine(Mp, K)
+    w = eng.make_weight(qtype, N, K, W)
+    xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * ldc * 4)
+    eng.quantize(xb, K, K, Mp, T)
+    ys = []
+    for _ in range(2):
+        cb.write(c0)
+        eng.matmul("test", w, Mp, cb, ldc, 0, acc)
+        ys.append(cb.read(np.float32, Mp * ldc).reshape(Mp, ldc))
+    for b in (xb, cb, w):
+        b.free()
+    eng.close()
+    y = ys[0]
+    assert np.array_equal(y.view(np.uint32), ys[1].view(np.uint32)) and np.array_equal(y[:, N:], c0[:, N:]) and np.isfinite(y).all()
+    assert np.array_equal(y[T:, :N], c0[T:, :N] if acc == 1 else np.zeros((Mp - T, N), np.float32))
+    rows = np.r_[0:200, N - 400:N]
+    Ws = np.ascontiguousarray(W.reshape(N, -1)[rows]).reshape(-1)
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, Ws, len(rows), K, aq[:T], np.ascontiguousarray(asc[:, :T]))
+    g = c0[:T, rows].astype(np.float64)
+    ref = ref + g if acc == 1 else ref * (g / (1.0 + np.exp(-g))) if acc == 2 else ref
+    assert mixed_err(y[:T, rows], ref) <= TOL
+
+
 @pytest.mark.parametrize("qtype,T,N,K,ldc,acc", [(az.Q4_0, 300, 11653, 4096, 11660, 1), (az.Q4_K, 640, 13308, 2560, 13312, 2), (az.Q6_K, 130, 17501, 4096, 17501, 0)])
-def test_gemm_on_digits_in_pieces_of_the_last_tiles(rt, qtype, T, N, K, ldc, acc):
+def test_gemm_on_digits_in_pieces_of_the_last_tiles(rt, monkeypatch, qtype, T, N, K, ldc, acc):
     """Tiles that full rounds of work-groups leave over go in pieces of K, the others whole (273, 520 and 274 tiles on a chip
     of 256 compute units): ragged rows and whole vectors, the three epilogues, run to run, the columns beside C's untouched.
     Against the oracle on the first and last rows."""
+    monkeypatch.setenv("ARCZ_GEMM_D64", "0")   # (read when an engine is made)
+    monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")
     print(f"last tiles in pieces {TYPE_NAMES[qtype]} T={T} N={N} K={K} acc={acc}", flush=True)
     Mp = (T + 127) // 128 * 128
     W = make_weights(qtype, N, K, seed=51)
