@@ -177,16 +177,20 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   // (the unit's base is a scalar; a lane adds its row of the group -- rows past the matrix: the last -- times the row
   //  stride, below 2^24, and its piece)
   const uint32_t row_stride = (uint32_t)nsb * QB, piece_off = (uint32_t)(lane % LPRW) * 16;
-  auto qload = [&](MmQ<QT>& q, int u) {  // u: the same in the whole wave, within the run
+  auto qload = [&](MmQ<QT>& q, int u, bool live) {  // u: the same in the whole wave, within the run
     const int gl = group_of(u), sb = u - gl * sbs;
     const int g0 = src.row0(gl);
     const uint8_t* base = src.raw(gl) + ((size_t)g0 * nsb + (s_begin + sb)) * QB;
+    // (past the stretch a buffer of no bytes: the load stays on every path, so that a wait counts the loads behind it, but
+    //  nothing is read.  Read again, the last unit was half of a short stretch's traffic: 8 tokens, us, 4096 x 4096 Q4_K 8.9 ->
+    //  8.0, Q4_0 8.7 -> 7.7, Q8_0 5120 x 17408 24.6 -> 22.0, 1024 x 8192 11.9 -> 10.1, IQ4_XS 8192 x 5120 12.9 -> 12.4)
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, live ? 0x7FFFFFFF : 0, 0x00027000);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
       const uint32_t rel = (uint32_t)min(i * RPI + lane / LPRW, N - 1 - g0);
       // (the main plane is read once per launch: non-temporal, so that the caches keep the tokens and the small planes
       //  -- 8 tokens, us: Q4_K 17408 x 5120 21.1 -> 20.5, 151936 x 5120 100 -> 96, Q8_0 155 -> 139)
-      q.r[i] = __builtin_nontemporal_load((const mm_u4*)(base + (__umul24(rel, row_stride) + piece_off)));
+      q.r[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(__umul24(rel, row_stride) + piece_off), 0, 2);  // (2: non-temporal)
     }
   };
   auto hload = [&](mm_u4& h, int ub) {  // the headers of units ub .. ub + 3 (past the stretch: its last)
@@ -276,7 +280,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   hload(hq1, u0 + 4);
   xload(xq, u0);
 #pragma unroll
-  for (int k = 0; k < D; ++k) qload(q[k], min(u0 + k, ulast));
+  for (int k = 0; k < D; ++k) qload(q[k], min(u0 + k, ulast), u0 + k < u1);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (!LEAN) {
 #pragma unroll
@@ -650,14 +654,13 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   };
   const int gf = group_of(min(u0, ulast));  // the stretch's first group
   v4f acc = {0.0f, 0.0f, 0.0f, 0.0f}, ph = acc, pt = acc;  // running sums; the cut group at the head, at the tail
-  // unit u: its rows out of qq through the wave's LDS, qq refilled with the unit D on (past the stretch the last unit
-  // again: the same loads on every path), the products
+  // unit u: its rows out of qq through the wave's LDS, qq refilled with the unit D on, the products
   auto sbstep = [&](MmQ<QT>& qq, int u, int j) {
     if (u < u1) {
 #pragma unroll
       for (int i = 0; i < NQ; ++i) *(mm_u4*)(WQ + wq[i]) = qq.r[i];
     }
-    qload(qq, min(u + D, ulast));
+    qload(qq, min(u + D, ulast), u + D < u1);
     if (u < u1) {
       const int gl = group_of(u), sb = u - gl * sbs;
       if constexpr (T8) {
@@ -739,6 +742,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
     batch(hq0, u + 8, u + 4);
 #pragma unroll
     for (int k = 0; k < 4; ++k) sbstep(q[k % D], u + k, k);
+    if (u + 4 >= u1) break;
     batch(hq1, u + 12, u + 8);
 #pragma unroll
     for (int k = 4; k < 8; ++k) sbstep(q[k % D], u + k, k - 4);
