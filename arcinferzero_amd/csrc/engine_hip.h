@@ -902,9 +902,12 @@ class Engine {
       // (17 - 64 rows: us at 17408 x 5120, 40 tokens, Q4_0 33 / 54, Q3_K 45 / 72, IQ4_XS 45 / 56, 5120 x 17408 34 / 67, 46 / 75, 46 /
       //  69; Q4_K 40 / 37, Q5_K 40 / 41, Q6_K 59 / 50: not)
       if (Mp <= 64 && (type == GGML_Q4_K || type == GGML_Q5_K || type == GGML_Q6_K)) return false;
-      // (these always: of 267 products, with digits 0.42 - 1.02 of the time without; IQ3_XXS 0.67 - 1.00, Q5_K 0.50 - 1.00)
+      // (these always: of 267 products, with digits 0.42 - 1.02 of the time without; Q5_K 0.50 - 1.00)
       if (type == GGML_Q3_K || type == GGML_IQ3_S || type == GGML_Q4_0 || type == GGML_MXFP4) return true;
-      if (type == GGML_IQ3_XXS ? Mp <= 128 : type == GGML_Q5_K && Mp >= 256) return true;
+      // (IQ3_XXS of few values, or of few rows, whose digits go in 16 pieces of K: not -- 9000 x 1024, 40 tokens 21 / 20, 896 x 12032, 506
+      //  tokens 50 / 47, 640 x 14336, 700 59 / 54, but 2500 103 / 110)
+      if (type == GGML_IQ3_XXS ? Mp <= 128 && (double)N * K >= (1 << 24) : type == GGML_Q5_K && Mp >= 256) return true;
+      if (type == GGML_IQ3_XXS && N <= 1024 && Mp <= 1024) return false;
       // (the others where they are priced cheaper by more than the prices' own error)
       const double d = digit_plan(digit_form(type), Mp, N, K / 256, true, rows).us;
       double i8 = 0.0;
