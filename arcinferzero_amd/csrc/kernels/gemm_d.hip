@@ -5,8 +5,8 @@
 //   J[m][n][b] = sum over the block's 32 k of x[m][k] * w[n][k], integers
 //
 // A kernel on packed weights unpacks them again for every tile of tokens, and the int8 matrix instruction leaves J as
-// int32, 16 conversions a lane.  Here both sides come as digits of four bits and a sign, written once per matmul by two
-// small kernels: x = 16 x1 + x0 and w = 256 w2 + 16 w1 + w0 (one to three digits, by the type's range).  A digit
+// int32, 16 conversions a lane.  Here both sides come as digits of four bits and a sign, written by two small kernels, the
+// tokens' once per matmul, the rows' when the weight is uploaded (or per matmul, where they are not kept): x = 16 x1 + x0 and w = 256 w2 + 16 w1 + w0 (one to three digits, by the type's range).  A digit
 // n = 0 .. 15 is the FP6 (E2M3) code n, the number n / 8 (16 is one too, 2.0, the largest top digit);
 // v_mfma_scale_f32_32x32x64_f8f6f4 takes 64 of them a row at four times the f16 rate, so a block's 32 k of x0 and of x1
 // lie in its two halves with scales 2^3 and 2^7 against the same 32 digits of w in both, and one instruction a weight
@@ -25,7 +25,7 @@
 // step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 863 TOP/s, two 651, three
 // 504 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650 and 375).
 // Q4_K and Q5_K with the min term, 17408 x 5120, us, int8 kernels and this: 8192 tokens Q4_K 2020 / 1850, 2048 544 / 470, Q5_K
-// 593 / 472, 300 110 / 100, 143 / 100.
+// 593 / 472, 300 115 / 104, 143 / 104 (weights from memory, 64-token tiles).
 // Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 136, MXFP4 183 / 135, IQ3_S
 // 201 / 147, Q3_K 293 / 182, Q6_K 277 / 234; x 4096: Q6_K 1094 / 790, IQ3_XXS 742 / 596.
 #include "digits.h"
