@@ -928,7 +928,8 @@ class Engine {
     }
   }
   // us of a product of Q4_K, Q5_K, IQ4_XS or IQ4_NL on the int8 kernels as gemm_dense launches them: pieces of K, 128 x 128 tiles
-  // (two work-groups a compute unit) or, Q4_K, 64 x 128 (three).  Fitted to eight matrices x 80 - 1500 tokens, 4 - 6 % off.
+  // (two work-groups a compute unit) or, Q4_K, 64 x 128 (three).  Fitted to eight matrices x 80 - 1500 tokens, 4 - 6 % off;
+  // Q4_K of a last round of 64 x 128 tiles from 1170 products with three engines in turn (17408 x 5120, 300 tokens: 113 us, priced 117).
   static double i8_price(uint32_t type, int Mp, int rows, int N, int nsb) {
     struct P { double base, pieces, round, ends, one, sums, out; };
     const P p = type == GGML_Q4_K ? P{9.0, 11.6, 26.0, 2.1, 0.62, 13.3e6, 14.6e6}
@@ -939,7 +940,7 @@ class Engine {
     const int full = t / (2 * cus), rest = t % (2 * cus), t64 = (rows + 63) / 64 * nt, f64 = t64 / (3 * cus), r64 = t64 % (3 * cus);
     const double c128 = full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : 1.0), c64 = 0.8 * f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.30 : r64 <= 2 * cus ? 0.48 : 0.8);
     if (type == GGML_Q4_K && c64 < 0.97 * c128)  // (gemm_dense's choice)
-      return p.base + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.5 : 0.63 + 0.37 * (r64 - cus) / (2.0 * cus))) * (19.9 * nsb / 4 + p.ends) + out;
+      return p.base + (f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.5 : r64 <= 2 * cus ? 0.68 : 1.05)) * (19.9 * nsb / 4 + p.ends) + out;
     return p.base + (full + (rest == 0 ? 0.0 : rest <= cus ? p.one : 1.0)) * (p.round * nsb / 4 + p.ends) + out;
   }
   // How a product on digits is launched: in tiles of 128 x 128 or, of a matrix whose rows' digits are kept, 64 tokens x 256 rows;
