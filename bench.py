@@ -20,10 +20,9 @@ sys.path.insert(0, ROOT)
 
 PEAK_INT8_TOPS = 5000.0   # MI355X dense int8 MFMA, published
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, published
-# HBM bytes one launch of the headline GEMM moves, from two counter runs of this script (FETCH_SIZE x 2.0 KiB read,
-# WRITE_SIZE x 1.0 KiB written, the factors calibrated on the 2 GiB copy in the same runs): 1,338,862 KiB x 2 = 2742.0 MB
-# read + 557,056 KiB = 570.4 MB written
-GEMM_HBM_BYTES_PER_LAUNCH = 3.312e9
+# HBM bytes one launch of the headline GEMM moves: a counter run (FETCH_SIZE x 2.0 KiB, the factor calibrated on a 2 GiB copy)
+# 1,678,970 KiB x 2 = 3438.5 MB read, and the output's 570.4 MB written
+GEMM_HBM_BYTES_PER_LAUNCH = 4.009e9
 
 
 def log(*a):
@@ -517,16 +516,15 @@ def main():
                    "M": M, "N": N, "K": K, "step": "quant_rows + gemm"},
         "roofline": {"bound": "mfma", "achieved": pre["kernel_tops"], "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                      "frac": pre["kernel_tops"] / PEAK_INT8_TOPS,
-                     # what the vector unit allows whatever the matrix unit does: per 32 x 32 x 32 int8 product (32
-                     # cycles of the matrix unit at the published peak) a lane converts 16 int32 sums and multiplies
-                     # them into 16 f32 accumulators with the block's scale tile: 32 vector instructions x 4 cycles
-                     "ceiling_frac": 0.25,
-                     "ceiling": "per-32 scales: 2 vector instructions (int32 -> f32, fma with the scale tile) per "
-                                "accumulator and block = 128 vector cycles per 32-cycle matrix instruction",
+                     # per 32 x 32 x 32 product (32 cycles of the matrix unit at the published int8 peak) this arithmetic
+                     # keeps a SIMD's vector unit 94 cycles (16 multiply-adds of the outputs with the scale tile and what
+                     # feeds the operands: counters) and the matrix unit 80 (digits 32, half a scale tile 32, min term 16)
+                     "ceiling_frac": 0.34,
+                     "ceiling": "per-32 scales: 94 vector cycles a 32-cycle product of the int8 peak, 80 of the matrix unit beside them",
                      "traffic": GEMM_HBM_BYTES_PER_LAUNCH,
-                     "traffic_source": "profiles/bench_hbm_traffic_fetch_write.txt (counter runs of this script; "
-                                       "a constant here, not read in this run)",
-                     "kernel": "gemm__QTYPE12_ACT321_AU3",
+                     "traffic_source": "profiles/kept_digits_kernels_counters_and_trace.txt (counter runs; a constant here, "
+                                       "not read in this run)",
+                     "kernel": "gemm_d__NW1_MN1",
                      "kernel_ms": pre["gemm_kernel_ms"], "kernel_ms_median": pre["gemm_kernel_ms_median"],
                      "kernel_ms_min": pre["gemm_kernel_ms_min"], "ops_per_launch": pre["ops"]},
         "parity_rel_err_sampled": pre["parity_rel_err"],
