@@ -1470,6 +1470,8 @@ class Engine {
   // 382 / 368 at 2000, 254 / 257 at 1000, 184 / 202 at 600; 32 x 8 of 1536 x 3072, 1000 461 / 433; 64 x 4 of 1024 x 1024 96 / 103.
   bool moe_on_digits(const MoeLayer& L, int T) const {
     if (!L.digits[1] || arcz_mem_size(L.digits[0]) == 0 || arcz_mem_size(L.digits[1]) == 0) return false;
+    // (the layer may be another engine's: this one has the records' room only if it kept a layer's digits itself)
+    if (arcz_mem_size(xr_) < (size_t)T * L.E * 2 || arcz_mem_size(sr_) < (size_t)slots_ * L.F * 2) return false;
     if (moe_digits_ > 1) return true;
     if (moe_dec_off_ || moe_mm_off_ || (moe_dec_set_ && T <= moe_dec_max_)) return false;  // (switches that name another form)
     const double slots = (double)T * L.NU / L.NE;

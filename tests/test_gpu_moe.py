@@ -566,3 +566,52 @@ def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E,
     for b in (xb, lb):
         b.free()
     eng.close()
+
+
+@pytest.mark.parametrize("own,env,rows,on_digits", [(az.Q4_0, {}, 64, True), (az.Q8_0, {}, 64, False), (az.Q4_0, {"ARCZ_MOE_DIGITS": "0"}, 64, False),
+                                                    (az.Q4_0, {"ARCZ_DIGITS_KEEP": "0"}, 64, False), (az.Q4_0, {}, 16, False)])
+def test_moe_layer_with_digits_on_another_engine(rt, monkeypatch, own, env, rows, on_digits):
+    """Engines share layers: one whose rows are kept as digits, on an engine with experts of the same shape that keeps none
+    itself -- they are Q8_0, a switch says so, its chunks are too short -- and so has no room for the records of a chunk:
+    the int8 forms, bit for bit what an engine without digits gives for its own upload; and on one that has the room: the
+    uploader's bits."""
+    NE, NU, E, F = 32, 16, 512, 512
+    T = Mp = rows
+    print(f"moe digits of another engine own={TYPE_NAMES[own]} {env} rows={rows}", flush=True)
+    Wg, Wu, Wd = make_weights(az.Q4_0, NE * F, E, seed=1), make_weights(az.Q4_0, NE * F, E, seed=2), make_weights(az.Q4_0, NE * E, F, seed=3)
+    x = make_acts(T, E, seed=4)
+    logits = np.random.default_rng(5).standard_normal((T, NE)).astype(np.float32)
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "2")   # (switches are read when an engine is made)
+    first = az.Engine(64, 512)
+    spare0 = az.lib.arcz_spare_bytes()
+    L = first.make_moe_layer(az.Q4_0, Wg, Wu, Wd, NE, NU, E, F)
+    assert az.lib.arcz_spare_bytes() > spare0
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", env.get("ARCZ_MOE_DIGITS", "2"))
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    eng = az.Engine(rows, 512)
+    Wo = Wg if own == az.Q4_0 else make_weights(own, NE * F, E, seed=6)
+    eng.make_moe_layer(own, Wo, Wo, Wo, NE, NU, E, F)   # (E == F: one tensor's bytes serve as all three)
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "0")
+    int8 = az.Engine(rows, 512)
+    Li = int8.make_moe_layer(az.Q4_0, Wg, Wu, Wd, NE, NU, E, F)
+    xb, lb = az.Runtime.from_numpy(x), az.Runtime.from_numpy(logits)
+
+    def run(e, layer):
+        ob = az.Runtime.alloc(T * E * 4).fill(0)
+        e.profile(True)
+        e.quantize(xb, E, E, Mp, T)
+        e.layer_moe(layer, lb, NE, ob, T, Mp)
+        y = ob.read(np.float32, T * E)
+        ob.free()
+        e.profile_collect()
+        return y.view(np.uint32), e.profile_get("act_records")[1]
+
+    y, records = run(eng, L)
+    want, _ = run(first, L) if on_digits else run(int8, Li)
+    assert records == (1 if on_digits else 0) and np.isfinite(y.view(np.float32)).all() and y.any()
+    assert np.array_equal(y, want)
+    for b in (xb, lb):
+        b.free()
+    for e in (eng, int8, first):   # (their layers with them)
+        e.close()
