@@ -1563,6 +1563,7 @@ class Engine {
   // usum (plain routing only): the routing launch also writes au_ = sa * S of the current chunk's rows of K values.
   void moe_route(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm, bool usum = false) {
     const int NE = L.NE, NU = L.NU, n = T * NU;
+    moe_room(L);
     if (T <= 0 || T > max_chunk || ldl < NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + NE) * 4)
       throw std::runtime_error("moe_route: router logits do not fit");
     const std::string defs = "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU) + " -DTM=" + std::to_string(tm) +
@@ -1604,7 +1605,7 @@ class Engine {
     for (int i = part; i < (part == 0 ? 2 : 3); ++i) {
       const int N = i == 2 ? E : F, K = i == 2 ? F : E;
       const GpuWeight wx = gemm_form(i == 2 ? "moe_down" : "moe_gateup", L.ex[i]);
-      const bool pre = i == 2 && L.wsv[2] && n_slots != 0;
+      const bool pre = i == 2 && L.wsv[2] && mhu_ && n_slots != 0;
       cl_kernel k = pre ? kernel("gemm", "-DQTYPE=12 -DACT32 -DMOE_TILES -DPRE=1 -DNE=" + std::to_string(NE), "gemm")
                         : gemm_kernel(wx.type, true, NE, wx.half_d);
       int M = i == 2 ? slots_ : Mp, NN = N, KK = K, ldc = N, acc = i == 1 ? 2 : 0, e0 = 0, e1 = NE, um = i == 2 ? 0 : 1,
@@ -1623,6 +1624,14 @@ class Engine {
       size_t gws[2] = {(size_t)(N + 127) / 128 * 256, (max_tiles + 7) / 8 * 8}, lws[2] = {256, 1};
       run(i == 2 ? "moe_down" : "moe_gateup", k, 2, gws, lws);
     }
+  }
+
+  // A layer may be another engine's: this one's buffers were sized for a layer of its own (moe_alloc), or not at all
+  void moe_room(const MoeLayer& L) const {
+    if (L.NE > moe_ne_ || L.NU > moe_nu_ || L.E > moe_e_ || L.F > moe_f_)
+      throw std::runtime_error("layer_moe: a layer of " + std::to_string(L.NE) + " x " + std::to_string(L.NU) + " experts of " + std::to_string(L.F) +
+                               " x " + std::to_string(L.E) + " on an engine with room for " + std::to_string(moe_ne_) + " x " + std::to_string(moe_nu_) +
+                               " of " + std::to_string(moe_f_) + " x " + std::to_string(moe_e_));
   }
 
   // Passes between the one-slot kernels, whose time goes with the pairs, and the tile GEMM, whose work-groups take about the
@@ -1732,6 +1741,7 @@ class Engine {
   // sgate = sigmoid of the router row's logit past the experts', column NE of a row of ldl > NE values).
   void layer_moe(const MoeLayer& L, cl_mem rl, int ldl, cl_mem x, int T, int Mp, cl_mem sh = nullptr) {
     const int E = L.E, F = L.F, NU = L.NU, n = T * NU;
+    moe_room(L);
     if (sh && arcz_mem_size(sh) < (size_t)T * E * 4) throw std::runtime_error("layer_moe: sh is too small");
     if (cur_T_ != T || cur_K_ != E || cur_Mp_ != Mp) throw std::runtime_error("layer_moe: the activations are not this chunk's");
     if (!cur_act32_) throw std::runtime_error("layer_moe: the expert kernels take per-32 activation scales (as the reference's, zero/kernels/gemm.cl:140-142)");
@@ -1847,7 +1857,7 @@ class Engine {
     // (the ready-made scale vectors: gate and up Q4_K with the quantizing epilogue; the token side's sa * S then comes
     //  from the routing launch, or from a launch of its own with the routing variants)
     const bool pre_gu = L.ex[0].type == GGML_Q4_K && L.ex[1].type == GGML_Q4_K && F % 128 == 0 && !moe_qfuse_off_ &&
-                        L.wsv[0] && L.wsv[1];
+                        L.wsv[0] && L.wsv[1] && mhu_;   // (none on an engine made with ARCZ_MOE_PRE=0, whose layer this need not be)
     moe_route(L, rl, ldl, T, tm, pre_gu && !L.variant());
     // the tile count is only known on the GPU: launch for the most tiles possible (zero/engine_moe.h:153)
     const size_t max_tiles = (size_t)(n + tm - 1) / tm + std::min(n, L.NE);
