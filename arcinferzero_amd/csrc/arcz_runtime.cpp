@@ -199,19 +199,28 @@ int arcz_device_cus(void) { return R.up ? R.prop.multiProcessorCount : 0; }
 size_t arcz_device_mem(void) { return R.up ? R.prop.totalGlobalMem : 0; }
 size_t arcz_device_bytes(void) { return R.device_bytes; }
 
-// Frees the spare buffers that no recorded list names; their handles stay, of size 0.
+// Frees a spare buffer, which no recorded list may name; its handle and its views' stay, of size 0.
+static bool give_back(arcz_mem* m) {
+  if (hipStreamSynchronize(R.stream) != hipSuccess || hipFree(m->ptr) != hipSuccess) return false;
+  R.device_bytes -= m->size;
+  R.spare_bytes -= m->size;
+  m->ptr = nullptr;
+  m->size = 0;
+  for (arcz_mem* v : R.mems)
+    if (v->parent == m) {
+      v->ptr = nullptr;
+      v->size = 0;
+    }
+  return true;
+}
+// ... all of them
 static bool give_back_spares() {
   bool any = false;
-  for (arcz_mem* m : R.mems) {
-    if (!m->spare || !m->ptr || arcz_mem_listed(m)) continue;
-    if (!any && hipStreamSynchronize(R.stream) != hipSuccess) return false;
-    if (hipFree(m->ptr) != hipSuccess) return any;
-    R.device_bytes -= m->size;
-    R.spare_bytes -= m->size;
-    m->ptr = nullptr;
-    m->size = 0;
-    any = true;
-  }
+  for (arcz_mem* m : R.mems)
+    if (m->spare && m->ptr && !arcz_mem_listed(m)) {
+      if (!give_back(m)) return any;
+      any = true;
+    }
   return any;
 }
 
@@ -279,6 +288,13 @@ int arcz_mem_spare(arcz_mem* m) {
   if (!m->spare) R.spare_bytes += m->size;
   m->spare = true;
   return ARCZ_OK;
+}
+int arcz_mem_give_back(arcz_mem* m) {
+  if (!m || !R.mems.count(m) || !m->spare) return fail(ARCZ_E_ARG_VALUE, "arcz_mem_give_back of a handle that is no spare buffer");
+  if (!m->ptr) return ARCZ_OK;
+  NOT_WHILE_RECORDING("arcz_mem_give_back", ARCZ_E_RECORDING);
+  if (arcz_mem_listed(m)) return fail(ARCZ_E_ARG_VALUE, "arcz_mem_give_back of a buffer that a live launch list names");
+  return give_back(m) ? ARCZ_OK : fail(ARCZ_E_DEVICE, "a spare buffer of %zu bytes is not freed", m->size);
 }
 size_t arcz_spare_bytes(void) { return R.spare_bytes; }
 size_t arcz_device_mem_free(void) {

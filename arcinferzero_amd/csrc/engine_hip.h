@@ -39,7 +39,7 @@ extern "C" void arcz_iq3xxs_grid(uint32_t* out);
 struct GpuWeight {
   uint32_t type = 0;
   int N = 0, K = 0;
-  cl_mem raw = nullptr;
+  cl_mem raw = nullptr;  // (who writes to it calls Engine::digits_drop first)
   size_t rows = 0;
   // > 0: this matrix is the output head of a model with final-logit soft-capping (the reference's lm_head_ with
   // hp.softcap, zero/engine.h:984-990): the GEMVs (1-8 tokens) write c * tanh(v / c)
@@ -1107,6 +1107,11 @@ class Engine {
     if (!xd_ || !(w.digits = try_buf(bytes))) return;
     CL_CHECK(arcz_mem_spare(w.digits));
     row_digits("keep_digits", w, 0, tiles, w.digits);
+  }
+  // ... and no more, since the planes they were written from may change: the memory is freed, the handle stays, of size 0
+  static void digits_drop(const GpuWeight& w) {
+    if (digits_kept(w) && arcz_mem_give_back(w.digits) != ARCZ_OK)
+      throw std::runtime_error(std::string("the rows' digits of this weight cannot be dropped: ") + arcz_last_error());
   }
   static bool digits_kept(const GpuWeight& w) { return w.digits && arcz_mem_size(w.digits) != 0; }
   // All the rows at once, or panels that give every compute unit a work-group: a launch of fewer takes as long as one that

@@ -44,6 +44,10 @@ arcz_weight* arcz_weight_upload_gguf(arcz_engine* e, const arcz_gguf* g, const c
 arcz_moe_layer* arcz_moe_layer_upload_gguf(arcz_engine* e, const arcz_gguf* g, const char* gate, const char* up,
                                            const char* down, int NU);
 int arcz_weight_free(arcz_engine* e, arcz_weight* w);
+/* The device planes, to read or to write: every later matmul takes what they then hold.  A second copy of the rows that the
+ * library keeps for chunks (their digits) is dropped with this call, since it would go on holding the values of the
+ * upload, and chunks take the kernels that read the planes.  NULL + arcz_engine_error() while a recorded launch list
+ * names that copy, or while one is being recorded (free the list first; or ask before anything is recorded). */
 arcz_mem* arcz_weight_raw(const arcz_weight* w);
 /* The row length the matmuls see: K, or -- Q8_0, Q4_0, IQ4_NL, MXFP4 rows of a K that is a multiple of 32 but not of
  * 256 -- K rounded up to whole superblocks, the rows having been padded with zero blocks as the reference's loader

@@ -58,8 +58,10 @@ arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes);
 int arcz_free(arcz_mem* m);
 /* Marks a buffer whose contents the caller can do without (weights laid out a second time for one of the kernels): where an
  * allocation finds no memory, all such buffers that no launch list names are freed before the out-of-memory hook is asked;
- * their handles stay live, of size 0, until arcz_free. */
+ * their handles, and their views', stay live, of size 0, until arcz_free. */
 int arcz_mem_spare(arcz_mem* m);
+/* Frees one of them now, likewise; ARCZ_E_ARG_VALUE while a live launch list names it. */
+int arcz_mem_give_back(arcz_mem* m);
 /* Bytes of such buffers held now. */
 size_t arcz_spare_bytes(void);
 size_t arcz_mem_size(const arcz_mem* m);

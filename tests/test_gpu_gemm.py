@@ -445,6 +445,55 @@ def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     assert az.lib.arcz_spare_bytes() == spare0
 
 
+@pytest.mark.parametrize("qtype,N,K", [(az.Q4_0, 4096, 2048), (az.Q4_K, 4100, 2304), (az.Q6_K, 4100, 4096)])
+def test_planes_rewritten_under_kept_digits(rt, qtype, N, K):
+    """A matrix whose rows are kept as digits, its planes asked for and rewritten: chunks multiply the new values, as the
+    passes of few tokens do -- bit for bit a weight uploaded with them whose digits were dropped too.  While a recorded
+    list names the digits the planes are not handed out, and the list goes on giving the old values."""
+    T = Mp = 512
+    print(f"planes rewritten {TYPE_NAMES[qtype]} N={N} K={K}", flush=True)
+    W = [make_weights(qtype, N, K, seed=s) for s in (71, 72)]
+    x = make_acts(T, K, seed=73)
+    eng = az.Engine(Mp, K)
+    spare0 = az.lib.arcz_spare_bytes()
+    w = eng.make_weight(qtype, N, K, W[0])
+    spare1 = az.lib.arcz_spare_bytes()
+    assert spare1 > spare0
+    xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * N * 4)
+
+    def step(v=None):
+        eng.quantize(xb, K, K, Mp, T)
+        eng.matmul("test", v or w, Mp, cb, N, 0, 0)
+
+    def out(f=step):
+        cb.fill(0xFFFFFFFF)
+        f()
+        return cb.read(np.uint32, Mp * N)
+
+    y0 = out()
+    lst = az.Runtime.record(step)
+    assert not az.lib.arcz_weight_raw(w.h) and b"launch list" in az.lib.arcz_engine_error()
+    assert az.lib.arcz_spare_bytes() == spare1 and np.array_equal(out(lst.run), y0) and np.array_equal(out(), y0)
+    lst.free()
+    az.lib.arcz_record_begin()
+    assert not az.lib.arcz_weight_raw(w.h)
+    az.lib.arcz_record_end(None)
+    raw = az.binding.Buffer(az.lib.arcz_weight_raw(w.h), owner=False)
+    assert raw.h and az.lib.arcz_spare_bytes() == spare0 and raw.size == az.planes_bytes(qtype, N, K)
+    raw.write(az.repack_planes(qtype, N, K, W[1]))
+    w1 = eng.make_weight(qtype, N, K, W[1])
+    assert az.lib.arcz_weight_raw(w1.h)
+    assert np.array_equal(out(), out(lambda: step(w1)))
+    rows = np.r_[0:200, N - 200:N]
+    y = out().view(np.float32).reshape(Mp, N)
+    aq, asc, _ = quantize_padded(x, Mp)
+    ref = orc.matmul_ref(qtype, np.ascontiguousarray(W[1].reshape(N, -1)[rows]).reshape(-1), len(rows), K, aq, asc)
+    assert np.isfinite(y).all() and rel_err_rows(y[:, rows], ref).max() <= TOL
+    for b in (w, w1, xb, cb):
+        b.free()
+    eng.close()
+
+
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q4_0, az.Q3_K, az.Q6_K])
 @pytest.mark.parametrize("T,Mp,N,K,acc,pieces", [(17, 32, 8200, 1024, 0, 1), (33, 128, 4099, 2304, 2, 4), (150, 256, 4228, 2048, 1, 1), (193, 208, 33000, 256, 0, 1), (260, 384, 4096, 2560, 2, 3)])
 def test_gemm_on_digits_tiles_of_64_tokens(rt, monkeypatch, qtype, T, Mp, N, K, acc, pieces):
