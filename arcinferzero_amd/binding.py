@@ -42,6 +42,7 @@ _sig("arcz_device_cus", _i)
 _sig("arcz_device_mem", _z)
 _sig("arcz_device_bytes", _z)
 _sig("arcz_spare_bytes", _z)
+_sig("arcz_give_back", _z, _z)
 _sig("arcz_alloc", _p, _z)
 _sig("arcz_view", _p, _p, _z, _z)
 _sig("arcz_free", _i, _p)
@@ -60,6 +61,7 @@ _sig("arcz_event_release", None, _p)
 _sig("arcz_event_record", _p)
 _sig("arcz_event_elapsed_ms", C.c_double, _p, _p)
 _sig("arcz_set_fake_oom", None, C.c_long)
+_sig("arcz_set_fake_mem", None, _z, _z)
 _sig("arcz_set_oom_hook", None, _p)
 _sig("arcz_launch_count", _u64)
 _sig("arcz_record_begin", _i)
@@ -338,6 +340,12 @@ class Runtime:
         if not h:
             raise ArczError(-4, lib.arcz_last_error().decode())
         return Buffer(h)
+
+    @staticmethod
+    def give_back(nbytes):
+        """Frees spare device memory (second copies of weights that chunks take where they are there), at least nbytes
+        of it or all, for another allocator that has run out; the bytes freed."""
+        return lib.arcz_give_back(nbytes)
 
     @staticmethod
     def from_numpy(a):

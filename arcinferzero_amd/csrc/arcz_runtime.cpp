@@ -56,6 +56,7 @@ struct Runtime {
   std::map<std::string, arcz_kernel*> kernels;
   int (*oom_hook)(void) = nullptr;
   long fake_oom = 0, allocs = 0;
+  size_t fake_total = 0, fake_free = 0;
   uint64_t launches = 0;
   std::string err;
   arcz_mem* scratch = nullptr;  // non-owning handle onto the device's static scratch array (arcz_scratch.hip)
@@ -196,7 +197,7 @@ void arcz_shutdown(void) {
 const char* arcz_last_error(void) { return R.err.c_str(); }
 const char* arcz_device_name(void) { return R.name.c_str(); }
 int arcz_device_cus(void) { return R.up ? R.prop.multiProcessorCount : 0; }
-size_t arcz_device_mem(void) { return R.up ? R.prop.totalGlobalMem : 0; }
+size_t arcz_device_mem(void) { return !R.up ? 0 : R.fake_total ? R.fake_total : R.prop.totalGlobalMem; }
 size_t arcz_device_bytes(void) { return R.device_bytes; }
 
 // Frees a spare buffer, which no recorded list may name; its handle and its views' stay, of size 0.
@@ -213,41 +214,61 @@ static bool give_back(arcz_mem* m) {
     }
   return true;
 }
-// ... all of them
-static bool give_back_spares() {
-  bool any = false;
-  for (arcz_mem* m : R.mems)
-    if (m->spare && m->ptr && !arcz_mem_listed(m)) {
-      if (!give_back(m)) return any;
-      any = true;
-    }
-  return any;
+// ... for an allocation of n bytes: the smallest that makes room for it by its size, or else the largest (further ones follow)
+static bool give_back_one(size_t n) {
+  arcz_mem* best = nullptr;
+  for (arcz_mem* m : R.mems) {
+    if (!m->spare || !m->ptr || arcz_mem_listed(m)) continue;
+    if (!best || (m->size >= n ? best->size < n || m->size < best->size : m->size > best->size)) best = m;
+  }
+  return best && give_back(best);
+}
+size_t arcz_give_back(size_t bytes) {
+  if (!R.up) return 0;
+  NOT_WHILE_RECORDING("arcz_give_back", 0);
+  const size_t before = R.spare_bytes;
+  while (before - R.spare_bytes < bytes && give_back_one(bytes - (before - R.spare_bytes))) {}
+  return before - R.spare_bytes;
 }
 
+static arcz_mem* new_mem(void* p, size_t bytes) {
+  arcz_mem* m = new arcz_mem{(char*)p, bytes, true};
+  R.mems.insert(m);
+  R.device_bytes += bytes;
+  return m;
+}
 arcz_mem* arcz_alloc(size_t bytes) {
   if (!R.up) { fail(ARCZ_E_DEVICE, "arcz_alloc before arcz_init"); return nullptr; }
   NOT_WHILE_RECORDING("arcz_alloc", nullptr);
   const size_t n = bytes < 64 ? 64 : bytes;
   void* p = nullptr;
   hipError_t e = hipSuccess;
-  ++R.allocs;
-  for (int attempt = 0; attempt <= 8; ++attempt) {
-    const bool fake = R.fake_oom > 0 && attempt == 0 && R.allocs % R.fake_oom == 0;
+  bool fake = R.fake_oom > 0 && ++R.allocs % R.fake_oom == 0;  // (once)
+  for (int attempt = 0; attempt <= 8;) {
     e = fake ? hipErrorOutOfMemory : hipMalloc(&p, n);
     if (e == hipSuccess) break;
     if (!fake) (void)hipGetLastError();
     if (e != hipErrorOutOfMemory) break;
-    if (give_back_spares()) continue;
+    fake = false;
+    if (give_back_one(n)) continue;
+    ++attempt;
     if (!(R.oom_hook && R.oom_hook())) break;  // nothing was freed: give up (clrt.h:474-487)
   }
   if (e != hipSuccess || !p) {
     fail(ARCZ_E_OOM, "allocation of %zu bytes failed: %s", n, hipGetErrorString(e));
     return nullptr;
   }
-  arcz_mem* m = new arcz_mem{(char*)p, bytes, true};
-  R.mems.insert(m);
-  R.device_bytes += bytes;
-  return m;
+  return new_mem(p, bytes);
+}
+arcz_mem* arcz_alloc_if_free(size_t bytes) {
+  if (!R.up || R.recording) return nullptr;
+  if (R.fake_oom > 0 && ++R.allocs % R.fake_oom == 0) return nullptr;
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes < 64 ? 64 : bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return new_mem(p, bytes);
 }
 
 arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes) {
@@ -299,6 +320,7 @@ int arcz_mem_give_back(arcz_mem* m) {
 size_t arcz_spare_bytes(void) { return R.spare_bytes; }
 size_t arcz_device_mem_free(void) {
   size_t free = 0, total = 0;
+  if (R.fake_total) return R.fake_free;
   return R.up && hipMemGetInfo(&free, &total) == hipSuccess ? free : 0;
 }
 int arcz_mem_listed(const arcz_mem* m) {
@@ -672,6 +694,7 @@ int arcz_list_free(arcz_list* l) {
 
 void arcz_set_oom_hook(int (*hook)(void)) { R.oom_hook = hook; }
 void arcz_set_fake_oom(long n) { R.fake_oom = n; R.allocs = 0; }
+void arcz_set_fake_mem(size_t total, size_t free) { R.fake_total = total; R.fake_free = free; }
 uint64_t arcz_launch_count(void) { return R.launches; }
 
 }  // extern "C"

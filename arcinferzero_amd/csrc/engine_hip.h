@@ -208,18 +208,11 @@ class Engine {
     mems_.push_back(m);
     return m;
   }
-  // ... or none, where memory has run out, for what a call can do without
+  // ... or none, where no memory is free, for what a call can do without
   cl_mem try_buf(size_t bytes) {
-    struct Throws {
-      bool was = zrt::oom_throws;
-      Throws() { zrt::oom_throws = true; }
-      ~Throws() { zrt::oom_throws = was; }
-    } throws;
-    try {
-      return buf(bytes);
-    } catch (const std::runtime_error&) {
-      return nullptr;
-    }
+    cl_mem m = arcz_alloc_if_free(bytes);
+    if (m) mems_.push_back(m);
+    return m;
   }
   // A recorded launch list keeps the device addresses its kernels were given, the engine's own workspaces among them:
   // a buffer that a live list names is not freed or replaced (the list would read and write freed memory).  The call
@@ -1095,14 +1088,18 @@ class Engine {
   // The rows' digits kept with the weight, so that no matmul writes them: 5 us of 4096 x 4096, 33 us of 17408 x 5120 with one
   // digit (512 tokens Q4_0 169 -> 140 us, 300 118 -> 87).  1 - 2.5 bytes a weight beside
   // the 0.4 - 0.8 of its planes: from 2^23 values on -- smaller ones are written in about a launch's time --, while such
-  // copies hold less than an eighth of the device's memory and a quarter of it stays free behind them; where an allocation
-  // finds no memory later they are given back (arcz_mem_spare) and the matmul writes digits again or takes the int8 kernels.
+  // copies hold less than an eighth of the device's memory and a quarter of it stays free behind them, first come, first
+  // served; where an allocation finds no memory later they are given back, as many as it needs (arcz_mem_spare), and the
+  // matmul writes digits again or takes the int8 kernels: they are written at uploads alone.
   // ARCZ_DIGITS_KEEP=0 when the engine is made: never.
+  static bool digits_fit(size_t bytes) {
+    const size_t total = arcz_device_mem();
+    return arcz_spare_bytes() + bytes <= total / 8 && arcz_device_mem_free() >= bytes + total / 4;
+  }
   void digits_keep(GpuWeight& w) {
     const int tiles = (w.N + 255) / 256 * 2;  // (whole pairs, for tiles of 256 rows)
-    const size_t bytes = (size_t)tiles * (w.K / 32) * digit_form(w.type).wimg, total = arcz_device_mem();
-    if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << 23)) return;
-    if (arcz_spare_bytes() + bytes > total / 8 || arcz_device_mem_free() < bytes + total / 4) return;
+    const size_t bytes = (size_t)tiles * (w.K / 32) * digit_form(w.type).wimg;
+    if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << 23) || !digits_fit(bytes)) return;
     digits_tokens();
     if (!xd_ || !(w.digits = try_buf(bytes))) return;
     CL_CHECK(arcz_mem_spare(w.digits));
@@ -1327,8 +1324,9 @@ class Engine {
     // 128 experts x 768 x 2048 at 4096 tokens: 0.80 -> 0.70 ms (gate / up 0.430 -> 0.375, down 0.256 -> 0.212: without
     // the scale registers both tile kernels fit three work-groups a compute unit) for 151 MB on top of the layer's 340.
     cl_mem wsv[3] = {nullptr, nullptr, nullptr};
-    // gate's and up's rows as digits, in the expert tiles' images (moe_d.hip), and down's; none, or given back: size 0
-    cl_mem digits[2] = {nullptr, nullptr};
+    // gate's and up's rows as digits, in the expert tiles' images (moe_d.hip), and down's, views of one buffer; none, or given
+    // back: size 0
+    cl_mem digits[2] = {nullptr, nullptr}, digits_mem = nullptr;
     bool variant() const { return escale || ebias; }
     std::string route_defs() const {
       if (ebias) {
@@ -1446,19 +1444,19 @@ class Engine {
     return rows / 256 * (K / 32) * (size_t)(f.nw * 6144 + 1024 + 2048 * f.mn);
   }
   void moe_digits_keep(MoeLayer& L) {
-    const size_t NE = L.NE, E = L.E, F = L.F, total = arcz_device_mem();
+    const size_t NE = L.NE, E = L.E, F = L.F;
     if (!digits_keep_ || !moe_digits_ || digits_env_ == 0 || moe_qfuse_off_ || !moe_pre_ || max_chunk < 32) return;
     if (L.ex[0].type != L.ex[1].type || !digit_form(L.ex[0].type).nw || !digit_form(L.ex[2].type).nw || NE * E * F < ((size_t)1 << 23)) return;
     // (32-bit offsets of the records, two bytes a value; the writing launches' grids)
     if ((size_t)max_chunk * E >= (1ull << 31) || (size_t)slots_ * F >= (1ull << 31) || NE * std::max(F / 128, E / 256) * 4 > 65535) return;
     const size_t bytes[2] = {moe_digit_bytes(L.ex[0].type, 2 * NE * F, L.E), moe_digit_bytes(L.ex[2].type, NE * E, L.F)};
-    if (arcz_spare_bytes() + bytes[0] + bytes[1] > total / 8 || arcz_device_mem_free() < bytes[0] + bytes[1] + total / 4) return;
+    if (!digits_fit(bytes[0] + bytes[1])) return;
     if (!xr_) xr_ = try_buf((size_t)max_chunk * E * 2);
     if (!sr_) sr_ = try_buf((size_t)slots_ * F * 2);
-    if (!xr_ || !sr_) return;
+    if (!xr_ || !sr_ || !(L.digits_mem = try_buf(bytes[0] + bytes[1]))) return;
+    CL_CHECK(arcz_mem_spare(L.digits_mem));  // (one buffer: half of them would serve no pass)
     for (int i = 0; i < 2; ++i) {
-      if (!(L.digits[i] = try_buf(bytes[i]))) return;
-      CL_CHECK(arcz_mem_spare(L.digits[i]));
+      L.digits[i] = view(L.digits_mem, i ? bytes[0] : 0, bytes[i]);
       const GpuWeight &a = L.ex[i ? 2 : 0], &b = L.ex[i ? 2 : 1];
       const size_t tiles = i ? a.rows / 256 : a.rows / 128;
       cl_kernel k = variant("gemm", {{"QTYPE", a.type}}, "row_digits_e");
@@ -1544,15 +1542,15 @@ class Engine {
     moe_sum(L, x, sh, T);
   }
   void free_moe_layer(MoeLayer& L) {
-    for (cl_mem m : L.digits) not_listed(m, "free_moe_layer");
+    not_listed(L.digits_mem, "free_moe_layer");
     for (int i = 0; i < 3; ++i) {
       free_weight(L.ex[i]);
       if (L.wsv[i]) release(L.wsv[i]);
       L.wsv[i] = nullptr;
     }
-    for (cl_mem& m : L.digits) {
-      if (m) release(m);
-      m = nullptr;
+    for (cl_mem* m : {&L.digits[0], &L.digits[1], &L.digits_mem}) {  // (views before their parent)
+      if (*m) release(*m);
+      *m = nullptr;
     }
     set_moe_routing(L, nullptr, nullptr, 1.0f);
   }

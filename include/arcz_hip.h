@@ -50,6 +50,8 @@ size_t arcz_device_mem_free(void);
 /* clCreateBuffer (clrt.h:744-751): device memory, at least 64 bytes, 256-byte aligned; NULL + error text on failure.
  * An allocation that fails calls the out-of-memory hook and is retried up to 8 times (clrt.h:474-487). */
 arcz_mem* arcz_alloc(size_t bytes);
+/* The same where there is room now: nothing is given back or retried for it, NULL without a message where there is none. */
+arcz_mem* arcz_alloc_if_free(size_t bytes);
 /* clCreateSubBuffer (clrt.h:752-762): a non-owning view; NULL if it would pass the parent's end. */
 arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes);
 /* clReleaseMemObject (clrt.h:763-769): waits for the stream, then frees (an owner) or forgets (a view).  The
@@ -57,11 +59,14 @@ arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes);
  * (ARCZ_E_ARG_VALUE, nothing freed). */
 int arcz_free(arcz_mem* m);
 /* Marks a buffer whose contents the caller can do without (weights laid out a second time for one of the kernels): where an
- * allocation finds no memory, all such buffers that no launch list names are freed before the out-of-memory hook is asked;
- * their handles, and their views', stay live, of size 0, until arcz_free. */
+ * arcz_alloc finds no memory, such buffers that no launch list names are freed one by one until it does, before the
+ * out-of-memory hook is asked; their handles, and their views', stay live, of size 0, until arcz_free. */
 int arcz_mem_spare(arcz_mem* m);
 /* Frees one of them now, likewise; ARCZ_E_ARG_VALUE while a live launch list names it. */
 int arcz_mem_give_back(arcz_mem* m);
+/* Frees as many of them as make `bytes` (all: SIZE_MAX), for another allocator of the process that has run out; the bytes
+ * freed. */
+size_t arcz_give_back(size_t bytes);
 /* Bytes of such buffers held now. */
 size_t arcz_spare_bytes(void);
 size_t arcz_mem_size(const arcz_mem* m);
@@ -134,6 +139,8 @@ int arcz_mem_listed(const arcz_mem* m);
 void arcz_set_oom_hook(int (*hook)(void));
 /* Test switch, the reference's ARC_FAKE_OOM (clrt.h:989-996): every n-th allocation "fails" once; 0 = off. */
 void arcz_set_fake_oom(long every_nth);
+/* Test switch: what arcz_device_mem and arcz_device_mem_free say; 0, 0 = the device's own figures. */
+void arcz_set_fake_mem(size_t total, size_t free);
 /* Launch count since start (the reference's ARC_LAUNCH_STATS, clrt.h:770-782). */
 uint64_t arcz_launch_count(void);
 

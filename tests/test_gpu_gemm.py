@@ -445,6 +445,77 @@ def test_digits_of_rows_kept_with_the_weight(rt, qtype, T, N, K):
     assert az.lib.arcz_spare_bytes() == spare0
 
 
+def test_limits_of_kept_digits(rt):
+    """Kept digits hold at most an eighth of the device's memory, over all engines, and leave a quarter of it free; a weight
+    beyond that is multiplied without them.  An allocation that finds no memory takes back as many as it needs, the
+    smallest that is large enough first, another allocator's request as many as make it; each weight's results agree
+    before and after."""
+    T = Mp = 256
+    print("limits of kept digits", flush=True)
+    sizes = [(4096, 2048), (8192, 2048), (12288, 2048)]
+    Ws = [make_weights(az.Q4_0, n, k, seed=81 + i) for i, (n, k) in enumerate(sizes)]
+    x = make_acts(T, 2048, seed=84)
+    engs = [az.Engine(Mp, 2048) for _ in range(2)]
+    xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * 12288 * 4)
+    base = az.lib.arcz_spare_bytes()
+    each = [n * k // 32 * 28 for n, k in sizes]                    # (24 bytes of digits and a scale for a block of 32)
+
+    def out(e, w):
+        e.quantize(xb, 2048, 2048, Mp, T)
+        e.profile(True)
+        e.profile_reset()
+        e.matmul("test", w, Mp, cb, w.N, 0, 0)
+        e.profile_collect()
+        return cb.read(np.float32, Mp * w.N).reshape(Mp, -1), e.profile_get("row_digits")[1] == 0 and e.profile_get("act_digits")[1] == 1
+
+    def upload(total, free, order=(0, 1, 2)):
+        az.lib.arcz_set_fake_mem(total, free)
+        try:
+            made = {i: engs[i % 2].make_weight(az.Q4_0, *sizes[i], Ws[i]) for i in order}
+        finally:
+            az.lib.arcz_set_fake_mem(0, 0)
+        return [made[i] for i in range(3)]
+
+    # the eighth holds the first and, uploaded next, the third; eight bytes fewer of memory: the second, uploaded last
+    big, eighth = 1 << 40, base + each[0] + each[2]
+    for total, kept in ((8 * eighth, [1, 0, 1]), (8 * eighth - 8, [1, 1, 0])):
+        ws = upload(total, big, (0, 2, 1))
+        assert az.lib.arcz_spare_bytes() - base == sum(b for b, k in zip(each, kept) if k)
+        for w, k in zip(ws, kept):
+            assert out(w.eng, w)[1] == bool(k)
+            w.free()
+        assert az.lib.arcz_spare_bytes() == base
+    # a quarter stays free
+    ws = upload(big, big // 4 + each[1])
+    assert az.lib.arcz_spare_bytes() - base == each[0] + each[1]
+    for w in ws:
+        w.free()
+    # taken back one by one
+    ws = upload(0, 0)
+    assert az.lib.arcz_spare_bytes() - base == sum(each)
+    ys = [out(w.eng, w)[0] for w in ws]
+    left = sum(each)
+    for need, gone in ((each[0] + 1, 1), (each[2] * 2, 2), (64, 0)):
+        az.lib.arcz_set_fake_oom(1)
+        try:
+            az.Runtime.alloc(need).free()
+        finally:
+            az.lib.arcz_set_fake_oom(0)
+        left -= each[gone]
+        assert az.lib.arcz_spare_bytes() - base == left
+    for w, y in zip(ws, ys):
+        z, kept = out(w.eng, w)
+        assert not kept and rel_err_rows(z, y).max() <= 2e-5          # (the same block sums, f32 from there on)
+        w.free()
+    ws = upload(0, 0)
+    assert az.Runtime.give_back(each[1]) == each[1] and az.Runtime.give_back(each[2] + 1) == each[0] + each[2]
+    assert az.lib.arcz_spare_bytes() == base
+    for b in (xb, cb, *ws):
+        b.free()
+    for e in engs:
+        e.close()
+
+
 @pytest.mark.parametrize("qtype,N,K", [(az.Q4_0, 4096, 2048), (az.Q4_K, 4100, 2304), (az.Q6_K, 4100, 4096)])
 def test_planes_rewritten_under_kept_digits(rt, qtype, N, K):
     """A matrix whose rows are kept as digits, its planes asked for and rewritten: chunks multiply the new values, as the
