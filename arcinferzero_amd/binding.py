@@ -136,14 +136,17 @@ _sig("arcz_gen_normal", None, _u64, _z, C.c_float, C.c_float, _p)
 _sig("arcz_gen_weights", _i, _u32, _u64, _z, _i, C.c_float, _p)
 
 
-# The calls of a forward pass: through the extension next to the library (csrc/pycall.c: the same functions, converted
-# faster), or through ctypes where it was not built for this interpreter.
+# The calls of a forward pass: through the extension next to the library (csrc/pycall.c: the same functions, plain arguments
+# converted faster), or through ctypes where it was not built for this interpreter.
+_quantize, _rmsnorm_quant, _swiglu_quant = lib.arcz_engine_quantize, lib.arcz_engine_rmsnorm_quant, lib.arcz_engine_swiglu_quant
+_matmul, _gemv_gu, _layer_moe = lib.arcz_engine_matmul, lib.arcz_engine_gemv_gu, lib.arcz_engine_layer_moe
 try:
+    from . import _pycall
+    _pycall.bind(_quantize, _rmsnorm_quant, _swiglu_quant, _matmul, _gemv_gu, _layer_moe)
     from ._pycall import gemv_gu as _gemv_gu, layer_moe as _layer_moe, matmul as _matmul, quantize as _quantize
     from ._pycall import rmsnorm_quant as _rmsnorm_quant, swiglu_quant as _swiglu_quant
 except ImportError:
-    _quantize, _rmsnorm_quant, _swiglu_quant = lib.arcz_engine_quantize, lib.arcz_engine_rmsnorm_quant, lib.arcz_engine_swiglu_quant
-    _matmul, _gemv_gu, _layer_moe = lib.arcz_engine_matmul, lib.arcz_engine_gemv_gu, lib.arcz_engine_layer_moe
+    pass
 
 
 def _check(code, engine=False):

@@ -205,3 +205,54 @@ def test_calls_of_a_pass_convert_their_arguments_alike(via):
             f(*good[:i], wrong, *good[i + 1:])
     with pytest.raises(TypeError):
         f(*good[:3])
+
+
+class _Indexable:
+    def __index__(self):
+        return 16
+
+
+@pytest.mark.parametrize("via", ["ctypes", "extension"])
+def test_calls_of_a_pass_take_what_ctypes_takes(via):
+    """... also what is no plain int, float or bytes: handles as c_void_p objects or by _as_parameter_, c_int objects,
+    numpy's integers and others with __index__ for an int (not for a handle), further arguments; a missing one is refused."""
+    import ctypes
+    f = az.lib.arcz_engine_matmul
+    if via == "extension":
+        f = pytest.importorskip("arcinferzero_amd._pycall").matmul
+    good = (None, b"m", None, 16, None, 4, 0, 0, 1)
+    as_parameter = type("H", (), {"_as_parameter_": None})()
+    for i, right in ((0, ctypes.c_void_p()), (0, as_parameter), (1, ctypes.c_char_p(b"m")), (1, None), (2, ctypes.c_void_p(0)), (3, ctypes.c_int(16)),
+                     (3, np.int64(16)), (3, np.int32(16)), (3, _Indexable()), (3, -1), (3, 2 ** 70), (4, b"c"), (5, True)):
+        assert f(*good[:i], right, *good[i + 1:]) == -100 and b"no weight" in az.lib.arcz_engine_error()
+    assert f(*good, 7) == -100
+    for i, wrong in ((3, None), (3, 16.0), (0, np.uint64(0)), (0, _Indexable()), (1, 16), (1, bytearray(b"m")), (2, object())):
+        with pytest.raises(ctypes.ArgumentError):
+            f(*good[:i], wrong, *good[i + 1:])
+    for n in range(9):
+        with pytest.raises(TypeError):
+            f(*good[:n])
+
+
+def test_extension_hands_other_arguments_to_ctypes():
+    """Which calls the extension hands on, shown by functions in the ctypes functions' place: every call with an argument
+    that is not plain (a float argument: an int, numpy's floats), with the arguments as they came."""
+    ext = pytest.importorskip("arcinferzero_amd._pycall")
+    seen = []
+    six = [getattr(az.lib, "arcz_engine_" + n) for n in ("quantize", "rmsnorm_quant", "swiglu_quant", "matmul", "gemv_gu", "layer_moe")]
+    plain = {"quantize": (None, None) + (1,) * 5, "rmsnorm_quant": (None, None, 0, None, 1, 1, 1, 1, 1e-6, None), "swiglu_quant": (None, None) + (1,) * 6,
+             "matmul": (None, b"m", None, 1, None, 1, 0, 0, 1), "gemv_gu": (None, None, None, 1, None), "layer_moe": (None, None, None, 1, None, 1, 1)}
+    try:
+        ext.bind(*[lambda *a, i=i: seen.append((i, a)) for i in range(6)])
+        for i, (name, args) in enumerate(plain.items()):
+            for k, a in enumerate(args):
+                other = [np.float32(1e-6), 1, "x"] if isinstance(a, float) else [1.5, "x"]
+                for o in other:
+                    call = args[:k] + (o,) + args[k + 1:]
+                    assert getattr(ext, name)(*call) is None and seen.pop() == (i, call) and not seen
+            assert getattr(ext, name)(*args, 1) is None and seen.pop() == (i, args + (1,))
+            assert getattr(ext, name)() is None and seen.pop() == (i, ())
+        with pytest.raises(TypeError):
+            ext.bind(*six[:5])
+    finally:
+        ext.bind(*six)
