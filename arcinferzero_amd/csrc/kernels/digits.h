@@ -106,9 +106,9 @@ __device__ inline void row_decode(const uint8_t* __restrict__ raw, const uint32_
   } else if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
     // blocks 2 q and 2 q + 1: the low and high nibbles of bytes 32 q .. 32 q + 31.  The values are taken around their middle
     // h = 8 or 16, which makes Q5_K's one digit (-16 is one) and leaves less to cancel between products and min term, v: d sc
-    // q - dmin mn = d sc (q - h) + (h d sc - dmin mn).  Off by, against 64 bits, K = 5120 and 17408, of the result's norm: Q4_K
-    // 1.2e-7 and 1.7e-7 (int8 kernels 1.6e-7, 2.4e-7), tokens with a mean of half their deviation 2.3e-7 and 3.8e-7 (2.8e-7,
-    // 3.3e-7; with the values as they are 9.7e-7, 1.8e-6), Q5_K 1.6e-7 and 2.5e-7.
+    // q - dmin mn = d sc (q - h) + (h d sc - dmin mn).  Off by, against 64 bits, 300 tokens x 2048 rows, K = 5120 and 17408 (in
+    // pieces), of the result's norm: Q4_K 1.2e-7 and 1.9e-7 (int8 kernels 1.6e-7, 2.4e-7), tokens with a mean of half their
+    // deviation 1.3e-7 and 1.9e-7 (2.7e-7, 3.2e-7); Q5_K the same.
     const PlanesQ4K pl = planes_q4k(rows_total, nsb);
     const u4v L[2] = {*(const u4v*)(raw + pl.qs + u * 128 + 32 * q), *(const u4v*)(raw + pl.qs + u * 128 + 32 * q + 16)};
     const u4v h = *(const u4v*)(raw + pl.hdr + u * 16);

@@ -404,7 +404,7 @@ struct G3ScaleRegs {
 // arithmetic, no loads into registers and no LDS stores are left in the loop.
 // PRE = 3 (Q4_K): the min term on the bf16 matrix instruction, which runs beside the vector ALU's work where the f32
 // one does not (measured in this kernel: without the min term a launch takes 13 % less, with it on the bf16
-// instruction 8 % less).  A float x is x1 + x2 + x3 exactly, three bf16 pieces by truncation; of the nine products of
+// instruction 8 % less).  A float x is x1 + x2 + x3 exactly, three bf16 pieces (split3); of the nine products of
 // two such splits the eight without x3 y3 carry everything above 2^-32 of the product and fill the eight k-slots a
 // lane half has in v_mfma_f32_32x32x16_bf16 (bf16 products are exact in f32, the sum is f32).  The pieces come
 // ready-made: au[K / 32][M] entries (u1 | u2 << 16, u3 | u3 << 16), and behind ws in wsv v[K / 32][N] entries

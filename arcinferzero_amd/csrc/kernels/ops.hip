@@ -389,7 +389,7 @@ extern "C" __global__ __launch_bounds__(256) void q4k_wscales(const uint8_t* __r
 }
 
 // The same two vectors as operands of the bf16 matrix instruction (the prefill GEMM's min term, its -DAU=3 form):
-// x = x1 + x2 + x3 exactly, each piece a bf16 by truncation (split3).  act_usum_bf16: au[b][m] = (u1 | u2 << 16,
+// x = x1 + x2 + x3 exactly, each piece a bf16 (split3).  act_usum_bf16: au[b][m] = (u1 | u2 << 16,
 // u3 | u3 << 16) of u = sa * S.  q4k_wscales_bf16: ws[b][n] = d * sc as f32, then v[b][n] = (v1 v1, v2 v2, v3 v3, v1 v2)
 // of v = -(dmin * mn), 16 bytes an entry.  Grids as act_usum and q4k_wscales.
 extern "C" __global__ __launch_bounds__(256) void act_usum_bf16(const float* __restrict__ asc, const short* __restrict__ absum,

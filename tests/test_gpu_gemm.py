@@ -739,6 +739,39 @@ def test_gemm_on_digits_with_a_minimum(rt, monkeypatch, qtype, T, Mp, N, K, acc)
 
 
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K])
+@pytest.mark.parametrize("T,N,K", [(300, 2048, 4096), (200, 768, 17408), (31, 2048, 5120)])
+def test_min_term_is_not_one_sided(rt, monkeypatch, qtype, T, N, K):
+    """The min term's pieces on the bf16 instruction, which cuts products off towards zero: tokens with a mean, against 64 bits,
+    K in one piece.  The results' errors have no mean of their own -- one piece by truncation leaves 0.5 - 3.1e-7 of the
+    results' deviation, a mean of this many errors of 2 - 7e-7 with the tokens' and rows' own in common is below 3e-8 -- and
+    their norm is no larger than with the int8 kernels, whose min term is an f32 instruction (to 2 %: other sums in f32)."""
+    print(f"min term {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    monkeypatch.setenv("ARCZ_Q4_SPLITK", "0")
+    Mp = (T + 127) // 128 * 128
+    W = make_weights(qtype, N, K, seed=61)
+    x = make_acts(T, K, seed=62, outliers=True) + np.float32(0.5)
+    aq, asc, _ = orc.quantize_act(x)
+    rb = len(W) // N
+    w64 = np.empty((N, K))
+    for n in range(N):
+        q, isc, imn, d, dmin = (a.astype(np.float64) for a in orc.decode_row_fields(qtype, W[n * rb:(n + 1) * rb], K))
+        w64[n] = q * np.repeat(isc * np.repeat(d, 2), 16) - np.repeat(imn * np.repeat(dmin, 2), 16)
+    ref = (aq * np.repeat(asc.astype(np.float64).T, 32, axis=1)) @ w64.T
+    off = {}
+    for digits, d64 in (("0", "0"), ("1", "0"), ("1", "1")):
+        monkeypatch.setenv("ARCZ_GEMM_DIGITS", digits)   # (read when an engine is made)
+        monkeypatch.setenv("ARCZ_GEMM_D64", d64)
+        eng = az.Engine(Mp, K)
+        e = run_gemm(eng, qtype, W, N, K, x, Mp)[:T] - ref
+        eng.close()
+        off[digits + d64] = np.linalg.norm(e) / np.linalg.norm(ref)
+        mean = e.mean() / ref.std()
+        print(f"  digits={digits} 64-token tiles={d64}: off {off[digits + d64]:.3g}, mean {mean:.2g}", flush=True)
+        assert abs(mean) <= 3e-8
+    assert max(off["10"], off["11"]) <= 1.02 * off["00"]
+
+
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K])
 def test_gemm_on_digits_with_a_minimum_exact(rt, monkeypatch, qtype):
     """... and exact where all is whole: scale and minimum one, random sub-scales and values, a token one block of values at
     the ends of the range; the largest products are 63 x 31 x 32 x 128 < 2^23."""
