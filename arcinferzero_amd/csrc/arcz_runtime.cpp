@@ -223,6 +223,15 @@ static bool give_back_one(size_t n) {
   }
   return best && give_back(best);
 }
+// Whether an allocation of n bytes has room in what is free and what can be given back: where it has none, nothing is given
+// back for it.
+static bool spares_make_room(size_t n) {
+  size_t room = 0, free = R.fake_free, total = 0;
+  if (!R.fake_total && hipMemGetInfo(&free, &total) != hipSuccess) return true;
+  for (arcz_mem* m : R.mems)
+    if (m->spare && m->ptr && !arcz_mem_listed(m)) room += m->size;
+  return n <= free + room;
+}
 size_t arcz_give_back(size_t bytes) {
   if (!R.up) return 0;
   NOT_WHILE_RECORDING("arcz_give_back", 0);
@@ -250,7 +259,7 @@ arcz_mem* arcz_alloc(size_t bytes) {
     if (!fake) (void)hipGetLastError();
     if (e != hipErrorOutOfMemory) break;
     fake = false;
-    if (give_back_one(n)) continue;
+    if (spares_make_room(n) && give_back_one(n)) continue;
     ++attempt;
     if (!(R.oom_hook && R.oom_hook())) break;  // nothing was freed: give up (clrt.h:474-487)
   }

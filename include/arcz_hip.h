@@ -59,8 +59,9 @@ arcz_mem* arcz_view(arcz_mem* parent, size_t offset, size_t bytes);
  * (ARCZ_E_ARG_VALUE, nothing freed). */
 int arcz_free(arcz_mem* m);
 /* Marks a buffer whose contents the caller can do without (weights laid out a second time for one of the kernels): where an
- * arcz_alloc finds no memory, such buffers that no launch list names are freed one by one until it does, before the
- * out-of-memory hook is asked; their handles, and their views', stay live, of size 0, until arcz_free. */
+ * arcz_alloc finds no memory, such buffers that no launch list names are freed one by one until it does -- none where all of
+ * them would not make room for it --, before the out-of-memory hook is asked; their handles, and their views', stay live, of
+ * size 0, until arcz_free. */
 int arcz_mem_spare(arcz_mem* m);
 /* Frees one of them now, likewise; ARCZ_E_ARG_VALUE while a live launch list names it. */
 int arcz_mem_give_back(arcz_mem* m);

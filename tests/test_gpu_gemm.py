@@ -516,6 +516,37 @@ def test_limits_of_kept_digits(rt):
         e.close()
 
 
+def test_allocations_that_kept_digits_make_no_room_for(rt):
+    """A request that is larger than what is free and what kept digits hold fails, and they stay; one byte fewer takes them."""
+    N, K = 4096, 2048
+    print("allocations that kept digits make no room for", flush=True)
+    eng = az.Engine(256, K)
+    spare0 = az.lib.arcz_spare_bytes()
+    ws = [eng.make_weight(az.Q4_0, N, K, make_weights(az.Q4_0, N, K, seed=91 + i)) for i in range(2)]
+    held = az.lib.arcz_spare_bytes()
+    assert held > spare0
+    with pytest.raises(az.ArczError):
+        az.Runtime.alloc(1 << 50)
+    assert az.lib.arcz_spare_bytes() == held
+    for free in (999, 1000):
+        az.lib.arcz_set_fake_mem(1 << 40, free)
+        az.lib.arcz_set_fake_oom(1)   # (every allocation finds no memory once)
+        try:
+            if free == 999:
+                with pytest.raises(az.ArczError):
+                    az.Runtime.alloc(held + 1000)
+                assert az.lib.arcz_spare_bytes() == held
+            else:
+                az.Runtime.alloc(held + 1000).free()
+                assert az.lib.arcz_spare_bytes() < held
+        finally:
+            az.lib.arcz_set_fake_oom(0)
+            az.lib.arcz_set_fake_mem(0, 0)
+    for w in ws:
+        w.free()
+    eng.close()
+
+
 @pytest.mark.parametrize("qtype,N,K", [(az.Q4_0, 4096, 2048), (az.Q4_K, 4100, 2304), (az.Q6_K, 4100, 4096)])
 def test_planes_rewritten_under_kept_digits(rt, qtype, N, K):
     """A matrix whose rows are kept as digits, its planes asked for and rewritten: chunks multiply the new values, as the
