@@ -1566,9 +1566,9 @@ class Engine {
   // usum (plain routing only): the routing launch also writes au_ = sa * S of the current chunk's rows of K values.
   void moe_route(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm, bool usum = false) {
     const int NE = L.NE, NU = L.NU, n = T * NU;
-    moe_room(L);
     if (T <= 0 || T > max_chunk || ldl < NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + NE) * 4)
       throw std::runtime_error("moe_route: router logits do not fit");
+    moe_room(L, T, true, false);
     const std::string defs = "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU) + " -DTM=" + std::to_string(tm) +
                              " -DNPART=" + std::to_string(moe_tpc_) + " -DNCH=" + std::to_string(moe_chunks(T));
     {
@@ -1629,12 +1629,16 @@ class Engine {
     }
   }
 
-  // A layer may be another engine's: this one's buffers were sized for a layer of its own (moe_alloc), or not at all
-  void moe_room(const MoeLayer& L) const {
-    if (L.NE > moe_ne_ || L.NU > moe_nu_ || L.E > moe_e_ || L.F > moe_f_)
-      throw std::runtime_error("layer_moe: a layer of " + std::to_string(L.NE) + " x " + std::to_string(L.NU) + " experts of " + std::to_string(L.F) +
-                               " x " + std::to_string(L.E) + " on an engine with room for " + std::to_string(moe_ne_) + " x " + std::to_string(moe_nu_) +
-                               " of " + std::to_string(moe_f_) + " x " + std::to_string(moe_e_));
+  // A layer may be another engine's: this one's buffers were sized for a layer of its own (moe_alloc), or not at all.  What T
+  // tokens of it take of them: routing in chunks, its counters; the experts, their inputs (of a block's scales slots_ next to each
+  // other, whatever T is) and outputs.
+  void moe_room(const MoeLayer& L, int T, bool chunks, bool experts) const {
+    const size_t n = (size_t)T * L.NU;
+    if (n > (size_t)slots_ || (chunks && (L.NE > moe_ne_ || moe_tpc_ * L.NU > 512 || (size_t)moe_chunks(T) * L.NE * 4 > arcz_mem_size(mcount_))) ||
+        (experts && (L.F > moe_f_ || n * L.E * 4 > arcz_mem_size(my_))))
+      throw std::runtime_error("layer_moe: " + std::to_string(T) + " tokens of a layer of " + std::to_string(L.NE) + " x " + std::to_string(L.NU) +
+                               " experts of " + std::to_string(L.F) + " x " + std::to_string(L.E) + " on an engine with room for " + std::to_string(max_chunk) +
+                               " of " + std::to_string(moe_ne_) + " x " + std::to_string(moe_nu_) + " of " + std::to_string(moe_f_) + " x " + std::to_string(moe_e_));
   }
 
   // Passes between the one-slot kernels, whose time goes with the pairs, and the tile GEMM, whose work-groups take about the
@@ -1744,9 +1748,9 @@ class Engine {
   // sgate = sigmoid of the router row's logit past the experts', column NE of a row of ldl > NE values).
   void layer_moe(const MoeLayer& L, cl_mem rl, int ldl, cl_mem x, int T, int Mp, cl_mem sh = nullptr) {
     const int E = L.E, F = L.F, NU = L.NU, n = T * NU;
-    moe_room(L);
     if (sh && arcz_mem_size(sh) < (size_t)T * E * 4) throw std::runtime_error("layer_moe: sh is too small");
     if (cur_T_ != T || cur_K_ != E || cur_Mp_ != Mp) throw std::runtime_error("layer_moe: the activations are not this chunk's");
+    moe_room(L, T, false, true);
     if (!cur_act32_) throw std::runtime_error("layer_moe: the expert kernels take per-32 activation scales (as the reference's, zero/kernels/gemm.cl:140-142)");
     if (arcz_mem_size(x) < (size_t)T * E * 4) throw std::runtime_error("layer_moe: x is too small");
     // A pass of 1-16 tokens (zero/engine_moe.h:86-262 has this form for 1-8): small tiles through the matrix-vector

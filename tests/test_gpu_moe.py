@@ -618,31 +618,37 @@ def test_moe_layer_with_digits_on_another_engine(rt, monkeypatch, own, env, rows
 
 
 def test_moe_layer_on_an_engine_without_room_for_it(rt, monkeypatch):
-    """An engine sizes the expert layer's buffers for the layers it made: another engine's that is larger in any count or
-    width is refused before anything is launched, also by the routing alone; one that is smaller in all of them gives its
-    uploader's bits.  A Q4_K layer with ready-made scale vectors on an engine that has no room for their sums
-    (ARCZ_MOE_PRE=0): the bits of that engine's own upload."""
-    NE, NU, E, F, T = 8, 2, 512, 512, 24
+    """An engine sizes the expert layer's buffers for the layers it made.  Passes of another engine's layer that they do not
+    hold are refused before anything is launched, the routing alone likewise; those that they do hold give the uploader's
+    bits, whatever the layer's counts and widths.  A Q4_K layer with ready-made scale vectors on an engine that has no room
+    for their sums (ARCZ_MOE_PRE=0): the bits of that engine's own upload."""
+    NE, NU, E, F = 8, 2, 512, 512
     monkeypatch.setenv("ARCZ_MOE_DIGITS", "0")
     print("moe layer on engines without room for it", flush=True)
 
     def layer(eng, ne, nu, e, f, q=az.Q4_K):
         return eng.make_moe_layer(q, make_weights(q, ne * f, e, seed=1), make_weights(q, ne * f, e, seed=2), make_weights(q, ne * e, f, seed=3), ne, nu, e, f)
 
-    def run(eng, L, t):
+    def run(eng, L, t, route=True):
+        """The layer's bits; None where it is refused.  route: whether the routing alone goes through (in chunks of tokens,
+        whatever t is, where a layer of up to 1024 pairs is routed by one work-group)."""
         xb, lb = az.Runtime.from_numpy(make_acts(t, E, seed=4)), az.Runtime.from_numpy(np.random.default_rng(5).standard_normal((t, NE)).astype(np.float32))
         ob = az.Runtime.alloc(t * E * 4).fill(0)
         try:
             eng.quantize(xb, E, E, t, t)
             launches = az.lib.arcz_launch_count()
-            try:
-                eng.layer_moe(L, lb, NE, ob, t, t)
-            except az.ArczError:
-                assert az.lib.arcz_launch_count() == launches
-                with pytest.raises(az.ArczError):
+            if route:
+                eng.moe_route(L, lb, NE, t, 16)
+            else:
+                with pytest.raises(az.ArczError, match="room for"):
                     eng.moe_route(L, lb, NE, t, 16)
                 assert az.lib.arcz_launch_count() == launches
-                raise
+            launches = az.lib.arcz_launch_count()
+            try:
+                eng.layer_moe(L, lb, NE, ob, t, t)
+            except az.ArczError as err:
+                assert "room for" in str(err) and az.lib.arcz_launch_count() == launches
+                return None
             y = ob.read(np.float32, t * E)
             assert np.isfinite(y).all() and y.any()
             return y.view(np.uint32)
@@ -650,23 +656,22 @@ def test_moe_layer_on_an_engine_without_room_for_it(rt, monkeypatch):
             for b in (xb, lb, ob):
                 b.free()
 
-    home = az.Engine(512, 768)
+    Ts = (1, 24, 400, 700)
+    home = az.Engine(768, 768)
     L = layer(home, NE, NU, E, F)
-    want = {t: run(home, L, t) for t in (1, T, 400)}
-    for dims in (None, (NE - 4, NU, E, F), (NE, NU - 1, E, F), (NE, NU, E - 256, F), (NE, NU, E, F - 256)):
-        eng = az.Engine(512, 768)
+    want = {t: run(home, L, t) for t in Ts}
+    #       the engine's own layer         tokens that it holds of this one, and that are routed alone
+    for dims, held, routed in ((None, (), ()), ((NE - 4, NU, E, F), (1, 24), ()), ((NE, NU - 1, E, F), (1, 24), ()),
+                               ((NE, NU, E - 256, F), (1, 24), Ts), ((NE, NU, E, F - 256), (), Ts), ((2 * NE, NU + 1, E, F + 256), Ts, Ts)):
+        eng = az.Engine(768, 768)
         if dims:
             layer(eng, *dims)
-        with pytest.raises(az.ArczError, match="room for"):
-            run(eng, L, T)
+        for t in Ts:
+            y = run(eng, L, t, t in routed)
+            assert np.array_equal(y, want[t]) if t in held else y is None, (dims, t)
         eng.close()
-    eng = az.Engine(512, 768)
-    layer(eng, 2 * NE, NU + 1, E, F + 256)
-    for t in want:
-        assert np.array_equal(run(eng, L, t), want[t])
-    eng.close()
     monkeypatch.setenv("ARCZ_MOE_PRE", "0")
-    eng = az.Engine(512, 768)
+    eng = az.Engine(768, 768)
     own = layer(eng, NE, NU, E, F)
     assert np.array_equal(run(eng, L, 400), run(eng, own, 400))
     eng.close()
