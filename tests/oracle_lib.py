@@ -70,6 +70,16 @@ def decode_row_fields(qtype, row, K):
     return q, isc, imn, d, dmin
 
 
+def dequant_rows64(qtype, W, N, K):
+    """GGUF rows -> f64 [N][K], exact (d * sc and dmin * mn of an f16 and at most eight bits each, times q)."""
+    rb = len(W) // N
+    out = np.empty((N, K))
+    for n in range(N):
+        q, isc, imn, d, dmin = (a.astype(np.float64) for a in decode_row_fields(qtype, W[n * rb:(n + 1) * rb], K))
+        out[n] = q * np.repeat(isc * np.repeat(d, 2), 16) - np.repeat(imn * np.repeat(dmin, 2), 16)
+    return out
+
+
 def quantize_act(x, act32=True, lib=None):
     """f32 [M][K] -> aq int8 [M][K], asc f32 [K/B][M], absum int16 [K/16][M]."""
     x = np.ascontiguousarray(x, dtype=np.float32)

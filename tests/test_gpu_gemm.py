@@ -614,14 +614,19 @@ def test_gemm_on_digits_tiles_of_64_tokens(rt, monkeypatch, qtype, T, Mp, N, K, 
     x = make_acts(T, K, seed=42, outliers=True)
     c0 = np.random.default_rng(43).standard_normal((Mp, ldc)).astype(np.float32)
     eng = az.Engine(Mp, K)
+    spare0 = az.lib.arcz_spare_bytes()
     w = eng.make_weight(qtype, N, K, W)
+    assert az.lib.arcz_spare_bytes() > spare0   # (kept digits: the switch then names these tiles alone)
     xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(Mp * ldc * 4)
     eng.quantize(xb, K, K, Mp, T)
     ys = []
+    eng.profile(True)
     for _ in range(2):
         cb.write(c0)
         eng.matmul("test", w, Mp, cb, ldc, 0, acc)
         ys.append(cb.read(np.float32, Mp * ldc).reshape(Mp, ldc))
+    eng.profile_collect()
+    assert eng.profile_get("act_digits")[1] == 2
     for b in (xb, cb, w):
         b.free()
     eng.close()
@@ -750,8 +755,8 @@ def test_gemm_on_digits_block_sums_exact(rt, monkeypatch, qtype, T, N):
 def test_gemm_on_digits_with_a_minimum(rt, monkeypatch, qtype, T, Mp, N, K, acc):
     """Q4_K and Q5_K on digits: the values around their middle in one digit, the min term with what that leaves on the bf16
     instruction; K shared out and not, ragged last tiles, the three epilogues.  Tokens with a mean, where products and min
-    term are both large: against 64 bits the result is no further off than the int8 kernels' (measured 1.1 - 2.3e-7 of its
-    norm, theirs 1.6 - 2.9e-7)."""
+    term are both large, against 64 bits (measured up to 2.3e-7 of the result's norm; test_min_term_is_not_one_sided has the
+    comparison with the int8 kernels)."""
     monkeypatch.setenv("ARCZ_GEMM_DIGITS", "1")
     print(f"digits with a minimum {TYPE_NAMES[qtype]} T={T} Mp={Mp} N={N} K={K} acc={acc}", flush=True)
     W = make_weights(qtype, N, K, seed=63)
@@ -782,12 +787,7 @@ def test_min_term_is_not_one_sided(rt, monkeypatch, qtype, T, N, K):
     W = make_weights(qtype, N, K, seed=61)
     x = make_acts(T, K, seed=62, outliers=True) + np.float32(0.5)
     aq, asc, _ = orc.quantize_act(x)
-    rb = len(W) // N
-    w64 = np.empty((N, K))
-    for n in range(N):
-        q, isc, imn, d, dmin = (a.astype(np.float64) for a in orc.decode_row_fields(qtype, W[n * rb:(n + 1) * rb], K))
-        w64[n] = q * np.repeat(isc * np.repeat(d, 2), 16) - np.repeat(imn * np.repeat(dmin, 2), 16)
-    ref = (aq * np.repeat(asc.astype(np.float64).T, 32, axis=1)) @ w64.T
+    ref = (aq * np.repeat(asc.astype(np.float64).T, 32, axis=1)) @ orc.dequant_rows64(qtype, W, N, K).T
     off = {}
     for digits, d64 in (("0", "0"), ("1", "0"), ("1", "1")):
         monkeypatch.setenv("ARCZ_GEMM_DIGITS", digits)   # (read when an engine is made)
@@ -829,6 +829,51 @@ def test_gemm_on_digits_with_a_minimum_exact(rt, monkeypatch, qtype):
         b.free()
     eng.close()
     assert np.array_equal(y, (aq.astype(np.float64) @ wi.T).astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype,N,K", [(az.Q4_0, 4096, 2048), (az.Q5_K, 4100, 2304), (az.MXFP4, 4100, 4096)])
+@pytest.mark.parametrize("T,rows", [(300, 384), (70, 80)])
+def test_kept_digits_on_another_engine(rt, qtype, N, K, T, rows):
+    """Engines share weights: one whose rows are kept as digits, on an engine that uploaded none (no room for its tokens'
+    digits: the int8 kernels, bit for bit those of an upload without digits) and on one that keeps digits itself, of a
+    smaller matrix in a shorter engine: the uploader's kernels and bits."""
+    print(f"kept digits on another engine {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=101)
+    x = make_acts(T, K, seed=102, outliers=True)
+    first, plain, own = az.Engine(512, max(K, 4096)), az.Engine(rows, K), az.Engine(rows, K)
+    spare0 = az.lib.arcz_spare_bytes()
+    w = first.make_weight(qtype, N, K, W)
+    assert az.lib.arcz_spare_bytes() > spare0
+    own.make_weight(az.Q4_0, 32768, 256, make_weights(az.Q4_0, 32768, 256, seed=103))
+    w8 = first.make_weight(qtype, N, K, W)
+    assert az.lib.arcz_weight_raw(w8.h)   # (handed out: without digits from here on)
+
+    def out(e, v):
+        xb, cb = az.Runtime.from_numpy(x), az.Runtime.alloc(rows * N * 4).fill(0xFFFFFFFF)
+        e.quantize(xb, K, K, rows, T)
+        e.profile(True)
+        e.profile_reset()
+        e.matmul("test", v, rows, cb, N, 0, 0)
+        e.profile_collect()
+        e.profile(False)
+        y = cb.read(np.uint32, rows * N)
+        for b in (xb, cb):
+            b.free()
+        return y, e.profile_get("act_digits")[1], e.profile_get("row_digits")[1]
+
+    y, acts, made = out(first, w)
+    assert made == 0 and (acts == 1 or T == 70)   # (of 70 tokens a type goes by price)
+    z = out(own, w)
+    assert z[1:] == (acts, 0) and np.array_equal(z[0], y)
+    z, z8 = out(plain, w), out(plain, w8)
+    assert z[1:] == z8[1:] == (0, 0) and np.array_equal(z[0], z8[0])
+    aq, asc, _ = quantize_padded(x, rows)
+    ref = orc.matmul_ref(qtype, W, N, K, aq, asc)
+    for got in (y, z[0]):
+        got = got.view(np.float32).reshape(rows, N)
+        assert np.isfinite(got).all() and not got[T:].any() and rel_err_rows(got[:T], ref[:T]).max() <= TOL
+    for e in (own, plain, first):
+        e.close()
 
 
 @pytest.mark.parametrize("qtype,T,N,K", [(az.Q4_0, 300, 12288, 512), (az.MXFP4, 512, 8192, 256), (az.Q6_K, 1024, 7808, 512), (az.Q3_K, 300, 4224, 2560)])

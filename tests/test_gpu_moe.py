@@ -568,6 +568,54 @@ def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E,
     eng.close()
 
 
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q4_0])
+def test_moe_tiles_on_digits_against_64_bits(rt, monkeypatch, qtype):
+    """The expert tiles' sums to f32 rounding: tokens with a mean, and up's rows gate's, so that the down projection's inputs
+    have one too (g^2 / (1 + exp(-g))) and the min terms of both kernels are large.  A piece of it lost would be 7e-6 and
+    more of the rows' norm; K / 32 roundings of a sum that walks, 2^-24 each, and silu's are below 1e-6."""
+    NE, NU, E, F, T, Mp = 16, 4, 1024, 768, 100, 112
+    print(f"moe digits against 64 bits {TYPE_NAMES[qtype]}", flush=True)
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "2")            # (read when the engine is made: whatever the rule says)
+    Wg, Wd = make_weights(qtype, NE * F, E, seed=1), make_weights(qtype, NE * E, F, seed=3)
+    x = make_acts(T, E, seed=4) + np.float32(0.5)
+    logits = np.random.default_rng(5).standard_normal((T, NE)).astype(np.float32)
+    eng = az.Engine(Mp, E)
+    L = eng.make_moe_layer(qtype, Wg, Wg.copy(), Wd, NE, NU, E, F)
+    xb, lb, ob = az.Runtime.from_numpy(x), az.Runtime.from_numpy(logits), az.Runtime.alloc(T * E * 4).fill(0)
+    eng.profile(True)
+    eng.quantize(xb, E, E, Mp, T)
+    eng.layer_moe(L, lb, NE, ob, T, Mp)
+    eng.profile_collect()
+    assert eng.profile_get("act_records")[1] == 1
+    S, n = eng.moe_slots, T * NU
+    inv = eng.moe_buffer("inv").read(np.int32, n).reshape(T, NU)
+    h, yr = eng.moe_buffer("h").read(np.float32, S * F).reshape(S, F), eng.moe_buffer("y").read(np.float32, S * E).reshape(S, E)
+    hq, hsc = eng.moe_buffer("hq").read(np.int8, S * F).reshape(S, F), eng.moe_buffer("hsc").read(np.float32, S * F // 32).reshape(F // 32, S)
+    for b in (xb, lb, ob):
+        b.free()
+    L.free()
+    eng.close()
+    aq, asc, _ = orc.quantize_act(x)
+    a64 = aq * np.repeat(asc.astype(np.float64).T, 32, axis=1)
+    ids = np.argsort(-logits, axis=1, kind="stable")[:, :NU]
+    wts = np.exp(np.take_along_axis(logits, ids, 1).astype(np.float64))
+    wts /= wts.sum(axis=1, keepdims=True)
+    rbg, rbd = len(Wg) // NE, len(Wd) // NE
+    off, norm = np.zeros(2), np.zeros(2)
+    for e in range(NE):
+        t, k = np.nonzero(ids == e)
+        s = inv[t, k]
+        h64 = hq[s] * np.repeat(hsc[:, s].astype(np.float64).T, 32, axis=1)
+        g = a64[t] @ orc.dequant_rows64(qtype, Wg[e * rbg:(e + 1) * rbg], F, E).T
+        want = g * g / (1.0 + np.exp(-g)), (h64 @ orc.dequant_rows64(qtype, Wd[e * rbd:(e + 1) * rbd], E, F).T) * wts[t, k][:, None]
+        for i, got in enumerate((h[s], yr[s])):
+            off[i] += ((got - want[i]) ** 2).sum()
+            norm[i] += (want[i] ** 2).sum()
+    off = np.sqrt(off / norm)
+    print(f"  gate / up off {off[0]:.3g}, down {off[1]:.3g}", flush=True)
+    assert off.max() <= 1e-6
+
+
 @pytest.mark.parametrize("own,env,rows,on_digits", [(az.Q4_0, {}, 64, True), (az.Q8_0, {}, 64, False), (az.Q4_0, {"ARCZ_MOE_DIGITS": "0"}, 64, False),
                                                     (az.Q4_0, {"ARCZ_DIGITS_KEEP": "0"}, 64, False), (az.Q4_0, {}, 16, False)])
 def test_moe_layer_with_digits_on_another_engine(rt, monkeypatch, own, env, rows, on_digits):
