@@ -941,7 +941,7 @@ class Engine {
   // 12288, 195 -> 93 us), or those that full rounds leave over, at most 512 pieces (SPLIT_BYTES).  Priced, in us: a full round
   // (two work-groups a compute unit) by 1024 values of K and for its ends, a last round of one work-group a unit 0.64 of that
   // and from there on by its work-groups, the pieces' sums 4 us and 12 TB/s, 3 % of
-  // a product of more than a round (at the power limit of the chip their traffic costs more).  Fitted to 666 products of nine
+  // a product of more than a round (fitted; the cause is not shown).  Fitted to 666 products of nine
   // types and eight matrices, 17 - 1500 tokens, weights from memory: 5 - 6 % off.
   struct DigitPlan { int th, whole, pieces; double us; };
   DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb, bool kept, int rows) const {
@@ -2065,7 +2065,7 @@ inline std::string engine_self_check() {
           for (int k2 = 0; k2 < K; ++k2) sm += (long long)aq[(size_t)m * K + k2] * wq[(size_t)n * K + k2];
           sums[(size_t)m * N + n] = (float)sm;
         }
-      const bool on_digits = e.digit_form(type).nw != 0;  // (the rule takes longer chunks; the kernels are the same)
+      const bool on_digits = e.digit_form(type).nw != 0;  // (the rule takes longer chunks; gemm_d alone: gemm_d64 and the expert tiles share its digits and loop)
       if (on_digits) e.digits_reserve(gw);
       for (int mode = 0; mode < 3; ++mode)
         for (int digits = 0; digits < (on_digits && e.digits_room(gw, M) ? 2 : 1); ++digits) {

@@ -19,11 +19,15 @@
 // most 128, two), ws is d; the others' ws is their block scale: Q4_0, MXFP4, IQ3_S, Q4_K and
 // Q5_K are one digit, IQ3_XXS, IQ4_XS and IQ4_NL two.
 //
-// Bound by power: at 17408 x 5120 x 8192 the chip runs this kernel below 1.9 GHz, without its DMA at 2.1, and every part
-// that is taken out -- operand reads from LDS, DMA, multiply-adds -- gives back about its share of the energy, not of the
-// cycles.  Hence few bytes and few instructions per product: a wave's operands serve 64 x 64 outputs, the addresses of a
-// step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 863 TOP/s, two 651, three
-// 504 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650 and 375).
+// Bound by the matrix and the vector unit, which run beside each other only in part.  At 17408 x 5120 x 8192 a 32 x 32 x 32
+// block-tile takes a SIMD 151, 185, 233 cycles with one, two, three digits and 170 with one and a minimum, at 2.2, 1.9, 1.9
+// and 2.0 GHz; the matrix unit is busy 64, 96, 128, 80 of them, vector instructions are 83, 94, 105, 94, and waves wait 39 -
+// 44 % of their cycles.  The loop's arithmetic alone, out of registers, takes 120 of the 170 at 2.3 GHz (product 33, scale
+// tile 32, multiply-adds 50, min term 17: the f32 scale tile adds to the multiply-adds in full); the rest are operand reads
+// from LDS, DMA and the meeting.  Hence few bytes and few instructions per product: a wave's operands serve 64 x 64 outputs,
+// the addresses of a step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 968 TOP/s,
+// two 706, three 548, one and a minimum 802 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650
+// and 375).
 // Q4_K and Q5_K with the min term, 17408 x 5120, us, int8 kernels and this: 8192 tokens Q4_K 2020 / 1850, 2048 544 / 470, Q5_K
 // 593 / 472, 300 115 / 104, 143 / 104 (weights from memory, 64-token tiles).
 // Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 136, MXFP4 183 / 135, IQ3_S
@@ -116,8 +120,9 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
 ROW_DIGITS(12) ROW_DIGITS(13) ROW_DIGITS(14) ROW_DIGITS(2) ROW_DIGITS(20) ROW_DIGITS(23) ROW_DIGITS(39) ROW_DIGITS(11) ROW_DIGITS(21) ROW_DIGITS(18)
 
 // ---- gemm_d: 128 tokens x 128 rows in four waves of 64 x 64, two work-groups a compute unit.  Blocks [b0, b1), an even number.
-// (Eight waves of 32 x 64, four a SIMD, hide more waits and read each row digit from LDS twice as often: 5 - 6 % slower, at
-// 17408 x 5120 x 8192 812 against 863 TOP/s with one digit, 632 / 651 with two, 476 / 504 with three.)
+// (Eight waves of 32 x 64, four a SIMD, hide more waits and read each row digit from LDS twice as often: 5 - 6 % slower, before
+// the rows' digits were kept, at 17408 x 5120 x 8192 812 against 863 TOP/s with one digit, 632 / 651 with two, 476 / 504 with
+// three.)
 template <int NW, int MN>
 __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __restrict__ xt, const uint8_t* __restrict__ wt,
                                             float* __restrict__ C, int M, int N, int ldc, int c_off, int accumulate, int m0,

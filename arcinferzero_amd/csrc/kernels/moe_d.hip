@@ -169,7 +169,7 @@ __device__ __forceinline__ bool tile_d_sums(uint8_t* lds_base, const uint8_t* __
     _Pragma("unroll") for (int ns = 0; ns < 2; ++ns) {                                                                  \
       v16f v[2];                                                                                                        \
       _Pragma("unroll") for (int i = 0; i < 16; ++i) {                                                                  \
-        v[0][i] = few ? res[0][ns][i] : res[0][ns][i];                                                                  \
+        v[0][i] = res[0][ns][i];                                                                  \
         v[1][i] = few ? 0.0f : res[1][ns][i];                                                                           \
       }                                                                                                                 \
       store_tile64(lds, v, y, N, 0, 0, r0, nr, chunk * 256 + ns * 128, N, swt, 1);                                      \

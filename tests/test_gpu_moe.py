@@ -497,8 +497,8 @@ def test_moe_layer_upload_checks_the_tensors_byte_counts(rt):
                                                         (az.IQ4_XS, az.IQ3_XXS, 8, 2, 1024, 1024, 1, 16), (az.IQ3_S, az.MXFP4, 16, 8, 768, 768, 300, 304)])
 def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E, F, T, Mp):
     """The expert tiles on digits against the int8 forms of the same layer, one to three digits a weight, with a minimum and
-    without, gate / up and down of different types; tiles of 1 to 64 slots, experts without a token.  h to f32 rounding,
-    its int8 form bit for bit the quantizer's on that h, the down projection's rows on that int8 form against the
+    without, gate / up and down of different types; tiles of 1 to 64 slots, experts without a token.  h to 1e-3 (to
+    f32 rounding: the next test), its int8 form bit for bit the quantizer's on that h, the down projection's rows on that int8 form against the
     oracle's sums, the layer run to run; digits given back: the other forms again."""
     print(f"moe digits {TYPE_NAMES[qtype]} {TYPE_NAMES[qdown]} NE={NE} NU={NU} E={E} F={F} T={T}", flush=True)
     monkeypatch.setenv("ARCZ_MOE_DIGITS", "2")            # (read when the engine is made: whatever the rule says)
