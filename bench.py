@@ -295,7 +295,7 @@ def bench_gemm_config(az, qtype, N, K, M, launches, seed, W=None):
 
 
 def bench_moe(az, launches, ready_made=True):
-    """The MoE configuration (configs[4] of the benchmark definition): 128 experts, top-8, 4096 tokens, hidden 2048, expert FFN 768, Q4_K; the whole layer
+    """The MoE configuration: 128 experts, top-8, 4096 tokens, hidden 2048, expert FFN 768, Q4_K; the whole layer
     (route, sort, gate/up tile GEMM with SwiGLU, expert-input quantization, down tile GEMM, combine) per launch.
     ready_made=False: an engine made with ARCZ_MOE_PRE=0 (the tile kernels form their scale vectors per tile and step
     instead of taking them ready-made from 8 more bytes per 32 expert weights)."""
@@ -512,7 +512,7 @@ def main():
         "warmup": args.warmup, "settle_steps": pre["settle_steps"], "ms_per_step": pre["ms_per_step"], "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "int8 x 4-bit weights, exact block sums (FP6 digit products summed in f32, below 2^24), f32 scale application", "data": "synthetic",
         "config": {"workload": "Q4_K dense prefill GEMM: weights 17408x5120 Q4_K, activations 8192x5120 f32 "
-                               "quantized to int8 per 32 in the step, out 8192x17408 f32 (configs[1] of the benchmark definition)",
+                               "quantized to int8 per 32 in the step, out 8192x17408 f32",
                    "M": M, "N": N, "K": K, "step": "quant_rows + gemm"},
         "roofline": {"bound": "mfma", "achieved": pre["kernel_tops"], "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                      "frac": pre["kernel_tops"] / PEAK_INT8_TOPS,
