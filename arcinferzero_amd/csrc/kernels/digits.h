@@ -211,10 +211,41 @@ __device__ inline void row_decode(const uint8_t* __restrict__ raw, const uint32_
 // (T, W); o: the lane's addresses of the first.  dma.at(step), dma(stage, i): where piece i of a step, KiB wave + 4 i of its
 // stage, comes from.  Every wave is behind its last reads of LDS when it returns, its last pieces have landed.
 struct DAddr { uint32_t A16, A8, SA, U, W16, W8, WS, V; };
+// Waits for a wave's pieces of stages of KB KiB but those of the last `later` steps: KB / 4 a step.  (The first waves have one more
+// where KB / 4 is not whole, and wait for as many of the last step's too: a branch on the wave costs more, 64-token tiles of
+// Q4_K, 300 tokens x 17408 rows, 111 -> 118 us.)
+template <int KB, int later> __device__ __forceinline__ void d_wait_but() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(later * (KB / 4)) : "memory");
+}
+// The work-group's waves meet; nothing but the wait before it is waited for
+__device__ __forceinline__ void d_meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+// Brings the first AHEAD steps (the last step in the place of those past it) and waits for the first of them -- for all, if these are
+// R - 1: 300 tokens x 17408 rows, 340 work-groups, otherwise 1 % slower.
+template <class I, class DMA> __device__ __forceinline__ void d_prologue(DMA& dma, int steps) {
+  constexpr int KB = I::STAGE / 1024, FIRST = I::R - 1;
+#pragma unroll
+  for (int q = 0; q < I::AHEAD; ++q) {
+    if (q == FIRST) {  // (a stage each is on its way; the last is asked for when the first is there)
+      d_wait_but<KB, FIRST - 1>();
+      d_meet();
+    }
+    dma.at(min(q, steps - 1));
+#pragma unroll
+    for (int i = 0; i < (KB + 3) / 4; ++i) dma(q * I::STAGE, i);
+  }
+  if (I::AHEAD == FIRST) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
+}
 template <int NW, int MN, class I, class DMA>
 __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int blocks, v16f (&res)[2][2]) {
   constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, KB = STAGE / 1024, ND = (KB + 3) / 4;
-  static_assert(R == 3 || (NB == 1 && ND == 5), "the wait counts below");
+  static_assert(ND <= (NB == 2 ? 8 : 6), "the slots below carry that many pieces");
   const int lane = threadIdx.x & 63, g = lane >> 5, steps = blocks / NB;
   struct F6 { u4v lo; u2v hi; };
   F6 A[2], W[2][NW];
@@ -274,15 +305,8 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
     const u4v a = {U[ms][0], U[ms][0], U[ms][0], U[ms][1]}, b = {v11, v22, V[ns][1], V[ns][0]};
     res[ms][ns] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), res[ms][ns], 0, 0, 0);
   };
-  // ---- prologue: the first R - 1 steps on their way, the first block's operands
-#pragma unroll
-  for (int q = 0; q < R - 1; ++q) {
-    dma.at(min(q, steps - 1));
-#pragma unroll
-    for (int i = 0; i < ND; ++i) dma(q * STAGE, i);
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  // ---- prologue: the first R steps on their way (the last of them behind the first one's arrival), the first block's operands
+  d_prologue<I>(dma, steps);
   at(0);
   ldA(0, 0); ldSA(0, 0);
   ldW(0, 0); ldWS(0);
@@ -290,11 +314,14 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
   ldSA(1, 0);
   uint32_t st = 0;
   int step = 0;
-  uint32_t stf = (R - 2) * STAGE;  // (the first turn's first pieces: of a step that the prologue brought, once more)
+  uint32_t stf = (I::AHEAD - 1) * STAGE;  // (the first turn's first pieces: of a step that the prologue brought, once more)
   // Two blocks a turn, four products a block: tiles (0,0) (0,1) (1,1) (1,0), then (0,1) (0,0) (1,0) (1,1), so that the operands
   // that come free first are those the next block begins with.  A product's values are added while the next one runs; a
-  // slot also carries a piece of the loads.  The stage of the step R - 1 on is refilled behind the meeting, when no wave
-  // reads the step before any more.
+  // slot also carries a piece of the loads.  Behind a step's meeting the stage of that very step is refilled, with the step R on
+  // (AHEAD = R: the products issued before the meeting wait for the last of the step's operands, no wave reads them any
+  // more), so that pieces have R - 1 steps to arrive; or (AHEAD = R - 1) the stage of the step before.  us with the first, before in
+  // the second way: Q4_K 17408 x 5120, 8192 tokens 1847 -> 1827, the 4096-token layer of Q4_K experts 631 -> 619, the 1000-token block
+  // of Q3_K 506 -> 498; but 300 tokens of Q4_K on gemm_d64 374 -> 382.
 #pragma unroll 1
   for (int b = 0; b < blocks; b += 2) {
 #pragma unroll
@@ -321,17 +348,13 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
       // -- the step's meeting: what the waves brought for the next step lies in LDS, the step before is read
       if (NB == 2 ? p == 6 : q == 2) {
         __builtin_amdgcn_sched_barrier(0);
-        // (of four stages the step after the next may still be on its way: five pieces a wave, or four)
-        if (R == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (wave < (KB & 3)) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        d_wait_but<KB, I::AHEAD - 2>();
+        d_meet();
         __builtin_amdgcn_sched_barrier(0);
-        stf = st == 0 ? (R - 1) * STAGE : st - STAGE;
+        stf = I::AHEAD == R ? st : st == 0 ? (R - 1) * STAGE : st - STAGE;
         st = st + STAGE == R * STAGE ? 0 : st + STAGE;
         at(st);
-        dma.at(min(step + R - 1, steps - 1));
+        dma.at(min(step + I::AHEAD, steps - 1));
         ++step;
       }
       // -- loads for later
@@ -372,7 +395,6 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
 template <int NW, int MN, class I, class DMA>
 __device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int wave, int blocks, v16f (&res)[2]) {
   constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, KB = STAGE / 1024, ND = (KB + 3) / 4;
-  static_assert(R == 3 || (NB == 1 && ND == 5), "the wait counts below");
   const int g = (threadIdx.x & 63) >> 5, steps = blocks / NB;
   struct F6 { u4v lo; u2v hi; };
   F6 A[2], W[2][2][NW];
@@ -407,14 +429,7 @@ __device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int wave, int
   const int sca = g ? 134 : 130, scb = 0x008A8682;
 #pragma unroll
   for (int e = 0; e < 16; ++e) res[0][e] = res[1][e] = 0.0f;
-#pragma unroll
-  for (int q = 0; q < R - 1; ++q) {
-    dma.at(min(q, steps - 1));
-#pragma unroll
-    for (int i = 0; i < ND; ++i) dma(q * STAGE, i);
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  d_prologue<I>(dma, steps);
   load(0, 0);
   int step = 0;
 #pragma unroll 1
@@ -433,15 +448,13 @@ __device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int wave, int
         }
       if (NB == 1 || k == 1) {  // (the step's meeting, as in d_loop)
         __builtin_amdgcn_sched_barrier(0);
-        if (R == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (wave < (KB & 3)) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the step's last operands: its stage is refilled)
+        d_wait_but<KB, I::AHEAD - 2>();
+        d_meet();
         __builtin_amdgcn_sched_barrier(0);
-        const uint32_t stf = st == 0 ? (R - 1) * STAGE : st - STAGE;
+        const uint32_t stf = I::AHEAD == R ? st : st == 0 ? (R - 1) * STAGE : st - STAGE;
         st = st + STAGE == R * STAGE ? 0 : st + STAGE;
-        dma.at(min(step + R - 1, steps - 1));
+        dma.at(min(step + I::AHEAD, steps - 1));
         ++step;
         load(1 - k, 0);
 #pragma unroll

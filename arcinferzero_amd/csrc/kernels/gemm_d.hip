@@ -43,7 +43,7 @@
 // x1 | x2 << 16, x3 | x3 << 16.
 template <int NW, int MN = 0> struct DImg {
   static constexpr int NB = NW == 3 ? 1 : 2;
-  static constexpr int R = NB == 2 ? 3 : 4;  // stages in LDS
+  static constexpr int R = NB == 2 ? 3 : 4, AHEAD = R;  // stages in LDS, steps on their way
   static constexpr int T = MN ? 7680 : NB == 2 ? 6656 : 7168, W = NB == 2 ? NW * 3072 + 512 + 1024 * MN : 10240;
   static constexpr int STAGE = NB * (T + W);
   static constexpr int TSA = 6144, TU = 6656, WWS = NW * 3072, WV = WWS + 512;
@@ -218,7 +218,7 @@ GEMM_D(NW1, 1, 0) GEMM_D(NW2, 2, 0) GEMM_D(NW3, 3, 0) GEMM_D(NW1_MN1, 1, 1)
 // 408 (Q4_K, K = 5120, 101 -> 95 us).  A tile of at most 32 tokens takes the loop for those.
 template <int NW, int MN> struct HImg {
   using D = DImg<NW, MN>;
-  static constexpr int NB = NW == 1 ? 2 : 1, R = NW == 2 ? 4 : 3;
+  static constexpr int NB = NW == 1 ? 2 : 1, R = NW == 2 ? 4 : 3, AHEAD = R - 1;  // (AHEAD = R: slower, digits.h)
   static constexpr int T = 4096, W = D::W, STAGE = NB * (T + 2 * W);  // (a block's tokens: 2 KiB, 1 KiB; sa, u)
   static constexpr int A_MS = 1024, A8_MS = 512, S_MS = 128, U_MS = 256, DIG = 3072;
 };

@@ -11,7 +11,7 @@
 #include "tile64.h"
 
 template <int NW, int MN> struct EImg {
-  static constexpr int NB = NW == 1 ? 2 : 1, R = NW == 2 ? 4 : 3;
+  static constexpr int NB = NW == 1 ? 2 : 1, R = NW == 2 ? 4 : 3, AHEAD = R;
   static constexpr int T = 4096, W = NW * 6144 + 1024 + 2048 * MN;
   static constexpr int STAGE = NB * (T + W);
   static constexpr int WWS = NW * 6144, WV = WWS + 1024;
