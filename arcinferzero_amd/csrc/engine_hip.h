@@ -85,6 +85,7 @@ class Engine {
     moe_mm_off_ = moe_dec_off_ || (getenv("ARCZ_MOE_MM") && atoi(getenv("ARCZ_MOE_MM")) == 0);
     digits_env_ = getenv("ARCZ_GEMM_DIGITS") ? atoi(getenv("ARCZ_GEMM_DIGITS")) : -1;
     digits_keep_ = !(getenv("ARCZ_DIGITS_KEEP") && atoi(getenv("ARCZ_DIGITS_KEEP")) == 0);
+    q8_wide_ = getenv("ARCZ_Q8_WK") ? atoi(getenv("ARCZ_Q8_WK")) : -1;
     digits64_ = getenv("ARCZ_GEMM_D64") ? atoi(getenv("ARCZ_GEMM_D64")) : -1;
     gemm_split_ = getenv("ARCZ_GEMM_SPLIT") ? std::max(0, atoi(getenv("ARCZ_GEMM_SPLIT"))) : 0;
     moe_tmd_ = getenv("ARCZ_MOE_TMD") ? atoi(getenv("ARCZ_MOE_TMD")) : 0;
@@ -852,6 +853,7 @@ class Engine {
   int digits_env_ = -1;                                                     // ARCZ_GEMM_DIGITS (-1: by rule)
   bool digits_keep_ = true;                                                 // ARCZ_DIGITS_KEEP (0: off)
   int digits64_ = -1;                                                       // ARCZ_GEMM_D64 (-1: by price, 0: never, 1: always)
+  int q8_wide_ = -1;                                                        // ARCZ_Q8_WK (-1: by price, 0: never, 1: always)
   int gemm_split_ = 0;                                                      // ARCZ_GEMM_SPLIT
   int q4_wm_ = 0, q4_wm_min_ = 2048;                                        // ARCZ_Q4_WM (0: by rule), ARCZ_Q4_WM_MIN (of =4)
   int moe_digits_ = 1;                                                      // ARCZ_MOE_DIGITS (0: off)
@@ -1068,6 +1070,27 @@ class Engine {
     if (price) *price = least;
     return best;
   }
+  // Q8_0 in tiles of eight waves (gemm8w_body), one work-group a compute unit: the pieces of K (1: none) with the lowest price in us,
+  // or 0 where the other kernel's is no higher.  A round takes 3 us and 1.4 for each superblock of a piece, the bytes of the weight
+  // 4.6 TB/s; the other kernel's own price is up to a sixth too low, 3.75 us for its launch left out.  Of eight matrices (1024 x 4096 -
+  // 17408 x 5120) x 20 - 2048 tokens 36 of 96 are taken and none got slower, on average 10 %, by up to 19 % faster: 4096 x 4096, 512 tokens 35.3 -> 28.8
+  // us, 2048 x 2048, 700 21.4 -> 17.3, 5120 x 17408, 300 119 -> 98, 4096 x 12288, 512 86 -> 72.
+  static int q8_wide_pieces(int Mp, int m64, int N, int nsb, bool one, double other) {
+    const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)m64 * ((N + 127) / 128);
+    int best = 0;
+    double least = 0.86 * other + 3.75;
+    for (int ny = 1; ny <= 8 && (ny == 1 || (ny <= nsb / 2 && !one)); ++ny) {
+      if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
+      const double rounds = (double)((tiles * ny + cus - 1) / cus) * (3.0 + 1.4 * ((nsb + ny - 1) / ny));
+      double us = 2.0 + std::max(rounds, 272.0 * N * nsb / 4.6e6);
+      if (ny > 1) us += 3.0 + 2.0 * ny * Mp * N * 4 / 5.0e6;
+      if (us < least) {
+        best = ny;
+        least = us;
+      }
+    }
+    return best;
+  }
   // Room for the digits: an engine makes it when it uploads a weight that the rule takes.  Without it such a weight runs on
   // the int8 kernels (it may be another engine's), or in panels of as many rows as there is room for: so an upload is not
   // refused where memory has run out or where a recorded list names the room that a larger matrix would replace.
@@ -1139,12 +1162,21 @@ class Engine {
         (m64 * nt128 + cus - 1) / cus == (m64_all * nt128 + cus - 1) / cus)
       m64 = m64_all;
     const int M64 = std::min(Mp, m64 * 64);
+    static const int q8_bm = getenv("ARCZ_Q8_BM") ? atoi(getenv("ARCZ_Q8_BM")) : 0;
     // Any type, a chunk so short that its tiles are fewer than two per compute unit: K is shared out over `ny`
     // work-groups per tile, which store partial tiles in a workspace, and splitk_reduce adds the slices in order (the
     // same bits on every run) and applies c_off and the accumulate mode.  One work-group needs 75 us for K = 5120, so
     // 64 tokens x 17408 rows took 100 us whatever the tile; now 136 tiles x 3 pieces, 42 us (128 tokens: 101 -> 71 us;
     // Q8_0 4096 x 4096: 64 tokens 41 -> 19 us, 256 tokens 44 -> 35 us).  ARCZ_Q4_SPLITK=0: off, =n: n pieces.
-    if (sk_force_ != 0) {
+    // (Q8_0: pieces of the eight-wave tiles, 0: the other kernel)
+    int q8w = 0;
+    if (w.type == GGML_Q8_0 && q8_bm != 128 && gemm_split_ <= 0 && q8_wide_ != 0) {
+      double other = 0.0;
+      split_pieces(w.type, 0, Mp, m64, N, K / 256, &other);
+      q8w = q8_wide_pieces(Mp, m64, N, K / 256, sk_force_ == 0, q8_wide_ > 0 ? 1e9 : other);
+      if (sk_force_ >= 2) q8w = q8_wide_ > 0 ? std::min(sk_force_, K / 256) : 0;
+    }
+    if (sk_force_ != 0 && q8w != 1) {
       // (tiles of 64 tokens up to 64 tokens, else of 128: the pieces of all tiles together must fit the resident slots,
       //  two work-groups per compute unit: one more piece than fits costs a whole second round)
       // (Q8_0, Q6_K: their dense kernels' 64-token tiles; IQ4_XS: the register-staged body's 128-token tiles)
@@ -1159,6 +1191,7 @@ class Engine {
       int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
       const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
       if (priced) ny = split_pieces(w.type, w.half_d, Mp, m64, N, nsb);
+      if (q8w) ny = q8w;
       if (sk_force >= 2) ny = std::min(sk_force, nsb);
       // (the others from three pieces on)
       if (ny >= (priced || sk_force >= 2 ? 2 : 3)) {
@@ -1178,11 +1211,13 @@ class Engine {
           sk_ws_bytes_ = need;
           ws = sk_ws_;
         }
-        cl_kernel k = variant("gemm", {{"QTYPE", w.type}, {"ACT32", 1}, {"BM", bm}, {"BN", 128}, {"SPLITK", 1}, {w.half_d ? "HDS" : nullptr, w.half_d}}, "gemm");
+        cl_kernel k = q8w ? variant("gemm", {{"QTYPE", w.type}, {"ACT32", 1}, {"WK", 4}}, "gemm")
+                         : variant("gemm", {{"QTYPE", w.type}, {"ACT32", 1}, {"BM", bm}, {"BN", 128}, {"SPLITK", 1}, {w.half_d ? "HDS" : nullptr, w.half_d}}, "gemm");
         cl_mem unused = nullptr;
         int zero = 0, one = 1, ldw = N, s1 = nsb;
         set_args(k, 0, w.raw, unused, aq_, asc_, absum_, ws, M, N, K, ldw, zero, zero, one, zero, s1);
-        size_t gws[2] = {tiles64 * 256, (size_t)ny}, lws[2] = {256, 1};
+        const size_t wg = q8w ? 512 : 256;
+        size_t gws[2] = {tiles64 * wg, (size_t)ny}, lws[2] = {wg, 1};
         run(name, k, 2, gws, lws);
         splitk_reduce(name, ws, ny, C, M, N, ldc, c_off, a, priced && M64 < Mp ? M64 : 0);
         return;
@@ -1190,7 +1225,6 @@ class Engine {
     }
     // tiles of 128 tokens x 128 rows (or 64 x 256) for Q4_K, 64 x 128 for Q6_K and Q8_0 (whose 64-token kernel measured 1.9 x the
     // 128-token one at 17408 x 5120 x 8192 and 3 x at 4096 x 4096 x 512; ARCZ_Q8_BM=128 brings the latter back)
-    static const int q8_bm = getenv("ARCZ_Q8_BM") ? atoi(getenv("ARCZ_Q8_BM")) : 0;
     const bool q8_small = w.type == GGML_Q8_0 && q8_bm != 128;
     static const int q4_bm = getenv("ARCZ_Q4_BM") ? atoi(getenv("ARCZ_Q4_BM")) : 0;
     // Q4_K: tiles of 64 tokens x 256 rows (the same work per work-group and the same rate as 128 x 128) when the last
@@ -1262,6 +1296,7 @@ class Engine {
       return;
     }
     cl_kernel k = wm4       ? kernel("gemm", "-DQTYPE=12 -DACT32 -DAU=3 -DWM=4", "gemm")
+                  : q8w == 1 ? kernel("gemm", "-DQTYPE=8 -DACT32 -DWK=4", "gemm")
                   : q8_small ? kernel("gemm", "-DQTYPE=8 -DACT32 -DBM=64", "gemm")
                   : q4_small ? kernel("gemm", "-DQTYPE=12 -DACT32 -DBM=64 -DBN=128", "gemm")
                   : q4_wide ? kernel("gemm", "-DQTYPE=12 -DACT32 -DBM=64", "gemm")
@@ -1276,7 +1311,7 @@ class Engine {
     const int bn = q4_wide && !q4_small ? 256 : 128;
     const bool m64_only = bm == 64 && (w.type == GGML_Q6_K || q8_small);
     const size_t tiles = (size_t)(m64_only ? m64 : (Mp + bm - 1) / bm) * ((N + bn - 1) / bn);
-    const size_t wg = wm4 ? 512 : 256;
+    const size_t wg = wm4 || q8w == 1 ? 512 : 256;
     size_t gws[1] = {tiles * wg}, lws[1] = {wg};
     if (au) {
       cl_kernel ku = kernel("ops", "", au3 ? "act_usum_bf16" : "act_usum");

@@ -79,6 +79,7 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "gemm", "MOE_TILES", "ppppppiiiiippiipipi", {"QTYPE", "ACT32", "MOE_TILES", nullptr},
      {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     {"gemm", "gemm", "SPLITK", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "BM", "BN", "SPLITK", nullptr}, {{nullptr, 0, false}}, 256},
+    {"gemm", "gemm", "WK", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "WK", nullptr}, {{nullptr, 0, false}}, 512},
     {"gemm", "gemm", "BN", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "BM", "BN", nullptr}, {{nullptr, 0, false}}, 256},
     {"gemm", "gemm", "WM", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "AU", "WM", nullptr}, {{nullptr, 0, false}}, 512},
     {"gemm", "gemm", "AU", "ppppppiiiiiiiii", {"QTYPE", "ACT32", "AU", nullptr}, {{nullptr, 0, false}}, 256},

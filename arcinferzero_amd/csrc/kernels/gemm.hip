@@ -1935,15 +1935,193 @@ __device__ __forceinline__ void gemm8_body(const uint8_t* __restrict__ raw, cons
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Q8_0, dense: 64 tokens x 128 rows a work-group of eight waves, one a compute unit.  Rows and tokens lie in LDS as they are and
+// go into the products unchanged; res += (sa[m][b] * d[n][b]) * (float)I.
+//
+// The waves share out a superblock by its blocks: wave w takes 64 tokens x rows 64 (w & 1) .. of blocks w / 2 and w / 2 + 4, a quarter
+// of K, and the four quarters meet in LDS behind the loop.  So a product of as many tiles as compute units needs no pieces of K
+// in memory: 4096 x 4096, 512 tokens are 256 tiles; gemm8_body takes them in two pieces of K, with 16.8 MB of partial sums out and
+// back and a launch of their own (33.9 + 5.5 us, now 26).  A wave's operands serve 2 x 2 tiles.  Three stages of a superblock in LDS,
+// refilled by DMA behind the meeting in which every wave has read its blocks.
+// Bound by vector instructions (32 a tile and lane, conversions among them) and the f32 scale tile, beside which none run: out of
+// 200 cycles a block-tile and SIMD 98 and 42; the meetings of eight waves cost 50, the DMA 30.  2.0 us of a launch go by until the
+// first superblock is there, 2.5 behind the loop.  Many rounds of work-groups, or few superblocks, are gemm8_body's, whose
+// two or three work-groups a compute unit overlap their ends (9000 x 1024, 1000 tokens 50 us here, 40 there); the engine prices both.
+#define G8W_STAGE 53248
+#define G8W_W 16384
+#define G8W_SA 49152
+#define G8W_D 51200
+#define G8W_R 3
+typedef __amdgpu_buffer_rsrc_t g8w_rsrc;
+__device__ __forceinline__ g8w_rsrc g8w_buffer(const void* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00020000); }
+__device__ __forceinline__ void gemm8w_body(const uint8_t* __restrict__ raw, const signed char* __restrict__ aq,
+                                           const float* __restrict__ asc, float* __restrict__ C, int M, int N, int K, int ldc,
+                                           int c_off, int accumulate, int s_begin, int s_end, int m0, int rows_valid, int n0) {
+  __shared__ alignas(1024) uint8_t lds[G8W_R * G8W_STAGE];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int l32 = lane & 31, g = lane >> 5, wn = wave & 1, blk = wave >> 1;
+  const int nsb = K >> 8, steps = s_end - s_begin;
+  const PlanesQ80 pl = planes_q80((size_t)N, nsb);
+  auto token_row = [&](int r) { return r < rows_valid ? r : 0; };  // rows past the tile read its first row
+  auto row = [&](int r) { return min(r, N - 1 - n0); };
+
+  // A wave's pieces of a step: twice four rows of tokens, four times four weight rows of 256 bytes each (16-byte unit u of row r lies
+  // at u ^ r % 16), and two blocks' 64 token scales (waves 0 - 3) or twice 16 rows' scales.
+  const g8w_rsrc abuf = g8w_buffer(aq + (size_t)m0 * K + s_begin * 256), wbuf = g8w_buffer(raw + pl.qs + ((size_t)n0 * nsb + s_begin) * 256),
+                sbuf = wave < 4 ? g8w_buffer(asc + ((size_t)s_begin * 8 + 2 * wave) * M + m0) : g8w_buffer(raw + pl.d + ((size_t)n0 * nsb + s_begin) * 16);
+  const uint32_t r4 = lane >> 4, snext = wave < 4 ? 32 * M : 16;
+  uint32_t aoff[2], woff[4], soff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t r = wave * 8 + i * 4 + r4;
+    aoff[i] = (uint32_t)token_row(r) * (uint32_t)K + 16u * ((lane & 15) ^ (r & 15));
+    soff[i] = wave < 4 ? ((uint32_t)i * M + token_row(lane)) * 4u : (uint32_t)row((wave & 3) * 32 + i * 16 + r4) * (uint32_t)nsb * 16u;
+  }
+  if (wave >= 4) {  // (a row's 16 bytes by four lanes)
+    soff[0] = (uint32_t)row((wave & 3) * 32 + (lane >> 2)) * (uint32_t)nsb * 16u + (lane & 3) * 4u;
+    soff[1] = (uint32_t)row((wave & 3) * 32 + 16 + (lane >> 2)) * (uint32_t)nsb * 16u + (lane & 3) * 4u;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t r = wave * 16 + i * 4 + r4;
+    woff[i] = (uint32_t)row(r) * (uint32_t)nsb * 256u + 16u * ((lane & 15) ^ (r & 15));
+  }
+  auto dma = [&](int st, uint32_t stage, int i) {
+    auto to = [&](uint32_t at) { return (__attribute__((address_space(3))) void*)(lds + stage + at); };
+    if (i < 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to(G8W_W + wave * 4096 + i * 1024), 16, woff[i & 3], st * 256, 0, 0);
+    else if (i < 6) __builtin_amdgcn_raw_ptr_buffer_load_lds(abuf, to(wave * 2048 + (i & 1) * 1024), 16, aoff[i & 1], st * 256, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(sbuf, to(G8W_SA + wave * 512 + (i & 1) * 256), 4, soff[i & 1], st * snext, 0, 0);
+  };
+  auto meet = [&](auto later) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(8 * decltype(later)::value) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // (block blk + 4 k of the superblock: 16-byte units 2 blk + g + 8 k)
+  const uint8_t* const opa[2] = {lds + l32 * 256 + (((2 * blk + g) ^ (l32 & 15)) * 16), lds + l32 * 256 + (((2 * blk + g + 8) ^ (l32 & 15)) * 16)};
+  v4i A[2][2], W[2][2];  // [buffer][tile]
+  float saop[2];
+  uint32_t wsop[2][2];  // (f16)
+  auto ldA = [&](int k, int ms, uint32_t stage) { A[k][ms] = *(const v4i*)(opa[k] + stage + ms * 8192); };
+  auto ldW = [&](int k, int ns, uint32_t stage) { W[k][ns] = *(const v4i*)(opa[k] + stage + G8W_W + wn * 16384 + ns * 8192); };
+  auto ldS = [&](int k, uint32_t stage) {
+    saop[k] = ((const float*)(lds + stage + G8W_SA))[(blk + 4 * k) * 64 + lane];
+#pragma unroll
+    for (int ns = 0; ns < 2; ++ns) wsop[k][ns] = ((const unsigned short*)(lds + stage + G8W_D))[(wn * 64 + ns * 32 + l32) * 8 + blk + 4 * k];
+  };
+  v16f res[2][2];
+  v16i I[2];
+  v32f P[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) res[i][0][e] = res[i][1][e] = 0.0f, I[i][e] = 0;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) P[i][e] = 0.0f;
+  }
+  auto mfma_p = [&](int k, int ns) {
+    v32f z;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) z[i] = 0.0f;
+    P[ns] = __builtin_amdgcn_mfma_f32_32x32x1f32(saop[k], f16_bits_to_f32(wsop[k][ns]), z, 0, 0, 0);
+  };
+  if (steps > 0) {
+    // ---- the first steps on their way (the last step in the place of those past it), the first block's operands
+#pragma unroll
+    for (int q = 0; q < G8W_R; ++q) {
+      if (q == G8W_R - 1) meet(std::integral_constant<int, G8W_R - 2>());
+#pragma unroll
+      for (int i = 0; i < 8; ++i) dma(min(q, steps - 1), q * G8W_STAGE, i);
+    }
+    ldA(0, 0, 0); ldW(0, 0, 0); ldS(0, 0); ldA(0, 1, 0); ldW(0, 1, 0);
+    mfma_p(0, 0);
+    uint32_t stage = 0, refill = (G8W_R - 1) * G8W_STAGE;  // (the first turn's first pieces: once more)
+    int next = min(G8W_R - 1, steps - 1);
+    // Eight products a step, of two blocks, tiles (0,0) (1,0) (1,1) (0,1) of each; a product's values are added while the next one
+    // runs.  The meeting of a step: the next one has landed, every wave has this one's operands.
+#pragma unroll 1
+    for (int st = 0; st < steps; ++st) {
+      asm volatile("" : "+v"(I[1]));  // (its conversion stays here: it was made at the turn's end too)
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        const int k = p >> 2, q = p & 3, ms = q == 1 || q == 2, ns = q >> 1;
+        {
+          v16i z;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) z[i] = 0;
+          I[p & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k][ms], W[k][ns], z, 0, 0, 0);
+        }
+        if (q == 1) mfma_p(k, 1);
+        if (p == 5) {
+          __builtin_amdgcn_sched_barrier(0);
+          meet(std::integral_constant<int, G8W_R - 2>());
+          __builtin_amdgcn_sched_barrier(0);
+          refill = stage;
+          stage = stage + G8W_STAGE == G8W_R * G8W_STAGE ? 0 : stage + G8W_STAGE;
+          next = min(st + G8W_R, steps - 1);
+        }
+        if (q == 1) { ldA(k ^ 1, 0, stage); ldW(k ^ 1, 0, stage); ldS(k ^ 1, stage); }
+        if (q == 2) { ldA(k ^ 1, 1, stage); ldW(k ^ 1, 1, stage); }
+        if (q == 3) mfma_p(k ^ 1, 0);
+        const int f = (p + 3) & 7;  // (two pieces a slot, 5, 6, 7 and, one turn on, 0)
+        if (f < 4) { dma(next, refill, 2 * f); dma(next, refill, 2 * f + 1); }
+        __builtin_amdgcn_sched_barrier(0);
+        const int qp = (p + 3) & 3, mp = qp == 1 || qp == 2, np = qp >> 1;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) res[mp][np][e] = __builtin_fmaf((float)I[(p + 1) & 1][e], P[np][16 * mp + e], res[mp][np][e]);
+        asm volatile("" : "+v"(res[mp][np]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    asm volatile("" : "+v"(I[1]));  // (the last product)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) res[0][1][e] = __builtin_fmaf((float)I[1][e], P[1][e], res[0][1][e]);
+  }
+  // ---- the quarters of K meet: [4][64][128] f32 in the place of the stages, added in their order
+  meet(std::integral_constant<int, 0>());
+  float* const part = (float*)lds;
+#pragma unroll
+  for (int ms = 0; ms < 2; ++ms)
+#pragma unroll
+    for (int ns = 0; ns < 2; ++ns)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        part[(blk * 64 + ms * 32 + 8 * (e >> 2) + 4 * g + (e & 3)) * 128 + wn * 64 + ns * 32 + l32] = res[ms][ns][e];
+  __syncthreads();
+  // (a thread: four columns of every sixteenth row, in whole vectors where C's rows are such)
+  const int c = 4 * (t & 31), n = n0 + c;
+  if (n >= N) return;
+  const bool wide = ((ldc | c_off) & 3) == 0 && ((uintptr_t)C & 15) == 0 && n + 4 <= N;
+  auto put = [&](float v, float old) { return accumulate == 1 ? v + old : accumulate == 2 ? v * (old / (1.0f + __expf(-old))) : v; };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (t >> 5) + 16 * i;
+    if (r >= rows_valid) break;
+    const v4f* p = (const v4f*)(part + r * 128 + c);
+    const v4f v = ((p[0] + p[2048]) + p[2 * 2048]) + p[3 * 2048];
+    float* cp = C + (size_t)(m0 + r) * ldc + c_off + n;
+    if (wide) {
+      const v4f old = accumulate ? *(const v4f*)cp : v;
+      *(v4f*)cp = (v4f){put(v[0], old[0]), put(v[1], old[1]), put(v[2], old[2]), put(v[3], old[3])};
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < N) cp[j] = put(v[j], accumulate ? cp[j] : 0.0f);
+    }
+  }
+}
+
 // A chunk laid out for M token rows whose last ones are padding: a launch of the 64-token tiles may leave out the tiles that
 // hold nothing else (their count comes from the grid).  The padding rows' results are zeros where a product is stored or
 // multiplied in (one that is added changes nothing): the mt work-groups of a row tile write a share of them each, behind
 // their own results (Q8_0, 300 tokens x 4096 rows, K = 1024: 12.8 us; by the last tile's alone, in front of its loads, 14.4;
 // no tile left out 13.6).
 __device__ inline void zero_tail(float* C, int ldc, int c_off, int accumulate, int tm, int mt, int M, int n0, int N) {
-  const int n = n0 + (threadIdx.x & 127);
+  const int n = n0 + (threadIdx.x & 127), per = blockDim.x >> 7;
   if (accumulate == 1 || n >= N) return;
-  for (int r = mt * G6_BM + 2 * tm + (threadIdx.x >> 7); r < M; r += 2 * mt) C[(size_t)r * ldc + c_off + n] = 0.0f;
+  for (int r = mt * G6_BM + per * tm + (threadIdx.x >> 7); r < M; r += per * mt) C[(size_t)r * ldc + c_off + n] = 0.0f;
 }
 
 // Tile of work-group `id` out of mt x nt tiles.  XCDs take work-groups in turn (id % 8), each running 64 at a time:
@@ -2218,6 +2396,20 @@ extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE8_ACT321_BM64(
   const int m0 = tm * G6_BM, n0 = tn * BN;
   gemm8_body<false>(raw, aq, asc, C, M, N, K, ldc, c_off, accumulate, s_begin, s_end, m0, min(G6_BM, M - m0), n0);
   zero_tail(C, ldc, c_off, accumulate, tm, mt, M, n0, N);
+}
+
+// Q8_0 -DWK=4: the tile of eight waves.  gridDim.y > 1: work-group (x, y) takes the y-th of gridDim.y pieces of K and leaves its
+// sums in C, [gridDim.y][M][ldc], for splitk_reduce.  grid (ceil(N / 128) * token tiles, pieces), local 512.
+extern "C" __global__ __launch_bounds__(512, 2) void gemm__QTYPE8_ACT321_WK4(
+    const uint8_t* raw, const uint8_t* wh_unused, const signed char* aq, const float* asc, const short* absum, float* C,
+    int M, int N, int K, int ldc, int c_off, int accumulate, int rgroup, int s_begin, int s_end) {
+  const int nt = (N + BN - 1) / BN, mt = gridDim.x / nt, y = blockIdx.y, ny = gridDim.y, ns = s_end - s_begin;
+  int tm, tn;
+  tile_of(blockIdx.x, mt, nt, tm, tn);
+  const int m0 = tm * G6_BM, n0 = tn * BN;
+  gemm8w_body(raw, aq, asc, C + (size_t)y * M * ldc, M, N, K, ldc, c_off, accumulate, s_begin + ns * y / ny, s_begin + ns * (y + 1) / ny, m0,
+             min(G6_BM, M - m0), n0);
+  if (ny == 1) zero_tail(C, ldc, c_off, accumulate, tm, mt, M, n0, N);
 }
 
 extern "C" __global__ __launch_bounds__(256, 2) void gemm__QTYPE12_ACT321(

@@ -306,6 +306,35 @@ def test_gemm_padding_rows(rt, qtype, T, Mp, N, K, acc):
     assert np.array_equal(y[T:], c0[T:] if acc == 1 else np.zeros((Mp - T, N), np.float32))
 
 
+@pytest.mark.parametrize("T,Mp,N,K,pieces", [(9, 16, 1, 256, 0), (63, 64, 129, 512, 0), (64, 64, 128, 768, 0), (65, 80, 127, 1024, 0),
+                                             (300, 384, 520, 1280, 0), (130, 256, 390, 4096, 0), (100, 112, 260, 512, 2),
+                                             (300, 300, 1030, 2048, 5)])
+@pytest.mark.parametrize("acc,ldc,c_off", [(0, 0, 0), (1, 1, 0), (2, 8, 4)])
+def test_gemm_q8_0_eight_waves(rt, monkeypatch, T, Mp, N, K, pieces, acc, ldc, c_off):
+    """Q8_0 in tiles of eight waves that share out each superblock's blocks: one superblock and more than the stages hold,
+    ragged last tiles, K in pieces besides, rows of whole vectors and not.  Against the oracle's formula, padding rows and the
+    columns around the result, and run to run."""
+    monkeypatch.setenv("ARCZ_Q8_WK", "1")   # (read when an engine is made)
+    monkeypatch.setenv("ARCZ_Q4_SPLITK", str(pieces))
+    print(f"eight waves T={T} Mp={Mp} N={N} K={K} pieces={pieces} acc={acc} ldc=N+{ldc + c_off} c_off={c_off}", flush=True)
+    eng = az.Engine(Mp, K)
+    W = make_weights(az.Q8_0, N, K, seed=111)
+    x = make_acts(T, K, seed=112, outliers=True)
+    ld = N + ldc + c_off
+    c0 = np.random.default_rng(113).standard_normal((Mp, ld)).astype(np.float32)
+    y, y2 = (run_gemm(eng, az.Q8_0, W, N, K, x, Mp, acc=acc, c_init=c0, ldc=ld, c_off=c_off) for _ in range(2))
+    eng.close()
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32))
+    aq, asc, absum = quantize_padded(x, Mp)
+    c = c0[:, c_off:c_off + N]
+    form = np.zeros((Mp, N), np.float64)
+    form[:T] = orc.matmul_formula(az.Q8_0, 1, W, N, K, aq[:T], asc, absum)
+    want = form + c if acc == 1 else form * (c.astype(np.float64) / (1.0 + np.exp(-c.astype(np.float64)))) if acc == 2 else form
+    assert mixed_err(y[:T, c_off:c_off + N], want[:T]) <= TIGHT
+    assert np.array_equal(y[T:, c_off:c_off + N], c[T:] if acc == 1 else np.zeros((Mp - T, N), np.float32))
+    assert np.array_equal(y[:, :c_off], c0[:, :c_off]) and np.array_equal(y[:, c_off + N:], c0[:, c_off + N:])
+
+
 @pytest.mark.parametrize("qtype,T,Mp,N,K,acc", [(az.Q3_K, 256, 256, 4096, 256, 0), (az.Q3_K, 300, 304, 3500, 1280, 1),
                                                 (az.Q4_0, 257, 260, 12289, 256, 0), (az.Q4_0, 1000, 1024, 3200, 768, 2),
                                                 (az.MXFP4, 385, 400, 8190, 512, 1), (az.IQ3_S, 390, 400, 8000, 1024, 0),
