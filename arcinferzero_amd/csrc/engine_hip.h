@@ -721,18 +721,22 @@ class Engine {
       int lpr = 0;
       for (int l : {32, 64, 128, 256})
         if (!lpr && (units + l - 1) / l <= 6 && (!force_lpr || l == force_lpr)) lpr = l;
-      // Rows of 128 or 256 lanes, two tokens: work-groups of 512 threads, one a compute unit, stage the tokens once per
-      // compute unit instead of twice (5120 x 17408 Q4_K: 15.0 -> 14.4 us; one token: 11.9 -> 12.2, so not taken there;
-      // ARCZ_GEMV_BT=256: never, =512: for one token too)
+      // Rows of 128 or 256 lanes, two token slots, and four of Q8_0: work-groups of 512 threads, one a compute unit, stage the
+      // tokens once per compute unit instead of twice (5120 x 17408 Q4_K: 15.0 -> 14.4 us, one token with two-pass inputs 14.8 -> 13.9;
+      // Q8_0 4096 x 12288, four slots 14.9 -> 13.5; one token: 11.9 -> 12.2, so not taken there; ARCZ_GEMV_BT=256: never, =512: for
+      // one token too)
       static const int bt_env = getenv("ARCZ_GEMV_BT") ? atoi(getenv("ARCZ_GEMV_BT")) : 0;
-      const int bt = lpr >= 128 && (T == 2 || (T == 1 && bt_env == 512)) && !q2_fuse_ && bt_env != 256 ? 512 : 256;
-      const int g = lpr ? bt / lpr : 1, wpr = lpr > 64 ? lpr / 64 : 1;
+      auto bt_of = [&](int slots) {
+        return lpr >= 128 && bt_env != 256 && (slots == 2 || (slots == 1 && bt_env == 512) || (slots == 4 && w.type == GGML_Q8_0)) ? 512 : 256;
+      };
+      const int wpr = lpr > 64 ? lpr / 64 : 1;
       // the kernel's token slots: T rounded up, or -- both halves of two-pass inputs in one launch -- 2 T rounded up
-      auto lds_of = [&](int slots) { return (size_t)slots * tokb(slots) + (wpr > 1 ? (size_t)16 * g * wpr * slots * 4 : 0); };  // (16: the kernels' GEMV_FLUSH)
+      auto lds_of = [&](int slots) { return (size_t)slots * tokb(slots) + (wpr > 1 ? (size_t)16 * (bt_of(slots) / lpr) * wpr * slots * 4 : 0); };  // (16: the kernels' GEMV_FLUSH)
       const int tb2 = T == 1 ? 2 : T == 2 ? 4 : 8;
       const bool q2f = q2_fuse_ && T <= 4 && lpr && lds_of(tb2) <= (w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536);
       const int tbl = q2f ? tb2 : T <= 2 ? T : T <= 4 ? 4 : 8;
       const size_t lds = lds_of(tbl);
+      const int bt = bt_of(tbl), g = lpr ? bt / lpr : 1;
       // (IQ3_S: 2 KiB of the work-group's LDS hold the codebook)
       const size_t lds_max = w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536;
       const bool fits = !force_v && lpr && lds <= lds_max;
@@ -768,7 +772,7 @@ class Engine {
         const int wpc = wpc_env > 0 ? wpc_env : bt == 512 || (tb == 1 && !codebook && !q6_mid) ? 1 : 2;
         size_t wgs = std::min<size_t>((size_t)(N + g - 1) / g, (size_t)arcz_device_cus() * wpc);
         if (wgs_env > 0) wgs = std::min<size_t>((size_t)(N + g - 1) / g, (size_t)wgs_env);
-        const int sched = gemv_sched(N, g, wgs, false, raw_bytes(w), lpr >= 128 && tb == 1 && bt == 256, !codebook && tb <= 2);
+        const int sched = gemv_sched(N, g, wgs, false, raw_bytes(w), lpr >= 128 && tb == 1 && bt == 256, !codebook && (tb <= 2 || (tb == 4 && w.type == GGML_Q8_0)));
         const std::string cap = head_defs(w);
         cl_kernel k = cap.empty() ? variant("decode", {{"QT", w.type}, {"LPR", lpr}, {"PF", pf}, {tb > 1 ? "TB" : nullptr, tb}, {bt == 512 ? "BT" : nullptr, 512},
                                                        {"LDS", (long)lds}, {q2f ? "Q2_AQ" : nullptr, (long)q2_aq_}, {q2f ? "Q2_SC" : nullptr, (long)(q2_sc_ / 4)},

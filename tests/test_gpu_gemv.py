@@ -95,6 +95,45 @@ def test_gemv_config_shapes_sampled(eng, qtype, N, K, T):
     assert err.max() <= TOL
 
 
+@pytest.mark.parametrize("N,K", [(33, 4096), (2050, 5120), (97, 6400), (259, 8192), (4100, 12288)])
+@pytest.mark.parametrize("T", [3, 4])
+def test_gemv_q8_0_four_slots(rt, N, K, T):
+    """Q8_0 with four token slots in registers: rows of one wave and of two (512 threads from 6400 values on), whole and short
+    last passes, three tokens and four."""
+    print(f"gemv Q8_0 four slots N={N} K={K} T={T}", flush=True)
+    W = make_weights(az.Q8_0, N, K, seed=13)
+    x = make_acts(T, K, seed=14, outliers=True)
+    e = az.Engine(16, K)
+    y, y2 = run_gemv(e, az.Q8_0, W, N, K, x, 16), run_gemv(e, az.Q8_0, W, N, K, x, 16)
+    e.close()
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32))
+    aq, asc, absum = quantize_padded(x, 16)
+    assert rel_err_rows(y, orc.matmul_formula(az.Q8_0, 1, W, N, K, aq[:T], asc, absum)).max() <= TIGHT
+
+
+@pytest.mark.parametrize("qtype,T,N,K", [(az.Q8_0, 2, 33, 4096), (az.Q8_0, 2, 259, 8192), (az.Q8_0, 1, 4100, 12288), (az.Q8_0, 2, 2050, 12288),
+                                         (az.Q4_K, 1, 259, 17408), (az.Q6_K, 1, 130, 17408), (az.IQ3_S, 1, 67, 13312)])
+def test_gemv_two_pass_long_rows(rt, qtype, T, N, K):
+    """Both halves of two-pass inputs in one launch, rows of two waves and more in work-groups of 512 threads, against a launch for
+    each half: the same bits for Q8_0.  The other types' one-token kernel, which those launches run, applies its scales in
+    integers and in f32 in another order: a lane's at most 2 * 6 * 4 terms and the row's tree of 8 sums round by 2^-24 of at most
+    the sum of their magnitudes each, 3.4e-6 of it, which is below six times a row's largest result here."""
+    print(f"gemv two-pass {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=15)
+    x = make_acts(T, K, seed=16, outliers=True)
+    ys = []
+    for fuse in (True, False):
+        e = az.Engine(16, K)
+        e.two_pass(True, fuse)
+        ys.append(run_gemv(e, qtype, W, N, K, x, 16))
+        e.close()
+    assert np.isfinite(ys[0]).all()
+    if qtype == az.Q8_0:
+        assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32))
+    else:
+        assert rel_err_rows(ys[0], ys[1]).max() <= TIGHT
+
+
 def test_gemv_accumulate_and_offset(eng):
     N, K, T, Mp = 128, 512, 3, 16
     W = make_weights(az.Q4_K, N, K, seed=8)
