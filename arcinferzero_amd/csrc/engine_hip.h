@@ -1550,14 +1550,14 @@ class Engine {
   }
   void moe_digits(const MoeLayer& L, cl_mem rl, int ldl, cl_mem x, int T, int Mp, cl_mem sh) {
     const int E = L.E, F = L.F, n = T * L.NU;
-    route_tiles(L, rl, ldl, T, 64);
+    const bool recorded = route_tiles(L, rl, ldl, T, 64, true);
     const size_t tiles = ((size_t)(n + 63) / 64 + std::min(n, L.NE) + 7) / 8 * 8;
     auto tile_kernel = [&](const char* name, uint32_t type) {
       const DigitForm f = digit_form(type);
       return variant("gemm", {{"NW", f.nw}, {f.mn ? "MN" : nullptr, 1}}, name);
     };
     size_t l[2] = {256, 1};
-    {
+    if (!recorded) {
       cl_kernel k = variant("gemm", {}, "act_records");
       int MM = Mp, KK = E, TT = T;
       set_args(k, 0, aq_, asc_, absum_, MM, KK, TT, xr_);
@@ -1603,7 +1603,7 @@ class Engine {
   // routing -> slots grouped by expert -> tiles (zero/engine_moe.h:95-134).  rl: router logits [T][ldl] f32.
   // tm: slots per tile.
   // usum (plain routing only): the routing launch also writes au_ = sa * S of the current chunk's rows of K values.
-  void moe_route(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm, bool usum = false) {
+  void moe_route(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm, bool usum = false, bool records = false) {
     const int NE = L.NE, NU = L.NU, n = T * NU;
     if (T <= 0 || T > max_chunk || ldl < NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + NE) * 4)
       throw std::runtime_error("moe_route: router logits do not fit");
@@ -1611,8 +1611,8 @@ class Engine {
     const std::string defs = "-DNE=" + std::to_string(NE) + " -DNU=" + std::to_string(NU) + " -DTM=" + std::to_string(tm) +
                              " -DNPART=" + std::to_string(moe_tpc_) + " -DNCH=" + std::to_string(moe_chunks(T));
     {
-      if (usum && L.variant()) throw std::logic_error("moe_route: the routing variants do not write the sums");
-      cl_kernel k = kernel("moe", defs + (usum ? " -DUSUM=1" : L.route_defs()), "moe_route");
+      if ((usum || records) && L.variant()) throw std::logic_error("moe_route: the routing variants write neither the sums nor the records");
+      cl_kernel k = kernel("moe", defs + (records ? " -DREC=1" : usum ? " -DUSUM=1" : L.route_defs()), "moe_route");
       int NR = ldl, TT = T;
       set_args(k, 0, rl, NR, TT, mids_, mwts_, sgate_, mcount_);
       if (L.escale) set_args(k, 7, L.escale);  // (zero/engine_moe.h:114-115)
@@ -1622,7 +1622,12 @@ class Engine {
         set_args(k, 7, asc_, absum_, MM, au_, nblk);
       }
       size_t g1 = (size_t)(T + 3) / 4 * 256, l1 = 256;
-      run("moe_route", k, 1, &g1, &l1);
+      if (records) {
+        int MM = cur_Mp_, KK = cur_K_;
+        set_args(k, 7, aq_, asc_, absum_, MM, KK, xr_);
+        g1 += (size_t)(KK / 256) * ((T + 63) / 64) * 256;
+      }
+      run(records ? "act_records" : "moe_route", k, 1, &g1, &l1);
     }
     {
       cl_kernel k = kernel("moe", defs, "moe_scan");
@@ -1768,10 +1773,11 @@ class Engine {
     run("moe_combine", k, 2, gws, lws);
   }
   // routing -> slots -> tiles of tm slots; few pairs: the three steps in one work-group (as three launches they took 19 us)
-  void route_tiles(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm) {
+  // records: the chunk's tokens as records of digits too, where that goes with the routing launch (true)
+  bool route_tiles(const MoeLayer& L, cl_mem rl, int ldl, int T, int tm, bool records = false) {
     if (T * L.NU > 1024 || L.NE > 512 || L.variant()) {
-      moe_route(L, rl, ldl, T, tm);
-      return;
+      moe_route(L, rl, ldl, T, tm, false, records && !L.variant());
+      return records && !L.variant();
     }
     if (ldl < L.NE || arcz_mem_size(rl) < ((size_t)(T - 1) * ldl + L.NE) * 4) throw std::runtime_error("layer_moe: router logits do not fit");
     cl_kernel k = variant("moe", {{"NE", L.NE}, {"NU", L.NU}, {"TM", tm}}, "moe_route_small");
@@ -1779,6 +1785,7 @@ class Engine {
     set_args(k, 0, rl, NR, TT, mids_, mwts_, sgate_, mtiles_, stok_, swt_, minv_);
     size_t g1 = 1024, l1 = 1024;
     run("moe_route", k, 1, &g1, &l1);
+    return false;
   }
 
   // x[t] += sum_k w_k * expert_k(h[t]) for the T tokens whose quantized h is the current activation chunk

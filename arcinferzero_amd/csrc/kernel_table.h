@@ -107,6 +107,7 @@ static const KernelSpec kKernelTable[] = {
     {"gemm", "moe_gateup_q", nullptr, "ppiipppipppp", {"QT", nullptr}, {{"NE", 0, true}, {nullptr, 0, false}}, 256},
     // ---- moe
     {"moe", "moe_route", "USUM", "piippppppipi", {"USUM", nullptr}, {{"NE", 0, true}, {"NU", 0, true}, {"NPART", 1, false}, {nullptr, 0, false}}, 256},
+    {"moe", "moe_route", "REC", "piipppppppiip", {"REC", nullptr}, {{"NE", 0, true}, {"NU", 0, true}, {"NPART", 1, false}, {nullptr, 0, false}}, 256},
     {"moe", "moe_route", "ESCALE", "piippppp", {"ESCALE", nullptr}, {{"NE", 0, true}, {"NU", 0, true}, {"NPART", 1, false}, {nullptr, 0, false}}, 256},
     {"moe", "moe_route", "ROUTE_DS", "piippppp", {"ROUTE_DS", nullptr},
      {{"NE", 0, true}, {"NU", 0, true}, {"NPART", 1, false}, {"RSCALE", 0x3F800000, false}, {nullptr, 0, false}}, 256},

@@ -20,47 +20,11 @@ template <int NW, int MN> struct EImg {
   static_assert(LDS >= 36352 && 2 * LDS <= 160 * 1024, "the epilogues' array; two work-groups a compute unit");
 };
 
-// act_records: aq [M][K], asc [K/32][M], absum [K/16][M] -> rec [rows][K/32][64 bytes].  64 rows x a superblock a work-group, the
-// eight lanes of a row next to each other (its 256 values in, its 512 bytes out; a row a lane, 16 bytes each of 64 lines, took
-// 20 us for 4096 x 2048, now 9); the scales and sums, a row of which is a block's, come through LDS.
-// grid (K / 256, ceil(rows / 64)), local 256.
+// act_records (digit_pack.h): grid (K / 256, ceil(rows / 64)), local 256.
 extern "C" __global__ __launch_bounds__(256) void act_records(const signed char* __restrict__ aq, const float* __restrict__ asc,
                                                               const short* __restrict__ absum, int M, int K, int rows,
                                                               uint8_t* __restrict__ rec) {
-  __shared__ float lsa[8][65];
-  __shared__ int ls[8][65];
-  const int s = blockIdx.x, m0 = blockIdx.y * 64, t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int b = (t >> 6) + 4 * i, r = t & 63, m = m0 + r;
-    if (m >= rows) continue;
-    const size_t at = (size_t)(s * 8 + b);
-    lsa[b][r] = asc[at * M + m];
-    ls[b][r] = (int)absum[2 * at * M + m] + (int)absum[(2 * at + 1) * M + m];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int b = t & 7, r = (t >> 3) + 32 * i, m = m0 + r;
-    if (m >= rows) continue;
-    const u4v* src = (const u4v*)(aq + (size_t)m * K + s * 256 + b * 32);
-    const u4v x[2] = {src[0], src[1]};
-    uint32_t c[2][8], o[2][6], w0, w1;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) digits_i8(x[k >> 2][k & 3], c[0][k], c[1][k]);
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      pack16(c[d], o[d]);
-      pack16(c[d] + 4, o[d] + 3);
-    }
-    const float sa = lsa[b][r];
-    split3(sa * (float)ls[b][r], w0, w1);
-    u4v* to = (u4v*)(rec + ((size_t)m * (K >> 5) + s * 8 + b) * 64);
-    to[0] = (u4v){o[0][0], o[0][1], o[0][2], o[0][3]};
-    to[1] = (u4v){o[1][0], o[1][1], o[1][2], o[1][3]};
-    to[2] = (u4v){o[0][4], o[0][5], o[1][4], o[1][5]};
-    to[3] = (u4v){w0, w1 | w1 << 16, __float_as_uint(sa), 0u};
-  }
+  act_records_body(aq, asc, absum, M, K, rows, rec, blockIdx.x, blockIdx.y);
 }
 
 // row_digits_e__QT: tiles of an expert tensor.  Tile i: rows i * step .. + 127 of raw0 for the waves' first 32 rows, i * step + second ..
