@@ -1514,6 +1514,7 @@ class Engine {
     if (!L.digits[1] || arcz_mem_size(L.digits[0]) == 0 || arcz_mem_size(L.digits[1]) == 0) return false;
     // (the layer may be another engine's: this one has the records' room only if it kept a layer's digits itself)
     if (arcz_mem_size(xr_) < (size_t)T * L.E * 2 || arcz_mem_size(sr_) < (size_t)slots_ * L.F * 2) return false;
+    if (std::max((size_t)T * L.E, (size_t)T * L.NU * L.F) * 2 > 0xFFFFFFFFu) return false;  // (the tiles' 32-bit offsets)
     if (moe_digits_ > 1) return true;
     if (moe_dec_off_ || moe_mm_off_ || (moe_dec_set_ && T <= moe_dec_max_)) return false;  // (switches that name another form)
     const double slots = (double)T * L.NU / L.NE;

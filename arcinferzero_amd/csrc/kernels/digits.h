@@ -9,9 +9,16 @@ typedef int i2v __attribute__((ext_vector_type(2)));
 
 // LDS by byte offset (the kernel's one shared array begins at 0)
 #define LDS_P(T, a) ((__attribute__((address_space(3))) T*)(uint32_t)(a))
-// 16 bytes a lane straight into LDS: lane l's land at the wave's base + 16 l
-__device__ inline void dma16(const void* src, uint32_t lds_wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, LDS_P(void, lds_wave_base), 16, 0, 0);
+// 16 bytes a lane straight into LDS: lane l's land at the wave's base + 16 l.  From a buffer: a base and an offset in scalar
+// registers and the lane's own offset, so that a step's pieces take no vector instruction.  (As 64-bit addresses they took ten a
+// turn of the loop.  us before / now: Q4_K 17408 x 5120, 8192 tokens 1827 / 1772, the 300-token block 381 / 364, the 4096-token
+// layer 622 / 613, the 1000-token block of Q3_K 499 / 493.)
+typedef __amdgpu_buffer_rsrc_t d_buf;
+__device__ __forceinline__ d_buf d_buffer(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ void dma16(d_buf b, uint32_t lane_off, uint32_t off, uint32_t lds_wave_base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, LDS_P(void, lds_wave_base), 16, lane_off, off, 0, 0);
 }
 
 // a block's digit (8 words of codes) of row r of an image

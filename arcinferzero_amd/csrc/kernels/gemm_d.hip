@@ -134,21 +134,21 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave & 1, wn = wave >> 1;
   struct {
-    const uint8_t *t0, *w0, *ts, *ws;
-    uint32_t lane16;
+    d_buf t, w;
+    uint32_t lane16, to, wo;
     int wave;
     __device__ void at(int step) {
-      ts = t0 + (size_t)step * TS;
-      ws = w0 + (size_t)step * WS;
+      to = step * TS + wave * 1024;
+      wo = step * WS + wave * 1024 - TS;
     }
     __device__ void operator()(uint32_t stage, int i) {  // (tokens, then rows)
       if (4 * i + 4 > KB && wave >= (KB & 3)) return;
-      const uint8_t* src = 4 * i + 4 <= TKB || (4 * i < TKB && wave + 4 * i < TKB) ? ts : ws;
-      asm volatile("" : "+v"(lane16));
-      dma16(src + i * 4096 + lane16, stage + wave * 1024 + i * 4096);
+      const uint32_t lds = stage + wave * 1024 + i * 4096;
+      if (4 * i + 4 <= TKB || (4 * i < TKB && wave + 4 * i < TKB)) dma16(t, lane16, to + i * 4096, lds);
+      else dma16(w, lane16, wo + i * 4096, lds);
     }
-  } dma = {xt + ((size_t)(m0 >> 7) * nblk + b0) * I::T + wave * 1024, wt + ((size_t)(n0 >> 7) * nblk + b0) * I::W + wave * 1024 - TS,
-           nullptr, nullptr, (uint32_t)lane * 16, wave};
+  } dma = {d_buffer(xt + ((size_t)(m0 >> 7) * nblk + b0) * I::T, (size_t)(b1 - b0) * I::T),
+           d_buffer(wt + ((size_t)(n0 >> 7) * nblk + b0) * I::W, (size_t)(b1 - b0) * I::W), (uint32_t)lane * 16, 0u, 0u, wave};
   const DAddr o = {wm * 2048u + lane * 16u, 4096u + wm * 1024u + lane * 8u, I::TSA + (wm * 64u + l32) * 4u, I::TU + g * I::T + (wm * 64u + l32) * 8u,
                    TS + (wn * 64u + l32) * 16u, TS + 2048u + (wn * 64u + l32) * 8u, TS + I::WWS + (wn * 64u + lane) * 4u,
                    TS + I::WV + g * I::W + (wn * 64u + l32) * 8u};
@@ -233,28 +233,31 @@ __device__ __forceinline__ void gemm_d64_body(uint8_t* lds_base, const uint8_t* 
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = (m0 >> 6) & 1;
   struct {
-    const uint8_t *t0, *w0, *ts, *ws;
-    uint32_t toff, lane16, gap;  // (gap: from a step's end in the first row tile's image to its start in the second's)
+    d_buf t, w;
+    uint32_t toff, lane16, split, gap, to, wo;  // (gap: from a step's end in the first row tile's image to its start in the second's)
     int wave;
     __device__ void at(int step) {
-      ts = t0 + (size_t)step * I::NB * D::T;
-      ws = w0 + (size_t)step * WS;
+      to = step * I::NB * D::T;
+      wo = step * WS + wave * 1024;
     }
     __device__ void operator()(uint32_t stage, int i) {
       if (4 * i + 4 > KB && wave >= (KB & 3)) return;
-      asm volatile("" : "+v"(toff), "+v"(lane16));
+      const uint32_t lds = stage + wave * 1024 + i * 4096;
       if (i < I::NB) {
-        dma16(ts + i * D::T + toff, stage + wave * 1024 + i * 4096);
+        dma16(t, toff, to + i * D::T, lds);
       } else {
-        const uint32_t off = (wave + 4 * (i - I::NB)) * 1024 + lane16;
-        dma16(ws + (off < WS ? off : off + gap), stage + wave * 1024 + i * 4096);
+        const int j = wave + 4 * (i - I::NB);  // (KiB j of the rows' part; the one that holds both tiles': its lanes differ)
+        dma16(w, WS % 1024 != 0 && i - I::NB == WS / 4096 ? split : lane16, wo + (i - I::NB) * 4096 + (j * 1024 >= WS ? gap : 0), lds);
       }
     }
-  } dma = {xt + ((size_t)(m0 >> 7) * nblk + b0) * D::T, wt + ((size_t)(n0 >> 7) * nblk + b0) * D::W, nullptr, nullptr,
+  } dma = {d_buffer(xt + ((size_t)(m0 >> 7) * nblk + b0) * D::T, (size_t)(b1 - b0) * D::T),
+           d_buffer(wt + ((size_t)(n0 >> 7) * nblk + b0) * D::W, (size_t)(nblk + b1 - b0) * D::W),
            // a wave's KiB of a block's tokens: both groups of 32's first 16 bytes, their other 8, sa and u
            wave < 2 ? half * 2048 + wave * 1024 + lane * 16u : wave == 2 ? 4096 + half * 1024 + lane * 16u
            : MN && lane >= 16 && lane < 48 ? D::TU + half * 512 + (lane - 16) * 16u : D::TSA + half * 256 + (lane & 15) * 16u,
-           (uint32_t)lane * 16, (uint32_t)(nblk * D::W - WS), wave};
+           (uint32_t)lane * 16, 0u, (uint32_t)(nblk * D::W - WS), 0u, 0u, wave};
+  // (NW = 2: KiB WS / 1024, a wave's, is the first tile's up to byte WS)
+  dma.split = lane * 16u + (wave == (WS / 1024 & 3) && WS / 1024 * 1024 + lane * 16 >= WS ? dma.gap : 0u);
   const uint32_t row = TS + (wave >> 1) * WS, r = (wave & 1) * 64;
   const DAddr o = {lane * 16u, 2048u + lane * 8u, 3072u + l32 * 4u, 3328u + g * I::T + l32 * 8u, row + (r + l32) * 16u, row + 2048u + (r + l32) * 8u,
                    row + D::WWS + (r + lane) * 4u, row + D::WV + g * I::W + (r + l32) * 8u};

@@ -71,24 +71,25 @@ __device__ __forceinline__ bool tile_d_sums(uint8_t* lds_base, const uint8_t* __
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   struct {
-    const uint8_t *r0, *w0, *rs, *ws;
-    uint32_t lane16, toff;
+    d_buf t, w;
+    uint32_t lane16, toff, to, wo;
     int wave;
     __device__ void at(int step) {
-      rs = r0 + (size_t)step * I::NB * 64;
-      ws = w0 + (size_t)step * WS;
+      to = step * I::NB * 64;
+      wo = step * WS + wave * 1024 - TS;
     }
     __device__ void operator()(uint32_t stage, int i) {  // (a block's 64 slots are four KiB)
       if (4 * i + 4 > KB && wave >= (KB & 3)) return;
-      asm volatile("" : "+v"(lane16), "+v"(toff));
-      if (i < I::NB) dma16(rs + i * 64 + toff, stage + wave * 1024 + i * 4096);
-      else dma16(ws + i * 4096 + lane16, stage + wave * 1024 + i * 4096);
+      const uint32_t lds = stage + wave * 1024 + i * 4096;
+      if (i < I::NB) dma16(t, toff, to + i * 64, lds);
+      else dma16(w, lane16, wo + i * 4096, lds);
     }
   } dma;
   {
+    // (the slot's records: 64 bytes a block; a pass's are below 4 GiB, the engine sees to it)
     const int r = 16 * wave + (lane >> 2), rr = r < rows_valid ? r : 0;  // (slots past the tile read its first)
-    dma = {rec, wt + wave * 1024 - TS, nullptr, nullptr, (uint32_t)lane * 16,
-           (uint32_t)(map ? map[m0 + rr] : m0 + rr) * (uint32_t)nblk * 64u + 16u * ((lane & 3) ^ ((r >> 2) & 3)), wave};
+    dma = {d_buffer(rec, 0xFFFFFFFFu), d_buffer(wt, (size_t)nblk * I::W), (uint32_t)lane * 16,
+           (uint32_t)(map ? map[m0 + rr] : m0 + rr) * (uint32_t)nblk * 64u + 16u * ((lane & 3) ^ ((r >> 2) & 3)), 0u, 0u, wave};
   }
   const uint32_t sw = (l32 >> 2) & 3, t = l32 * 64u;  // (piece p of slot r at 16 (p ^ r / 4 % 4))
   const DAddr o = {t + ((g ^ sw) << 4), t + ((2 ^ sw) << 4) + g * 8u, t + ((3 ^ sw) << 4) + 8u, g * I::T + t + ((3 ^ sw) << 4),
