@@ -257,29 +257,25 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
   struct F6 { u4v lo; u2v hi; };
   F6 A[2], W[2][NW];
   float saop[2], wsop;
-  // addresses of the step the loads are in
-  uint32_t pA16, pA8, pW16, pW8, pSA, pWS, pU = 0, pV = 0;
-  auto at = [&](uint32_t stage) {
-    pA16 = o.A16 + stage; pA8 = o.A8 + stage; pW16 = o.W16 + stage; pW8 = o.W8 + stage; pSA = o.SA + stage; pWS = o.WS + stage;
-    asm volatile("" : "+v"(pA16), "+v"(pA8), "+v"(pW16), "+v"(pW8), "+v"(pSA), "+v"(pWS));
-    if constexpr (MN) {
-      pU = o.U + stage; pV = o.V + stage;
-      asm volatile("" : "+v"(pU), "+v"(pV));
-    }
-  };
+  // the lane's addresses in the first stage; st, the stage that the loads are in, and what else a place adds are immediate offsets
+  uint32_t pA16 = o.A16, pA8 = o.A8, pW16 = o.W16, pW8 = o.W8, pSA = o.SA, pWS = o.WS, pU = o.U, pV = o.V;
+  asm volatile("" : "+v"(pA16), "+v"(pA8), "+v"(pW16), "+v"(pW8), "+v"(pSA), "+v"(pWS));
+  if constexpr (MN) asm volatile("" : "+v"(pU), "+v"(pV));
+  static_assert((R - 1) * STAGE + (NB - 1) * I::W + (NW - 1) * I::DIG + 512 < 65536 && (R - 1) * STAGE + (NB - 1) * I::T + 2 * I::A_MS < 65536, "16 bits");
+  int st = 0;
   auto ldA = [&](int ms, int blk) {
-    A[ms].lo = *LDS_P(const u4v, pA16 + (NB == 2 ? blk : 0) * I::T + ms * I::A_MS);
-    A[ms].hi = *LDS_P(const volatile u2v, pA8 + (NB == 2 ? blk : 0) * I::T + ms * I::A8_MS);
+    A[ms].lo = *LDS_P(const u4v, pA16 + st * STAGE + (NB == 2 ? blk : 0) * I::T + ms * I::A_MS);
+    A[ms].hi = *LDS_P(const volatile u2v, pA8 + st * STAGE + (NB == 2 ? blk : 0) * I::T + ms * I::A8_MS);
   };
   auto ldW = [&](int ns, int blk) {
 #pragma unroll
     for (int d = 0; d < NW; ++d) {
-      W[ns][d].lo = *LDS_P(const u4v, pW16 + (NB == 2 ? blk : 0) * I::W + d * I::DIG + ns * 512);
-      W[ns][d].hi = *LDS_P(const volatile u2v, pW8 + (NB == 2 ? blk : 0) * I::W + d * I::DIG + ns * 256);
+      W[ns][d].lo = *LDS_P(const u4v, pW16 + st * STAGE + (NB == 2 ? blk : 0) * I::W + d * I::DIG + ns * 512);
+      W[ns][d].hi = *LDS_P(const volatile u2v, pW8 + st * STAGE + (NB == 2 ? blk : 0) * I::W + d * I::DIG + ns * 256);
     }
   };
-  auto ldSA = [&](int ms, int blk) { saop[ms] = *LDS_P(const float, pSA + (NB == 2 ? blk : 0) * I::T + ms * I::S_MS); };
-  auto ldWS = [&](int blk) { wsop = *LDS_P(const float, pWS + (NB == 2 ? blk : 0) * I::W); };
+  auto ldSA = [&](int ms, int blk) { saop[ms] = *LDS_P(const float, pSA + st * STAGE + (NB == 2 ? blk : 0) * I::T + ms * I::S_MS); };
+  auto ldWS = [&](int blk) { wsop = *LDS_P(const float, pWS + st * STAGE + (NB == 2 ? blk : 0) * I::W); };
   auto six = [](const F6& f) {
     const i4v a = __builtin_bit_cast(i4v, f.lo);
     const i2v b = __builtin_bit_cast(i2v, f.hi);
@@ -304,24 +300,21 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
   // The min term, u x v of both blocks of a step in one bf16 instruction, added straight to the results: a lane half takes a
   // block, its eight k are the products of the pieces but u3 v3 (2^-32 of the whole).
   u2v U[2], V[2];
-  auto ldU = [&](int ms) { U[ms] = *LDS_P(const u2v, pU + ms * I::U_MS); };
-  auto ldV = [&](int ns) { V[ns] = *LDS_P(const u2v, pV + ns * 256); };
+  auto ldU = [&](int ms) { U[ms] = *LDS_P(const u2v, pU + st * STAGE + ms * I::U_MS); };
+  auto ldV = [&](int ns) { V[ns] = *LDS_P(const u2v, pV + st * STAGE + ns * 256); };
   auto mfma_min = [&](int ms, int ns) {
     typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-    const uint32_t v11 = __builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x01000100u), v22 = __builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x03020302u);
-    const u4v a = {U[ms][0], U[ms][0], U[ms][0], U[ms][1]}, b = {v11, v22, V[ns][1], V[ns][0]};
+    const uint32_t v11 = __builtin_amdgcn_perm(V[ns][1], V[ns][1], 0x01000100u), v22 = __builtin_amdgcn_perm(V[ns][1], V[ns][1], 0x03020302u);
+    const u4v a = {U[ms][0], U[ms][0], U[ms][0], U[ms][1]}, b = {v11, v22, V[ns][0], V[ns][1]};
     res[ms][ns] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), res[ms][ns], 0, 0, 0);
   };
   // ---- prologue: the first R steps on their way (the last of them behind the first one's arrival), the first block's operands
   d_prologue<I>(dma, steps);
-  at(0);
   ldA(0, 0); ldSA(0, 0);
   ldW(0, 0); ldWS(0);
   mfma_p(0);
   ldSA(1, 0);
-  uint32_t st = 0;
   int step = 0;
-  uint32_t stf = (I::AHEAD - 1) * STAGE;  // (the first turn's first pieces: of a step that the prologue brought, once more)
   // Two blocks a turn, four products a block: tiles (0,0) (0,1) (1,1) (1,0), then (0,1) (0,0) (1,0) (1,1), so that the operands
   // that come free first are those the next block begins with.  A product's values are added while the next one runs; a
   // slot also carries a piece of the loads.  Behind a step's meeting the stage of that very step is refilled, with the step R on
@@ -329,8 +322,11 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
   // more), so that pieces have R - 1 steps to arrive; or (AHEAD = R - 1) the stage of the step before.  us with the first, before in
   // the second way: Q4_K 17408 x 5120, 8192 tokens 1847 -> 1827, the 4096-token layer of Q4_K experts 631 -> 619, the 1000-token block
   // of Q3_K 506 -> 498; but 300 tokens of Q4_K on gemm_d64 374 -> 382.
-#pragma unroll 1
-  for (int b = 0; b < blocks; b += 2) {
+  // Turn u of as many as bring the stages round, so that every place in LDS is a constant (with the stage in registers, eight more
+  // vector instructions a turn.  us: Q4_K 17408 x 5120, 8192 tokens 1713 -> 1686, the 4096-token layer 595 -> 586, the 1000-token block of
+  // Q3_K 476 -> 467.)
+  auto turn = [&](auto u_) {
+    constexpr int u = decltype(u_)::value;
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
       const int blk = p >> 2, q = p & 3, ms = q >> 1, ns = blk ? (q == 0 || q == 3) : (q == 1 || q == 2);
@@ -358,13 +354,11 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
         d_wait_but<KB, I::AHEAD - 2>();
         d_meet();
         __builtin_amdgcn_sched_barrier(0);
-        stf = I::AHEAD == R ? st : st == 0 ? (R - 1) * STAGE : st - STAGE;
-        st = st + STAGE == R * STAGE ? 0 : st + STAGE;
-        at(st);
         dma.at(min(step + I::AHEAD, steps - 1));
         ++step;
       }
       // -- loads for later
+      st = (NB == 2 ? u + (p >= 6) : 2 * u + (p >= 2) + (p >= 6)) % R;
       const int nb = (p + 2) >> 2 & 1;  // (block of the loads below: from p == 2 the second, from 6 the next step's first)
       if (q == 0) { ldW(blk ? 0 : 1, blk); ldA(1, blk); }
       if (q == 2) { ldA(0, nb); ldSA(0, nb); ldWS(nb); }
@@ -376,6 +370,8 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
       {
         // (two blocks a step: two pieces a slot, 6, 7 and, one turn on, 0, 1; one: three each)
         const int f = NB == 2 ? (p + 2 & 7) * 2 : q == 2 ? 0 : q == 3 ? 3 : ND;
+        // (the first turn's first pieces are of a step that the prologue brought, once more)
+        const int met = NB == 2 ? u + R - (p < 6) : 2 * u + blk, stf = (I::AHEAD == R ? met : met + R - 1) % R * STAGE;
         if (f < ND) dma(stf, f);
         if (f + 1 < ND) dma(stf, f + 1);
         if (NB == 1 && f + 2 < ND) dma(stf, f + 2);
@@ -390,7 +386,21 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  constexpr int TURNS = NB == 2 ? R : R % 2 ? R : R / 2;
+  int b = 0;
+#pragma unroll 1
+  for (; b + 2 * TURNS <= blocks; b += 2 * TURNS) {
+    turn(std::integral_constant<int, 0>());
+    turn(std::integral_constant<int, 1>());
+    if constexpr (TURNS > 2) turn(std::integral_constant<int, 2>());
   }
+  if (b < blocks) {
+    turn(std::integral_constant<int, 0>());
+    if constexpr (TURNS > 2)
+      if (b + 2 < blocks) turn(std::integral_constant<int, 1>());
+  }
+  static_assert(TURNS == 2 || TURNS == 3, "the turns above");
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // the last product: tile (1, 1) of the second block
 #pragma unroll
@@ -449,7 +459,7 @@ __device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int wave, int
           const u4v a = {U[0], U[0], U[0], U[1]};
 #pragma unroll
           for (int ns = 0; ns < 2; ++ns) {
-            const u4v v = {__builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x01000100u), __builtin_amdgcn_perm(V[ns][0], V[ns][0], 0x03020302u), V[ns][1], V[ns][0]};
+            const u4v v = {__builtin_amdgcn_perm(V[ns][1], V[ns][1], 0x01000100u), __builtin_amdgcn_perm(V[ns][1], V[ns][1], 0x03020302u), V[ns][0], V[ns][1]};
             res[ns] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, v), res[ns], 0, 0, 0);
           }
         }

@@ -40,7 +40,7 @@
 //   per digit [128][16 bytes], [128][8 bytes]; then [128] f32 ws
 // A tile's blocks follow each other.  NB: blocks a step of the GEMM takes; steps are whole KiB.
 // Types with a minimum (MN: Q4_K, Q5_K) have behind sa [128][8 bytes] u = sa * S, and behind ws v, of the min term: bf16 pieces
-// x1 | x2 << 16, x3 | x3 << 16.
+// u1 | u2 << 16, u3 | u3 << 16 and v3 | v3 << 16, v1 | v2 << 16 (so that both lie as the products take them).
 template <int NW, int MN = 0> struct DImg {
   static constexpr int NB = NW == 3 ? 1 : 2;
   static constexpr int R = NB == 2 ? 3 : 4, AHEAD = R;  // stages in LDS, steps on their way
@@ -108,7 +108,7 @@ __device__ inline void row_digits(const uint8_t* __restrict__ raw, const uint32_
     if constexpr (MN) {
       uint32_t w0, w1;
       split3(in ? d.mv[i] : 0.0f, w0, w1);
-      *(u2v*)(img + I::WV + r * 8) = (u2v){w0, w1 | w1 << 16};
+      *(u2v*)(img + I::WV + r * 8) = (u2v){w1 | w1 << 16, w0};
     }
   }
 }

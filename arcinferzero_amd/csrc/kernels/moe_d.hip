@@ -49,7 +49,7 @@ __device__ inline void row_digits_e(const uint8_t* __restrict__ raw0, const uint
     if constexpr (MN) {
       uint32_t w0, w1;
       split3(d.mv[i], w0, w1);
-      *(u2v*)(img + I::WV + pos * 8) = (u2v){w0, w1 | w1 << 16};
+      *(u2v*)(img + I::WV + pos * 8) = (u2v){w1 | w1 << 16, w0};
     }
   }
 }
