@@ -103,6 +103,10 @@ template <int QT> struct MmSb8 {
 };
 // The types with products of their own for at most eight tokens (mm_slice, T8).
 constexpr bool mm_t8(int qt) { return qt != QT_IQ3_S && qt != QT_Q3_K && qt != QT_IQ3_XXS; }
+// ... and, in the expert tiles, for at most four (T4).  us a layer of 128 x 8 experts of 768 x 2048, 40 tokens, without / with:
+// IQ4_XS 94.0 / 92.5, Q4_K 83.7 / 81.9, Q6_K 119.5 / 118.0, Q4_0 81.5 / 80.3, MXFP4 91.5 / 90.5; not Q8_0 (115.6 / 115.5) and
+// IQ4_NL (91.9 / 92.1), nor Q5_K, whose kernel then keeps 40 bytes a lane in scratch memory (106 / 113).
+constexpr bool mm_t4(int qt) { return mm_t8(qt) && qt != QT_Q5_K && qt != QT_Q8_0 && qt != QT_IQ4_NL; }
 
 // The rows a work-group multiplies, one slice of K at a time: ng groups of 16 rows, group gl at row row0(gl) of the
 // planes at raw(gl), which hold `rows` rows; token t is row tok(t) of the activations.  Here: groups gb0 .. of a matrix.
@@ -121,13 +125,15 @@ struct MmRows {
 // the tokens with the second block's values zero, rows 8 - 15 the tokens with the first one's, so a lane's four sums are of
 // block 2 p + g / 2 and tokens 4 (g & 1) .., and the scale step, a third of the vector instructions and half wasted on
 // eight tokens otherwise, is halved.  Lane (n, g) supplies 16 values of row n: block 2 p + g / 2, half g & 1.  The halves of
-// the lanes meet when a group is stored.
-template <int QT, bool LEAN, bool T8, class SRC, class STORE>
+// the lanes meet when a group is stored.  T4: at most four tokens.  Two such instructions into the same sums, rows 4 j .. 4 j + 3 the
+// tokens with block j of four: lane (n, g)'s sums are of block g, and the scale step is halved once more.
+template <int QT, bool LEAN, int TS, class SRC, class STORE>
 __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& src, int K,
                                 const signed char* __restrict__ aq, const float* __restrict__ asc,
                                 const short* __restrict__ absum, int M, int T, int s_begin, int s_end, STORE store) {
   using TT = MmT<QT>;
   using LL = MmL<QT>;
+  constexpr bool T8 = TS <= 8, T4 = TS <= 4;
   constexpr int QB = TT::QB, NQ = QB / 64, D = LEAN ? TT::DX : TT::D, LPRW = QB / 16, RPI = 64 / LPRW;
   constexpr bool Q45 = QT == QT_Q4_K || QT == QT_Q5_K;
   constexpr bool B16 = qt_nib16(QT) || QT == QT_IQ4_XS;  // a block is 16 bytes: low nibbles values 0..15, high 16..31
@@ -235,25 +241,34 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   // ---- staging.  Loads first: the tokens' int8 rows (wave w: rows 2 w and 2 w + 1, 16-byte pieces lane, lane + 64, ..),
   // their scales and sums (asc [K / 32][M], absum [K / 16][M]), then the wave's first superblocks right behind them:
   // loads come back in order, so the stores below wait for the tokens alone while the weights are on their way.
-  constexpr int NCH = LEAN ? 1 : (TT::SB * 16 + 63) / 64;  // pieces per lane and row at most
-  constexpr int NSC = LEAN ? 1 : (TT::SB * 8 * 16 + 511) / 512;  // (block, token) pairs per thread at most
-  const int cpr = Ks >> 4;
+  // LEAN, whose tiles hold a few of the 16 tokens, likewise (piece by piece, one after the other, the loads of the weights
+  // waited behind six round trips of tokens): the tokens that the tile has, no others -- a slot from T on may hold anything, for its scale is zero -- and, of the
+  // smaller tiles, a row of zeros, the ninth.
+  constexpr int NCH = (TT::SB * 16 + 63) / 64;  // pieces per lane and row at most
+  constexpr int TL = LEAN && TS < 16 ? 3 : 4, NSC = (TT::SB * (8 << TL) + 511) / 512;  // (block, token) pairs per thread at most
+  const int cpr = Ks >> 4, ts = tid & ((1 << TL) - 1);
   mm_u4 va[2][NCH];
   float vs[NSC];
   int vu[NSC];
-  if constexpr (LEAN) {  // (the registers are for two work-groups: piece by piece)
-    for (int i = tid; i < 16 * cpr; i += 512) {
-      const int t = i / cpr, k16 = i - t * cpr;
-      mm_u4 v = mm_u4{0, 0, 0, 0};
-      if (t < T) v = *(const mm_u4*)(aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256 + k16 * 16);
-      *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = v;
+  if constexpr (LEAN) {
+    const int t2 = src.tok(min(ts, T - 1));
+#pragma unroll
+    for (int r2 = 0; r2 < (TS < 16 ? 1 : 2); ++r2) {
+      const int t = wave + 8 * r2;
+      if (t < T) {
+        const signed char* ap = aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i)
+          if (64 * i < cpr) va[r2][i] = *(const mm_u4*)(ap + min(lane + 64 * i, cpr - 1) * 16);
+      }
     }
-    for (int i = tid; i < nb * 16; i += 512) {
-      const int b = s_begin * 8 + (i >> 4), t = i & 15, tt = src.tok(t < T ? t : 0);
-      const float sa = t < T ? asc[(size_t)b * M + tt] : 0.0f;
-      SA[i] = sa;
-      if constexpr (TT::MIN) U[i] = sa * (float)((int)absum[(size_t)(2 * b) * M + tt] + (int)absum[(size_t)(2 * b + 1) * M + tt]);
-    }
+#pragma unroll
+    for (int i = 0; i < NSC; ++i)
+      if (512 * i < nb << TL) {
+        const int b = s_begin * 8 + min((tid + 512 * i) >> TL, nb - 1);
+        vs[i] = asc[(size_t)b * M + t2];
+        if constexpr (TT::MIN) vu[i] = (int)absum[(size_t)(2 * b) * M + t2] + (int)absum[(size_t)(2 * b + 1) * M + t2];
+      }
   }
   if constexpr (!LEAN) {
 #pragma unroll
@@ -282,6 +297,33 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
 #pragma unroll
   for (int k = 0; k < D; ++k) qload(q[k], min(u0 + k, ulast), u0 + k < u1);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (LEAN) {
+    if constexpr (TS < 16) {
+      if (tid < cpr) *(mm_u4*)(A + 8 * Ks + tid * 16) = mm_u4{0, 0, 0, 0};
+      if constexpr (TT::MIN)
+        for (int i = tid; i < nb * 2; i += 512) *(v4f*)(U + (i >> 1) * 16 + 8 + (i & 1) * 4) = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int r2 = 0; r2 < (TS < 16 ? 1 : 2); ++r2) {
+      const int t = wave + 8 * r2;
+      if (t < T) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+          const int k16 = min(lane + 64 * i, cpr - 1);  // (clamped lanes store the same bytes again)
+          if (64 * i < cpr) *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = va[r2][i];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NSC; ++i) {
+      const int b = (tid + 512 * i) >> TL;
+      if (b < nb) {
+        const float sa = ts < T ? vs[i] : 0.0f;
+        SA[b * 16 + ts] = sa;
+        if constexpr (TT::MIN) U[b * 16 + ts] = sa * (float)vu[i];
+      }
+    }
+  }
   if constexpr (!LEAN) {
 #pragma unroll
   for (int r2 = 0; r2 < 2; ++r2) {
@@ -329,13 +371,15 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
 
   // the products of one superblock (sbk: its index within the slice) of the lane's row, into acc
   // (T8; row8: the token row of the lane's 16 values, or the first of the zero rows)
-  const int row8 = (n16 < 8) == (g < 2) ? (n16 & 7) : 8, hi = g >> 1, lo1 = g & 1;
+  // (T4: of the first and of the second instruction of four blocks)
+  const int hi = g >> 1, lo1 = g & 1;
+  const int row8 = T4 ? (n16 >> 2 == hi ? n16 & 3 : 8) : (n16 < 8) == (g < 2) ? (n16 & 7) : 8, row8b = n16 >> 2 == 2 + hi ? n16 & 3 : 8;
   auto products8 = [&](const MmSb8<QT>& h, int sbk, v4f& acc) {
     const int b0 = sbk * 8;
-    const uint8_t* ar = A + row8 * Ks;
     float ua = 0.0f, ub = 0.0f, va = 0.0f, vb = 0.0f, d = 0.0f, dmin = 0.0f;
     uint32_t G[4];
     v4f part = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4i Ia, Ib;
     if constexpr (Q45) {
       d = f16_bits_to_f32(h.h.x);
       dmin = f16_bits_to_f32(h.h.x >> 16);
@@ -355,10 +399,19 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       if (LEAN && p) __builtin_amdgcn_sched_barrier(0);
-      const v4i av = *(const v4i*)(ar + (((sbk * 16 + 4 * p + g) ^ row8) << 4));
-      const float4 sa = *(const float4*)(SA + (b0 + 2 * p + hi) * 16 + 4 * lo1);
+      const int row = T4 && (p & 1) ? row8b : row8;
+      const v4i av = *(const v4i*)(A + row * Ks + (((sbk * 16 + 4 * p + g) ^ row) << 4));
+      // (T4: with the second of two instructions, whose sums are of block 2 (p - 1) + g; the first leaves them in I, Ib)
+      const bool end = !T4 || (p & 1);
+      const int bw = T4 ? (p >> 1) * 4 + g : 2 * p + hi;  // the block of the lane's sums, its pair and place in the pair
+      const int odd = T4 ? lo1 : hi;
+      float4 sa;
+      if (end) sa = *(const float4*)(SA + (b0 + bw) * 16 + (T4 ? 0 : 4 * lo1));
       const float sa4[4] = {sa.x, sa.y, sa.z, sa.w};
-      const v4i z = {0, 0, 0, 0};
+      if (!T4 || !(p & 1)) Ia = Ib = v4i{0, 0, 0, 0};
+      auto of = [&](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {  // of the words of four pairs of blocks, the lane's sums'
+        return T4 ? (p < 2 ? (hi ? b : a) : (hi ? d : c)) : p == 0 ? a : p == 1 ? b : p == 2 ? c : d;
+      };
       v4i wv;
       if constexpr (QT == QT_Q6_K) {
         const mm_u4 L = h.c[p >> 1], H = h.x[p >> 1];
@@ -372,9 +425,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
           wv[k] = (int)(w & keep);
           wb[k] = (int)(w & ~keep & 0xFCFCFCFCu);
         }
-        const v4i Ia = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, z, 0, 0, 0);
-        const v4i Ib = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wb, z, 0, 0, 0);
-        const uint32_t sw = (p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi);
+        Ia = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, Ia, 0, 0, 0);
+        Ib = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wb, Ib, 0, 0, 0);
+        if (!end) continue;
+        const uint32_t sw = of(h.h.x, h.h.y, h.h.z, h.h.w) >> (16 * odd);
         const int sca = (int)(signed char)sw, scb = (int)(signed char)(sw >> 8);
 #pragma unroll
         for (int i = 0; i < 4; ++i) part[i] = fmaf((float)(__mul24(sca, Ia[i]) + __mul24(scb, Ib[i])), sa4[i], part[i]);
@@ -388,7 +442,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
             wv[k] = (int)((c[k] >> (4 * hi)) & 0x0F0F0F0Fu);
             if constexpr (QT == QT_Q5_K) wv[k] |= (int)((H5 >> k) & 0x10101010u);
           }
-          ws = d * (float)((G[p] >> (12 * hi)) & 63u);
+          if (end) ws = d * (float)((of(G[0], G[1], G[2], G[3]) >> (12 * odd)) & 63u);
         } else if constexpr (B16) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
@@ -397,21 +451,22 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
             else if constexpr (QT == QT_MXFP4) wv[k] = (int)mxfp4_lookup(q);
             else wv[k] = (int)nib_vals<QT>(q);
           }
-          if constexpr (QT == QT_IQ4_XS) {
-            const int b = 2 * p + hi;
-            ws = d * (float)((int)(((h.h.y >> (4 * b)) & 0xFu) | ((((h.h.x >> 16) >> (2 * b)) & 3u) << 4)) - 32);
+          if (!end) {
+          } else if constexpr (QT == QT_IQ4_XS) {
+            ws = d * (float)((int)(((h.h.y >> (4 * bw)) & 0xFu) | ((((h.h.x >> 16) >> (2 * bw)) & 3u) << 4)) - 32);
           } else if constexpr (QT == QT_MXFP4) {
-            ws = e8m0_half((p < 2 ? h.h.x : h.h.y) >> (16 * (p & 1) + 8 * hi));
+            ws = e8m0_half((p < 2 ? h.h.x : h.h.y) >> (T4 ? 8 * g : 16 * (p & 1) + 8 * hi));
           } else {
-            ws = f16_bits_to_f32((p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi));
+            ws = f16_bits_to_f32(of(h.h.x, h.h.y, h.h.z, h.h.w) >> (16 * odd));
           }
         } else {  // Q8_0
           wv = __builtin_bit_cast(v4i, c);
-          ws = f16_bits_to_f32((p == 0 ? h.h.x : p == 1 ? h.h.y : p == 2 ? h.h.z : h.h.w) >> (16 * hi));
+          ws = f16_bits_to_f32(of(h.h.x, h.h.y, h.h.z, h.h.w) >> (16 * odd));
         }
-        const v4i I = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, z, 0, 0, 0);
+        Ia = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, Ia, 0, 0, 0);
+        if (!end) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = fmaf((float)I[i], sa4[i] * ws, acc[i]);
+        for (int i = 0; i < 4; ++i) acc[i] = fmaf((float)Ia[i], sa4[i] * ws, acc[i]);
       }
     }
     if constexpr (Q45) {  // (rows 8 - 15, no tokens, have U = 0)
@@ -649,7 +704,10 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   auto put = [&](v4f v, int gl) {
     if constexpr (T8)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] += __shfl_xor(v[i], 32, 64);
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (T4) v[i] += __shfl_xor(v[i], 16, 64);
+        v[i] += __shfl_xor(v[i], 32, 64);
+      }
     store(v, gl);
   };
   const int gf = group_of(min(u0, ulast));  // the stretch's first group
@@ -808,7 +866,7 @@ __device__ inline void mm_kernel(uint8_t* lds, const uint8_t* __restrict__ raw, 
   for (int sl = 0; sl < slices; ++sl) {
     if (sl) __syncthreads();  // (the tokens and partial sums of the slice before have been read)
     const bool first = sl == 0, last = sl == slices - 1, add = GA ? accumulate : (accumulate || sl);
-    mm_slice<QT, false, T8>(lds, grid, src, K, aq, asc, absum, M, T, s_begin + all * sl / slices,
+    mm_slice<QT, false, (T8 ? 8 : 16)>(lds, grid, src, K, aq, asc, absum, M, T, s_begin + all * sl / slices,
                              s_begin + all * (sl + 1) / slices, [&](v4f v, int gl) {
       const int n = src.row0(gl) + n16;
       if (GA) {
@@ -882,16 +940,17 @@ extern "C" __global__ __launch_bounds__(256) void gemv_mm_reduce(const float* __
 // the tile GEMM's 64 or 128, whose work-groups then walk K alone; here a work-group takes 128 rows, and a wave reads whole
 // groups of 16 of them in order, so it streams the expert's weights once for all the tile's slots.  Bound by instruction
 // issue (the scale step is taken for 16 slots whatever the tile holds), then by memory: 40 tokens, 128 x 8 experts of 768 x
-// 2048, IQ4_XS: gate / up 61 us (3.2 TB/s), down 35, where the tile GEMM took 3 x 100.  Q6_K and Q3_K, two products a
+// 2048, IQ4_XS: gate / up 50 us, down 29, where the tile GEMM took 3 x 100.  Q6_K and Q3_K, two products a
 // block, need the registers of one work-group a compute unit.
 struct MmExpert {
   const uint8_t *w0, *w1;  // group 2 i of w0, group 2 i + 1 of w1 (PAIR) or both of w0
   int rows, r0, ng;
   bool pair;
-  const int* st;           // the slots' token rows (LDS)
+  const int* st;           // the slots' token rows (down: nullptr, the slots themselves, from s0 on)
+  int s0;
   __device__ const uint8_t* raw(int gl) const { return pair && (gl & 1) ? w1 : w0; }
   __device__ int row0(int gl) const { return r0 + 16 * (pair ? gl >> 1 : gl); }
-  __device__ int tok(int t) const { return st[t]; }
+  __device__ int tok(int t) const { return st ? st[t] : s0 + t; }
 };
 constexpr int MMX_HS = 132;  // floats of a slot's 128 rows in LDS
 
@@ -904,17 +963,14 @@ __device__ inline void moe_gateup_mm(uint8_t* lds, const uint8_t* __restrict__ r
                                      const float* __restrict__ asc, const short* __restrict__ absum, int M,
                                      const int* __restrict__ tiles, const int* __restrict__ stok, float* __restrict__ h, int S,
                                      signed char* __restrict__ hq, float* __restrict__ hsc, short* __restrict__ hbs, int NE) {
-  __shared__ int st[16];
   const int ti = blockIdx.y;
   if (ti >= tiles[0]) return;
   const int e = tiles[1 + 3 * ti], r0 = tiles[2 + 3 * ti], nr = tiles[3 + 3 * ti];
-  if (threadIdx.x < 16) st[threadIdx.x] = stok[r0 + min((int)threadIdx.x, nr - 1)];
   float* hs = (float*)(lds + (K >> 8) * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ);
   uint32_t* grid = (uint32_t*)(hs + 16 * MMX_HS);
   mm_grid<QT>(grid, tabs);
-  __syncthreads();
   MmExpert src;
-  src.w0 = rg; src.w1 = ru; src.rows = NE * F; src.r0 = e * F + blockIdx.x * 128; src.ng = 16; src.pair = true; src.st = st;
+  src.w0 = rg; src.w1 = ru; src.rows = NE * F; src.r0 = e * F + blockIdx.x * 128; src.ng = 16; src.pair = true; src.st = stok + r0; src.s0 = 0;
   const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
   v4f gate = {0.0f, 0.0f, 0.0f, 0.0f};
   auto both = [&](v4f v, int gl) {
@@ -925,8 +981,9 @@ __device__ inline void moe_gateup_mm(uint8_t* lds, const uint8_t* __restrict__ r
       for (int i = 0; i < 4; ++i) hs[(4 * g + i) * MMX_HS + 8 * (gl & ~1) + n16] = gate[i] / (1.0f + __expf(-gate[i])) * v[i];
     }
   };
-  if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT)>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
-  else mm_slice<QT, true, false>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
+  if (mm_t4(QT) && nr <= 4) mm_slice<QT, true, mm_t4(QT) ? 4 : 16>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
+  else if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT) ? 8 : 16>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
+  else mm_slice<QT, true, 16>(lds, grid, src, K, aq, asc, absum, M, nr, 0, K >> 8, both);
   __syncthreads();
   const int hl = threadIdx.x & 31;
   for (int b = threadIdx.x >> 5; b < 4 * nr; b += 16) {
@@ -955,20 +1012,15 @@ __device__ inline void moe_down_mm(uint8_t* lds, const uint8_t* __restrict__ raw
                                    const signed char* __restrict__ hq, const float* __restrict__ hsc,
                                    const short* __restrict__ hbs, int S, const int* __restrict__ tiles,
                                    const float* __restrict__ swt, float* __restrict__ y, int gpw, int NE) {
-  __shared__ int st[16];
   __shared__ float sw[16];
   const int ti = blockIdx.y;
   if (ti >= tiles[0]) return;
   const int e = tiles[1 + 3 * ti], r0 = tiles[2 + 3 * ti], nr = tiles[3 + 3 * ti];
-  if (threadIdx.x < 16) {
-    st[threadIdx.x] = r0 + min((int)threadIdx.x, nr - 1);
-    sw[threadIdx.x] = swt[r0 + min((int)threadIdx.x, nr - 1)];
-  }
+  if (threadIdx.x < 16) sw[threadIdx.x] = swt[r0 + min((int)threadIdx.x, nr - 1)];
   uint32_t* grid = (uint32_t*)(lds + (K >> 8) * MmL<QT>::TOK + MM_WAVES * MmL<QT>::WSZ);
   mm_grid<QT>(grid, tabs);
-  __syncthreads();
   MmExpert src;
-  src.w0 = src.w1 = raw; src.rows = NE * N; src.ng = 8 * gpw; src.r0 = e * N + blockIdx.x * src.ng * 16; src.pair = false; src.st = st;
+  src.w0 = src.w1 = raw; src.rows = NE * N; src.ng = 8 * gpw; src.r0 = e * N + blockIdx.x * src.ng * 16; src.pair = false; src.st = nullptr; src.s0 = r0;
   const int n16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
   auto rows = [&](v4f v, int gl) {
     const int n = (blockIdx.x * src.ng + gl) * 16 + n16;
@@ -976,8 +1028,9 @@ __device__ inline void moe_down_mm(uint8_t* lds, const uint8_t* __restrict__ raw
     for (int i = 0; i < 4; ++i)
       if (4 * g + i < nr) y[(size_t)(r0 + 4 * g + i) * N + n] = sw[4 * g + i] * v[i];
   };
-  if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT)>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
-  else mm_slice<QT, true, false>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
+  if (mm_t4(QT) && nr <= 4) mm_slice<QT, true, mm_t4(QT) ? 4 : 16>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
+  else if (mm_t8(QT) && nr <= 8) mm_slice<QT, true, mm_t8(QT) ? 8 : 16>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
+  else mm_slice<QT, true, 16>(lds, grid, src, K, hq, hsc, hbs, S, nr, 0, K >> 8, rows);
 }
 
 // WPE: waves a SIMD the registers are kept to.  4 (128 registers: two work-groups a compute unit, where LDS holds two -- not
