@@ -410,18 +410,26 @@ extern "C" __global__ __launch_bounds__(256) void moe_combine(float* __restrict_
                                                               const int* __restrict__ inv, int N, int NU) {
   const int c = (blockIdx.x * 256 + threadIdx.x) * 4, t = blockIdx.y;
   if (c >= N) return;
+  float4* xp = (float4*)(x + (size_t)t * N + c);
+  float4 o = *xp;
   float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int k = 0; k < NU; ++k) {
-    const float4 a = *(const float4*)(y + (size_t)inv[t * NU + k] * N + c);
-    v.x += a.x; v.y += a.y; v.z += a.z; v.w += a.w;
-  }
+  auto rows = [&](auto n_, int k) {
+    constexpr int n = decltype(n_)::value;
+    float4 a[n];
+#pragma unroll
+    for (int i = 0; i < n; ++i) a[i] = *(const float4*)(y + (size_t)inv[t * NU + k + i] * N + c);
+#pragma unroll
+    for (int i = 0; i < n; ++i) { v.x += a[i].x; v.y += a[i].y; v.z += a[i].z; v.w += a[i].w; }
+  };
+  int k = 0;
+  for (; k + 8 <= NU; k += 8) rows(std::integral_constant<int, 8>(), k);
+  if (k + 4 <= NU) { rows(std::integral_constant<int, 4>(), k); k += 4; }
+  for (; k < NU; ++k) rows(std::integral_constant<int, 1>(), k);
   if (sh) {
     const float gt = sgate[t];
     const float4 a = *(const float4*)(sh + (size_t)t * N + c);
     v.x += gt * a.x; v.y += gt * a.y; v.z += gt * a.z; v.w += gt * a.w;
   }
-  float4* xp = (float4*)(x + (size_t)t * N + c);
-  float4 o = *xp;
   o.x += v.x; o.y += v.y; o.z += v.z; o.w += v.w;
   *xp = o;
 }
