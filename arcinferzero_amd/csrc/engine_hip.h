@@ -945,39 +945,45 @@ class Engine {
   // How a product on digits is launched: in tiles of 128 x 128 or, of a matrix whose rows' digits are kept, 64 tokens x 256 rows;
   // the first `whole` tiles a work-group each, the others in `pieces` of K -- all of them (512 tokens x 4096 rows of Q3_K, K =
   // 12288, 195 -> 93 us), or those that full rounds leave over, at most 512 pieces (SPLIT_BYTES).  Priced, in us: a full round
-  // (two work-groups a compute unit) by 1024 values of K and for its ends, a last round of one work-group a unit 0.64 of that
-  // and from there on by its work-groups, the pieces' sums 4 us and 12 TB/s, 3 % of
-  // a product of more than a round (fitted; the cause is not shown).  Fitted to 666 products of nine
-  // types and eight matrices, 17 - 1500 tokens, weights from memory: 5 - 6 % off.
+  // (two work-groups a compute unit) by 1024 values of K and for its ends; a launch of no full round, `part`, 0.64 - 0.69 of
+  // that up to one work-group a unit, then by its work-groups; `last`, the round behind full ones, whose work-groups start as
+  // places come free; the pieces' sums 4 us and 8 TB/s, a second turn of loads from nine on.  Fitted to 2000 launches of four
+  // forms and twelve matrices, 20 - 1400 tokens, weights from memory: 7 % off, and what it takes is 1.2 % slower than the best of
+  // them on average, 14 % at most.
   struct DigitPlan { int th, whole, pieces; double us; };
   DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb, bool kept, int rows) const {
     const int cus = arcz_device_cus(), slots = 2 * cus, most = (int)std::min<size_t>(slots, SPLIT_BYTES / 65536);
-    const double k1024 = f.mn ? 21.3 : f.nw == 1 ? 17.4 : f.nw == 2 ? 23.7 : 30.7, ends = f.mn ? 5.6 : f.nw == 1 ? 4.4 : 8.0;
-    const double two = f.nw == 1 && !f.mn ? 0.84 : 0.76;
+    const double k1024 = f.mn ? 17.2 : f.nw == 1 ? 14.6 : f.nw == 2 ? 19.8 : 26.4, ends = f.mn ? 2.7 : f.nw == 1 ? 0.5 : f.nw == 2 ? 4.9 : 3.2;
+    const double one = rows <= 32 ? 0.77 : f.nw == 3 ? 0.68 : 0.63, two = f.nw < 3 ? 0.89 : 0.81;
     // (tiles of 64 tokens: fewer stages in flight with two and three digits; at most 32 tokens: half the products)
-    const double k64 = (f.nw == 1 ? 1.02 : f.nw == 2 ? 1.10 : 1.12) * (rows <= 32 && f.nw < 3 ? 0.7 : 1.0), e64 = ends + (f.nw == 1 ? 0.7 : f.nw == 2 ? 1.5 : 2.0);
+    const double k64 = (f.mn ? 1.02 : f.nw == 1 ? 1.05 : f.nw == 2 ? 1.07 : 1.12) * (rows <= 32 && f.nw < 3 ? 0.7 : 1.0);
+    const double e64 = ends + (f.mn ? 0.7 : f.nw == 1 ? 0.15 : f.nw == 2 ? 1.8 : 1.9);
     int th = 128;
     auto tile = [&](int p) { return (th == 128 ? k1024 : k64 * k1024) * ((nsb + p - 1) / p) / 4 + (th == 128 ? ends : e64); };
-    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? 0.64 : two + (1.0 - two) * (wgs - cus) / cus; };
+    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? one + 0.05 * wgs / cus : two + (1.0 - two) * (wgs - cus) / cus; };
+    auto last = [&](int full, int wgs, int p) {
+      if (!full || !wgs) return part(wgs);
+      return p == 1 ? std::max(0.54, 0.36 + 0.84 * wgs / slots) : 0.19 + 1.08 * wgs / slots;
+    };
     DigitPlan best = {128, 0, 1, 1e30};
     for (th = 128; th >= 64; th -= 64) {
       if (th == 64 ? !kept || digits64_ == 0 : kept && digits64_ == 1) continue;
       const int n = th == 64 ? (rows + 63) / 64 * ((N + 255) / 256) : (Mp + 127) / 128 * ((N + 127) / 128);
       const int full = n / slots, rest = n % slots;
       auto take = [&](int whole, int p, double us) {
-        if (p > 1) us += 4.0 + (n - whole) * p * 0.131 / 12.0;
+        if (p > 1) us += 3.8 + (p > 8 ? 1.0 : 0.0) + (n - whole) * p * 0.131 / 8.2;
         if (us < best.us) best = {th, whole, p, us};
       };
-      take(n, 1, (full + part(rest)) * tile(1));
+      take(n, 1, (full + last(full, rest, 1)) * tile(1));
       for (int p = 2; p <= 16 && p <= nsb / 2; ++p) {
         if (n * p <= most) take(0, p, part(n * p) * tile(p));
-        if (full && rest && rest * p <= most) take(n - rest, p, 1.03 * (full * tile(1) + part(rest * p) * tile(p)));
+        if (full && rest && rest * p <= most) take(n - rest, p, 1.01 * (full * tile(1) + last(full, rest * p, p) * tile(p)));
         // (the second places of a round of one work-group a unit: beside it a piece runs as in a full round)
-        if (rest > cus && (rest - cus) * p <= std::min(cus, most)) take(n - rest + cus, p, (full + 0.64 + 0.36 / p) * tile(1) + 4.0);
+        if (rest > cus && (rest - cus) * p <= std::min(cus, most)) take(n - rest + cus, p, (full + 0.68) * tile(1) + 0.185 * tile(p));
       }
     }
     // (the tokens' digits and the launches; the rows' digits from memory)
-    best.us += (f.mn ? 5.4 : f.nw == 1 ? 6.2 : f.nw == 2 ? 2.5 : 1.9) + Mp * (nsb * 256) / 1.7e6 +
+    best.us += (f.mn ? 4.9 : f.nw == 1 ? 6.0 : f.nw == 2 ? 2.8 : 1.9) + Mp * (nsb * 256) / 1.7e6 +
                (double)((N + 127) / 128) * nsb * 8 * f.wimg / (f.nw == 3 ? 18.0e6 : 40.0e6) + rows * (double)N * 4 / 9.0e6;
     return best;
   }
