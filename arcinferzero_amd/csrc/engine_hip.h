@@ -915,7 +915,9 @@ class Engine {
       else i8 = i8_price(type, Mp, rows, N, K / 256);
       if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes)
       const double less = type == GGML_IQ3_XXS || type == GGML_Q6_K ? 1.0 : type == GGML_Q4_K ? (K <= 1024 ? 0.9 : 0.94) : type == GGML_Q5_K ? 0.95 : 0.93;
-      return d < less * i8;  // (Q4_K 9000 x 1024, 1500 tokens: 65 / 60 us)
+      // (... and matrices below 2^23 values by 8 % more: Q4_K 1856 x 3584, 251 tokens 25.5 / 23.1, IQ4_NL 1712 x 1536 18.0 / 16.6)
+      const double small = (double)N * K < (1 << 23) && type != GGML_Q6_K && type != GGML_IQ3_XXS ? 0.08 : 0.0;
+      return d < (less - small) * i8;  // (Q4_K 9000 x 1024, 1500 tokens: 65 / 60 us)
     }
     if (Mp < 256) return false;
     switch (type) {
@@ -1120,11 +1122,15 @@ class Engine {
   }
   // The rows' digits kept with the weight, so that no matmul writes them: 5 us of 4096 x 4096, 33 us of 17408 x 5120 with one
   // digit (512 tokens Q4_0 169 -> 140 us, 300 118 -> 87).  1 - 2.5 bytes a weight beside
-  // the 0.4 - 0.8 of its planes: from 2^23 values on -- smaller ones are written in about a launch's time --, while such
-  // copies hold less than an eighth of the device's memory and a quarter of it stays free behind them, first come, first
+  // the 0.4 - 0.8 of its planes: from 2^21 values on (Q4_K and IQ3_S, whose int8 kernels are ahead up to there, 2^22; short
+  // rows, whose digits are few steps, 2^23), while such copies hold less than an eighth of the device's memory and a quarter of it stays free behind them, first come, first
   // served; where an allocation finds no memory later they are given back, as many as it needs (arcz_mem_spare), and the
   // matmul writes digits again or takes the int8 kernels: they are written at uploads alone.
   // ARCZ_DIGITS_KEEP=0 when the engine is made: never.
+  // (From 2^23 on before: the time without against that with them, 20 - 4000 tokens, on average and at worst, matrices of 2^22 -
+  // 2^23 values: IQ3_S 1.24, 1.15; IQ4_NL 1.23, 1.03; IQ4_XS 1.23, 0.94; MXFP4 1.17, 1.06; Q3_K 1.37, 1.18; Q4_0 1.41, 1.09; Q4_K 1.15,
+  // 0.97; Q5_K 1.30, 1.10; Q6_K 1.18, 0.97; of 2^21 - 2^22: IQ4_NL 1.26, 1.22; IQ4_XS 1.34, 1.03; MXFP4 1.34, 1.03; Q3_K 1.17, 0.95; Q4_0
+  // 1.19, 0.94; Q5_K 1.23, 1.03; but IQ3_S 1.04, 0.93; Q4_K 1.01, 0.88; and Q3_K 1072 x 1024 0.90 - 0.92, 4096 x 1024 about 1.)
   static bool digits_fit(size_t bytes) {
     const size_t total = arcz_device_mem();
     return arcz_spare_bytes() + bytes <= total / 8 && arcz_device_mem_free() >= bytes + total / 4;
@@ -1132,7 +1138,8 @@ class Engine {
   void digits_keep(GpuWeight& w) {
     const int tiles = (w.N + 255) / 256 * 2;  // (whole pairs, for tiles of 256 rows)
     const size_t bytes = (size_t)tiles * (w.K / 32) * digit_form(w.type).wimg;
-    if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << 23) || !digits_fit(bytes)) return;
+    const int least = w.K < 1024 || (w.type == GGML_Q3_K && w.K == 1024) ? 23 : w.type == GGML_Q4_K || w.type == GGML_IQ3_S ? 22 : 21;
+    if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << least) || !digits_fit(bytes)) return;
     digits_tokens();
     if (!xd_ || !(w.digits = try_buf(bytes))) return;
     CL_CHECK(arcz_mem_spare(w.digits));
