@@ -20,16 +20,17 @@
 // Q5_K are one digit, IQ3_XXS, IQ4_XS and IQ4_NL two.
 //
 // Bound by the matrix and the vector unit, which run beside each other only in part.  At 17408 x 5120 x 8192 a 32 x 32 x 32
-// block-tile takes a SIMD 151, 185, 233 cycles with one, two, three digits and 170 with one and a minimum, at 2.2, 1.9, 1.9
-// and 2.0 GHz; the matrix unit is busy 64, 96, 128, 80 of them, vector instructions are 83, 94, 105, 94, and waves wait 39 -
-// 44 % of their cycles.  The loop's arithmetic alone, out of registers, takes 120 of the 170 at 2.3 GHz (product 33, scale
-// tile 32, multiply-adds 50, min term 17: the f32 scale tile adds to the multiply-adds in full); the rest are operand reads
-// from LDS, DMA and the meeting.  Hence few bytes and few instructions per product: a wave's operands serve 64 x 64 outputs,
-// the addresses of a step are six registers and immediate offsets.  Kernel alone, 17408 x 5120 x 8192: one digit 968 TOP/s,
-// two 706, three 548, one and a minimum 802 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x 4096 x 4096 650
-// and 375).
-// Q4_K and Q5_K with the min term, 17408 x 5120, us, int8 kernels and this: 8192 tokens Q4_K 2020 / 1850, 2048 544 / 470, Q5_K
-// 593 / 472, 300 115 / 104, 143 / 104 (weights from memory, 64-token tiles).
+// block-tile takes a SIMD 131, 162, 207 cycles with one, two, three digits and 148 with one and a minimum, at 2.0, 1.8, 1.8
+// and 1.9 GHz, which is what the power limit leaves; the matrix unit is busy 64, 96, 128, 80 of them, vector instructions are
+// 76, 84, 93, 83, and waves wait 45 - 50 % of their cycles.  The loop's arithmetic alone, out of registers, takes 120 of the 148
+// at 2.3 GHz (product 33, scale tile 32, multiply-adds 50, min term 17: the f32 scale tile adds to the multiply-adds in full);
+// the rest are operand reads from LDS, DMA and the meeting.  Hence few bytes and few instructions per product: a wave's operands
+// serve 64 x 64 outputs, the addresses of a step are six registers and immediate offsets, its pieces' are scalars.  (Before the
+// latter, with the stage in registers: 151, 185, 233, 170 cycles at 2.2, 1.9, 1.9, 2.0 GHz.)  Kernel alone, 17408 x 5120 x 8192:
+// one digit 1014 TOP/s, two 751, three 578, one and a minimum 859 (the int8 kernels on packed weights: Q4_0 and Q3_K at 12288 x
+// 4096 x 4096 650 and 375).
+// Q4_K and Q5_K with the min term, 17408 x 5120, us, int8 kernels and this: 8192 tokens Q4_K 2020 / 1700, 2048 544 / 470, Q5_K
+// 593 / 472, 300 115 / 93, 143 / 93 (weights from memory, 64-token tiles).
 // Matmul with both writing kernels, us, before and now, 12288 x 4096 x 1024: Q4_0 173 / 136, MXFP4 183 / 135, IQ3_S
 // 201 / 147, Q3_K 293 / 182, Q6_K 277 / 234; x 4096: Q6_K 1094 / 790, IQ3_XXS 742 / 596.
 #include "digits.h"

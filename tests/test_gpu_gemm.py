@@ -385,6 +385,26 @@ def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
 
 
+@pytest.mark.parametrize("qtype,N,K,digits", [(az.Q4_0, 2048, 1024, 1), (az.Q4_0, 2047, 1024, 0), (az.MXFP4, 513, 4096, 1), (az.Q4_0, 4096, 768, 0),
+                                              (az.Q3_K, 1024, 2048, 1), (az.Q3_K, 4096, 1024, 0), (az.IQ3_S, 1024, 4096, 1),
+                                              (az.IQ3_S, 1023, 4096, 0)])
+def test_smallest_matrices_that_keep_digits(rt, qtype, N, K, digits):
+    """The sizes from which a weight's rows are kept as digits, by type and row length, and those below (41 tokens, which only kept
+    digits take): which kernels ran, and the oracle."""
+    T, Mp = 41, 48
+    print(f"kept digits type={qtype} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=91)
+    x = make_acts(T, K, seed=92, outliers=True)
+    eng = az.Engine(Mp, K)
+    eng.profile(True)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp)
+    eng.profile_collect()
+    assert eng.profile_get("act_digits")[1] == digits and eng.profile_get("keep_digits")[1] == digits
+    eng.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    assert rel_err_rows(y[:T], orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
+
+
 @pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "1", "ARCZ_Q4_SPLITK": "2"}, 1, 2), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
                                                  ({"ARCZ_Q4_SPLITK": "2"}, 1, 2),
                                                  ({"ARCZ_GEMM_SPLIT": "3", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])

@@ -170,10 +170,11 @@ def test_moe_matrix_pipe_tiles_of_16_slots(rt, monkeypatch, qtype, NE, NU, E, F,
 
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q8_0, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q3_K, az.IQ3_S,
                                    az.IQ3_XXS])
-@pytest.mark.parametrize("NE,NU,E,F,T", [(32, 4, 512, 256, 14), (16, 4, 768, 512, 20), (8, 4, 4096, 256, 13)])
+@pytest.mark.parametrize("NE,NU,E,F,T", [(32, 4, 512, 256, 14), (16, 4, 768, 512, 20), (8, 4, 4096, 256, 13), (16, 13, 512, 256, 9)])
 def test_moe_matrix_pipe_tiles_of_few_slots(rt, monkeypatch, qtype, NE, NU, E, F, T):
     """Tiles of one to four slots (of these there are two to ten experts each here), of five to eight and of more, which have
-    products of their own; rows whose tokens take one and several loads a lane.  Against the oracle as the others."""
+    products of their own; rows whose tokens take one and several loads a lane; thirteen experts a token, summed in eights, fours and ones.
+    Against the oracle as the others."""
     monkeypatch.setenv("ARCZ_MOE_DECODE_MAX", "0")
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 32)
 
