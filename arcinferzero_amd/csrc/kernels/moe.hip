@@ -156,19 +156,32 @@ extern "C" __global__ __launch_bounds__(1024) void moe_route_small(const float* 
   __shared__ int eoff[512], wtot[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = T * NU;
   for (int i = tid; i < 16 * 512 / 2; i += 1024) ((uint32_t*)wc)[i] = 0;
-  for (int t = wave; t < T; t += 16) {
-    const float* lg = logits + (size_t)t * ldl;
-    int mysel;
-    float mywt;
-    route_one_token(lg, NE, NU, lane, mysel, mywt);
-    if (lane < NU) {
-      sid[t * NU + lane] = (short)mysel;
-      sw[t * NU + lane] = mywt;
-      ids[(size_t)t * NU + lane] = mysel;
-      wts[(size_t)t * NU + lane] = mywt;
+  // (the next token's logits are on their way while one is routed.  Layers of 128 x 8 experts, us: 40 tokens of IQ4_XS 90.3 -> 89.5, one
+  // of Q4_K, whose logits are loaded the same way, 16.9 -> 16.6)
+  auto tokens = [&](auto pl_) {
+    constexpr int PL = decltype(pl_)::value;
+    float next[PL];
+    if (wave < T) route_logits(logits + (size_t)wave * ldl, NE, lane, next);
+    for (int t = wave; t < T; t += 16) {
+      const float* lg = logits + (size_t)t * ldl;
+      float v[PL];
+#pragma unroll
+      for (int i = 0; i < PL; ++i) v[i] = next[i];
+      route_logits(logits + (size_t)min(t + 16, T - 1) * ldl, NE, lane, next);
+      int mysel;
+      float mywt;
+      route_one_token_pl(v, lg, NE, NU, lane, mysel, mywt);
+      if (lane < NU) {
+        sid[t * NU + lane] = (short)mysel;
+        sw[t * NU + lane] = mywt;
+        ids[(size_t)t * NU + lane] = mysel;
+        wts[(size_t)t * NU + lane] = mywt;
+      }
+      if (lane == 0 && sgate) sgate[t] = ldl > NE ? 1.0f / (1.0f + expf(-lg[NE])) : 0.0f;
     }
-    if (lane == 0 && sgate) sgate[t] = ldl > NE ? 1.0f / (1.0f + expf(-lg[NE])) : 0.0f;
-  }
+  };
+  if (NE <= 128) tokens(std::integral_constant<int, 2>());
+  else tokens(std::integral_constant<int, ROUTE_PER_LANE>());
   __syncthreads();
   const bool live = tid < n;
   const int e = live ? sid[tid] : 0;

@@ -38,14 +38,20 @@ __device__ inline float route_ds_sp(float g) { return sqrtf(g > 20.0f ? g + log1
 // The choices one after the other: the largest key of the wave, and of the lanes that hold it the lowest expert, by a
 // ballot.  A round is a chain of about ten instructions -- with the (value, expert) pairs compared step by step, which it
 // was, 60 -- and the exponentials are taken once at the end, lane k its own; their sum in the order of the choices.
+// v: the lane's logits, of experts lane, lane + 64, .. (route_logits).
 template <int PL>
-__device__ inline void route_one_token_pl(const float* __restrict__ lg, int NE, int NU, int lane, int& sel, float& wt,
+__device__ inline void route_logits(const float* __restrict__ lg, int NE, int lane, float (&v)[PL]) {
+#pragma unroll
+  for (int i = 0; i < PL; ++i) v[i] = lg[min(i * 64 + lane, NE - 1)];
+}
+template <int PL>
+__device__ inline void route_one_token_pl(const float (&v)[PL], const float* __restrict__ lg, int NE, int NU, int lane, int& sel, float& wt,
                                           const RouteVariant rv = RouteVariant()) {
   uint32_t key[PL];
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = i * 64 + lane;
-    key[i] = e < NE ? route_key(rv.ebias ? route_ds_sp(lg[e]) + rv.ebias[e] : lg[e]) : 0u;
+    key[i] = e < NE ? route_key(rv.ebias ? route_ds_sp(v[i]) + rv.ebias[e] : v[i]) : 0u;
   }
   uint32_t mykey = 0, top = 0;
   int mysel = 0;
@@ -77,10 +83,16 @@ __device__ inline void route_one_token_pl(const float* __restrict__ lg, int NE, 
 }
 
 // (two logits a lane serve up to 128 experts, the common case; the same steps either way)
+template <int PL>
+__device__ inline void route_one_token_of(const float* __restrict__ lg, int NE, int NU, int lane, int& sel, float& wt, const RouteVariant rv) {
+  float v[PL];
+  route_logits(lg, NE, lane, v);
+  route_one_token_pl(v, lg, NE, NU, lane, sel, wt, rv);
+}
 __device__ inline void route_one_token(const float* __restrict__ lg, int NE, int NU, int lane, int& sel, float& wt,
                                        const RouteVariant rv = RouteVariant()) {
-  if (NE <= 128) route_one_token_pl<2>(lg, NE, NU, lane, sel, wt, rv);
-  else route_one_token_pl<ROUTE_PER_LANE>(lg, NE, NU, lane, sel, wt, rv);
+  if (NE <= 128) route_one_token_of<2>(lg, NE, NU, lane, sel, wt, rv);
+  else route_one_token_of<ROUTE_PER_LANE>(lg, NE, NU, lane, sel, wt, rv);
 }
 // The shared expert's gate of a token (moe.cl:40, 46): sigmoid of the logit past the experts' when the row holds one;
 // 1 with the -DROUTE_DS routing.
