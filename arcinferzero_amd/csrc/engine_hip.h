@@ -902,6 +902,9 @@ class Engine {
       //  69; Q4_K 40 / 37, Q5_K 40 / 41, Q6_K 59 / 50: not)
       if (Mp <= 64 && (type == GGML_Q4_K || type == GGML_Q5_K || type == GGML_Q6_K)) return false;
       // (these always: of 267 products, with digits 0.42 - 1.02 of the time without; Q5_K 0.50 - 1.00)
+      // (but Q4_0 and MXFP4 of few short rows: 1840 x 1280, 49 tokens of MXFP4 18.5 us, in five pieces on the int8 kernels 13.2)
+      if ((type == GGML_Q4_0 || type == GGML_MXFP4) && (double)N * K < (1 << 23) && K < 1536 &&
+          (Mp + 127) / 128 * ((N + 127) / 128) <= arcz_device_cus() / 4) return false;
       if (type == GGML_Q3_K || type == GGML_IQ3_S || type == GGML_Q4_0 || type == GGML_MXFP4) return true;
       // (IQ3_XXS of few values, or of few rows, whose digits go in 16 pieces of K: not -- 9000 x 1024, 40 tokens 21 / 20, 896 x 12032, 506
       //  tokens 50 / 47, 640 x 14336, 700 59 / 54, but 2500 103 / 110)
@@ -928,6 +931,13 @@ class Engine {
       default: return false;
     }
   }
+  // Pieces of K at most, where their number is not priced: of two superblocks; of one where rows are shorter than six of them, which
+  // would go in one piece otherwise, and tiles few (us before / now: 1568 x 1024, 30 tokens of Q4_K 21.9 / 7.9, 1696 x 1024, 217
+  // of Q5_K 1.69x, 288 x 1280, 108 of Q4_0 30.3 / 12.0, 992 x 1280, 56 of IQ4_XS 31.3 / 12.3; but 65 tiles, 1552 x 1024, 591 tokens of
+  // Q4_K 17.9 / 19.4, 112 tiles 21.4 / 27.3; Q4_K not from 256 rows on, where its dense kernel has the scale vectors ready).
+  static int sk_most(uint32_t type, int nsb, size_t tiles, int Mp) {
+    return nsb < 6 && tiles <= (size_t)arcz_device_cus() / 4 && (type != GGML_Q4_K || Mp < 256) ? nsb : nsb / 2;
+  }
   // us of a product of Q4_K, Q5_K, IQ4_XS or IQ4_NL on the int8 kernels as gemm_dense launches them: pieces of K, 128 x 128 tiles
   // (two work-groups a compute unit) or, Q4_K, 64 x 128 (three).  Fitted to eight matrices x 80 - 1500 tokens, 4 - 6 % off;
   // Q4_K of a last round of 64 x 128 tiles from 1170 products with three engines in turn (17408 x 5120, 300 tokens: 113 us, priced 117).
@@ -935,7 +945,7 @@ class Engine {
     struct P { double base, pieces, round, ends, one, sums, out; };
     const P p = type == GGML_Q4_K ? P{9.0, 11.6, 26.0, 2.1, 0.62, 13.3e6, 14.6e6}
                 : type == GGML_Q5_K ? P{7.2, 11.7, 26.7, 3.1, 0.61, 11.3e6, 10.1e6} : P{7.2, 9.8, 26.1, 2.9, 0.69, 13.4e6, 12.6e6};
-    const int cus = arcz_device_cus(), nt = (N + 127) / 128, t = (Mp + 127) / 128 * nt, ny = std::min({8, nsb / 2, 2 * cus / t});
+    const int cus = arcz_device_cus(), nt = (N + 127) / 128, t = (Mp + 127) / 128 * nt, ny = std::min({8, sk_most(type, nsb, t, Mp), 2 * cus / t});
     const double out = rows * (double)N * 4 / p.out;
     if (ny >= 3) return p.pieces + (t * ny <= cus ? p.one : 1.0) * (p.round * nsb / 4 / ny + p.ends) + 2.0 * ny * Mp * N * 4 / p.sums + out;
     const int full = t / (2 * cus), rest = t % (2 * cus), t64 = (rows + 63) / 64 * nt, f64 = t64 / (3 * cus), r64 = t64 % (3 * cus);
@@ -1205,7 +1215,7 @@ class Engine {
       const size_t tiles64 = (size_t)(tm == 64 && !q45 ? m64 : (Mp + tm - 1) / tm) * ((N + 127) / 128), slots = (bm == 32 ? 3 : 2) * (size_t)arcz_device_cus();
       const int nsb = K / 256;
       const int sk_force = sk_force_;
-      int ny = (int)std::min<size_t>({(size_t)8, (size_t)nsb / 2, slots / std::max<size_t>(tiles64, 1)});
+      int ny = (int)std::min<size_t>({(size_t)8, (size_t)sk_most(w.type, nsb, tiles64, Mp), slots / std::max<size_t>(tiles64, 1)});
       const bool priced = w.type == GGML_Q8_0 || w.type == GGML_Q6_K;
       if (priced) ny = split_pieces(w.type, w.half_d, Mp, m64, N, nsb);
       if (q8w) ny = q8w;

@@ -385,7 +385,27 @@ def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
 
 
-@pytest.mark.parametrize("qtype,N,K,digits", [(az.Q4_0, 2048, 1024, 1), (az.Q4_0, 2047, 1024, 0), (az.MXFP4, 513, 4096, 1), (az.Q4_0, 4096, 768, 0),
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4])
+@pytest.mark.parametrize("T,Mp,N,K", [(40, 48, 272, 768), (33, 48, 1040, 1024), (120, 128, 528, 1280), (24, 32, 256, 1280)])
+def test_short_rows_in_pieces_of_a_superblock(rt, qtype, T, Mp, N, K):
+    """Rows of three to five superblocks of few tiles: a piece of K each, on the int8 kernels (the product and its reduction), against
+    the oracle, into a wider C."""
+    print(f"pieces of a superblock {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=93)
+    x = make_acts(T, K, seed=94, outliers=True)
+    eng = az.Engine(Mp, K)
+    eng.profile(True)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp, ldc=N + 5, c_off=3)
+    eng.profile_collect()
+    assert eng.profile_get("act_digits")[1] == 0 and eng.profile_get("test")[1] >= 2
+    eng.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    assert rel_err_rows(y[:T, 3:3 + N], orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
+    assert not y[T:, 3:3 + N].any()
+    assert (np.delete(y, np.s_[3:3 + N], axis=1).view(np.uint32) == 0xFFFFFFFF).all()
+
+
+@pytest.mark.parametrize("qtype,N,K,digits", [(az.Q4_0, 1024, 2048, 1), (az.Q4_0, 1023, 2048, 0), (az.MXFP4, 513, 4096, 1), (az.Q4_0, 4096, 768, 0),
                                               (az.Q3_K, 1024, 2048, 1), (az.Q3_K, 4096, 1024, 0), (az.IQ3_S, 1024, 4096, 1),
                                               (az.IQ3_S, 1023, 4096, 0)])
 def test_smallest_matrices_that_keep_digits(rt, qtype, N, K, digits):
