@@ -931,10 +931,11 @@ class Engine {
       default: return false;
     }
   }
-  // Pieces of K at most, where their number is not priced: of two superblocks; of one where rows are shorter than six of them, which
-  // would go in one piece otherwise, and tiles few (us before / now: 1568 x 1024, 30 tokens of Q4_K 21.9 / 7.9, 1696 x 1024, 217
-  // of Q5_K 1.69x, 288 x 1280, 108 of Q4_0 30.3 / 12.0, 992 x 1280, 56 of IQ4_XS 31.3 / 12.3; but 65 tiles, 1552 x 1024, 591 tokens of
-  // Q4_K 17.9 / 19.4, 112 tiles 21.4 / 27.3; Q4_K not from 256 rows on, where its dense kernel has the scale vectors ready).
+  // Pieces of K at most: of two superblocks; of one where rows are shorter than six of them, which would go in one piece or two
+  // otherwise, and tiles few (us before / now: 1568 x 1024, 30 tokens of Q4_K 21.9 / 7.9, 1696 x 1024, 217 of Q5_K 1.69x, 288 x
+  // 1280, 108 of Q4_0 30.3 / 12.0, 992 x 1280, 56 of IQ4_XS 31.3 / 12.3, of Q6_K 16.3 / 10.3; but 65 tiles, 1552 x 1024, 591 of
+  // Q4_K 17.9 / 19.4, 112 tiles 21.4 / 27.3, 68 tiles of Q6_K 15.3 / 16.7).  Q4_K not from 256 token rows on, where its dense kernel
+  // has the scale vectors ready.
   static int sk_most(uint32_t type, int nsb, size_t tiles, int Mp) {
     return nsb < 6 && tiles <= (size_t)arcz_device_cus() / 4 && (type != GGML_Q4_K || Mp < 256) ? nsb : nsb / 2;
   }
@@ -1078,7 +1079,7 @@ class Engine {
     const size_t cus = (size_t)arcz_device_cus(), slots = (q8 ? 3 : 2) * cus, tiles = (size_t)m64 * ((N + 127) / 128);
     int best = 1;
     double least = 0.0;
-    for (int ny = 1; ny <= 8 && (ny == 1 || ny <= nsb / 2); ++ny) {
+    for (int ny = 1; ny <= 8 && (ny == 1 || ny <= sk_most(type, nsb, tiles, Mp)); ++ny) {
       if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const size_t full = tiles * ny / slots, rest = tiles * ny % slots;
       const double part = rest == 0 ? 0.0 : rest <= cus ? (q8 ? 0.46 : 0.62) : rest <= 2 * cus ? (q8 ? 0.65 : 1.0) : 1.0;

@@ -385,7 +385,7 @@ def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
 
 
-@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4])
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q6_K, az.Q3_K, az.IQ3_XXS])
 @pytest.mark.parametrize("T,Mp,N,K", [(40, 48, 272, 768), (33, 48, 1040, 1024), (120, 128, 528, 1280), (24, 32, 256, 1280)])
 def test_short_rows_in_pieces_of_a_superblock(rt, qtype, T, Mp, N, K):
     """Rows of three to five superblocks of few tiles: a piece of K each, on the int8 kernels (the product and its reduction), against
