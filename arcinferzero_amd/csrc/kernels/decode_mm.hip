@@ -118,7 +118,7 @@ struct MmRows {
   __device__ int tok(int t) const { return t; }
 };
 
-// one slice of K, superblocks [s_begin, s_end): at most MmT<QT>::SB of them; store(v, gl): group gl's sums of the slice,
+// one slice of K, superblocks [s_begin, s_end): at most MmT<QT>::SB of them, with LEAN as many as LDS holds; store(v, gl): group gl's sums of the slice,
 // lane (n16, g) with tokens 4 g .. 4 g + 3 of its row n16.  LEAN: within 128 registers, so that two work-groups share a
 // compute unit -- fewer superblocks in flight, the tokens' values and scales of two blocks at a time instead of eight.
 // T8: at most eight tokens.  Two neighbouring blocks go through one v_mfma_i32_16x16x64_i8: the instruction's rows 0 - 7 are
@@ -243,15 +243,25 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   // loads come back in order, so the stores below wait for the tokens alone while the weights are on their way.
   // LEAN, whose tiles hold a few of the 16 tokens, likewise (piece by piece, one after the other, the loads of the weights
   // waited behind six round trips of tokens): the tokens that the tile has, no others -- a slot from T on may hold anything, for its scale is zero -- and, of the
-  // smaller tiles, a row of zeros, the ninth.
-  constexpr int NCH = (TT::SB * 16 + 63) / 64;  // pieces per lane and row at most
-  constexpr int TL = LEAN && TS < 16 ? 3 : 4, NSC = (TT::SB * (8 << TL) + 511) / 512;  // (block, token) pairs per thread at most
+  // smaller tiles, a row of zeros, the ninth.  Its rows come whole: what SB superblocks' pieces do not cover (the launcher gives it as
+  // many as LDS holds, 28 of Q4_0's gate / up, 30 of its down) is staged before them, piece by piece.
+  constexpr int NCH = (TT::SB * 16 + 63) / 64;  // pieces per lane and row in the registers below
+  constexpr int TL = LEAN && TS < 16 ? 3 : 4, NSC = (TT::SB * (8 << TL) + 511) / 512;  // (block, token) pairs per thread
   const int cpr = Ks >> 4, ts = tid & ((1 << TL) - 1);
   mm_u4 va[2][NCH];
   float vs[NSC];
   int vu[NSC];
   if constexpr (LEAN) {
     const int t2 = src.tok(min(ts, T - 1));
+    for (int k16 = 64 * NCH + lane; k16 < cpr; k16 += 64)
+      for (int t = wave; t < T; t += 8)
+        *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = *(const mm_u4*)(aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256 + k16 * 16);
+    for (int i = tid + 512 * NSC; i < nb << TL; i += 512) {  // (512 is whole tokens: ts is this pair's too)
+      const int b = i >> TL, at = s_begin * 8 + b;
+      const float sa = ts < T ? asc[(size_t)at * M + t2] : 0.0f;
+      SA[b * 16 + ts] = sa;
+      if constexpr (TT::MIN) U[b * 16 + ts] = sa * (float)((int)absum[(size_t)(2 * at) * M + t2] + (int)absum[(size_t)(2 * at + 1) * M + t2]);
+    }
 #pragma unroll
     for (int r2 = 0; r2 < (TS < 16 ? 1 : 2); ++r2) {
       const int t = wave + 8 * r2;

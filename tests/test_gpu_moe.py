@@ -179,6 +179,22 @@ def test_moe_matrix_pipe_tiles_of_few_slots(rt, monkeypatch, qtype, NE, NU, E, F
     _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, 32)
 
 
+# The longest rows that the launcher gives each kernel of the matrix pipe's expert tiles (what its 159 KiB of LDS hold), and
+# the first ones past the 24 superblocks (Q6_K: 20) that a work-group stages in one turn.
+@pytest.mark.parametrize("qtype,E,F", [(az.Q4_K, 6400, 256), (az.Q5_K, 5632, 256), (az.Q6_K, 5120, 256), (az.Q8_0, 6144, 256), (az.Q4_0, 6400, 256),
+                                       (az.Q4_0, 7168, 256), (az.IQ4_XS, 7168, 256), (az.IQ4_NL, 7168, 256), (az.MXFP4, 7168, 256), (az.IQ3_S, 5888, 256),
+                                       (az.Q4_K, 256, 6400), (az.Q4_K, 256, 6912), (az.Q5_K, 256, 5888), (az.Q6_K, 256, 5376), (az.Q6_K, 256, 5632),
+                                       (az.Q8_0, 256, 6656), (az.Q4_0, 256, 7680), (az.IQ4_XS, 256, 6400), (az.IQ4_XS, 256, 7680), (az.IQ4_NL, 256, 7680),
+                                       (az.MXFP4, 256, 7680), (az.Q3_K, 256, 6656), (az.IQ3_S, 256, 6400), (az.IQ3_XXS, 256, 6400)])
+def test_moe_matrix_pipe_tiles_of_long_rows(rt, monkeypatch, qtype, E, F):
+    """Rows of more values than a work-group stages in one turn, to the longest that the form takes; tiles of 16, 14, 8, 6, 5 and 1
+    slots (the three forms of the products).  Against the oracle as the others."""
+    monkeypatch.setenv("ARCZ_MOE_DECODE_MAX", "0")
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "0")
+    counts = _moe_layer_vs_oracle(qtype, 8, 3, E, F, 17, 32, bias=[3.0, 0.0, 1.2, 1.0, 0.5, 0.0, -1.0, -1.0])
+    assert counts["moe_route"] == 1 and counts["moe_scan"] == 0   # (the tile GEMMs are routed in three launches)
+
+
 @pytest.mark.parametrize("qtype,T", [(az.Q4_K, 6), (az.Q5_K, 7), (az.Q6_K, 8), (az.Q4_K, 5), (az.Q8_0, 8)])
 def test_moe_matrix_pipe_tiles_from_six_tokens(rt, monkeypatch, qtype, T):
     """The first token counts that the 16-slot tiles take (48 pairs; Q4_K - Q6_K), and the last that they do not."""
@@ -244,7 +260,7 @@ def test_moe_ready_made_scale_vectors_change_no_bit(rt, monkeypatch, variant, NE
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
 
 
-def _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, Mp):
+def _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, Mp, bias=0.0):
     print(f"moe layer {TYPE_NAMES[qtype]} NE={NE} NU={NU} E={E} F={F} T={T}", flush=True)
     eng = az.Engine(Mp, max(E, F))
     try:
@@ -256,6 +272,7 @@ def _moe_layer_vs_oracle(qtype, NE, NU, E, F, T, Mp):
         rng = np.random.default_rng(5)
         logits = rng.standard_normal((T, NE)).astype(np.float32)
         logits[:, 1] -= 50.0                                  # an expert that gets no token
+        logits += np.float32(bias)                            # (of each expert, where a test wants its own numbers of slots)
         xb = az.Runtime.from_numpy(x)
         eng.quantize(xb, E, E, Mp, T)
         lb = az.Runtime.from_numpy(logits)
