@@ -724,21 +724,25 @@ class Engine {
       // Rows of 128 or 256 lanes, two token slots, and four of Q8_0: work-groups of 512 threads, one a compute unit, stage the
       // tokens once per compute unit instead of twice (5120 x 17408 Q4_K: 15.0 -> 14.4 us, one token with two-pass inputs 14.8 -> 13.9;
       // Q8_0 4096 x 12288, four slots 14.9 -> 13.5; one token: 11.9 -> 12.2, so not taken there; ARCZ_GEMV_BT=256: never, =512: for
-      // one token too)
+      // one token too).  Where LDS does not hold their sums beside the tokens, 256 (us with the kernels beyond LDS / so: Q8_0 4096 x
+      // 12800, four tokens 20.3 / 18.0, a block of 12800 with two-pass inputs of two tokens 53.5 / 45.1; one token's, Q4_0 4096 x 25856
+      // 55.9 / 48.6; two tokens, Q6_K 4096 x 25856 40.9 / 26.2)
       static const int bt_env = getenv("ARCZ_GEMV_BT") ? atoi(getenv("ARCZ_GEMV_BT")) : 0;
-      auto bt_of = [&](int slots) {
-        return lpr >= 128 && bt_env != 256 && (slots == 2 || (slots == 1 && bt_env == 512) || (slots == 4 && w.type == GGML_Q8_0)) ? 512 : 256;
-      };
       const int wpr = lpr > 64 ? lpr / 64 : 1;
+      // (IQ3_S: 2 KiB of the work-group's LDS hold the codebook)
+      const size_t lds_max = w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536;
+      auto lds_at = [&](int slots, int bt) { return (size_t)slots * tokb(slots) + (wpr > 1 ? (size_t)16 * (bt / lpr) * wpr * slots * 4 : 0); };  // (16: the kernels' GEMV_FLUSH)
+      auto bt_of = [&](int slots) {
+        return lpr >= 128 && bt_env != 256 && (slots == 2 || (slots == 1 && bt_env == 512) || (slots == 4 && w.type == GGML_Q8_0)) &&
+               lds_at(slots, 512) <= lds_max ? 512 : 256;
+      };
       // the kernel's token slots: T rounded up, or -- both halves of two-pass inputs in one launch -- 2 T rounded up
-      auto lds_of = [&](int slots) { return (size_t)slots * tokb(slots) + (wpr > 1 ? (size_t)16 * (bt_of(slots) / lpr) * wpr * slots * 4 : 0); };  // (16: the kernels' GEMV_FLUSH)
+      auto lds_of = [&](int slots) { return lds_at(slots, bt_of(slots)); };
       const int tb2 = T == 1 ? 2 : T == 2 ? 4 : 8;
-      const bool q2f = q2_fuse_ && T <= 4 && lpr && lds_of(tb2) <= (w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536);
+      const bool q2f = q2_fuse_ && T <= 4 && lpr && lds_of(tb2) <= lds_max;
       const int tbl = q2f ? tb2 : T <= 2 ? T : T <= 4 ? 4 : 8;
       const size_t lds = lds_of(tbl);
       const int bt = bt_of(tbl), g = lpr ? bt / lpr : 1;
-      // (IQ3_S: 2 KiB of the work-group's LDS hold the codebook)
-      const size_t lds_max = w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536;
       const bool fits = !force_v && lpr && lds <= lds_max;
       static const int mm_env = getenv("ARCZ_GEMV_MM_MIN") ? atoi(getenv("ARCZ_GEMV_MM_MIN")) : 0;
       const double mvals = (double)N * K / (1 << 20);

@@ -134,6 +134,36 @@ def test_gemv_two_pass_long_rows(rt, qtype, T, N, K):
         assert rel_err_rows(ys[0], ys[1]).max() <= TIGHT
 
 
+@pytest.mark.parametrize("qtype,T,N,K,two_pass", [(az.Q8_0, 3, 67, 12800, False), (az.Q8_0, 4, 2050, 12800, False), (az.Q8_0, 2, 259, 12800, True),
+                                                  (az.Q4_0, 1, 67, 25856, True), (az.Q6_K, 1, 33, 25856, True), (az.IQ3_S, 1, 35, 25088, True),
+                                                  (az.IQ4_XS, 2, 67, 25856, False)])
+def test_gemv_rows_that_fit_256_threads_alone(rt, qtype, T, N, K, two_pass):
+    """Rows as long as 64 KiB of LDS hold beside the sums of 256 threads, but not of 512: the LDS-staged kernels take them all the
+    same, both halves of two-pass inputs in one launch.  Against the oracle; Q8_0's rows with the bits of the one-token launch (the
+    other kernels add a row up in another order)."""
+    print(f"gemv 256 threads {TYPE_NAMES[qtype]} N={N} K={K} T={T} two_pass={two_pass}", flush=True)
+    W = make_weights(qtype, N, K, seed=17)
+    x = make_acts(T, K, seed=18, outliers=True)
+    e = az.Engine(16, K)
+    e.two_pass(two_pass)
+    e.profile(True)
+    y = run_gemv(e, qtype, W, N, K, x, 16)
+    e.profile_collect()
+    assert e.profile_get("test")[1] == 1
+    if two_pass:
+        e.two_pass(True, False)
+        one = run_gemv(e, qtype, W, N, K, x, 16)
+    else:
+        one = np.concatenate([run_gemv(e, qtype, W, N, K, x[t:t + 1], 16) for t in range(T)])
+    e.close()
+    assert np.isfinite(y).all() and rel_err_rows(y, one).max() <= TIGHT
+    if qtype == az.Q8_0:
+        assert np.array_equal(y.view(np.uint32), one.view(np.uint32))
+    if not two_pass:
+        aq, asc, _ = quantize_padded(x, 16)
+        assert rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
+
+
 def test_gemv_accumulate_and_offset(eng):
     N, K, T, Mp = 128, 512, 3, 16
     W = make_weights(az.Q4_K, N, K, seed=8)
