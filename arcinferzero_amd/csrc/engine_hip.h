@@ -1656,7 +1656,7 @@ class Engine {
         set_args(k, 7, aq_, asc_, absum_, MM, KK, xr_);
         g1 += (size_t)(KK / 256) * ((T + 63) / 64) * 256;
       }
-      run(records ? "act_records" : "moe_route", k, 1, &g1, &l1);
+      run(records ? "moe_route_records" : "moe_route", k, 1, &g1, &l1);  // (two launches' work: neither one's time)
     }
     {
       cl_kernel k = kernel("moe", defs, "moe_scan");

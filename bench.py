@@ -336,7 +336,7 @@ def bench_moe(az, launches, ready_made=True):
     az.Runtime.sync()
     eng.profile_collect()
     parts = {}
-    for name in ("moe_route", "act_records", "moe_scan", "moe_scatter", "moe_gateup", "moe_quant", "moe_down", "moe_combine"):
+    for name in ("moe_route", "act_records", "moe_route_records", "moe_scan", "moe_scatter", "moe_gateup", "moe_quant", "moe_down", "moe_combine"):
         t, n = eng.profile_get(name)
         parts[name + "_ms"] = t / launches   # per layer, however many launches the step takes
     ops = T * NU * 3 * 2.0 * F * E

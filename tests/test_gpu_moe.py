@@ -555,7 +555,9 @@ def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E,
     eng.profile(True)
     y1 = run()
     eng.profile_collect()
-    assert eng.profile_get("act_records")[1] == 1
+    # (more pairs than one work-group routes: the routing launch writes the records as well)
+    launched = tuple(eng.profile_get(k)[1] for k in ("moe_route", "act_records", "moe_route_records"))
+    assert launched == ((0, 0, 1) if n > 1024 else (1, 1, 0))
     eng.profile(False)
     assert np.array_equal(y1.view(np.uint32), run().view(np.uint32))
     inv = eng.moe_buffer("inv").read(np.int32, n).reshape(T, NU)
@@ -594,6 +596,42 @@ def test_moe_tiles_on_digits(rt, monkeypatch, tmp_path, qtype, qdown, NE, NU, E,
     for b in (xb, lb):
         b.free()
     eng.close()
+
+
+@pytest.mark.parametrize("qtype,T,Mp", [(az.Q4_K, 128, 128), (az.Q4_K, 129, 144), (az.IQ4_XS, 193, 208), (az.Q6_K, 320, 320)])
+def test_moe_records_with_the_routing_launch(rt, monkeypatch, qtype, T, Mp):
+    """More than 1024 pairs: the routing launch writes the tokens' records too.  An expert scale of 1.0 is a routing variant, whose
+    passes write them in a launch of their own, and changes no weight: the same bits.  With the shared expert's gate in the rows of
+    logits; token counts around whole work-groups of records (64) and of routed tokens (4)."""
+    NE, NU, E, F = 64, 8, 512, 256
+    print(f"moe records with the routing {TYPE_NAMES[qtype]} T={T}", flush=True)
+    monkeypatch.setenv("ARCZ_MOE_DIGITS", "2")            # (read when the engine is made: whatever the rule says)
+    Wg, Wu, Wd = make_weights(qtype, NE * F, E, seed=1), make_weights(qtype, NE * F, E, seed=2), make_weights(qtype, NE * E, F, seed=3)
+    rng = np.random.default_rng(5)
+    eng = az.Engine(Mp, E)
+    L = eng.make_moe_layer(qtype, Wg, Wu, Wd, NE, NU, E, F)
+    xb, sb = az.Runtime.from_numpy(make_acts(T, E, seed=4)), az.Runtime.from_numpy(rng.standard_normal((T, E)).astype(np.float32))
+    lb = az.Runtime.from_numpy(rng.standard_normal((T, NE + 1)).astype(np.float32))
+
+    def run():
+        ob = az.Runtime.alloc(T * E * 4).fill(0)
+        eng.profile(True)
+        eng.quantize(xb, E, E, Mp, T)
+        eng.layer_moe(L, lb, NE + 1, ob, T, Mp, sb)
+        y = ob.read(np.uint32, T * E)
+        ob.free()
+        eng.profile_collect()
+        return y, [eng.profile_get(k)[1] for k in ("moe_route", "act_records", "moe_route_records")]
+
+    y, fused = run()
+    eng.set_moe_routing(L, escale=np.ones(NE, np.float32))
+    want, apart = run()
+    for b in (xb, sb, lb):
+        b.free()
+    eng.close()   # (the layer with it)
+    assert fused == ([0, 0, 1] if T * NU > 1024 else [1, 1, 0])
+    assert [b - a for a, b in zip(fused, apart)] == [1, 1, 0]   # (the counts add up)
+    assert np.isfinite(y.view(np.float32)).all() and y.any() and np.array_equal(y, want)
 
 
 @pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q6_K, az.Q4_0])
