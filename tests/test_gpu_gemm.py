@@ -385,11 +385,11 @@ def test_caller_quantized_rows_are_multiplied_as_given(rt, qtype, T, Mp, N, K):
     assert np.isfinite(y).all() and rel_err_rows(y, orc.matmul_ref(qtype, W, N, K, aq, asc)).max() <= TOL
 
 
-@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q6_K, az.Q3_K, az.IQ3_XXS])
+@pytest.mark.parametrize("qtype", [az.Q4_K, az.Q5_K, az.Q4_0, az.IQ4_XS, az.IQ4_NL, az.MXFP4, az.Q6_K, az.Q8_0, az.Q3_K, az.IQ3_S, az.IQ3_XXS])
 @pytest.mark.parametrize("T,Mp,N,K", [(40, 48, 272, 768), (33, 48, 1040, 1024), (120, 128, 528, 1280), (24, 32, 256, 1280)])
 def test_short_rows_in_pieces_of_a_superblock(rt, qtype, T, Mp, N, K):
     """Rows of three to five superblocks of few tiles: a piece of K each, on the int8 kernels (the product and its reduction), against
-    the oracle, into a wider C."""
+    the oracle, into a wider C; the reduction's other two epilogues on the same sums."""
     print(f"pieces of a superblock {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
     W = make_weights(qtype, N, K, seed=93)
     x = make_acts(T, K, seed=94, outliers=True)
@@ -398,7 +398,16 @@ def test_short_rows_in_pieces_of_a_superblock(rt, qtype, T, Mp, N, K):
     y = run_gemm(eng, qtype, W, N, K, x, Mp, ldc=N + 5, c_off=3)
     eng.profile_collect()
     assert eng.profile_get("act_digits")[1] == 0 and eng.profile_get("test")[1] >= 2
+    eng.profile(False)
+    c0 = az.gen_normal(95, (Mp, N + 5))
+    ya, ys = (run_gemm(eng, qtype, W, N, K, x, Mp, acc=acc, c_init=c0, ldc=N + 5, c_off=3) for acc in (1, 2))
     eng.close()
+    y0, g = y[:, 3:3 + N], c0[:, 3:3 + N].astype(np.float64)
+    want = y0.astype(np.float64) * (g / (1.0 + np.exp(-g)))
+    assert np.array_equal(ya[:, 3:3 + N], y0 + c0[:, 3:3 + N])
+    assert np.abs(ys[:, 3:3 + N] - want).max() <= 1e-5 * np.abs(want).max()   # (three f32 roundings and the exponential's)
+    for other in (ya, ys):
+        assert np.array_equal(np.delete(other, np.s_[3:3 + N], axis=1), np.delete(c0, np.s_[3:3 + N], axis=1))
     aq, asc, _ = quantize_padded(x, Mp)
     assert rel_err_rows(y[:T, 3:3 + N], orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
     assert not y[T:, 3:3 + N].any()
