@@ -309,6 +309,7 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (LEAN) {
     if constexpr (TS < 16) {
+      static_assert((MM_LDS_MAX - MM_WAVES * LL::WSZ) / LL::TOK * 16 <= 512, "a piece of the row of zeros a thread, of the longest rows that LDS holds");
       if (tid < cpr) *(mm_u4*)(A + 8 * Ks + tid * 16) = mm_u4{0, 0, 0, 0};
       if constexpr (TT::MIN)
         for (int i = tid; i < nb * 2; i += 512) *(v4f*)(U + (i >> 1) * 16 + 8 + (i & 1) * 4) = v4f{0.0f, 0.0f, 0.0f, 0.0f};

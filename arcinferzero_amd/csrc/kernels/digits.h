@@ -250,7 +250,7 @@ template <class I, class DMA> __device__ __forceinline__ void d_prologue(DMA& dm
   }
 }
 template <int NW, int MN, class I, class DMA>
-__device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int blocks, v16f (&res)[2][2]) {
+__device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int blocks, v16f (&res)[2][2]) {
   constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, KB = STAGE / 1024, ND = (KB + 3) / 4;
   static_assert(ND <= (NB == 2 ? 8 : 6), "the slots below carry that many pieces");
   const int lane = threadIdx.x & 63, g = lane >> 5, steps = blocks / NB;
@@ -410,7 +410,7 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int wave, int b
 // The same for 32 tokens: an expert's tile of at most 32 slots.  Both row tiles of a block one after the other, the next block's
 // operands read before the products.
 template <int NW, int MN, class I, class DMA>
-__device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int wave, int blocks, v16f (&res)[2]) {
+__device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int blocks, v16f (&res)[2]) {
   constexpr int NB = I::NB, R = I::R, STAGE = I::STAGE, KB = STAGE / 1024, ND = (KB + 3) / 4;
   const int g = (threadIdx.x & 63) >> 5, steps = blocks / NB;
   struct F6 { u4v lo; u2v hi; };

@@ -154,7 +154,7 @@ __device__ __forceinline__ void gemm_d_body(uint8_t* lds_base, const uint8_t* __
                    TS + (wn * 64u + l32) * 16u, TS + 2048u + (wn * 64u + l32) * 8u, TS + I::WWS + (wn * 64u + lane) * 4u,
                    TS + I::WV + g * I::W + (wn * 64u + l32) * 8u};
   v16f res[2][2];
-  d_loop<NW, MN, I>(o, dma, wave, b1 - b0, res);
+  d_loop<NW, MN, I>(o, dma, b1 - b0, res);
 
   // ---- epilogue: lane = weight row n, accumulator i = token row 8 * (i / 4) + 4 * g + i % 4
 #pragma unroll
@@ -264,11 +264,11 @@ __device__ __forceinline__ void gemm_d64_body(uint8_t* lds_base, const uint8_t* 
                    row + D::WWS + (r + lane) * 4u, row + D::WV + g * I::W + (r + l32) * 8u};
   v16f res[2][2];
   if (valid - m0 <= 32) {
-    d_loop32<NW, MN, I>(o, dma, wave, b1 - b0, res[0]);
+    d_loop32<NW, MN, I>(o, dma, b1 - b0, res[0]);
 #pragma unroll
     for (int i = 0; i < 16; ++i) res[1][0][i] = res[1][1][i] = 0.0f;
   } else {
-    d_loop<NW, MN, I>(o, dma, wave, b1 - b0, res);
+    d_loop<NW, MN, I>(o, dma, b1 - b0, res);
   }
 #pragma unroll
   for (int ms = 0; ms < 2; ++ms)

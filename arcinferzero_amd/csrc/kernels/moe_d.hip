@@ -96,8 +96,8 @@ __device__ __forceinline__ bool tile_d_sums(uint8_t* lds_base, const uint8_t* __
                    TS + (wave * 64u + l32) * 16u, TS + 4096u + (wave * 64u + l32) * 8u, TS + I::WWS + (wave * 64u + lane) * 4u,
                    TS + I::WV + g * I::W + (wave * 64u + l32) * 8u};
   const bool few = rows_valid <= 32;
-  if (few) d_loop32<NW, MN, I>(o, dma, wave, nblk, res[0]);
-  else d_loop<NW, MN, I>(o, dma, wave, nblk, res);
+  if (few) d_loop32<NW, MN, I>(o, dma, nblk, res[0]);
+  else d_loop<NW, MN, I>(o, dma, nblk, res);
   __syncthreads();  // (the stages are the epilogue's)
   return few;
 }
