@@ -971,13 +971,16 @@ class Engine {
   DigitPlan digit_plan(const DigitForm& f, int Mp, int N, int nsb, bool kept, int rows) const {
     const int cus = arcz_device_cus(), slots = 2 * cus, most = (int)std::min<size_t>(slots, SPLIT_BYTES / 65536);
     const double k1024 = f.mn ? 17.2 : f.nw == 1 ? 14.6 : f.nw == 2 ? 19.8 : 26.4, ends = f.mn ? 2.7 : f.nw == 1 ? 0.5 : f.nw == 2 ? 4.9 : 3.2;
-    const double one = rows <= 32 ? 0.77 : f.nw == 3 ? 0.68 : 0.63, two = f.nw < 3 ? 0.89 : 0.81;
+    // (two digits, at most 32 tokens, a loop of their own: 1440 launches of 160 products, pieces 0.1 % over the best of them, 2.3 % at
+    //  most; with the others' figures, fitted before its waits were mended, 0.7 and 15 %)
+    const bool few2 = rows <= 32 && f.nw == 2;
+    const double one = few2 ? 0.72 : rows <= 32 ? 0.77 : f.nw == 3 ? 0.68 : 0.63, two = few2 ? 0.95 : f.nw < 3 ? 0.89 : 0.81;
     // (tiles of 64 tokens: fewer stages in flight with two and three digits; at most 32 tokens: half the products)
     const double k64 = (f.mn ? 1.02 : f.nw == 1 ? 1.05 : f.nw == 2 ? 1.07 : 1.12) * (rows <= 32 && f.nw < 3 ? 0.7 : 1.0);
     const double e64 = ends + (f.mn ? 0.7 : f.nw == 1 ? 0.15 : f.nw == 2 ? 1.8 : 1.9);
     int th = 128;
     auto tile = [&](int p) { return (th == 128 ? k1024 : k64 * k1024) * ((nsb + p - 1) / p) / 4 + (th == 128 ? ends : e64); };
-    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? one + 0.05 * wgs / cus : two + (1.0 - two) * (wgs - cus) / cus; };
+    auto part = [&](int wgs) { return wgs == 0 ? 0.0 : wgs <= cus ? one + (few2 ? 0.0 : 0.05) * wgs / cus : two + (1.0 - two) * (wgs - cus) / cus; };
     auto last = [&](int full, int wgs, int p) {
       if (!full || !wgs) return part(wgs);
       return p == 1 ? std::max(0.54, 0.36 + 0.84 * wgs / slots) : 0.19 + 1.08 * wgs / slots;
@@ -1000,7 +1003,7 @@ class Engine {
       }
     }
     // (the tokens' digits and the launches; the rows' digits from memory)
-    best.us += (f.mn ? 4.9 : f.nw == 1 ? 6.0 : f.nw == 2 ? 2.8 : 1.9) + Mp * (nsb * 256) / 1.7e6 +
+    best.us += (f.mn ? 4.9 : f.nw == 1 ? 6.0 : few2 ? 1.3 : f.nw == 2 ? 2.8 : 1.9) + Mp * (nsb * 256) / 1.7e6 +
                (double)((N + 127) / 128) * nsb * 8 * f.wimg / (f.nw == 3 ? 18.0e6 : 40.0e6) + rows * (double)N * 4 / 9.0e6;
     return best;
   }

@@ -220,9 +220,10 @@ __device__ inline void row_decode(const uint8_t* __restrict__ raw, const uint32_
 struct DAddr { uint32_t A16, A8, SA, U, W16, W8, WS, V; };
 // Waits for a wave's pieces of stages of KB KiB but those of the last `later` steps: KB / 4 a step.  (The first waves have one more
 // where KB / 4 is not whole, and wait for as many of the last step's too: a branch on the wave costs more, 64-token tiles of
-// Q4_K, 300 tokens x 17408 rows, 111 -> 118 us.)
-template <int KB, int later> __device__ __forceinline__ void d_wait_but() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(later * (KB / 4)) : "memory");
+// Q4_K, 300 tokens x 17408 rows, 111 -> 118 us.  EXACT: by the wave, where the last step's pieces were asked for just before.)
+template <int KB, int later, bool EXACT> __device__ __forceinline__ void d_wait_but(int wave) {
+  if (EXACT && later && KB % 4 && wave < KB % 4) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(later * (KB / 4 + 1)) : "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(later * (KB / 4)) : "memory");
 }
 // The work-group's waves meet; nothing but the wait before it is waited for
 __device__ __forceinline__ void d_meet() {
@@ -237,7 +238,7 @@ template <class I, class DMA> __device__ __forceinline__ void d_prologue(DMA& dm
 #pragma unroll
   for (int q = 0; q < I::AHEAD; ++q) {
     if (q == FIRST) {  // (a stage each is on its way; the last is asked for when the first is there)
-      d_wait_but<KB, FIRST - 1>();
+      d_wait_but<KB, FIRST - 1, false>(0);
       d_meet();
     }
     dma.at(min(q, steps - 1));
@@ -351,7 +352,7 @@ __device__ __forceinline__ void d_loop(const DAddr& o, DMA& dma, int blocks, v16
       // -- the step's meeting: what the waves brought for the next step lies in LDS, the step before is read
       if (NB == 2 ? p == 6 : q == 2) {
         __builtin_amdgcn_sched_barrier(0);
-        d_wait_but<KB, I::AHEAD - 2>();
+        d_wait_but<KB, I::AHEAD - 2, (I::AHEAD < R)>(dma.wave);
         d_meet();
         __builtin_amdgcn_sched_barrier(0);
         dma.at(min(step + I::AHEAD, steps - 1));
@@ -465,8 +466,8 @@ __device__ __forceinline__ void d_loop32(const DAddr& o, DMA& dma, int blocks, v
         }
       if (NB == 1 || k == 1) {  // (the step's meeting, as in d_loop)
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the step's last operands: its stage is refilled)
-        d_wait_but<KB, I::AHEAD - 2>();
+        if (I::AHEAD == R) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the step's last operands: its stage is refilled)
+        d_wait_but<KB, I::AHEAD - 2, (I::AHEAD < R)>(dma.wave);
         d_meet();
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t stf = I::AHEAD == R ? st : st == 0 ? (R - 1) * STAGE : st - STAGE;
