@@ -912,19 +912,19 @@ class Engine {
       if (type == GGML_Q3_K || type == GGML_IQ3_S || type == GGML_Q4_0 || type == GGML_MXFP4) return true;
       // (IQ3_XXS of few values, or of few rows, whose digits go in 16 pieces of K: not -- 9000 x 1024, 40 tokens 21 / 20, 896 x 12032, 506
       //  tokens 50 / 47, 640 x 14336, 700 59 / 54, but 2500 103 / 110)
-      if (type == GGML_IQ3_XXS ? Mp <= 128 && (double)N * K >= (1 << 24) : type == GGML_Q5_K && Mp >= 256) return true;
+      if (type == GGML_IQ3_XXS ? Mp <= 128 && (double)N * K >= (1 << 24) : type == GGML_Q5_K && Mp >= 256 && (double)N * K >= (1 << 23)) return true;
       if (type == GGML_IQ3_XXS && N <= 1024 && Mp <= 1024) return false;
-      // (the others where they are priced cheaper by more than the prices' own error)
+      // (the others where they are priced cheaper by more than the prices' own error: of 2000 products, half of them below 2^23 values,
+      //  0.2 % over the better of both on average, 13 % at most)
       const double d = digit_plan(digit_form(type), Mp, N, K / 256, true, rows).us;
       double i8 = 0.0;
       if (type == GGML_Q6_K || type == GGML_IQ3_XXS)
         split_pieces(type, type == GGML_IQ3_XXS ? 1 : 0, Mp, (rows + 63) / 64, N, K / 256, &i8);  // (tiles of padding are left out)
       else i8 = i8_price(type, Mp, rows, N, K / 256);
       if (type == GGML_IQ3_XXS) i8 += 1.5 + (double)N * K / 7.5e6;  // (about half of what writing it out as Q6_K takes)
-      const double less = type == GGML_IQ3_XXS || type == GGML_Q6_K ? 1.0 : type == GGML_Q4_K ? (K <= 1024 ? 0.9 : 0.94) : type == GGML_Q5_K ? 0.95 : 0.93;
-      // (... and matrices below 2^23 values by 8 % more: Q4_K 1856 x 3584, 251 tokens 25.5 / 23.1, IQ4_NL 1712 x 1536 18.0 / 16.6)
-      const double small = (double)N * K < (1 << 23) && type != GGML_Q6_K && type != GGML_IQ3_XXS ? 0.08 : 0.0;
-      return d < (less - small) * i8;  // (Q4_K 9000 x 1024, 1500 tokens: 65 / 60 us)
+      const double less = type == GGML_IQ3_XXS || type == GGML_Q6_K ? 1.0 : type == GGML_Q4_K && K <= 1024 ? 0.9
+                          : (type == GGML_Q4_K || type == GGML_Q5_K) && (double)N * K < (1 << 23) ? 0.92 : 0.95;  // (their digits' price is 9 % short there)
+      return d < less * i8;  // (Q4_K 9000 x 1024, 1500 tokens: 65 / 60 us)
     }
     if (Mp < 256) return false;
     switch (type) {
@@ -946,13 +946,15 @@ class Engine {
   // us of a product of Q4_K, Q5_K, IQ4_XS or IQ4_NL on the int8 kernels as gemm_dense launches them: pieces of K, 128 x 128 tiles
   // (two work-groups a compute unit) or, Q4_K, 64 x 128 (three).  Fitted to eight matrices x 80 - 1500 tokens, 4 - 6 % off;
   // Q4_K of a last round of 64 x 128 tiles from 1170 products with three engines in turn (17408 x 5120, 300 tokens: 113 us, priced 117).
+  // Pieces by their whole superblocks: 486 products of 2^21 values and more, 4.5 % off; by their average, as before, 9 %, and
+  // too high by up to a fifth where the pieces are even (IQ4_XS 816 x 3072, 241 tokens: 18.8 us, priced 21.6 and now 18.4).
   static double i8_price(uint32_t type, int Mp, int rows, int N, int nsb) {
-    struct P { double base, pieces, round, ends, one, sums, out; };
-    const P p = type == GGML_Q4_K ? P{9.0, 11.6, 26.0, 2.1, 0.62, 13.3e6, 14.6e6}
-                : type == GGML_Q5_K ? P{7.2, 11.7, 26.7, 3.1, 0.61, 11.3e6, 10.1e6} : P{7.2, 9.8, 26.1, 2.9, 0.69, 13.4e6, 12.6e6};
+    struct P { double base, round, ends, one, out, pieces, superblock, half, sums; };
+    const P p = type == GGML_Q4_K ? P{9.0, 26.0, 2.1, 0.62, 14.6e6, 7.6, 7.26, 0.64, 7.9e6}
+                : type == GGML_Q5_K ? P{7.2, 26.7, 3.1, 0.61, 10.1e6, 7.5, 8.01, 0.64, 6.9e6} : P{7.2, 26.1, 2.9, 0.69, 12.6e6, 7.6, 6.92, 0.69, 6.5e6};
     const int cus = arcz_device_cus(), nt = (N + 127) / 128, t = (Mp + 127) / 128 * nt, ny = std::min({8, sk_most(type, nsb, t, Mp), 2 * cus / t});
     const double out = rows * (double)N * 4 / p.out;
-    if (ny >= 3) return p.pieces + (t * ny <= cus ? p.one : 1.0) * (p.round * nsb / 4 / ny + p.ends) + 2.0 * ny * Mp * N * 4 / p.sums + out;
+    if (ny >= 3) return p.pieces + (t * ny <= cus ? p.half : 1.0) * p.superblock * ((nsb + ny - 1) / ny) + 2.0 * ny * Mp * N * 4 / p.sums + out;
     const int full = t / (2 * cus), rest = t % (2 * cus), t64 = (rows + 63) / 64 * nt, f64 = t64 / (3 * cus), r64 = t64 % (3 * cus);
     const double c128 = full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : 1.0), c64 = 0.8 * f64 + (r64 == 0 ? 0.0 : r64 <= cus ? 0.30 : r64 <= 2 * cus ? 0.48 : 0.8);
     if (type == GGML_Q4_K && c64 < 0.97 * c128)  // (gemm_dense's choice)

@@ -434,6 +434,24 @@ def test_smallest_matrices_that_keep_digits(rt, qtype, N, K, digits):
     assert rel_err_rows(y[:T], orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
 
 
+@pytest.mark.parametrize("qtype,T,Mp,N,K", [(az.IQ4_XS, 241, 256, 816, 3072), (az.IQ4_NL, 65, 80, 1504, 2048), (az.Q5_K, 418, 512, 1888, 2048),
+                                            (az.IQ4_XS, 56, 64, 1408, 1536)])
+def test_kept_digits_left_for_even_pieces_of_k(rt, qtype, T, Mp, N, K):
+    """Small matrices whose K goes in even pieces on the int8 kernels, which are then ahead of the kept digits: which kernels
+    ran, and the oracle."""
+    print(f"even pieces {TYPE_NAMES[qtype]} T={T} N={N} K={K}", flush=True)
+    W = make_weights(qtype, N, K, seed=97)
+    x = make_acts(T, K, seed=98, outliers=True)
+    eng = az.Engine(Mp, K)
+    eng.profile(True)
+    y = run_gemm(eng, qtype, W, N, K, x, Mp)
+    eng.profile_collect()
+    assert eng.profile_get("keep_digits")[1] == 1 and eng.profile_get("act_digits")[1] == 0 and eng.profile_get("test")[1] == 2
+    eng.close()
+    aq, asc, _ = quantize_padded(x, Mp)
+    assert rel_err_rows(y[:T], orc.matmul_ref(qtype, W, N, K, aq[:T], asc)).max() <= TOL
+
+
 @pytest.mark.parametrize("env,digits,products", [({}, 1, None), ({"ARCZ_GEMM_DIGITS": "1", "ARCZ_Q4_SPLITK": "2"}, 1, 2), ({"ARCZ_GEMM_DIGITS": "0"}, 0, None), ({"ARCZ_Q4_SPLITK": "0"}, 1, 1),
                                                  ({"ARCZ_Q4_SPLITK": "2"}, 1, 2),
                                                  ({"ARCZ_GEMM_SPLIT": "3", "ARCZ_Q4_SPLITK": "0"}, 0, 4)])
