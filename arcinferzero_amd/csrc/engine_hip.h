@@ -1104,13 +1104,14 @@ class Engine {
   }
   // Q8_0 in tiles of eight waves (gemm8w_body), one work-group a compute unit: the pieces of K (1: none) with the lowest price in us,
   // or 0 where the other kernel's is no higher.  A round takes 3 us and 1.4 for each superblock of a piece, the bytes of the weight
-  // 4.6 TB/s; the other kernel's own price is up to a sixth too low, 3.75 us for its launch left out.  Of eight matrices (1024 x 4096 -
+  // 4.6 TB/s; the other kernel's own price is up to a sixth too low, 3.75 us for its launch left out
+  // (0.2 less here: of 540 products none that is taken is then more than 3 % slower).  Of eight matrices (1024 x 4096 -
   // 17408 x 5120) x 20 - 2048 tokens 36 of 96 are taken and none got slower, on average 10 %, by up to 19 % faster: 4096 x 4096, 512 tokens 35.3 -> 28.8
   // us, 2048 x 2048, 700 21.4 -> 17.3, 5120 x 17408, 300 119 -> 98, 4096 x 12288, 512 86 -> 72.
   static int q8_wide_pieces(int Mp, int m64, int N, int nsb, bool one, double other) {
     const size_t cus = (size_t)arcz_device_cus(), tiles = (size_t)m64 * ((N + 127) / 128);
     int best = 0;
-    double least = 0.86 * other + 3.75;
+    double least = 0.86 * other + 3.55;
     for (int ny = 1; ny <= 8 && (ny == 1 || (ny <= nsb / 2 && !one)); ++ny) {
       if (ny > 1 && (size_t)ny * Mp * N * 4 > SPLIT_BYTES) break;
       const double rounds = (double)((tiles * ny + cus - 1) / cus) * (3.0 + 1.4 * ((nsb + ny - 1) / ny));
@@ -1210,7 +1211,8 @@ class Engine {
     if (w.type == GGML_Q8_0 && q8_bm != 128 && gemm_split_ <= 0 && q8_wide_ != 0) {
       double other = 0.0;
       split_pieces(w.type, 0, Mp, m64, N, K / 256, &other);
-      q8w = q8_wide_pieces(Mp, m64, N, K / 256, sk_force_ == 0, q8_wide_ > 0 ? 1e9 : other);
+      // (two superblocks: never, the price is 0.6 us short there; 16000 x 512, 91 tokens 9.1 us, with these 10.1, 3712 x 512, 508 9.2 / 9.9)
+      q8w = q8_wide_pieces(Mp, m64, N, K / 256, sk_force_ == 0, q8_wide_ > 0 ? 1e9 : K < 768 ? 0.0 : other);
       if (sk_force_ >= 2) q8w = q8_wide_ > 0 ? std::min(sk_force_, K / 256) : 0;
     }
     if (sk_force_ != 0 && q8w != 1) {
