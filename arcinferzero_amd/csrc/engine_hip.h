@@ -727,14 +727,23 @@ class Engine {
       // one token too).  Where LDS does not hold their sums beside the tokens, 256 (us with the kernels beyond LDS / so: Q8_0 4096 x
       // 12800, four tokens 20.3 / 18.0, a block of 12800 with two-pass inputs of two tokens 53.5 / 45.1; one token's, Q4_0 4096 x 25856
       // 55.9 / 48.6; two tokens, Q6_K 4096 x 25856 40.9 / 26.2)
+      // Of so few rows that 256 threads' work-groups are no more than the compute units: 256 too, or half of those have nothing to do
+      // (470 products: 0.88 of the time with 512 on average, of more rows 1.08; IQ4_XS 128 x 12800, one token of two-pass inputs, 5.5 / 4.3
+      // us); and the table types' two-pass inputs of more rows than one round of 512 threads takes, whose 256 threads go two to a
+      // unit (MXFP4 1152 x 16896 8.9 / 7.5, IQ4_NL 5360 x 12800 14.6 / 13.6)
+      const bool codebook = w.type == GGML_IQ4_XS || w.type == GGML_IQ3_S || w.type == GGML_IQ4_NL || w.type == GGML_MXFP4 ||
+                            w.type == GGML_IQ3_XXS;
       static const int bt_env = getenv("ARCZ_GEMV_BT") ? atoi(getenv("ARCZ_GEMV_BT")) : 0;
       const int wpr = lpr > 64 ? lpr / 64 : 1;
       // (IQ3_S: 2 KiB of the work-group's LDS hold the codebook)
       const size_t lds_max = w.type == GGML_IQ3_S || w.type == GGML_IQ3_XXS ? 65536 - 2048 : 65536;
       auto lds_at = [&](int slots, int bt) { return (size_t)slots * tokb(slots) + (wpr > 1 ? (size_t)16 * (bt / lpr) * wpr * slots * 4 : 0); };  // (16: the kernels' GEMV_FLUSH)
       auto bt_of = [&](int slots) {
-        return lpr >= 128 && bt_env != 256 && (slots == 2 || (slots == 1 && bt_env == 512) || (slots == 4 && w.type == GGML_Q8_0)) &&
-               lds_at(slots, 512) <= lds_max ? 512 : 256;
+        const bool two = slots == 2 || (slots == 4 && w.type == GGML_Q8_0);
+        if (lpr < 128 || bt_env == 256 || !(two || (slots == 1 && bt_env == 512)) || lds_at(slots, 512) > lds_max) return 256;
+        if (bt_env == 512) return 512;
+        const int cus = arcz_device_cus();
+        return N <= cus * (256 / lpr) || (codebook && q2_fuse_ && N > cus * (512 / lpr)) ? 256 : 512;
       };
       // the kernel's token slots: T rounded up, or -- both halves of two-pass inputs in one launch -- 2 T rounded up
       auto lds_of = [&](int slots) { return lds_at(slots, bt_of(slots)); };
@@ -764,8 +773,6 @@ class Engine {
         // 17408 x 5120: 20.2 against 25.7 with one; three or four per unit are slower everywhere).
         static const int wpc_env = getenv("ARCZ_GEMV_WPC") ? atoi(getenv("ARCZ_GEMV_WPC")) : 0;
         static const int wgs_env = getenv("ARCZ_GEMV_WGS") ? atoi(getenv("ARCZ_GEMV_WGS")) : 0;
-        const bool codebook = w.type == GGML_IQ4_XS || w.type == GGML_IQ3_S || w.type == GGML_IQ4_NL || w.type == GGML_MXFP4 ||
-                              w.type == GGML_IQ3_XXS;
         // (Q6_K, one token, since its kernel takes the - 32 off the sums: two work-groups a unit are ahead on matrices
         //  of layer size -- 17408 x 5120 16.4 -> 15.9 us, 5120 x 17408 16.3 -> 15.9, 8192 x 8192 12.8 -> 12.3 -- and
         //  behind on the 151936 x 5120 output head, 106.3 -> 110.3)

@@ -134,6 +134,25 @@ def test_gemv_two_pass_long_rows(rt, qtype, T, N, K):
         assert rel_err_rows(ys[0], ys[1]).max() <= TIGHT
 
 
+@pytest.mark.parametrize("qtype,T,K,lanes,two_pass", [(az.Q8_0, 2, 17408, 256, False), (az.Q8_0, 4, 8192, 128, False), (az.Q4_K, 2, 17408, 128, False),
+                                                      (az.Q8_0, 2, 12288, 128, True), (az.Q6_K, 1, 17408, 128, True), (az.IQ3_S, 1, 13312, 128, True)])
+def test_gemv_512_threads_from_their_first_rows(rt, qtype, T, K, lanes, two_pass):
+    """Work-groups of 512 threads are for more rows than 256 threads' work-groups on every compute unit take: the last number of
+    rows below and the first above, whose rows have the same bits (a row's lanes add it up in the same order), against the oracle."""
+    N = az.lib.arcz_device_cus() * (256 // lanes)
+    print(f"gemv 512 threads {TYPE_NAMES[qtype]} N={N} K={K} T={T} two_pass={two_pass}", flush=True)
+    W = make_weights(qtype, N + 3, K, seed=19)
+    x = make_acts(T, K, seed=20, outliers=True)
+    e = az.Engine(16, K)
+    e.two_pass(two_pass)
+    ys = [run_gemv(e, qtype, W[:len(W) // (N + 3) * n], n, K, x, 16) for n in (N, N + 3)]
+    e.close()
+    assert np.isfinite(ys[1]).all() and np.array_equal(ys[0].view(np.uint32), np.ascontiguousarray(ys[1][:, :N]).view(np.uint32))
+    if not two_pass:
+        aq, asc, _ = quantize_padded(x, 16)
+        assert rel_err_rows(ys[1], orc.matmul_ref(qtype, W, N + 3, K, aq[:T], asc)).max() <= TOL
+
+
 @pytest.mark.parametrize("qtype,T,N,K,two_pass", [(az.Q8_0, 3, 67, 12800, False), (az.Q8_0, 4, 2050, 12800, False), (az.Q8_0, 2, 259, 12800, True),
                                                   (az.Q4_0, 1, 67, 25856, True), (az.Q6_K, 1, 33, 25856, True), (az.IQ3_S, 1, 35, 25088, True),
                                                   (az.IQ4_XS, 2, 67, 25856, False)])
