@@ -253,14 +253,16 @@ __device__ inline void mm_slice(uint8_t* lds, const uint32_t* grid, const SRC& s
   int vu[NSC];
   if constexpr (LEAN) {
     const int t2 = src.tok(min(ts, T - 1));
-    for (int k16 = 64 * NCH + lane; k16 < cpr; k16 += 64)
-      for (int t = wave; t < T; t += 8)
-        *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = *(const mm_u4*)(aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256 + k16 * 16);
-    for (int i = tid + 512 * NSC; i < nb << TL; i += 512) {  // (512 is whole tokens: ts is this pair's too)
-      const int b = i >> TL, at = s_begin * 8 + b;
-      const float sa = ts < T ? asc[(size_t)at * M + t2] : 0.0f;
-      SA[b * 16 + ts] = sa;
-      if constexpr (TT::MIN) U[b * 16 + ts] = sa * (float)((int)absum[(size_t)(2 * at) * M + t2] + (int)absum[(size_t)(2 * at + 1) * M + t2]);
+    if (__builtin_expect(cpr > 64 * NCH || nb << TL > 512 * NSC, 0)) {  // (out of the other tiles' way)
+      for (int k16 = 64 * NCH + lane; k16 < cpr; k16 += 64)
+        for (int t = wave; t < T; t += 8)
+          *(mm_u4*)(A + t * Ks + ((k16 ^ t) << 4)) = *(const mm_u4*)(aq + (size_t)src.tok(t) * K + (size_t)s_begin * 256 + k16 * 16);
+      for (int i = tid + 512 * NSC; i < nb << TL; i += 512) {  // (512 is whole tokens: ts is this pair's too)
+        const int b = i >> TL, at = s_begin * 8 + b;
+        const float sa = ts < T ? asc[(size_t)at * M + t2] : 0.0f;
+        SA[b * 16 + ts] = sa;
+        if constexpr (TT::MIN) U[b * 16 + ts] = sa * (float)((int)absum[(size_t)(2 * at) * M + t2] + (int)absum[(size_t)(2 * at + 1) * M + t2]);
+      }
     }
 #pragma unroll
     for (int r2 = 0; r2 < (TS < 16 ? 1 : 2); ++r2) {
