@@ -921,8 +921,8 @@ class Engine {
       //  tokens 50 / 47, 640 x 14336, 700 59 / 54, but 2500 103 / 110)
       if (type == GGML_IQ3_XXS ? Mp <= 128 && (double)N * K >= (1 << 24) : type == GGML_Q5_K && Mp >= 256 && (double)N * K >= (1 << 23)) return true;
       if (type == GGML_IQ3_XXS && N <= 1024 && Mp <= 1024) return false;
-      // (the others where they are priced cheaper by more than the prices' own error: of 2000 products, half of them below 2^23 values,
-      //  0.2 % over the better of both on average, 13 % at most)
+      // (the others where they are priced cheaper by more than the prices' own error: of 1225 products, half of them below 2^23 values,
+      //  0.2 % over the better of both on average, 14 % at most)
       const double d = digit_plan(digit_form(type), Mp, N, K / 256, true, rows).us;
       double i8 = 0.0;
       if (type == GGML_Q6_K || type == GGML_IQ3_XXS)
@@ -1166,7 +1166,7 @@ class Engine {
   void digits_keep(GpuWeight& w) {
     const int tiles = (w.N + 255) / 256 * 2;  // (whole pairs, for tiles of 256 rows)
     const size_t bytes = (size_t)tiles * (w.K / 32) * digit_form(w.type).wimg;
-    const int least = w.K < 1024 || (w.type == GGML_Q3_K && w.K == 1024) ? 23 : w.type == GGML_Q4_K || w.type == GGML_IQ3_S ? 22 : 21;
+    const int least = w.K < (w.type == GGML_Q3_K ? 1280 : 1024) ? 23 : w.type == GGML_Q4_K || w.type == GGML_IQ3_S ? 22 : 21;
     if (!digits_keep_ || (size_t)w.N * w.K < ((size_t)1 << least) || !digits_fit(bytes)) return;
     digits_tokens();
     if (!xd_ || !(w.digits = try_buf(bytes))) return;
